@@ -139,6 +139,7 @@ SIGNATURES = {
     "ft_model_read_param": [_P, _SZ, _P],
     "ft_model_write_param": [_P, _SZ, _P],
     "ft_model_read_grad": [_P, _SZ, _P],
+    "ft_model_read_grads": [_P, _P],
     "ft_model_forward_logits": [_P, _P, _SZ, _SZ, _P],
     "ft_model_eval_chunk": [_P, _P, _P, _P, _SZ, _SZ, _P, _P],
     "ft_trainer_create": [_P, C.POINTER(TrainerConfigC), C.POINTER(_P)],

@@ -923,6 +923,13 @@ struct StepControl {
     int apply;       // 0 when the norm is not finite: the update is skipped
 };
 
+// Pieces of many small tensors into one array (w <- g), which may be pinned host memory: 512 gradients of an adapter set
+// one copy and wait each took 4.5 ms of a 20 ms step, this and one wait 0.2 ms.
+__global__ __launch_bounds__(256) void multi_copy_kernel(const ft_segment* __restrict__ segs) {
+    const ft_segment s = segs[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < s.n; i += 256) s.w[i] = s.g[i];
+}
+
 __global__ __launch_bounds__(256) void multi_sum_squares_kernel(const ft_segment* __restrict__ segs,
                                                                 float* __restrict__ partials) {
     __shared__ float red[4];
@@ -1170,6 +1177,13 @@ int ft_internal_multi_grad_norm(ft_context* ctx, const ft_segment* segs_dev, siz
     FT_LAUNCH_CHECK();
     hipLaunchKernelGGL(grad_norm_finish_kernel, dim3(1), dim3(256), 0, ctx->stream, partials_dev, nseg, max_norm,
                        control_dev);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}
+
+int ft_internal_multi_copy(ft_context* ctx, const ft_segment* segs_dev, size_t nseg) {
+    if (nseg == 0) return FT_OK;
+    hipLaunchKernelGGL(multi_copy_kernel, dim3((unsigned)nseg), dim3(256), 0, ctx->stream, segs_dev);
     FT_LAUNCH_CHECK();
     return FT_OK;
 }

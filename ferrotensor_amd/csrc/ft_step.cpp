@@ -56,6 +56,7 @@ int ft_internal_attention_backward_rope(ft_context* ctx, const float* q, const f
                                         const float* out, const float* d_out, float* dq, float* dk, float* dv,
                                         float* stats, size_t B, size_t S, size_t H, size_t Hkv,
                                         const ft_attention_options* opts, const float* rope_table);
+int ft_internal_multi_copy(ft_context* ctx, const ft_segment* segs_dev, size_t nseg);
 int ft_internal_multi_adamw(ft_context* ctx, const ft_segment* segs_dev, size_t nseg, const ft_adam_params* p,
                             float grad_scale, const float* control_dev);
 
@@ -119,6 +120,11 @@ struct ft_model {
     LinearW lm_head;
     std::vector<ParamRef> params;
     bool params_dirty = true;
+    // ft_model_read_grads: the gradients' pieces and the pinned array they are gathered into, made at its first call
+    // and given back when the set of trainable tensors changes.
+    ft_segment* grad_segs = nullptr;
+    size_t grad_nseg = 0;
+    float* grad_host = nullptr;
     // Bumped whenever an adapter's buffers are (re)allocated: a trainer holds raw pointers into
     // them and sizes its moments from them, so it is only valid for the generation it was made in.
     uint64_t param_generation = 0;
@@ -292,10 +298,22 @@ int ensure_workspace(ft_model* m, size_t B, size_t S) {
     return FT_OK;
 }
 
+void free_grad_gather(ft_model* m) {
+    if (m->grad_segs) (void)ft_free(m->ctx, m->grad_segs);
+    if (m->grad_host) {
+        (void)hipStreamSynchronize(m->ctx->stream);
+        (void)hipHostFree(m->grad_host);
+    }
+    m->grad_segs = nullptr;
+    m->grad_host = nullptr;
+    m->grad_nseg = 0;
+}
+
 // The trainable tensors in reporting order. With a trainable base (model_builder.rs:353-357) the
 // linear weights and the norm scales are in it too, and their gradient buffers are made here.
 int rebuild_params(ft_model* m) {
     m->params.clear();
+    free_grad_gather(m);
     const bool base = m->cfg.trainable_base != 0;
     const size_t H = m->cfg.hidden_size;
     auto grad_buf = [&](float** g, size_t n) -> int {
@@ -931,6 +949,7 @@ int ft_model_create(ft_context* ctx, const ft_model_config* cfg, ft_model** out)
 int ft_model_destroy(ft_model* m) {
     if (!m) return FT_OK;
     ws_free(m);
+    free_grad_gather(m);
     ft_context* ctx = m->ctx;
     auto rel = [&](void* p) {
         if (p) (void)ft_free(ctx, p);
@@ -1142,6 +1161,52 @@ int ft_model_write_param(ft_model* m, size_t index, const float* host) {
 int ft_model_read_grad(ft_model* m, size_t index, float* out_host) {
     FT_CHECK_ARG(m && out_host && !m->params_dirty && index < m->params.size(), "ft_model_read_grad: bad argument");
     return ft_download(m->ctx, out_host, m->params[index].g, m->params[index].n * sizeof(float));
+}
+
+int ft_model_read_grads(ft_model* m, float* out_host) {
+    return guarded([&]() -> int {
+        FT_CHECK_ARG(m && out_host && !m->params_dirty, "ft_model_read_grads: bad argument");
+        size_t total = 0;
+        for (const auto& p : m->params) total += p.n;
+        if (total == 0) return FT_OK;
+        ft_context* ctx = m->ctx;
+        FT_HIP(hipSetDevice(ctx->device));
+        // Many small tensors (adapters) are gathered by one kernel into pinned memory; a trainable base is few large
+        // ones, which the pinned array would only copy twice.
+        if (total > (size_t)16 << 20) {
+            for (const auto& p : m->params) {
+                FT_TRY(ft_download(ctx, out_host, p.g, p.n * sizeof(float)));
+                out_host += p.n;
+            }
+            return FT_OK;
+        }
+        if (!m->grad_segs) {
+            FT_HIP(hipHostMalloc((void**)&m->grad_host, total * sizeof(float), hipHostMallocDefault));
+            std::vector<ft_segment> segs;
+            float* dst = m->grad_host;
+            for (const auto& p : m->params) {
+                for (size_t off = 0; off < p.n; off += FT_SUM_SQUARES_CHUNK) {
+                    const size_t n = std::min<size_t>(p.n - off, FT_SUM_SQUARES_CHUNK);
+                    segs.push_back(ft_segment{dst + off, p.g + off, nullptr, nullptr, (uint32_t)n});
+                }
+                dst += p.n;
+            }
+            ft_segment* dev = nullptr;
+            int rc = ft_alloc(ctx, segs.size() * sizeof(ft_segment), (void**)&dev);
+            if (rc == FT_OK) rc = ft_upload(ctx, dev, segs.data(), segs.size() * sizeof(ft_segment));
+            if (rc != FT_OK) {
+                if (dev) (void)ft_free(ctx, dev);
+                free_grad_gather(m);
+                return rc;
+            }
+            m->grad_segs = dev;
+            m->grad_nseg = segs.size();
+        }
+        FT_TRY(ft_internal_multi_copy(ctx, m->grad_segs, m->grad_nseg));
+        FT_HIP(hipStreamSynchronize(ctx->stream));
+        std::memcpy(out_host, m->grad_host, total * sizeof(float));
+        return FT_OK;
+    });
 }
 
 int ft_model_forward_logits(ft_model* m, const uint32_t* rows, size_t B, size_t S, float* logits_host) {

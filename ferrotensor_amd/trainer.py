@@ -155,7 +155,15 @@ class Lfm2Model:
         return {n: self._read(self._lib.ft_model_read_param, i, k) for i, (n, k) in enumerate(self.named_params())}
 
     def grads(self) -> Dict[str, np.ndarray]:
-        return {n: self._read(self._lib.ft_model_read_grad, i, k) for i, (n, k) in enumerate(self.named_params())}
+        """Views of one array, in the order of `named_params`."""
+        named = self.named_params()
+        flat = np.empty(sum(k for _, k in named), np.float32)
+        check(self._lib.ft_model_read_grads(self.handle, flat.ctypes.data_as(C.c_void_p)))
+        out, at = {}, 0
+        for n, k in named:
+            out[n] = flat[at:at + k]
+            at += k
+        return out
 
     def forward_batch(self, rows) -> np.ndarray:
         """`Lfm2Model::forward_batch`: logits [B, S, vocab] on the host."""

@@ -158,6 +158,12 @@ impl Lfm2Model {
         ok(unsafe { sys::ft_model_read_grad(self.raw, index, out.as_mut_ptr()) })?;
         Ok(out)
     }
+    /// All gradients one after the other, in the order of the parameters (`numel` values in total).
+    pub fn read_grads(&self, numel: usize) -> Result<Vec<f32>, TrainError> {
+        let mut out = vec![0.0f32; numel];
+        ok(unsafe { sys::ft_model_read_grads(self.raw, out.as_mut_ptr()) })?;
+        Ok(out)
+    }
     /// `Lfm2Model::forward_batch` (lfm.rs:590-623): logits `[B * S, vocab]` of equally long rows.
     pub fn forward_batch(&self, rows: &[&[u32]], vocab_size: usize) -> Result<Vec<f32>, TrainError> {
         let b = rows.len();

@@ -1267,3 +1267,42 @@ def test_engine_ops_step_matches_the_oracle_and_the_fused_driver(ctx, f16):
             assert_close(f"step {step} weight {n}", got.reshape(-1), w.reshape(-1), atol=1e-6, rtol=1e-4)
     assert et.calls > 200     # op by op: hundreds of engine calls where the fused driver makes a few dozen launches
 
+
+
+@pytest.mark.parametrize("trainable_base", [False, True])
+def test_all_gradients_at_once_match_single_reads(trainable_base):
+    """ft_model_read_grads against ft_model_read_grad, bit for bit: after a step, after an adapter of another rank
+    replaced one (other tensors, other total), and for pieces longer than one copy block."""
+    from ferrotensor_amd import HipContext
+    from ferrotensor_amd.trainer import Lfm2Model, ModelConfig, Trainer
+    rng = np.random.default_rng(5)
+    H, F, V, D = 256, 320, 128, 64
+    ctx = HipContext(0)
+    try:
+        m = Lfm2Model(ctx, ModelConfig(vocab_size=V, hidden_size=H, intermediate_size=F, num_hidden_layers=2,
+                                       num_attention_heads=4, num_key_value_heads=2, tie_word_embeddings=True,
+                                       f16_linears=not trainable_base, trainable_base=trainable_base))
+        t = {"model.embed_tokens.weight": rng.standard_normal((V, H)), "model.norm.weight": np.ones(H)}
+        for l in range(2):
+            p = "model.layers.%d." % l
+            t[p + "input_layernorm.weight"] = t[p + "post_attention_layernorm.weight"] = np.ones(H)
+            for n, s in {"self_attn.q_proj": (4 * D, H), "self_attn.k_proj": (2 * D, H), "self_attn.v_proj": (2 * D, H),
+                         "self_attn.o_proj": (H, 4 * D), "mlp.gate_proj": (F, H), "mlp.up_proj": (F, H),
+                         "mlp.down_proj": (H, F)}.items():
+                t[p + n + ".weight"] = rng.standard_normal(s) * 0.05
+        m.load_tensors({k: v.astype(np.float32) for k, v in t.items()})
+        rows = rng.integers(0, V, (2, 32)).astype(np.uint32)
+        for rank in (4, 32):
+            for name in m.linear_prefixes(["q_proj", "o_proj"]):
+                i, o = m.linear_dims(name)
+                m.set_lora(name, rng.standard_normal((i, rank)).astype(np.float32) * 0.05,
+                           rng.standard_normal((rank, o)).astype(np.float32) * 0.05, 8.0)
+            Trainer(m, lr=1e-3, weight_decay=0.0).train_chunk(rows, np.roll(rows, -1, 1), np.ones((2, 32), np.uint8))
+            got = m.grads()
+            named = m.named_params()
+            assert list(got) == [n for n, _ in named] and any(k > 4096 for _, k in named) == (rank == 32 or trainable_base)
+            for i, (n, k) in enumerate(named):
+                np.testing.assert_array_equal(got[n], m._read(m._lib.ft_model_read_grad, i, k))
+            assert any(np.any(v != 0) for v in got.values())
+    finally:
+        ctx.close()
