@@ -787,12 +787,9 @@ __host__ __device__ constexpr int b_swizzle(int k4) {
 // KW = 2: eight waves; a stage holds two consecutive K tiles and waves 4-7 multiply the second
 // one of every stage for the same 64x64 output tile (the two sums meet in LDS after the loop):
 // twice the waves per SIMD for products whose tiles leave a CU with at most two workgroups.
-template <int BM, int BN, int WM, int WN, int LAYOUT, int NSEG, int EPI = kEpiPlain, int KW = 1, bool BF32 = false>
-__global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGateUp) - BF32 : 2) void gemm_async_kernel(AsyncBatch g) {
-    static_assert(LAYOUT == 0 || LAYOUT == 1 || (LAYOUT == 2 && BF32 && NSEG == 1 && EPI == kEpiPlain), "a @ b, a @ b^T; f32: a^T @ b");
-    constexpr bool A_KM = LAYOUT == 2;   // a is [K, M]
-    constexpr bool B_KC = LAYOUT == 1;   // b is [N, K]
-    constexpr int B_SIZE = BF32 ? 4 : 2;
+template <int BM, int BN, int WM, int WN, int LAYOUT, int NSEG, int EPI = kEpiPlain, int KW = 1>
+__global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 2) void gemm_async_kernel(AsyncBatch g) {
+    static_assert(LAYOUT == 0 || LAYOUT == 1, "a is k-contiguous on this path");
     static_assert(NSEG == 1 || NSEG == kAsyncMaxSeg, "one segment, or the general case");
     static_assert(EPI == kEpiPlain || NSEG == 1, "fused epilogues take one segment");
     constexpr int NST = 3;
@@ -809,12 +806,12 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     constexpr int CB = BN / 32;         // column blocks of a wave in the loop
     static_assert(FM == 1 && FN == CB / KS && (KS == 1 || KS == 2), "a wave's block after the exchange");
     constexpr int A_FLOATS = BM * 32;             // f32 tile
-    constexpr int B_FLOATS = BN * 8 * B_SIZE;     // in float units
+    constexpr int B_FLOATS = BN * 16;             // f16 tile, in float units
     constexpr int SUB = A_FLOATS + NB * B_FLOATS;  // one K tile of 32
     constexpr int STAGE = KW * SUB;
     static_assert(KW == 1 || (KW == 2 && BM == 64), "K-sharing waves: tiles of 64 rows");
     constexpr int A_CH = BM / 8 / 4;              // 1 KiB chunks per wave
-    constexpr int B_CH = BN * B_SIZE / 32 / 4;
+    constexpr int B_CH = BN / 16 / 4;
     constexpr int LPT = A_CH + NB * B_CH;         // load instructions per wave per tile
     constexpr int WAIT = (NST - 2) * LPT;         // loads that may still be in flight when tile t is needed
     using ExA = FastTile<BM, true, 16>;
@@ -986,7 +983,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
         abase[s] = sg.a;
         bbase[s] = sg.b;
         lda_b[s] = sg.lda * 4;
-        ldb_b[s] = sg.ldb * B_SIZE;
+        ldb_b[s] = sg.ldb * 2;
         tend[s] = (s > 0 ? tend[s - 1] : 0) + (s < p.nseg ? sg.nt : 0);
         has_ext[s] = NB == 1 && grp == 0 && s < p.nseg && sg.a2 != nullptr;
     }
@@ -1008,38 +1005,19 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     // bytes) + col. The products are formed once per segment (offA / offB), so
     // the K loop itself carries no per-lane address arithmetic.
     unsigned rowA[A_CH], colA[A_CH], rowB[B_CH], colB[B_CH], offA[A_CH], offB[B_CH];
-    // Chunk c of an f32 tile: eight k-contiguous rows of 128 bytes, or four k of 64 columns (k-major; the 16-byte
-    // columns of rows with bit 3 of k set swap halves, so that the two k of a read lie in different banks).
-    auto f32_octets = [&](int c, int base, int extent, unsigned& row, unsigned& col) {
-        const int r = lane / 8, cs = lane % 8, at = base + 8 * c + r;
-        row = (unsigned)(at < extent ? at : extent - 1);
-        col = (unsigned)((cs ^ ((4 * c + (r >> 1)) & 7)) * 16);
-    };
-    auto f32_rows = [&](int c, int base, int extent, unsigned& row, unsigned& col) {
-        const int k = 4 * c + lane / 16;
-        int at = base + ((lane % 16) ^ (k & 8)) * 4;
-        at = at + 4 <= extent ? at : extent - 4;
-        row = (unsigned)k;
-        col = (unsigned)(at * 4);
-    };
 #pragma unroll
     for (int j = 0; j < A_CH; j++) {
-        const int c = wave + 4 * j;
-        if constexpr (A_KM) {
-            f32_rows(c, m0, M, rowA[j], colA[j]);
-        } else {
-            f32_octets(c, m0, M, rowA[j], colA[j]);
-        }
+        const int c = wave + 4 * j, r = lane / 8, cs = lane % 8;
+        int row = m0 + 8 * c + r;
+        row = row < M ? row : M - 1;
+        rowA[j] = (unsigned)row;
+        colA[j] = (unsigned)((cs ^ ((4 * c + (r >> 1)) & 7)) * 16);
         offA[j] = rowA[j] * (unsigned)lda_b[0] + colA[j];
     }
 #pragma unroll
     for (int j = 0; j < B_CH; j++) {
         const int c = wave + 4 * j;
-        if constexpr (BF32 && B_KC) {
-            f32_octets(c, n0, p.N, rowB[j], colB[j]);
-        } else if constexpr (BF32) {
-            f32_rows(c, n0, p.N, rowB[j], colB[j]);
-        } else if constexpr (B_KC) {
+        if constexpr (LAYOUT == 1) {
             const int r = lane / 4, cs = lane % 4;
             int n = n0 + 16 * c + r;
             n = n < p.N ? n : p.N - 1;
@@ -1060,7 +1038,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     int seg_end = NSEG > 1 ? tend[0] : 1 << 30;
     const char* aseg = abase[0];
     const char* bseg = bbase[0];
-    long b_step = B_KC ? 32L * B_SIZE : 32L * ldb_b[0];  // bytes per K tile
+    long b_step = LAYOUT == 1 ? 64L : 32L * ldb_b[0];  // bytes per K tile
 
     auto issue = [&](int t, float* st) {
         t = t < nt ? t : nt - 1;  // past the end: re-read the last tile into a stage nobody reads
@@ -1074,7 +1052,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
                 const int la = seg_pick<NSEG>(lda_b, seg_cur), lb = seg_pick<NSEG>(ldb_b, seg_cur);
                 aseg = seg_pick<NSEG>(abase, seg_cur);
                 bseg = seg_pick<NSEG>(bbase, seg_cur);
-                b_step = B_KC ? 32L * B_SIZE : 32L * lb;
+                b_step = LAYOUT == 1 ? 64L : 32L * lb;
 #pragma unroll
                 for (int j = 0; j < A_CH; j++) offA[j] = rowA[j] * (unsigned)la + colA[j];
 #pragma unroll
@@ -1082,7 +1060,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
             }
         }
         const int tl = t - seg_first;
-        const char* at = aseg + (long)tl * (A_KM ? 32L * lda_b[0] : 128L);
+        const char* at = aseg + (long)tl * 128;
         const char* bt = bseg + (long)tl * b_step;
 #pragma unroll
         for (int j = 0; j < A_CH; j++) glds16(at, offA[j], st + (wave + 4 * j) * 256);
@@ -1096,37 +1074,26 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     };
     // A K tile's operands as this lane feeds them: k = 16 * S + 8 * half + 0..7 of its row (a: f32 as read, then
     // its f16 halves) and its column (b, f16), S = k step.
-    float4 raw[NS][2], rawb[BF32 ? CB * NB : 1][NS][2];
-    half8_t bfr[2][CB * NB][NS], bfl[BF32 ? 2 : 1][BF32 ? CB * NB : 1][NS], hi[2][NS], lo[2][NS];
-    RowScale rs, cs[BF32 ? CB * NB : 1];  // (an f32 b is split as a is, under a scale per column)
-    auto f32_frag = [&](const float* tile, bool kc, int idx, int S, float4 (&out)[2]) {
-        if (kc) {
+    float4 raw[NS][2];
+    half8_t bfr[2][CB * NB][NS], hi[2][NS], lo[2][NS];
+    RowScale rs;
+    auto read_frags = [&](const float* st, half8_t (&bf)[CB * NB][NS]) {
+        const int row = rm0 + l32;
+#pragma unroll
+        for (int u = 0; u < NS; u++)
 #pragma unroll
             for (int q = 0; q < 2; q++) {
-                const int kq = 4 * S + 2 * half + q;
-                out[q] = *reinterpret_cast<const float4*>(tile + idx * 32 + ((kq ^ ((idx >> 1) & 7)) * 4));
+                const int kq = 4 * (u + ks) + 2 * half + q;
+                raw[u][q] = *reinterpret_cast<const float4*>(st + row * 32 + ((kq ^ ((row >> 1) & 7)) * 4));
             }
-        } else {
-            const float* q = tile + (16 * S + 8 * half) * 64 + ((idx >> 2) ^ (8 * half)) * 4 + (idx & 3);
-            out[0] = make_float4(q[0], q[64], q[128], q[192]);
-            out[1] = make_float4(q[256], q[320], q[384], q[448]);
-        }
-    };
-    static_assert(!(A_KM && BM != 64) && !(BF32 && BN != 64), "k-major f32 tiles are 64 columns wide");
-    auto read_frags = [&](const float* st, half8_t (&bf)[CB * NB][NS]) {
-#pragma unroll
-        for (int u = 0; u < NS; u++) f32_frag(st, !A_KM, rm0 + l32, u + ks, raw[u]);
 #pragma unroll
         for (int j = 0; j < CB * NB; j++) {
-            const float* tile = st + A_FLOATS + (j / CB) * B_FLOATS;
-            const char* bs = reinterpret_cast<const char*>(tile);
+            const char* bs = reinterpret_cast<const char*>(st + A_FLOATS + (j / CB) * B_FLOATS);
             const int nw = (j % CB) * 32;
 #pragma unroll
             for (int u = 0; u < NS; u++) {
                 const int S = u + ks;
-                if constexpr (BF32) {
-                    f32_frag(tile, B_KC, nw + l32, S, rawb[j][u]);
-                } else if constexpr (B_KC) {
+                if constexpr (LAYOUT == 1) {
                     const int n = nw + l32, col = (2 * S + half) ^ ((n >> 2) & 3);
                     bf[j][u] = *reinterpret_cast<const half8_t*>(bs + n * 64 + col * 16);
                 } else {
@@ -1141,52 +1108,33 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     // Sums of rows whose scale has changed, brought to the new scale: the lanes' ratios are handed to the
     // accumulators' rows by shuffles. Rare: a scale changes at a row's first tile that is not all zeros and at a value
     // more than eight times larger than any before.
-    auto rescale = [&](float ratio, const float (&cratio)[BF32 ? CB * NB : 1]) {
+    auto rescale = [&](float ratio) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const float f = __shfl(ratio, (r / 4) * 8 + half * 4 + (r % 4));
 #pragma unroll
-            for (int j = 0; j < CB * NB; j++) {
-                sum[j][r] *= f;  // (a ratio above 1 means a row or column of zeros so far; two of them may pass the f32 range together)
-                if constexpr (BF32) sum[j][r] *= cratio[j];
-            }
+            for (int j = 0; j < CB * NB; j++) sum[j][r] *= f;
         }
     };
-    auto frag_max = [&](const float4 (&v)[NS][2]) {
+    auto tile_max = [&]() {
         float mx = 0.0f;
 #pragma unroll
         for (int u = 0; u < NS; u++)
 #pragma unroll
-            for (int q = 0; q < 2; q++) mx = abs_max(abs_max(mx, v[u][q].x, v[u][q].y), v[u][q].z, v[u][q].w);
+            for (int q = 0; q < 2; q++) mx = abs_max(abs_max(mx, raw[u][q].x, raw[u][q].y), raw[u][q].z, raw[u][q].w);
         return mx;
     };
-    auto grow = [&](RowScale& sc, float mx) { return sc.grow(fmaxf(mx, __shfl_xor(mx, 32))); };
-    // What was read into raw and rawb, split into buffer BUF.
-    auto split_tile = [&](auto buf) {
-        constexpr int BUF = decltype(buf)::value;
-#pragma unroll
-        for (int u = 0; u < NS; u++) {
-            split8(raw[u][0], raw[u][1], rs.scale, hi[BUF][u], lo[BUF][u]);
-            if constexpr (BF32) {
-#pragma unroll
-                for (int j = 0; j < CB * NB; j++) split8(rawb[j][u][0], rawb[j][u][1], cs[j].scale, bfr[BUF][j][u], bfl[BUF][j][u]);
-            }
-        }
-    };
-    // MFMAs first .. last - 1 of a tile whose halves are in buffer BUF: lo a * b, hi a * b, or with an f32 b
-    // lo a * hi b, hi a * lo b, hi a * hi b (lo a * lo b is below the last place of either: 2^-22 of the product).
-    constexpr int TERMS = BF32 ? 3 : 2;
+    // MFMAs FIRST .. LAST - 1 of the 2 * NS * CB * NB of a tile whose halves are in buffer BUF.
     auto mfmas = [&](auto buf, int first, int last) {
         constexpr int BUF = decltype(buf)::value;
 #pragma unroll
-        for (int e = 0; e < TERMS * NS * CB * NB; e++) {
+        for (int e = 0; e < 2 * NS * CB * NB; e++) {
             if (e < first || e >= last) continue;
-            const int u = e / (TERMS * CB * NB), term = (e / (CB * NB)) % TERMS, j = e % (CB * NB);
-            const half8_t& bh = BF32 && term == 1 ? bfl[BF32 ? BUF : 0][BF32 ? j : 0][u] : bfr[BUF][j][u];
-            sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(term == 0 ? lo[BUF][u] : hi[BUF][u], bh, sum[j], 0, 0, 0);
+            const int u = e / (2 * CB * NB), low = (e / (CB * NB)) % 2 == 0, j = e % (CB * NB);
+            sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(low ? lo[BUF][u] : hi[BUF][u], bfr[BUF][j][u], sum[j], 0, 0, 0);
         }
     };
-    constexpr int ALL = TERMS * NS * CB * NB, EARLY = ALL / 2;  // half of the MFMAs in front of the split of the next tile
+    constexpr int EARLY = NS * CB * NB, ALL = 2 * EARLY;  // half of the MFMAs in front of the split of the next tile
     // Tile t, whose operands are in hi, lo and bfr of buffer BUF; `stage` is the one it came from, `next` holds tile
     // t + 1. Tile t + 1 is read while the first MFMAs of tile t run and split between the others: 16 to 32
     // instructions that fit into the time the matrix pipe takes (with the split in front of all MFMAs the waves of a
@@ -1203,37 +1151,21 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
         read_frags(next + grp * SUB, bfr[BUF ^ 1]);
         __builtin_amdgcn_sched_barrier(0);
         mfmas(here, 0, EARLY);
-        const float mx = frag_max(raw);
-        bool over = mx > rs.limit;
-        float cmx[BF32 ? CB * NB : 1], cratio[BF32 ? CB * NB : 1], ratio = 1.0f;
-        if constexpr (BF32) {
-#pragma unroll
-            for (int j = 0; j < CB * NB; j++) {
-                cmx[j] = frag_max(rawb[j]);
-                cratio[j] = 1.0f;
-                over = over || cmx[j] > cs[j].limit;
-            }
-        }
-        const bool grown = __builtin_amdgcn_ballot_w64(over) != 0;
-        if (grown) {
-            ratio = grow(rs, mx);
-            if constexpr (BF32) {
-#pragma unroll
-                for (int j = 0; j < CB * NB; j++) cratio[j] = grow(cs[j], cmx[j]);
-            }
-        }
+        const float mx = tile_max();
+        const bool grown = __builtin_amdgcn_ballot_w64(mx > rs.limit) != 0;
+        float ratio = 1.0f;
+        if (grown) ratio = rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
         mfmas(here, EARLY, ALL);  // (still under the old scales)
-        constexpr std::integral_constant<int, BUF ^ 1> there{};
-        split_tile(there);
+#pragma unroll
+        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[BUF ^ 1][u], lo[BUF ^ 1][u]);
 #pragma unroll
         for (int e = EARLY; e < ALL; e++) {
-            constexpr int SPLIT = 24 * NS * (BF32 ? 1 + CB * NB : 1);  // instructions of the split
-            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                                          // one MFMA,
-            __builtin_amdgcn_sched_group_barrier(0x2, (SPLIT + ALL - EARLY - 1) / (ALL - EARLY), 0);  // its share of the split
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                              // one MFMA,
+            __builtin_amdgcn_sched_group_barrier(0x2, (24 * NS + EARLY - 1) / EARLY, 0);  // its share of the split
         }
 #pragma unroll
         for (int u = 0; u < NS; u++) asm volatile("" : "+v"(hi[BUF ^ 1][u]), "+v"(lo[BUF ^ 1][u]));  // split here, not at the use
-        if (grown) rescale(ratio, cratio);
+        if (grown) rescale(ratio);
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -1263,15 +1195,15 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
     __builtin_amdgcn_sched_barrier(0);
     issue(t0 + 2, St2);
     read_frags(St0 + grp * SUB, bfr[0]);
+    {
+        const float mx = tile_max();
+        rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
+#pragma unroll
+        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[0][u], lo[0][u]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
-    grow(rs, frag_max(raw));
-    if constexpr (BF32) {
-#pragma unroll
-        for (int j = 0; j < CB * NB; j++) grow(cs[j], frag_max(rawb[j]));
-    }
-    split_tile(even);
-    __builtin_amdgcn_sched_barrier(0);
     for (int t = t0; t < nt; t += 2 * NST) {
         iter(t, St0, St1, even);
         if (t + 1 < nt) iter(t + 1, St1, St2, odd);
@@ -1289,7 +1221,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
         const int e = __shfl(rs.exponent, (r / 4) * 8 + half * 4 + (r % 4));
 #pragma unroll
         for (int j = 0; j < CB * NB; j++) {
-            sum[j][r] = __builtin_amdgcn_ldexpf(sum[j][r], BF32 ? -(e + cs[BF32 ? j : 0].exponent) : -e);
+            sum[j][r] = __builtin_amdgcn_ldexpf(sum[j][r], -e);
             probe = fmaf(sum[j][r], 0.0f, probe);
         }
     }
@@ -1305,23 +1237,19 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
             if constexpr (NSEG > 1) s = t >= tend[1] ? 2 : (t >= tend[0] ? 1 : 0);
             const int tl = t - (NSEG > 1 && s > 0 ? (s == 1 ? tend[0] : tend[NSEG > 1 ? 1 : 0]) : 0);
             const int la = seg_pick<NSEG>(lda_b, s), lb = seg_pick<NSEG>(ldb_b, s);
-            const long r = row < M ? row : M - 1;
-            const char* at = seg_pick<NSEG>(abase, s) + (A_KM ? r * 4 : r * la);
+            const char* at = seg_pick<NSEG>(abase, s) + (long)tl * 128 + (long)(row < M ? row : M - 1) * la;
             const char* bt = seg_pick<NSEG>(bbase, s);
 #pragma unroll 1
             for (int q = 2 * ks; q < 2 * (ks + NS); q++) {
-                const long k = 32L * tl + 8 * q + 4 * half;
-                auto a_k = [&](int e) { return *reinterpret_cast<const float*>(at + (A_KM ? (k + e) * la : (k + e) * 4)); };
-                const float4 af = make_float4(a_k(0), a_k(1), a_k(2), a_k(3));
+                const int kq = 8 * q + 4 * half;
+                const float4 af = *reinterpret_cast<const float4*>(at + kq * 4);
 #pragma unroll
                 for (int j = 0; j < CB * NB; j++) {
                     int n = n0 + (j % CB) * 32 + l32;
                     n = n < p.N ? n : p.N - 1;
-                    const char* bb = j < CB ? bt : balt;
-                    auto at_k = [&](int e) {
-                        const char* q = bb + (B_KC ? (long)n * lb + (k + e) * B_SIZE : (k + e) * lb + (long)n * B_SIZE);
-                        return BF32 ? *reinterpret_cast<const float*>(q) : (float)*reinterpret_cast<const _Float16*>(q);
-                    };
+                    const long k = 32L * tl + kq, step = LAYOUT == 1 ? 2 : lb;
+                    const char* bb = (j < CB ? bt : balt) + (LAYOUT == 1 ? (long)n * lb + k * 2 : k * lb + n * 2);
+                    auto at_k = [&](int e) { return (float)*reinterpret_cast<const _Float16*>(bb + e * step); };
                     sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.x, at_k(0), sum[j], 0, 0, 0);
                     sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.y, at_k(1), sum[j], 0, 0, 0);
                     sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.z, at_k(2), sum[j], 0, 0, 0);
@@ -1535,6 +1463,152 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? 4 - (EPI == kEpiGa
 }
 
 // ---------------------------------------------------------------------------
+// f32 x f32 on the same pipeline (global -> LDS DMA, three stages, explicit
+// waits): the plain matmul / matmul_bt / matmul_at of the engine, where b is an
+// f32 tensor. An operand tile is either
+//   KC  k-contiguous in memory (a[M,K]; b[N,K]): [64 rows][32 k], 128 B per row,
+//       swizzled as in gemm_async_kernel, one ds_read_b128 per k-quad, or
+//   KM  k-major (a[K,M] of matmul_at; b[K,N]): [32 k][64] exactly as in memory
+//       (4 k rows per DMA instruction), four ds_read_b32 per k-quad.
+// 64x64 tiles, 32x32 per wave; K a multiple of 32, M / N multiples of 4 where an
+// operand is KM. Tile order as in gemm_async_kernel.
+// ---------------------------------------------------------------------------
+struct F32AsyncArgs {
+    const float* a;
+    const float* b;
+    float* out;
+    int M, N, nt;        // nt = K / 32
+    int lda, ldb, ldc;
+    int tiles_m, tiles_n, xcds, panel;
+    int splits;          // shares of the K tiles (blockIdx.y); > 1: partial tiles go to `partial` [splits][M][N]
+    float* partial;
+};
+
+template <bool A_KM, bool B_KM>
+__global__ __launch_bounds__(256) void gemm_f32_async_kernel(F32AsyncArgs g) {
+    constexpr int NST = 3, TILE = 64 * 32, STAGE = 2 * TILE;
+    constexpr int LPT = 4;                         // 2 + 2 load instructions per wave per K tile
+    __shared__ __attribute__((aligned(16))) float St0[STAGE];
+    __shared__ __attribute__((aligned(16))) float St1[STAGE];
+    __shared__ __attribute__((aligned(16))) float St2[STAGE];
+    int bid = (int)blockIdx.x;
+    if (g.xcds > 1) {
+        const int total = (int)gridDim.x, x = bid % g.xcds, q = total / g.xcds, r = total % g.xcds;
+        bid = x * q + (x < r ? x : r) + bid / g.xcds;
+    }
+    const int per_panel = g.tiles_m * g.panel;
+    const int last = (g.tiles_n - 1) / g.panel;
+    int pnl = bid / per_panel;
+    pnl = pnl < last ? pnl : last;
+    const int rem = bid - pnl * per_panel;
+    const int width = pnl == last ? g.tiles_n - last * g.panel : g.panel;
+    const int m0 = (rem / width) * 64, n0 = (pnl * g.panel + rem % width) * 64;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int wm0 = (wave / 2) * 32, wn0 = (wave % 2) * 32;
+    const int l32 = lane % 32, half = lane / 32;
+
+    // Per-lane byte offsets of the two DMA instructions a wave issues per operand and K tile.
+    unsigned offA[2], offB[2];
+    auto offsets = [&](bool km, int base0, int extent, int ld, unsigned (&off)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int c = wave + 4 * j;  // chunk of 1 KiB
+            if (km) {
+                const int kr = lane / 16, cs = lane % 16;
+                int col = base0 + cs * 4;
+                col = col + 4 <= extent ? col : extent - 4;
+                off[j] = (unsigned)(4 * c + kr) * (unsigned)ld * 4u + (unsigned)col * 4u;
+            } else {
+                const int r = lane / 8, cs = lane % 8;
+                int row = base0 + 8 * c + r;
+                row = row < extent ? row : extent - 1;
+                off[j] = (unsigned)row * (unsigned)ld * 4u + (unsigned)((cs ^ ((4 * c + (r >> 1)) & 7)) * 16);
+            }
+        }
+    };
+    offsets(A_KM, m0, g.M, g.lda, offA);
+    offsets(B_KM, n0, g.N, g.ldb, offB);
+    const long a_step = A_KM ? 32L * g.lda * 4 : 128L, b_step = B_KM ? 32L * g.ldb * 4 : 128L;
+    const char* abase = reinterpret_cast<const char*>(g.a);
+    const char* bbase = reinterpret_cast<const char*>(g.b);
+    // This workgroup's share of the K tiles: [t0, nt).
+    const int split = (int)blockIdx.y;
+    const int t0 = (int)(((long)g.nt * split) / g.splits);
+    const int nt = (int)(((long)g.nt * (split + 1)) / g.splits);
+    auto issue = [&](int t, float* st) {
+        t = t < nt ? t : nt - 1;  // past the end: re-read the last tile into a stage nobody reads
+        const char* at = abase + (long)t * a_step;
+        const char* bt = bbase + (long)t * b_step;
+#pragma unroll
+        for (int j = 0; j < 2; j++) glds16(at, offA[j], st + (wave + 4 * j) * 256);
+#pragma unroll
+        for (int j = 0; j < 2; j++) glds16(bt, offB[j], st + TILE + (wave + 4 * j) * 256);
+    };
+    auto frag = [&](const float* tile, bool km, int s, int idx) -> float4 {
+        const int kq = 2 * s + half;
+        if (km) {
+            const float* q = tile + (4 * kq) * 64 + idx;
+            return make_float4(q[0], q[64], q[128], q[192]);
+        }
+        return *reinterpret_cast<const float4*>(tile + idx * 32 + ((kq ^ ((idx >> 1) & 7)) * 4));
+    };
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    // Rotated like the loop of gemm_async_kernel: wait, barrier, refill and the first fragment
+    // reads of tile t + 1 come before the last MFMA group of tile t.
+    float4 af[2], bf[2];
+    auto iter = [&](int t, float* cur, const float* next) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int c = s & 1, nx = c ^ 1;
+            if (s + 1 < 4) {
+                af[nx] = frag(cur, A_KM, s + 1, wm0 + l32);
+                bf[nx] = frag(cur + TILE, B_KM, s + 1, wn0 + l32);
+            } else {
+                // own reads of the stage complete, tile t + 1 landed (tile t + 2 may be in flight)
+                __builtin_amdgcn_s_waitcnt(0x0070 | LPT);
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                issue(t + NST, cur);
+                af[nx] = frag(next, A_KM, 0, wm0 + l32);
+                bf[nx] = frag(next + TILE, B_KM, 0, wn0 + l32);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c].x, bf[c].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c].y, bf[c].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c].z, bf[c].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[c].w, bf[c].w, acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    issue(t0, St0);
+    issue(t0 + 1, St1);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | LPT);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(t0 + 2, St2);
+    af[0] = frag(St0, A_KM, 0, wm0 + l32);
+    bf[0] = frag(St0 + TILE, B_KM, 0, wn0 + l32);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t = t0; t < nt; t += NST) {
+        iter(t, St0, St1);
+        if (t + 1 < nt) iter(t + 1, St1, St2);
+        if (t + 2 < nt) iter(t + 2, St2, St0);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // nothing may still be landing in LDS when the workgroup retires
+    const int col = n0 + wn0 + l32;
+    if (col >= g.N) return;
+    float* dst = g.splits > 1 ? g.partial + (long)split * g.M * g.N : g.out;
+    const int ld = g.splits > 1 ? g.N : g.ldc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int row = m0 + wm0 + (r / 4) * 8 + half * 4 + (r % 4);
+        if (row < g.M) dst[(long)row * ld + col] = acc[r];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // out[R, C] (C <= 32) = scale * X[R, Kr] @ Y[Kr, C].
 //   XT:  X is stored [Kr, R] (element (row,k) at x[k*ldx + row])
 //   YT:  Y is stored [C, Kr] (element (k,col) at y[col*ldy + k])
@@ -1691,7 +1765,7 @@ bool aligned16p(const void* q) { return (((uintptr_t)q) & 15) == 0; }
 static int ft_gemm_xcds(ft_context* ctx) { return ctx->num_cus % 8 == 0 && ctx->num_cus >= 64 ? 8 : 1; }
 
 template <int BM, int BN, int WM, int WN>
-int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain, bool f32b = false) {
+int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain) {
     const int tiles_m = (g.M + BM - 1) / BM;
     int tiles_n = 0, max_seg = 1;
     double flops = 0.0, bytes = 0.0, a_bytes = 0.0, b_bytes = 0.0;
@@ -1703,13 +1777,13 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain,
         double a_this = 0.0;  // the products of a batch share their a operand
         for (int s = 0; s < p.nseg; s++) {
             a_this += 4.0 * g.M * 32.0 * p.seg[s].nt;
-            b_bytes += (f32b ? 4.0 : 2.0) * p.N * 32.0 * p.seg[s].nt * (epi == kEpiGateUp ? 2 : 1);
+            b_bytes += 2.0 * p.N * 32.0 * p.seg[s].nt * (epi == kEpiGateUp ? 2 : 1);
         }
         if (a_this > a_bytes) a_bytes = a_this;
         for (int s = 0; s < p.nseg; s++) {
             const double k = 32.0 * p.seg[s].nt, k2 = p.seg[s].a2 ? (double)p.seg[s].K2 : 0.0;
             flops += 2.0 * g.M * (double)p.N * (k + k2);
-            bytes += 4.0 * g.M * (k + k2) + (f32b ? 4.0 : 2.0) * p.N * k + 4.0 * p.N * k2;
+            bytes += 4.0 * g.M * (k + k2) + 2.0 * p.N * k + 4.0 * p.N * k2;
         }
         bytes += (p.add ? 8.0 : 4.0) * g.M * (double)p.N;
     }
@@ -1751,7 +1825,7 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain,
     const bool few_tiles = (size_t)tiles * 4 <= (size_t)ctx->num_cus * 5;
     const bool long_k = (size_t)tiles * 2 < 3 * (size_t)ctx->num_cus && min_kt >= 512;
     // Eight waves on a tile (two K tiles per stage, see the kernel) need whole pairs of tiles in every segment.
-    bool pairs_ok = BM == 64 && epi == kEpiPlain && !any_rope && !f32b && min_kt >= 8;
+    bool pairs_ok = BM == 64 && epi == kEpiPlain && !any_rope && min_kt >= 8;
     for (int i = 0; i < g.count && pairs_ok; i++)
         for (int s = 0; s < g.p[i].nseg; s++) pairs_ok = pairs_ok && g.p[i].seg[s].nt % 2 == 0;
     bool pairs = false;
@@ -1884,29 +1958,6 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain,
         return FT_OK;
     };
     char name[96];
-    if constexpr (BM == 64 && BN == 64) {
-        if (f32b) {
-            const bool gu = epi == kEpiGateUp;
-            snprintf(name, sizeof(name), "gemm_async_kernel<64, 64, 32, 32, %d, %d, %d, 1, true>", layout,
-                     max_seg > 1 ? kAsyncMaxSeg : 1, epi);
-            const double mn = (double)g.M * g.p[0].N;
-            ft_prof_scope prof(ctx, name, gu ? 2.0 * flops : flops,
-                               bytes + (gu ? 128.0 * g.p[0].N * g.p[0].seg[0].nt + 8.0 * mn : epi == kEpiSiluBwd ? 12.0 * mn : 0.0));
-#define FT_F32B(L, S, E) \
-    hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, L, S, E, 1, true>), grid, dim3(256), 0, ctx->stream, g)
-            if (gu) FT_F32B(0, 1, kEpiGateUp);
-            else if (epi == kEpiSiluBwd) FT_F32B(1, 1, kEpiSiluBwd);
-            else if (layout == 2) FT_F32B(2, 1, kEpiPlain);
-            else if (max_seg > 1) {
-                if (layout == 0) FT_F32B(0, kAsyncMaxSeg, kEpiPlain); else FT_F32B(1, kAsyncMaxSeg, kEpiPlain);
-            } else {
-                if (layout == 0) FT_F32B(0, 1, kEpiPlain); else FT_F32B(1, 1, kEpiPlain);
-            }
-#undef FT_F32B
-            FT_LAUNCH_CHECK();
-            return epi == kEpiPlain ? reduce_shares() : FT_OK;
-        }
-    }
     if (epi != kEpiPlain) {
         // both fused forms: one product, one segment, tiles of 64 rows
         if constexpr (BM == 64) {
@@ -1994,8 +2045,7 @@ bool wide_tiles(const ft_context* ctx, size_t M, size_t N) {
     return N >= 512 && ((M + 63) / 64) * ((N + 127) / 128) >= 4 * (size_t)ctx->num_cus;
 }
 
-int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout, bool f32b = false) {
-    if (f32b) return launch_async<64, 64, 32, 32>(ctx, g, layout, kEpiPlain, true);
+int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout) {
     size_t tiles128 = 0;
     for (int i = 0; i < g.count; i++) tiles128 += (size_t)((g.M + 127) / 128) * (size_t)((g.p[i].N + 127) / 128);
     if (tiles128 >= 8 * (size_t)ctx->num_cus) return launch_async<128, 128, 32, 128>(ctx, g, layout);
@@ -2028,36 +2078,31 @@ int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout, bool f32
     return launch_async<64, 64, 32, 32>(ctx, g, layout);
 }
 
-// Can out[M,N] (+)= a @ b (`layout`; b f16, or f32: `f32b`) + a2[M,K2] @ b2 run on the asynchronous path?
+// Can out[M,N] (+)= a[M,K] @ b (f16, `layout`) + a2[M,K2] @ b2 run on the asynchronous path?
 bool async_eligible(int layout, const float* a, const void* b, const float* out, const float* add, size_t M, size_t K,
-                    size_t N, const float* a2, const float* b2, size_t K2, bool f32b = false) {
-    if (layout != 0 && layout != 1 && !(layout == 2 && f32b)) return false;
+                    size_t N, const float* a2, const float* b2, size_t K2) {
+    if (layout != 0 && layout != 1) return false;
     if (M == 0 || N == 0 || K < 32 || K % 32 != 0) return false;
     if (!aligned16p(a) || !aligned16p(b) || !aligned16p(out) || !out || !a || !b) return false;
     // The residual is read in 16-byte groups (epilogue and split-K reduce kernel alike).
     if (add && !aligned16p(add)) return false;
-    const size_t group = f32b ? 4 : 8;  // 16 bytes of a row of b
-    if (layout != 1 && (N % group != 0 || N < group)) return false;
-    if (layout == 2 && (M % 4 != 0 || M < 4)) return false;
-    if (f32b && M * N < 128 * 128) return false;  // tiny f32 products: the register-staged kernels
+    if (layout == 0 && (N % 8 != 0 || N < 8)) return false;
     if (K2 > 0 && (K2 > 16 || K2 % 4 != 0 || !aligned16p(a2) || !aligned16p(b2))) return false;
     // Per-lane operand offsets are 32-bit byte offsets from a uniform base.
     const double lim = 4294967296.0;
-    const double a_span = layout == 2 ? 4.0 * 36 * (double)M : 4.0 * (double)M * (double)K + 4.0 * 64 * (double)K;
     const double ldb = layout == 1 ? (double)K : (double)N;
-    const double b_span = f32b ? 4.0 * ldb * (layout == 1 ? (double)N + 64 : 36.0)
-                               : 2.0 * ldb * (double)(layout == 1 ? N : K) + 2.0 * 64 * ldb;
-    return a_span < lim && b_span < lim;
+    return 4.0 * (double)M * (double)K + 4.0 * 64 * (double)K < lim &&
+           2.0 * ldb * (double)(layout == 1 ? N : K) + 2.0 * 64 * ldb < lim;
 }
 
 AsyncSeg make_seg(int layout, const float* a, const void* b, size_t K, size_t N, const float* a2, const float* b2,
-                  size_t K2, size_t M = 0) {
+                  size_t K2) {
     AsyncSeg sg{};
     sg.a = a;
     sg.b = b;
     sg.a2 = K2 > 0 ? a2 : nullptr;
     sg.b2 = K2 > 0 ? b2 : nullptr;
-    sg.lda = layout == 2 ? (int)M : (int)K;
+    sg.lda = (int)K;
     sg.ldb = layout == 1 ? (int)K : (int)N;
     sg.lda2 = (int)K2;
     sg.ldb2 = layout == 1 ? (int)K2 : (int)N;
@@ -2101,6 +2146,82 @@ int launch_cfg(ft_context* ctx, GemmArgs p, int layout, bool half_b, bool fast) 
     return FT_OK;
 }
 
+// Operands of the f32 DMA kernel: 16-byte aligned, K in whole tiles, at least two of them per
+// workgroup, k-major operands in whole float4 groups, 32-bit per-lane offsets.
+bool f32_async_eligible(int layout, const float* a, const void* b, const float* out, size_t M, size_t K, size_t N) {
+    if (M == 0 || N == 0 || K < 64 || K % 32 != 0) return false;
+    if (!aligned16p(a) || !aligned16p(b) || !out) return false;
+    const bool a_km = layout == 2, b_km = layout != 1;
+    if (a_km && (M % 4 != 0 || M < 4)) return false;
+    if (b_km && (N % 4 != 0 || N < 4)) return false;
+    if (M * N < 128 * 128) return false;  // tiny products: the register-staged kernels
+    const double lim = 4294967296.0;
+    const double a_span = a_km ? 4.0 * 36 * (double)M : 4.0 * ((double)M + 64) * (double)K;
+    const double b_span = b_km ? 4.0 * 36 * (double)N : 4.0 * ((double)N + 64) * (double)K;
+    return a_span < lim && b_span < lim;
+}
+
+int launch_f32_async(ft_context* ctx, int layout, const float* a, const float* b, float* out, size_t M, size_t K,
+                     size_t N) {
+    F32AsyncArgs g{};
+    g.a = a;
+    g.b = b;
+    g.out = out;
+    g.M = (int)M;
+    g.N = (int)N;
+    g.nt = (int)(K / 32);
+    g.lda = layout == 2 ? (int)M : (int)K;
+    g.ldb = layout == 1 ? (int)K : (int)N;
+    g.ldc = (int)N;
+    g.tiles_m = (int)((M + 63) / 64);
+    g.tiles_n = (int)((N + 63) / 64);
+    g.xcds = ft_gemm_xcds(ctx);
+    // panels of about sqrt(96) n tiles: equal bytes of a and b per XCD-resident block of tiles
+    int panels = (int)((double)g.tiles_n / 10.0 + 0.5);
+    if (panels < 1) panels = 1;
+    g.panel = (g.tiles_n + panels - 1) / panels;
+    // Split K when the tiles occupy at most half of the CUs and K is long enough to share out
+    // (at least 4 K tiles per share); the shares are added in order. (At 216 tiles of K = 2048
+    // a three-way split measured no gain: 44.4 us against 42.6.)
+    const size_t tiles = (size_t)g.tiles_m * g.tiles_n;
+    g.splits = 1;
+    if (tiles * 2 <= (size_t)ctx->num_cus && (M * N) % 4 == 0) {
+        int want = (int)((2 * (size_t)ctx->num_cus + tiles - 1) / tiles);
+        if (want > 8) want = 8;
+        if (want > g.nt / 4) want = g.nt / 4;
+        if (want >= 2 && M * N * (size_t)want <= kSplitScratchFloats) {
+            if (!ctx->gemm_scratch) {
+                FT_HIP(hipSetDevice(ctx->device));
+                FT_HIP(hipMalloc((void**)&ctx->gemm_scratch, kSplitScratchFloats * sizeof(float)));
+            }
+            g.splits = want;
+            g.partial = ctx->gemm_scratch;
+        }
+    }
+    const dim3 grid((unsigned)tiles, (unsigned)g.splits);
+    char name[64];
+    snprintf(name, sizeof(name), "gemm_f32_async_kernel<%d>", layout);
+    ft_prof_scope prof(ctx, name, 2.0 * M * (double)N * K, 4.0 * ((double)M * K + (double)N * K + (double)M * N));
+    if (layout == 0)
+        hipLaunchKernelGGL((gemm_f32_async_kernel<false, true>), grid, dim3(256), 0, ctx->stream, g);
+    else if (layout == 1)
+        hipLaunchKernelGGL((gemm_f32_async_kernel<false, false>), grid, dim3(256), 0, ctx->stream, g);
+    else
+        hipLaunchKernelGGL((gemm_f32_async_kernel<true, true>), grid, dim3(256), 0, ctx->stream, g);
+    FT_LAUNCH_CHECK();
+    if (g.splits > 1) {
+        SplitReduceArgs ra{};
+        ra.partial[0] = g.partial;
+        ra.add[0] = nullptr;
+        ra.out[0] = out;
+        ra.n4[0] = (long)(M * N / 4);
+        ra.splits = g.splits;
+        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(ft_div_up(M * N / 4, 256), 1), dim3(256), 0, ctx->stream, ra);
+        FT_LAUNCH_CHECK();
+    }
+    return FT_OK;
+}
+
 int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, const float* a, const void* b,
                   float* out, size_t M, size_t K, size_t N, const float* a2, const float* b2, size_t K2,
                   const float* add = nullptr) {
@@ -2126,18 +2247,20 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     p.ldc = (long)N;
     p.lda2 = (long)K2;
     p.ldb2 = layout == 1 ? (long)K2 : (long)N;
-    if (K > 0 && async_eligible(layout, a, b, out, add, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0, !half_b)) {
+    if (half_b && K > 0 && async_eligible(layout, a, b, out, add, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0)) {
         AsyncBatch g{};
         g.count = 1;
         g.M = (int)M;
-        g.p[0].seg[0] = make_seg(layout, a, b, K, N, p.a2, p.b2, p.a2 ? K2 : 0, M);
+        g.p[0].seg[0] = make_seg(layout, a, b, K, N, p.a2, p.b2, p.a2 ? K2 : 0);
         g.p[0].nseg = 1;
         g.p[0].out = out;
         g.p[0].add = add;
         g.p[0].N = (int)N;
         g.p[0].ldc = (int)N;
-        return launch_async_auto(ctx, g, layout, !half_b);
+        return launch_async_auto(ctx, g, layout);
     }
+    if (!half_b && !p.a2 && !add && f32_async_eligible(layout, a, b, out, M, K, N))
+        return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N);
     // Tile choice for the register-staged kernels, from measurements on MI355X at
     // M = 2048: 128x128 tiles when there are many per CU, else 64x64; a deep K
     // loop on few tiles prefers BK = 64 (half the barriers per MFMA).
@@ -2273,7 +2396,6 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
                  "ft_lora_linear_group: 1..%d linears per call", kAsyncMaxProb);
     bool batch = M < (1u << 30) && K < (1u << 30) && M > 0;
     bool any_rope = false;
-    const bool f32b = linears[0].w_dtype == FT_DTYPE_F32;
     for (size_t i = 0; i < count; i++) {
         const ft_lora_linear_desc& d = linears[i];
         FT_CHECK_ARG(d.w_dtype == FT_DTYPE_F32 || d.w_dtype == FT_DTYPE_F16, "ft_lora_linear_group: dtype %d",
@@ -2285,8 +2407,8 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
             any_rope = true;
         }
         FT_CHECK_ARG(d.r == 0 || (d.t && d.b), "ft_lora_linear_group: linear %zu has a rank but no factors", i);
-        batch = batch && d.w_dtype == linears[0].w_dtype && d.N < (1u << 30) &&
-                async_eligible(0, x, d.w, d.y, d.residual, M, K, d.N, d.t, d.b, d.r, f32b);
+        batch = batch && d.w_dtype == FT_DTYPE_F16 && d.N < (1u << 30) &&
+                async_eligible(0, x, d.w, d.y, d.residual, M, K, d.N, d.t, d.b, d.r);
     }
     if (batch && count > 1) {
         AsyncBatch g{};
@@ -2303,8 +2425,8 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
             g.p[i].rope = reinterpret_cast<const float2*>(d.rope_table);
             g.p[i].rope_seq = (int)d.rope_seq;
         }
-        if (!any_rope) return launch_async_auto(ctx, g, 0, f32b);
-        return launch_async<64, 64, 32, 32>(ctx, g, 0, kEpiPlain, f32b);  // the rotation lives in the 64x64 epilogue
+        if (!any_rope) return launch_async_auto(ctx, g, 0);
+        return launch_async<64, 64, 32, 32>(ctx, g, 0);  // the rotation lives in the 64x64 epilogue
     }
     for (size_t i = 0; i < count; i++) {
         const ft_lora_linear_desc& d = linears[i];
@@ -2322,14 +2444,13 @@ int ft_lora_linear_dx_group(ft_context* ctx, const ft_lora_dx_desc* linears, siz
                  "ft_lora_linear_dx_group: 1..%d linears per call", kAsyncMaxSeg);
     bool batch = M < (1u << 30) && K < (1u << 30) && M > 0 && K > 0;
     size_t tiles = 0;
-    const bool f32b = linears[0].w_dtype == FT_DTYPE_F32;
     for (size_t i = 0; i < count; i++) {
         const ft_lora_dx_desc& d = linears[i];
         FT_CHECK_ARG(d.w_dtype == FT_DTYPE_F32 || d.w_dtype == FT_DTYPE_F16, "ft_lora_linear_dx_group: dtype %d",
                      d.w_dtype);
         FT_CHECK_ARG(d.r == 0 || (d.dt && d.a), "ft_lora_linear_dx_group: linear %zu has a rank but no factors", i);
-        batch = batch && d.w_dtype == linears[0].w_dtype && d.N < (1u << 30) &&
-                async_eligible(1, d.dy, d.w, dx, residual, M, d.N, K, d.dt, d.a, d.r, f32b);
+        batch = batch && d.w_dtype == FT_DTYPE_F16 && d.N < (1u << 30) &&
+                async_eligible(1, d.dy, d.w, dx, residual, M, d.N, K, d.dt, d.a, d.r);
         tiles += d.N / 32;
     }
     if (batch && count > 1 && tiles < (1u << 30)) {
@@ -2345,7 +2466,7 @@ int ft_lora_linear_dx_group(ft_context* ctx, const ft_lora_dx_desc* linears, siz
         g.p[0].add = residual;
         g.p[0].N = (int)K;
         g.p[0].ldc = (int)K;
-        return launch_async_auto(ctx, g, 1, f32b);
+        return launch_async_auto(ctx, g, 1);
     }
     for (size_t i = 0; i < count; i++) {
         const ft_lora_dx_desc& d = linears[i];
@@ -2360,10 +2481,9 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
     FT_CHECK_ARG(ctx && x && w_gate && w_up && gate && up && act, "ft_mlp_gate_up: NULL argument");
     FT_CHECK_ARG(w_dtype == FT_DTYPE_F32 || w_dtype == FT_DTYPE_F16, "ft_mlp_gate_up: dtype %d", w_dtype);
     if (M == 0 || N == 0) return FT_OK;
-    const bool f32b = w_dtype == FT_DTYPE_F32;
-    const bool fused = M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
-                       async_eligible(0, x, w_up, up, nullptr, M, K, N, nullptr, nullptr, 0, f32b) &&
-                       async_eligible(0, x, w_gate, gate, nullptr, M, K, N, nullptr, nullptr, 0, f32b) && aligned16p(act);
+    const bool fused = w_dtype == FT_DTYPE_F16 && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
+                       async_eligible(0, x, w_up, up, nullptr, M, K, N, nullptr, nullptr, 0) &&
+                       async_eligible(0, x, w_gate, gate, nullptr, M, K, N, nullptr, nullptr, 0) && aligned16p(act);
     if (fused) {
         AsyncBatch g{};
         g.count = 1;
@@ -2376,8 +2496,8 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
         g.p[0].out3 = act;
         g.p[0].N = (int)N;
         g.p[0].ldc = (int)N;
-        return !f32b && wide_tiles(ctx, M, N) ? launch_async<64, 128, 32, 64>(ctx, g, 0, kEpiGateUp)
-                                              : launch_async<64, 64, 32, 32>(ctx, g, 0, kEpiGateUp, f32b);
+        return wide_tiles(ctx, M, N) ? launch_async<64, 128, 32, 64>(ctx, g, 0, kEpiGateUp)
+                                     : launch_async<64, 64, 32, 32>(ctx, g, 0, kEpiGateUp);
     }
     FT_TRY(ft_lora_linear(ctx, x, w_up, w_dtype, nullptr, nullptr, nullptr, up, M, K, N, 0));
     FT_TRY(ft_lora_linear(ctx, x, w_gate, w_dtype, nullptr, nullptr, nullptr, gate, M, K, N, 0));
@@ -2390,9 +2510,8 @@ int ft_mlp_down_backward(ft_context* ctx, const float* dy, const void* w_down, i
     FT_CHECK_ARG(w_dtype == FT_DTYPE_F32 || w_dtype == FT_DTYPE_F16, "ft_mlp_down_backward: dtype %d", w_dtype);
     if (M == 0 || F == 0) return FT_OK;
     // d_act[M,F] = dy[M,H] @ w_down[F,H]^T: layout 1 with output width F, reduction H.
-    const bool f32b = w_dtype == FT_DTYPE_F32;
-    const bool fused = M < (1u << 30) && F < (1u << 30) && H < (1u << 30) &&
-                       async_eligible(1, dy, w_down, d_gate, nullptr, M, H, F, nullptr, nullptr, 0, f32b);
+    const bool fused = w_dtype == FT_DTYPE_F16 && M < (1u << 30) && F < (1u << 30) && H < (1u << 30) &&
+                       async_eligible(1, dy, w_down, d_gate, nullptr, M, H, F, nullptr, nullptr, 0);
     if (fused) {
         AsyncBatch g{};
         g.count = 1;
@@ -2405,8 +2524,8 @@ int ft_mlp_down_backward(ft_context* ctx, const float* dy, const void* w_down, i
         g.p[0].e2 = up;
         g.p[0].N = (int)F;
         g.p[0].ldc = (int)F;
-        return !f32b && wide_tiles(ctx, M, F) ? launch_async<64, 128, 32, 64>(ctx, g, 1, kEpiSiluBwd)
-                                              : launch_async<64, 64, 32, 32>(ctx, g, 1, kEpiSiluBwd, f32b);
+        return wide_tiles(ctx, M, F) ? launch_async<64, 128, 32, 64>(ctx, g, 1, kEpiSiluBwd)
+                                     : launch_async<64, 64, 32, 32>(ctx, g, 1, kEpiSiluBwd);
     }
     FT_CHECK_ARG(scratch, "ft_mlp_down_backward: this operand combination needs the [M,F] scratch buffer");
     FT_TRY(ft_lora_linear_dx(ctx, dy, w_down, w_dtype, nullptr, nullptr, nullptr, scratch, M, F, H, 0));

@@ -257,37 +257,13 @@ def test_f16_split_keeps_f32_accuracy_over_the_exponent_range(g, M, K, N, layout
     assert np.all(err <= bound), (np.argwhere(err > bound)[:5], np.max(err / bound))
 
 
-@pytest.mark.parametrize("M,K,N", [(256, 32, 64), (132, 288, 136), (600, 96, 320), (300, 2048, 964)])
-@pytest.mark.parametrize("layout", [0, 1, 2])
-def test_f32_split_keeps_f32_accuracy_over_the_exponent_range(g, M, K, N, layout):
-    """As above with both operands f32 and split (rows of a and columns of b over the exponent range): the dropped product
-    of the low halves adds 2^-22 sum|x||w| at most, a value far below its column's largest the second floor term. A result
-    among the subnormals is the sum of up to 16 partial sums (two k halves, eight shares) rounded to 2^-149 each: 16 * 2^-150."""
-    ctx, eng = g
-    x = split_rows(M + K + N, M, K)
-    w = np.ascontiguousarray(split_rows(N + K, N, K).T)
-    x /= np.maximum(np.abs(x).max(axis=1, keepdims=True) / np.float32(1e12), 1)   # (products and sums stay in the f32 range)
-    w /= np.maximum(np.abs(w).max(axis=0, keepdims=True) / np.float32(1e12), 1)
-    a = x if layout != 2 else np.ascontiguousarray(x.T)
-    b = w if layout != 1 else np.ascontiguousarray(w.T)
-    out = empty(ctx, M, N)
-    (eng.matmul, eng.matmul_bt, eng.matmul_at)[layout](ctx, up(ctx, a), up(ctx, b), out)
-    x64, w64 = x.astype(np.float64), w.astype(np.float64)
-    ax, aw = np.abs(x64), np.abs(w64)
-    bound = ((K / 8 + 8) * 2.0 ** -24 + 2.0 ** -22) * (ax @ aw) + 2.0 ** -36 * (
-        ax.max(axis=1, keepdims=True) * aw.sum(axis=0) + ax.sum(axis=1, keepdims=True) * aw.max(axis=0)) + \
-        2.0 ** -147 * (2 + aw.sum(axis=0) + ax.sum(axis=1, keepdims=True))
-    err = np.abs(out.to_numpy().reshape(M, N) - x64 @ w64)
-    assert np.all(err <= bound), (np.argwhere(err > bound)[:5], np.max(err / bound))
-
-
-@pytest.mark.parametrize("layout,f16", [(0, True), (1, True), (0, False), (1, False), (2, False)])
-def test_f16_split_products_of_infinities_and_nans(g, layout, f16):
+@pytest.mark.parametrize("layout", [0, 1])
+def test_f16_split_products_of_infinities_and_nans(g, layout):
     """An infinity or NaN among the operands gives what f32 arithmetic gives, in its row or column only; a sum past the
     f32 range is an infinity; values at the end of the range are kept."""
     from ferrotensor_amd import UnifiedTensor
     ctx, eng = g
-    M, K, N = 132, 256, 136
+    M, K, N = 130, 256, 136
     x, w = rnd(1, M, K), rnd(2, K, N, scale=0.05)
     x[3, 7] = np.inf
     x[40, 200] = -np.inf
@@ -297,18 +273,13 @@ def test_f16_split_products_of_infinities_and_nans(g, layout, f16):
     w[:, 17] = np.abs(w[:, 17]) + 1.0     # row 90 overflows in this column
     x[100, 31] = np.finfo(np.float32).max
     w[9, 77] = np.inf
-    stored = np.ascontiguousarray(w.T if layout == 1 else w)
+    stored = np.ascontiguousarray(w if layout == 0 else w.T)
+    w16 = UnifiedTensor.from_f32_as_f16(ctx, stored, list(stored.shape))
     out = empty(ctx, M, N)
-    if f16:
-        w16 = UnifiedTensor.from_f32_as_f16(ctx, stored, list(stored.shape))
-        (eng.matmul_f16b if layout == 0 else eng.matmul_bt_f16b)(ctx, up(ctx, x), w16, out)
-        w = cpu.round_f16(w).reshape(K, N)
-    else:
-        a = up(ctx, np.ascontiguousarray(x.T) if layout == 2 else x)
-        (eng.matmul, eng.matmul_bt, eng.matmul_at)[layout](ctx, a, up(ctx, stored), out)
+    (eng.matmul_f16b if layout == 0 else eng.matmul_bt_f16b)(ctx, up(ctx, x), w16, out)
     got = out.to_numpy().reshape(M, N)
     with np.errstate(all="ignore"):
-        want = x.astype(np.float64) @ w.astype(np.float64)
+        want = x.astype(np.float64) @ cpu.round_f16(w).astype(np.float64)
         want = np.where(np.isinf(want.astype(np.float32)), want * np.inf, want)  # past the largest f32
     sure = np.ones((M, N), bool)
     sure[90] = False                      # sums near the end of the range: an intermediate sum may overflow
