@@ -26,7 +26,6 @@
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
@@ -748,20 +747,12 @@ __device__ __forceinline__ float abs_max(float m, float a, float b) {
     return m;
 }
 
-// (Packed conversions of f32 results: v_fma_mixlo/mixhi_f16, which would scale, subtract and round in one instruction,
-// take 10 cycles a wave against 4 to 5 of each of these.)
 __device__ __forceinline__ void split8(const float4& x, const float4& y, float s, half8_t& hi, half8_t& lo) {
     const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-        const half2_t h = __builtin_convertvector(float2_t{v[e] * s, v[e + 1] * s}, half2_t);
-        const half2_t l = __builtin_convertvector(
-            float2_t{__builtin_fmaf(v[e], s, -(float)h.x), __builtin_fmaf(v[e + 1], s, -(float)h.y)}, half2_t);
-        hi[e] = h.x;
-        hi[e + 1] = h.y;
-        lo[e] = l.x;
-        lo[e + 1] = l.y;
-    }
+    for (int e = 0; e < 8; e++) hi[e] = (_Float16)__builtin_fmaf(v[e], s, 0.0f);
+#pragma unroll
+    for (int e = 0; e < 8; e++) lo[e] = (_Float16)__builtin_fmaf(v[e], s, -(float)hi[e]);
 }
 
 // Four f16 of one column from four k rows of a [k][n] tile in LDS: in each group of 16 lanes, lane 4 j + c gives
@@ -788,7 +779,7 @@ __host__ __device__ constexpr int b_swizzle(int k4) {
 // one of every stage for the same 64x64 output tile (the two sums meet in LDS after the loop):
 // twice the waves per SIMD for products whose tiles leave a CU with at most two workgroups.
 template <int BM, int BN, int WM, int WN, int LAYOUT, int NSEG, int EPI = kEpiPlain, int KW = 1>
-__global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 2) void gemm_async_kernel(AsyncBatch g) {
+__global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 2) void gemm_async_kernel(AsyncBatch g) {
     static_assert(LAYOUT == 0 || LAYOUT == 1, "a is k-contiguous on this path");
     static_assert(NSEG == 1 || NSEG == kAsyncMaxSeg, "one segment, or the general case");
     static_assert(EPI == kEpiPlain || NSEG == 1, "fused epilogues take one segment");
@@ -809,7 +800,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     constexpr int B_FLOATS = BN * 16;             // f16 tile, in float units
     constexpr int SUB = A_FLOATS + NB * B_FLOATS;  // one K tile of 32
     constexpr int STAGE = KW * SUB;
-    static_assert(KW == 1 || (KW == 2 && BM == 64), "K-sharing waves: tiles of 64 rows");
+    static_assert(KW == 1 || (KW == 2 && BM == 64 && BN == 64), "K-sharing waves: 64x64 tiles");
     constexpr int A_CH = BM / 8 / 4;              // 1 KiB chunks per wave
     constexpr int B_CH = BN / 16 / 4;
     constexpr int LPT = A_CH + NB * B_CH;         // load instructions per wave per tile
@@ -817,10 +808,9 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     using ExA = FastTile<BM, true, 16>;
     using ExB = FastTile<BN, LAYOUT == 1, 16>;
 
-    __shared__ __attribute__((aligned(16))) float St[NST * STAGE];
-    float* const St0 = St;
-    float* const St1 = St + STAGE;
-    float* const St2 = St + 2 * STAGE;
+    __shared__ __attribute__((aligned(16))) float St0[STAGE];
+    __shared__ __attribute__((aligned(16))) float St1[STAGE];
+    __shared__ __attribute__((aligned(16))) float St2[STAGE];
     // The rank-r products' operand tiles take the first stage's place once the K loop is over:
     // a stage set of their own would cost the 128x128 tile its second workgroup per CU.
     static_assert(ExA::LDS_FLOATS % 4 == 0 && ExA::LDS_FLOATS + ExB::LDS_FLOATS <= STAGE, "rank-r tiles fit a stage");
@@ -960,7 +950,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     if (pi != 0) p = pin_prob(g.p[pi], read_prob(g.p[pi]));
     const int m0 = tm * BM;
     const int n0 = (tn - p.tile_begin) * BN;
-    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64)) % 4;
+    const int lane = threadIdx.x % 64, wave = (threadIdx.x / 64) % 4;
     const int grp = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 256));  // wave-uniform
     const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
     const int l32 = lane % 32, half = lane / 32;
@@ -1035,7 +1025,6 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     }
     int seg_cur = 0;           // segment the offsets are formed for
     int seg_first = 0;         // its first tile
-    int seg_end = NSEG > 1 ? tend[0] : 1 << 30;
     const char* aseg = abase[0];
     const char* bseg = bbase[0];
     long b_step = LAYOUT == 1 ? 64L : 32L * ldb_b[0];  // bytes per K tile
@@ -1045,13 +1034,15 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
         t = KW * t + grp;         // this wave group's tile of the pair
         st += grp * SUB;
         if constexpr (NSEG > 1) {
-            while (t >= seg_end) {  // uniform, taken once per segment (t never goes back)
-                seg_cur++;
-                seg_first = seg_end;
-                seg_end = seg_cur < NSEG - 1 ? seg_pick<NSEG>(tend, seg_cur) : 1 << 30;
-                const int la = seg_pick<NSEG>(lda_b, seg_cur), lb = seg_pick<NSEG>(ldb_b, seg_cur);
-                aseg = seg_pick<NSEG>(abase, seg_cur);
-                bseg = seg_pick<NSEG>(bbase, seg_cur);
+            int s = 0;
+            if (t >= tend[0]) s = 1;
+            if (t >= tend[1]) s = 2;
+            if (s != seg_cur) {  // uniform, taken once per segment
+                seg_cur = s;
+                seg_first = s == 1 ? tend[0] : tend[1];
+                const int la = seg_pick<NSEG>(lda_b, s), lb = seg_pick<NSEG>(ldb_b, s);
+                aseg = seg_pick<NSEG>(abase, s);
+                bseg = seg_pick<NSEG>(bbase, s);
                 b_step = LAYOUT == 1 ? 64L : 32L * lb;
 #pragma unroll
                 for (int j = 0; j < A_CH; j++) offA[j] = rowA[j] * (unsigned)la + colA[j];
@@ -1072,10 +1063,10 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
             for (int j = 0; j < B_CH; j++) glds16(bt2, offB[j], st + A_FLOATS + B_FLOATS + (wave + 4 * j) * 256);
         }
     };
-    // A K tile's operands as this lane feeds them: k = 16 * S + 8 * half + 0..7 of its row (a: f32 as read, then
-    // its f16 halves) and its column (b, f16), S = k step.
+    // A K tile's operands as this lane feeds them: k = 16 * S + 8 * half + 0..7 of its row (a, f32) and its
+    // column (b, f16), S = k step.
     float4 raw[NS][2];
-    half8_t bfr[2][CB * NB][NS], hi[2][NS], lo[2][NS];
+    half8_t bfr[2][CB * NB][NS];
     RowScale rs;
     auto read_frags = [&](const float* st, half8_t (&bf)[CB * NB][NS]) {
         const int row = rm0 + l32;
@@ -1105,10 +1096,12 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
             }
         }
     };
-    // Sums of rows whose scale has changed, brought to the new scale: the lanes' ratios are handed to the
-    // accumulators' rows by shuffles. Rare: a scale changes at a row's first tile that is not all zeros and at a value
-    // more than eight times larger than any before.
-    auto rescale = [&](float ratio) {
+    // Row scales for a tile that holds a value too large for the present one (the first tile of a row that is
+    // not all zeros; a later tile with a value more than eight times larger than any before): rare, so the
+    // lanes' scales are brought to the accumulators' rows by shuffles.
+    auto rescale = [&](float mx, bool first) {
+        const float ratio = rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
+        if (first) return;  // the sums are still zero
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const float f = __shfl(ratio, (r / 4) * 8 + half * 4 + (r % 4));
@@ -1116,56 +1109,38 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
             for (int j = 0; j < CB * NB; j++) sum[j][r] *= f;
         }
     };
-    auto tile_max = [&]() {
+    // Tile t, whose operands are in `raw` and bfr[BUF]; `stage` is the one it came from, `next` holds tile t + 1.
+    // Split into f16 halves, then the wait for tile t + 1, the barrier, the refill of the stage and the reads of
+    // tile t + 1 in front of the MFMAs, whose run covers those reads.
+    auto iter = [&](int t, float* stage, const float* next, auto buf) {
+        constexpr int BUF = decltype(buf)::value;
         float mx = 0.0f;
 #pragma unroll
         for (int u = 0; u < NS; u++)
 #pragma unroll
             for (int q = 0; q < 2; q++) mx = abs_max(abs_max(mx, raw[u][q].x, raw[u][q].y), raw[u][q].z, raw[u][q].w);
-        return mx;
-    };
-    // MFMAs FIRST .. LAST - 1 of the 2 * NS * CB * NB of a tile whose halves are in buffer BUF.
-    auto mfmas = [&](auto buf, int first, int last) {
-        constexpr int BUF = decltype(buf)::value;
+        if (__builtin_amdgcn_ballot_w64(mx > rs.limit) != 0) rescale(mx, t == t0);
+        half8_t hi[NS], lo[NS];
 #pragma unroll
-        for (int e = 0; e < 2 * NS * CB * NB; e++) {
-            if (e < first || e >= last) continue;
-            const int u = e / (2 * CB * NB), low = (e / (CB * NB)) % 2 == 0, j = e % (CB * NB);
-            sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(low ? lo[BUF][u] : hi[BUF][u], bfr[BUF][j][u], sum[j], 0, 0, 0);
-        }
-    };
-    constexpr int EARLY = NS * CB * NB, ALL = 2 * EARLY;  // half of the MFMAs in front of the split of the next tile
-    // Tile t, whose operands are in hi, lo and bfr of buffer BUF; `stage` is the one it came from, `next` holds tile
-    // t + 1. Tile t + 1 is read while the first MFMAs of tile t run and split between the others: 16 to 32
-    // instructions that fit into the time the matrix pipe takes (with the split in front of all MFMAs the waves of a
-    // SIMD, which the barrier keeps in step, did it at the same time and left the pipe idle meanwhile).
-    auto iter = [&](int t, float* stage, const float* next, auto buf) {
-        constexpr int BUF = decltype(buf)::value;
-        constexpr std::integral_constant<int, BUF> here{};
-        // Tile t + 1 has landed (at most tile t + 2's loads in flight); after the barrier that holds for every
-        // wave, and every wave has read tile t, so its stage can take tile t + 3.
+        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[u], lo[u]);
+        // This wave's reads of the stage are complete (lgkmcnt 0) and tile t + 1 has landed (at
+        // most tile t + 2's loads in flight); after the barrier that holds for every wave, so
+        // the stage can take tile t + 3.
         __builtin_amdgcn_s_waitcnt(0x0070 | (WAIT & 15) | ((WAIT >> 4) << 14));
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         issue(t + NST, stage);
         read_frags(next + grp * SUB, bfr[BUF ^ 1]);
         __builtin_amdgcn_sched_barrier(0);
-        mfmas(here, 0, EARLY);
-        const float mx = tile_max();
-        const bool grown = __builtin_amdgcn_ballot_w64(mx > rs.limit) != 0;
-        float ratio = 1.0f;
-        if (grown) ratio = rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
-        mfmas(here, EARLY, ALL);  // (still under the old scales)
 #pragma unroll
-        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[BUF ^ 1][u], lo[BUF ^ 1][u]);
+        for (int u = 0; u < NS; u++) {
 #pragma unroll
-        for (int e = EARLY; e < ALL; e++) {
-            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                              // one MFMA,
-            __builtin_amdgcn_sched_group_barrier(0x2, (24 * NS + EARLY - 1) / EARLY, 0);  // its share of the split
+            for (int j = 0; j < CB * NB; j++)
+                sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[u], bfr[BUF][j][u], sum[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < CB * NB; j++)
+                sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[u], bfr[BUF][j][u], sum[j], 0, 0, 0);
         }
-#pragma unroll
-        for (int u = 0; u < NS; u++) asm volatile("" : "+v"(hi[BUF ^ 1][u]), "+v"(lo[BUF ^ 1][u]));  // split here, not at the use
-        if (grown) rescale(ratio);
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -1195,12 +1170,6 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     __builtin_amdgcn_sched_barrier(0);
     issue(t0 + 2, St2);
     read_frags(St0 + grp * SUB, bfr[0]);
-    {
-        const float mx = tile_max();
-        rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
-#pragma unroll
-        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[0][u], lo[0][u]);
-    }
     __builtin_amdgcn_sched_barrier(0);
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
@@ -1235,7 +1204,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
             const int t = KW * tp + grp;
             int s = 0;
             if constexpr (NSEG > 1) s = t >= tend[1] ? 2 : (t >= tend[0] ? 1 : 0);
-            const int tl = t - (NSEG > 1 && s > 0 ? (s == 1 ? tend[0] : tend[NSEG > 1 ? 1 : 0]) : 0);
+            const int tl = t - (NSEG > 1 && s > 0 ? (s == 1 ? tend[0] : tend[1]) : 0);
             const int la = seg_pick<NSEG>(lda_b, s), lb = seg_pick<NSEG>(ldb_b, s);
             const char* at = seg_pick<NSEG>(abase, s) + (long)tl * 128 + (long)(row < M ? row : M - 1) * la;
             const char* bt = seg_pick<NSEG>(bbase, s);
@@ -1266,8 +1235,8 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     // cos and sin): requested here, so that the exchange and the rank-r term run under their latency (in front of the
     // K loop they would hold 32 registers through it, which costs the SIMD its fourth wave).
     // Out-of-range elements read element 0 instead of branching around the load.
-    constexpr bool PRE = BM == 64 && ((BN == 64 && NSEG == 1 && EPI == kEpiPlain) || EPI == kEpiSiluBwd);
-    float2 pre[PRE ? FN : 1][PRE ? 16 : 1];  // plain: .x = residual, or (cos, sin); SiLU backward: (gate, up)
+    constexpr bool PRE = BM == 64 && BN == 64 && NSEG == 1 && (EPI == kEpiPlain || EPI == kEpiSiluBwd);
+    float2 pre[PRE ? 16 : 1];  // plain: .x = residual, or (cos, sin); SiLU backward: (gate, up)
     bool pre_add = false;
     if constexpr (PRE) {
         const GlobalF* s1 = EPI == kEpiSiluBwd ? p.e1 : p.add;
@@ -1282,19 +1251,16 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
                 if (pos >= p.rope_seq) pos -= p.rope_seq;
                 if (pos >= p.rope_seq) pos %= p.rope_seq;  // sequences shorter than a tile
                 const CosSin cs = p.rope[(long)pos * 32 + l32];
-                pre[0][r] = make_float2(cs.x, cs.y);
+                pre[r] = make_float2(cs.x, cs.y);
             }
         } else if (pre_add) {
+            const int col = n0 + wn0 + l32;
 #pragma unroll
-            for (int j = 0; j < FN; j++) {
-                const int col = n0 + wn0 + j * 32 + l32;
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int row = m0 + wm0 + (r / 4) * 8 + half * 4 + (r % 4);
-                    const long o = row < M && col < p.N ? (long)row * p.ldc + col : 0;
-                    pre[j][r].x = s1[o];
-                    if constexpr (EPI == kEpiSiluBwd) pre[j][r].y = p.e2[o];
-                }
+            for (int r = 0; r < 16; r++) {
+                const int row = m0 + wm0 + (r / 4) * 8 + half * 4 + (r % 4);
+                const long o = row < M && col < p.N ? (long)row * p.ldc + col : 0;
+                pre[r].x = s1[o];
+                if constexpr (EPI == kEpiSiluBwd) pre[r].y = p.e2[o];
             }
         }
     }
@@ -1308,10 +1274,10 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
         for (int j = 0; j < FN * NB; j++) acc[0][j] = sum[j];
     } else {
         // Two waves of a row block: each hands the other the sums of the columns that one finishes.
+        static_assert(KS == 1 || 2 * KW * FN * NB * 1024 <= STAGE, "the exchange fits the stages");
         constexpr int PER = FN * NB * 1024;  // floats a wave hands over
-        static_assert(4 * KW * PER <= (KW == 1 ? NST : 2) * STAGE, "the exchange fits the stages");
         const int slot = grp * 4 + wave;
-        auto place = [&](int sl) { return St + sl * PER + lane; };
+        auto place = [&](int sl) { return (KW == 2 ? (sl < 4 ? St0 : St1) + (sl & 3) * PER : (sl < 2 ? St0 : St1) + (sl & 1) * PER) + lane; };
         float* give = place(slot ^ 1);
         const float* take = place(slot);
 #pragma unroll
@@ -1342,7 +1308,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     };
     if constexpr (KW == 2) {
         // The second wave group hands its sums over through the third stage and retires.
-        static_assert(FN * NB * 16 * 256 <= STAGE, "the hand-over fits a stage");
+        static_assert(KW == 1 || FN * NB * 16 * 256 <= STAGE, "the hand-over fits a stage");
         float* red = St2 + wave * 64 + lane;
         if (grp == 1) {
 #pragma unroll
@@ -1395,7 +1361,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
                 if (row < M && col < p.N) {
                     float2 cs;
                     if constexpr (PRE) {
-                        cs = pre[0][r];
+                        cs = pre[r];
                     } else {
                         const CosSin t = p.rope[(long)(row % p.rope_seq) * 32 + l32];
                         cs = make_float2(t.x, t.y);
@@ -1435,7 +1401,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
     } else if constexpr (EPI == kEpiSiluBwd) {
         emit_all([&](int i, int j, int r, int row, int col) {
             const long o = (long)row * p.ldc + col;
-            const float d = acc[i][j][r], x = pre[j][r].x, y = pre[j][r].y;
+            const float d = acc[i][j][r], x = pre[r].x, y = pre[r].y;
             const float sg = 1.0f / (1.0f + __expf(-x));
             store_streaming(&p.out2[o], d * (x * sg));
             store_streaming(&p.out[o], d * y * (sg * (1.0f + x * (1.0f - sg))));
@@ -1448,7 +1414,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 && BN == 64 ? (EPI == kEpiGateUp
         emit_all([&](int i, int j, int r, int row, int col) { dst[(long)row * p.N + col] = acc[i][j][r]; });
     } else if (PRE && pre_add) {
         emit_all([&](int i, int j, int r, int row, int col) {
-            store_streaming(&p.out[(long)row * p.ldc + col], acc[i][j][r] + pre[PRE ? j : 0][PRE ? r : 0].x);
+            store_streaming(&p.out[(long)row * p.ldc + col], acc[i][j][r] + pre[PRE ? r : 0].x);
         });
     } else if (p.add) {
         emit_all([&](int i, int j, int r, int row, int col) {
@@ -1831,7 +1797,7 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
     bool pairs = false;
     g.tail_first = tiles;
     g.tail_shift = 0;
-    if (BM == 64 && BN == 64 && epi == kEpiPlain && tiles > ctx->num_cus && !long_k) {
+    if (BM == 64 && epi == kEpiPlain && tiles > ctx->num_cus && !long_k) {
         // A remainder over the CUs of at most a quarter of them (288 tiles: the 576-column products of the 135M
         // shape; 800: q/k/v at 360M): its tiles (the last of the order) must be plain ones (no RoPE epilogue,
         // whole float4 groups).
@@ -1885,7 +1851,7 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
         // ceil(288 w / 256) of them, 2, 3, 4 for w = 1, 2, 3, i.e. 2, 1.5, 1.33 tiles' worth; measured,
         // three shares beat two (and four) in the 135M-shaped step. (Only where the tail split above does not
         // apply: it leaves a CU with one whole tile and an eighth, 15.3 -> 14.9 ms per 135M step.)
-        if (BN == 64 && tiles > ctx->num_cus) want = 3;
+        if (BM == 64 && tiles > ctx->num_cus) want = 3;
         // 128x128 tiles hold two workgroups on a CU: the shares must fit one round of them
         if (BM == 128) want = (int)(2 * (size_t)ctx->num_cus / tiles);
         if (want > 8) want = 8;
@@ -1918,7 +1884,7 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
     if (defer) *defer = ft_deferred_sum{};
     auto reduce_shares = [&]() -> int {
         if (g.tail_shift > 0) {
-            if (defer && g.count == 1 && epi == kEpiPlain && g.p[0].ldc == g.p[0].N) {
+            if (defer && BM == 64 && g.count == 1 && epi == kEpiPlain && g.p[0].ldc == g.p[0].N) {
                 defer->partial = g.partial;
                 defer->add = g.p[0].add;
                 defer->out = g.p[0].out;
@@ -1959,32 +1925,32 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
     };
     char name[96];
     if (epi != kEpiPlain) {
-        // both fused forms: one product, one segment, tiles of 64 rows
+        // both fused forms: one product, one segment, 64x64 tiles (the only instantiation)
         if constexpr (BM == 64) {
             const bool gu = epi == kEpiGateUp;
-            snprintf(name, sizeof(name), "gemm_async_kernel<%d, %d, %d, %d, %d, 1, %s>", BM, BN, WM, WN, layout,
+            snprintf(name, sizeof(name), "gemm_async_kernel<64, 64, 32, 32, %d, 1, %s>", layout,
                      gu ? "gate_up" : "silu_bwd");
             const double mn = (double)g.M * g.p[0].N;
             ft_prof_scope prof(ctx, name, gu ? 2.0 * flops : flops,
                                gu ? bytes + 64.0 * g.p[0].N * g.p[0].seg[0].nt + 8.0 * mn : bytes + 12.0 * mn);
             // Fewer tiles than CUs (one sequence per pass): eight waves share the K loop of a tile.
             const bool few = (size_t)tiles <= (size_t)ctx->num_cus && g.p[0].seg[0].nt % 2 == 0 && g.p[0].seg[0].nt >= 8;
-            if (gu && few && BN == 64)
+            if (gu && few)
                 hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 0, 1, kEpiGateUp, 2>), grid, dim3(512), 0,
                                    ctx->stream, g);
             else if (gu)
-                hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 0, 1, kEpiGateUp>), grid, dim3(256), 0,
+                hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 0, 1, kEpiGateUp>), grid, dim3(256), 0,
                                    ctx->stream, g);
-            else if (few && BN == 64)
+            else if (few)
                 hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 1, 1, kEpiSiluBwd, 2>), grid, dim3(512), 0,
                                    ctx->stream, g);
             else
-                hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 1, 1, kEpiSiluBwd>), grid, dim3(256), 0,
+                hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 1, 1, kEpiSiluBwd>), grid, dim3(256), 0,
                                    ctx->stream, g);
             FT_LAUNCH_CHECK();
             return FT_OK;
         } else {
-            return ft_set_error(FT_ERR_INVALID, "fused epilogues use tiles of 64 rows");
+            return ft_set_error(FT_ERR_INVALID, "fused epilogues use 64x64 tiles");
         }
     }
     // Eight waves on a tile when the tiles alone leave at most two workgroups on a CU and the K
@@ -1997,17 +1963,17 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
             ft_prof_scope prof(ctx, name, flops, bytes);
             if (max_seg == 1) {
                 if (layout == 0)
-                    hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 0, 1, kEpiPlain, 2>), grid, dim3(512), 0,
+                    hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 0, 1, kEpiPlain, 2>), grid, dim3(512), 0,
                                        ctx->stream, g);
                 else
-                    hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 1, 1, kEpiPlain, 2>), grid, dim3(512), 0,
+                    hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 1, 1, kEpiPlain, 2>), grid, dim3(512), 0,
                                        ctx->stream, g);
             } else {
                 if (layout == 0)
-                    hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 0, kAsyncMaxSeg, kEpiPlain, 2>), grid,
+                    hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 0, kAsyncMaxSeg, kEpiPlain, 2>), grid,
                                        dim3(512), 0, ctx->stream, g);
                 else
-                    hipLaunchKernelGGL((gemm_async_kernel<BM, BN, WM, WN, 1, kAsyncMaxSeg, kEpiPlain, 2>), grid,
+                    hipLaunchKernelGGL((gemm_async_kernel<64, 64, 32, 32, 1, kAsyncMaxSeg, kEpiPlain, 2>), grid,
                                        dim3(512), 0, ctx->stream, g);
             }
             FT_LAUNCH_CHECK();
@@ -2035,16 +2001,10 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
 }
 
 // Tile choice, from measurements of the whole step on MI355X at M = 2048: 128x128
-// tiles (32x128 per wave) reach the highest MFMA rate but only pay off when there
-// are many of them per CU (the vocabulary head); the rest runs as 64x128 or
-// 64x64 tiles, up to four workgroups of the latter resident per CU.
-// The fused MLP halves take 64x128 tiles with at least four of them per CU (as 8192 x 2048 x 2048: 201 -> 167 us). At
-// 2048 x 2560 (640 tiles, two and a half per CU) they lose what the wider tile gains to the thin last round: gate and
-// up 52.8 -> 55.2 us, SiLU backward 49.2 -> 51.9.
-bool wide_tiles(const ft_context* ctx, size_t M, size_t N) {
-    return N >= 512 && ((M + 63) / 64) * ((N + 127) / 128) >= 4 * (size_t)ctx->num_cus;
-}
-
+// tiles (64x64 per wave) reach the highest MFMA rate but only pay off when there
+// are many of them per CU (the vocabulary head); everything else runs best as
+// 64x64 tiles, four workgroups resident per CU (three with two b tiles per stage; 128x64
+// and 64x128 tiles were measured too: no gain inside the step).
 int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout) {
     size_t tiles128 = 0;
     for (int i = 0; i < g.count; i++) tiles128 += (size_t)((g.M + 127) / 128) * (size_t)((g.p[i].N + 127) / 128);
@@ -2062,19 +2022,6 @@ int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout) {
     }
     if (plain && min_kt >= 512 && tiles128 * 2 <= 2 * (size_t)ctx->num_cus && tiles128 * 8 >= 2 * (size_t)ctx->num_cus)
         return launch_async<128, 128, 32, 128>(ctx, g, layout);
-    size_t tiles = 0;
-    bool rope = false, wide = true;
-    for (int i = 0; i < g.count; i++) {
-        tiles += (size_t)((g.M + 63) / 64) * (size_t)((g.p[i].N + 127) / 128);
-        rope = rope || g.p[i].rope != nullptr;
-        wide = wide && (g.p[i].N % 128 == 0 || g.p[i].N >= 512);
-    }
-    // 64x128 tiles with two of them per CU (2048 x 960 x 2560 41 -> 34 us, 8192 x 2048 x 2048 201 -> 167: a value of a is
-    // read and split for twice the columns), or with a long K over 129 to 256 of them (two K shares per tile: 70 -> 61 us
-    // at 2048 x 5120 x 960; at K = 2560 the partial tiles cost what the tile gains, 38.4 against 38.6, at 960 16.1 -> 25.9).
-    const size_t cus = (size_t)ctx->num_cus;
-    if (!rope && wide && (tiles >= 2 * cus || (plain && min_kt >= 100 && tiles <= cus && tiles * 2 > cus)))
-        return launch_async<64, 128, 32, 64>(ctx, g, layout);
     return launch_async<64, 64, 32, 32>(ctx, g, layout);
 }
 
@@ -2496,8 +2443,7 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
         g.p[0].out3 = act;
         g.p[0].N = (int)N;
         g.p[0].ldc = (int)N;
-        return wide_tiles(ctx, M, N) ? launch_async<64, 128, 32, 64>(ctx, g, 0, kEpiGateUp)
-                                     : launch_async<64, 64, 32, 32>(ctx, g, 0, kEpiGateUp);
+        return launch_async<64, 64, 32, 32>(ctx, g, 0, kEpiGateUp);
     }
     FT_TRY(ft_lora_linear(ctx, x, w_up, w_dtype, nullptr, nullptr, nullptr, up, M, K, N, 0));
     FT_TRY(ft_lora_linear(ctx, x, w_gate, w_dtype, nullptr, nullptr, nullptr, gate, M, K, N, 0));
@@ -2524,8 +2470,7 @@ int ft_mlp_down_backward(ft_context* ctx, const float* dy, const void* w_down, i
         g.p[0].e2 = up;
         g.p[0].N = (int)F;
         g.p[0].ldc = (int)F;
-        return wide_tiles(ctx, M, F) ? launch_async<64, 128, 32, 64>(ctx, g, 1, kEpiSiluBwd)
-                                     : launch_async<64, 64, 32, 32>(ctx, g, 1, kEpiSiluBwd);
+        return launch_async<64, 64, 32, 32>(ctx, g, 1, kEpiSiluBwd);
     }
     FT_CHECK_ARG(scratch, "ft_mlp_down_backward: this operand combination needs the [M,F] scratch buffer");
     FT_TRY(ft_lora_linear_dx(ctx, dy, w_down, w_dtype, nullptr, nullptr, nullptr, scratch, M, F, H, 0));
