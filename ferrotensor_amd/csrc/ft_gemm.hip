@@ -1,5 +1,4 @@
-// f32 matrix products on the gfx950 matrix cores: v_mfma_f32_32x32x16_f16 on operands split into f16 halves
-// (gemm_async_kernel, the f16-weight products), v_mfma_f32_32x32x2_f32 elsewhere.
+// f32 matrix products on the gfx950 matrix cores (v_mfma_f32_32x32x2_f32).
 //
 // gemm_kernel: out[M,N] = op(a) @ op(b) (+ a2[M,K2] @ op(b2)) for the three
 // layouts of the reference's tile kernel (a@b, a@b^T, a^T@b), with b stored as
@@ -21,13 +20,11 @@
 #include "ft_thin.h"
 
 #include <cmath>
-#include <type_traits>
 
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
 constexpr int BK = 32;
 constexpr int KQ = BK / 4;
@@ -533,12 +530,8 @@ __global__ __launch_bounds__(256) void gemm_fast_kernel(GemmArgs p) {
 //            runs at the rate of a linear read (c ^ (r & 7) takes twice as long).
 //   b tile   layout 1 (b[N,K]): [BN rows][32 k] f16, 64 B per row, 16 rows per
 //            instruction, 16-byte column c holds k-octet c ^ ((r >> 2) & 3) (likewise measured).
-//            layout 0 (b[K,N]): [32 k][BN n] f16 as in memory, columns swizzled (b_swizzle), read
-//            transposed (ds_read_b64_tr_b16: a lane receives four k of its column).
-// The products run on v_mfma_f32_32x32x16_f16 with every f32 of `a` split into two f16 numbers (RowScale below).
-// Measured against the same pipeline with v_mfma_f32_32x32x2_f32, M = 2048: 960x960 (o projection) 39.8 -> 18.5 us,
-// 960x1600 (q/k/v) 66.8 -> 29.1, gate and up 960x2560 each 160 -> 56, its input gradient K = 5120 170 -> 70,
-// the head 1446x960x49152 1058 -> 340 us (402 TFLOP/s); relative error against f64 at K = 960 5.4e-7 -> 2.8e-7.
+//            layout 0 (b[K,N]): [32 k][BN n] f16 exactly as in memory; a lane
+//            reads its column's 4 k values as four 16-bit loads.
 // The K loop is unrolled over the stages; the waits are explicit (s_waitcnt
 // vmcnt(n) + s_barrier, not __syncthreads, whose fence would drain every
 // outstanding load).
@@ -718,68 +711,11 @@ __device__ __forceinline__ T pinned(T v) {
     return ft_pinned(v);
 }
 
-// f32 operands on the f16 matrix instructions. A value x of a row with the power-of-two scale s is x * s =
-// hi + lo, two f16 numbers rounded to nearest: 22 to 24 significant bits, and at the row's largest value
-// scaled to 2^11 .. 2^15 everything below it keeps an absolute error of 2^-25 / 2^11 of that value or less.
-// b is f16 already, so a @ b = (hi @ b + lo @ b) / s, two v_mfma_f32_32x32x16_f16 with f32 sums in place of
-// eight v_mfma_f32_32x32x2_f32 at a sixteenth of the rate. The instruction adds 16 products at a time, so a
-// sum over K is rounded K / 8 times instead of K / 2.
-struct RowScale {
-    float scale = 1.0f;
-    float limit = 0.0f;  // largest |x| that this scale takes (f16 ends at 65504)
-    int exponent = 0;    // scale = 2^exponent
-    // Takes in the row's largest |x|; returns new scale / old scale.
-    __device__ __forceinline__ float grow(float m) {
-        if (!(m > limit)) return 1.0f;
-        const unsigned bits = __float_as_uint(m);
-        int e = 138 - (int)((bits < 0x7f7fffffu ? bits : 0x7f7fffffu) >> 23);  // m * 2^e in [2^11, 2^12)
-        e = e < 127 ? e : 127;
-        const float ratio = __builtin_amdgcn_ldexpf(1.0f, e - exponent);
-        exponent = e;
-        scale = __builtin_amdgcn_ldexpf(1.0f, e);
-        limit = __builtin_amdgcn_ldexpf(1.0f, 15 - e < 127 ? 15 - e : 127);
-        return ratio;
-    }
-};
-
-__device__ __forceinline__ float abs_max(float m, float a, float b) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));  // (fmaxf quiets its operands first: an instruction each)
-    return m;
-}
-
-__device__ __forceinline__ void split8(const float4& x, const float4& y, float s, half8_t& hi, half8_t& lo) {
-    const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
-#pragma unroll
-    for (int e = 0; e < 8; e++) hi[e] = (_Float16)__builtin_fmaf(v[e], s, 0.0f);
-#pragma unroll
-    for (int e = 0; e < 8; e++) lo[e] = (_Float16)__builtin_fmaf(v[e], s, -(float)hi[e]);
-}
-
-// Four f16 of one column from four k rows of a [k][n] tile in LDS: in each group of 16 lanes, lane 4 j + c gives
-// the address of row j, columns 4 c .. 4 c + 3, and lane i receives column i of rows 0 .. 3.
-__device__ __forceinline__ half4_t lds_read_tr(const char* q) {
-    typedef __fp16 v4 __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) v4*)q));
-}
-
-// LDS accesses of this wave complete, then the workgroup's barrier: __syncthreads without its wait for loads from
-// global memory, which may stay in flight here.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// 16-byte column c of row k of a [32 k][BN n] f16 tile holds columns 8 (c ^ b_swizzle(k % 4)): the four rows that half
-// a wave reads at once (64 bytes each) then lie in different banks.
-template <int BN>
-__host__ __device__ constexpr int b_swizzle(int k4) {
-    return BN == 64 ? 4 * (k4 >> 1) : 4 * k4;
-}
-
 // KW = 2: eight waves; a stage holds two consecutive K tiles and waves 4-7 multiply the second
 // one of every stage for the same 64x64 output tile (the two sums meet in LDS after the loop):
 // twice the waves per SIMD for products whose tiles leave a CU with at most two workgroups.
 template <int BM, int BN, int WM, int WN, int LAYOUT, int NSEG, int EPI = kEpiPlain, int KW = 1>
-__global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 2) void gemm_async_kernel(AsyncBatch g) {
+__global__ __launch_bounds__(256 * KW) void gemm_async_kernel(AsyncBatch g) {
     static_assert(LAYOUT == 0 || LAYOUT == 1, "a is k-contiguous on this path");
     static_assert(NSEG == 1 || NSEG == kAsyncMaxSeg, "one segment, or the general case");
     static_assert(EPI == kEpiPlain || NSEG == 1, "fused epilogues take one segment");
@@ -788,14 +724,6 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
     constexpr int FM = WM / 32, FN = WN / 32;
     constexpr int WAVES_N = BN / WN;
     static_assert((BM / WM) * (BN / WN) == 4, "4 waves per workgroup");
-    // In the K loop a wave owns 32 rows and all columns of the tile, so that a value of a is split into its f16
-    // halves by one wave only (two waves with half the columns each would both do it, and read it twice). With 64
-    // rows that leaves two waves a row block: each takes 16 of a K tile's 32 k, and they exchange sums after the loop
-    // for the WM x WN block each of them writes.
-    constexpr int KS = 4 * 32 / BM;     // waves that share a row block
-    constexpr int NS = 2 / KS;          // MFMA k steps (16) of a K tile per wave
-    constexpr int CB = BN / 32;         // column blocks of a wave in the loop
-    static_assert(FM == 1 && FN == CB / KS && (KS == 1 || KS == 2), "a wave's block after the exchange");
     constexpr int A_FLOATS = BM * 32;             // f32 tile
     constexpr int B_FLOATS = BN * 16;             // f16 tile, in float units
     constexpr int SUB = A_FLOATS + NB * B_FLOATS;  // one K tile of 32
@@ -955,12 +883,13 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
     const int wm0 = (wave / WAVES_N) * WM, wn0 = (wave % WAVES_N) * WN;
     const int l32 = lane % 32, half = lane / 32;
 
-    const int rm0 = (wave / KS) * 32, ks = KS == 1 ? 0 : wave % KS;  // loop: row block and share of the k steps
-    floatx16 sum[CB * NB];  // loop: column block j % CB of b matrix j / CB
+    floatx16 acc[FM][FN * NB];
 #pragma unroll
-    for (int j = 0; j < CB * NB; j++)
+    for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) sum[j][r] = 0.0f;
+        for (int j = 0; j < FN * NB; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
 
     // Uniform description of the segments (a missing one repeats the last: never reached).
     const char* abase[NSEG];
@@ -1016,7 +945,7 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
         } else {
             constexpr int LPR = BN / 8, RPC = 64 / LPR;
             const int kr = lane / LPR, cs = lane % LPR;
-            int col = n0 + (cs ^ b_swizzle<BN>((c * RPC + kr) & 3)) * 8;
+            int col = n0 + cs * 8;
             col = col + 8 <= p.N ? col : p.N - 8;
             rowB[j] = (unsigned)(c * RPC + kr);
             colB[j] = (unsigned)(col * 2);
@@ -1063,66 +992,55 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
             for (int j = 0; j < B_CH; j++) glds16(bt2, offB[j], st + A_FLOATS + B_FLOATS + (wave + 4 * j) * 256);
         }
     };
-    // A K tile's operands as this lane feeds them: k = 16 * S + 8 * half + 0..7 of its row (a, f32) and its
-    // column (b, f16), S = k step.
-    float4 raw[NS][2];
-    half8_t bfr[2][CB * NB][NS];
-    RowScale rs;
-    auto read_frags = [&](const float* st, half8_t (&bf)[CB * NB][NS]) {
-        const int row = rm0 + l32;
-#pragma unroll
-        for (int u = 0; u < NS; u++)
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const int kq = 4 * (u + ks) + 2 * half + q;
-                raw[u][q] = *reinterpret_cast<const float4*>(st + row * 32 + ((kq ^ ((row >> 1) & 7)) * 4));
-            }
-#pragma unroll
-        for (int j = 0; j < CB * NB; j++) {
-            const char* bs = reinterpret_cast<const char*>(st + A_FLOATS + (j / CB) * B_FLOATS);
-            const int nw = (j % CB) * 32;
-#pragma unroll
-            for (int u = 0; u < NS; u++) {
-                const int S = u + ks;
-                if constexpr (LAYOUT == 1) {
-                    const int n = nw + l32, col = (2 * S + half) ^ ((n >> 2) & 3);
-                    bf[j][u] = *reinterpret_cast<const half8_t*>(bs + n * 64 + col * 16);
-                } else {
-                    // Transposed reads: 16 lanes fetch 4 k rows of 16 columns, a lane receives 4 k of one column.
-                    const int kr = (lane % 16) / 4, n = nw + (l32 & 16) + (lane % 4) * 4;
-                    const char* q = bs + ((16 * S + 8 * half + kr) * BN + ((n >> 3) ^ b_swizzle<BN>(kr)) * 8 + (n & 7)) * 2;
-                    bf[j][u] = __builtin_shufflevector(lds_read_tr(q), lds_read_tr(q + 4 * BN * 2), 0, 1, 2, 3, 4, 5, 6, 7);
-                }
-            }
+    auto a_frag = [&](const float* st, int s, int row) -> float4 {
+        const int kq = 2 * s + half;
+        return *reinterpret_cast<const float4*>(st + row * 32 + ((kq ^ ((row >> 1) & 7)) * 4));
+    };
+    auto b_frag = [&](const float* st, int s, int n, int jb) -> float4 {
+        const char* bs = reinterpret_cast<const char*>(st + A_FLOATS + jb * B_FLOATS);
+        if constexpr (LAYOUT == 1) {
+            const int kq = 2 * s + half;
+            const int col = (kq >> 1) ^ ((n >> 2) & 3);
+            const half4_t h = *reinterpret_cast<const half4_t*>(bs + n * 64 + col * 16 + (kq & 1) * 8);
+            return make_float4((float)h.x, (float)h.y, (float)h.z, (float)h.w);
+        } else {
+            const _Float16* q = reinterpret_cast<const _Float16*>(bs) + (8 * s + 4 * half) * BN + n;
+            return make_float4((float)q[0], (float)q[BN], (float)q[2 * BN], (float)q[3 * BN]);
         }
     };
-    // Row scales for a tile that holds a value too large for the present one (the first tile of a row that is
-    // not all zeros; a later tile with a value more than eight times larger than any before): rare, so the
-    // lanes' scales are brought to the accumulators' rows by shuffles.
-    auto rescale = [&](float mx, bool first) {
-        const float ratio = rs.grow(fmaxf(mx, __shfl_xor(mx, 32)));
-        if (first) return;  // the sums are still zero
+    auto mfma_step = [&](const float4 (&af)[FM], const float4 (&bf)[FN * NB]) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float f = __shfl(ratio, (r / 4) * 8 + half * 4 + (r % 4));
+        for (int i = 0; i < FM; i++)
 #pragma unroll
-            for (int j = 0; j < CB * NB; j++) sum[j][r] *= f;
-        }
+            for (int j = 0; j < FN * NB; j++) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].x, bf[j].x, acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].y, bf[j].y, acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].z, bf[j].z, acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].w, bf[j].w, acc[i][j], 0, 0, 0);
+            }
     };
-    // Tile t, whose operands are in `raw` and bfr[BUF]; `stage` is the one it came from, `next` holds tile t + 1.
-    // Split into f16 halves, then the wait for tile t + 1, the barrier, the refill of the stage and the reads of
-    // tile t + 1 in front of the MFMAs, whose run covers those reads.
-    auto iter = [&](int t, float* stage, const float* next, auto buf) {
-        constexpr int BUF = decltype(buf)::value;
-        float mx = 0.0f;
+    // The K loop, rotated by three quarters of a tile: the wait for tile t + 1, the barrier, the
+    // refill of the stage tile t has just left and the first fragment reads of tile t + 1 all sit
+    // in front of the LAST group of MFMAs of tile t, so a wave comes out of the barrier with 4 MFMAs
+    // still to issue while its first reads of the new tile are in flight (with the barrier at the
+    // top of a tile every wave of the workgroup met that LDS latency at the same moment).
+    float4 af[2][FM], bf[2][FN * NB];
+    auto read_frags = [&](const float* cur, int s, int buf) {
 #pragma unroll
-        for (int u = 0; u < NS; u++)
+        for (int i = 0; i < FM; i++) af[buf][i] = a_frag(cur, s, wm0 + i * 32 + l32);
 #pragma unroll
-            for (int q = 0; q < 2; q++) mx = abs_max(abs_max(mx, raw[u][q].x, raw[u][q].y), raw[u][q].z, raw[u][q].w);
-        if (__builtin_amdgcn_ballot_w64(mx > rs.limit) != 0) rescale(mx, t == t0);
-        half8_t hi[NS], lo[NS];
+        for (int j = 0; j < FN * NB; j++) bf[buf][j] = b_frag(cur, s, wn0 + (j % FN) * 32 + l32, j / FN);
+    };
+    // Tile t: `stage` holds it, `next` holds tile t + 1; fragments of its first k-quads are in af[0] / bf[0].
+    auto iter = [&](int t, float* stage, const float* next) {
+        const float* cur = stage + grp * SUB;
 #pragma unroll
-        for (int u = 0; u < NS; u++) split8(raw[u][0], raw[u][1], rs.scale, hi[u], lo[u]);
+        for (int s = 0; s < 3; s++) {
+            read_frags(cur, s + 1, (s + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma_step(af[s & 1], bf[s & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // This wave's reads of the stage are complete (lgkmcnt 0) and tile t + 1 has landed (at
         // most tile t + 2's loads in flight); after the barrier that holds for every wave, so
         // the stage can take tile t + 3.
@@ -1130,110 +1048,19 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         issue(t + NST, stage);
-        read_frags(next + grp * SUB, bfr[BUF ^ 1]);
+        read_frags(next + grp * SUB, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < NS; u++) {
-#pragma unroll
-            for (int j = 0; j < CB * NB; j++)
-                sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo[u], bfr[BUF][j][u], sum[j], 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < CB * NB; j++)
-                sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi[u], bfr[BUF][j][u], sum[j], 0, 0, 0);
-        }
+        mfma_step(af[1], bf[1]);
         __builtin_amdgcn_sched_barrier(0);
     };
 
     // Prologue: tiles t0 .. t0+2 requested, the first one landed, its first fragments read.
     issue(t0, St0);
     issue(t0 + 1, St1);
-    // The rank-r products' operands: ordinary loads, consumed last (with several segments requested after the loop,
-    // for the registers).
-    ExA xa[NSEG];
-    ExB xb[NSEG];
-    auto load_ext = [&]() {
-#pragma unroll
-        for (int s = 0; s < NSEG; s++) {
-            if (has_ext[s]) {
-                const AsyncSeg& sg = p.seg[s];
-                xa[s].set_offsets(sg.lda2, m0, M, 4);
-                xb[s].set_offsets(sg.ldb2, n0, p.N, 4);
-                xa[s].template load<float, true>(reinterpret_cast<const char*>(sg.a2), 0, sg.K2);
-                xb[s].template load<float, true>(reinterpret_cast<const char*>(sg.b2), 0, sg.K2);
-            }
-        }
-    };
-    if constexpr (NSEG == 1) load_ext();
-
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (WAIT & 15) | ((WAIT >> 4) << 14));
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    issue(t0 + 2, St2);
-    read_frags(St0 + grp * SUB, bfr[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    constexpr std::integral_constant<int, 0> even{};
-    constexpr std::integral_constant<int, 1> odd{};
-    for (int t = t0; t < nt; t += 2 * NST) {
-        iter(t, St0, St1, even);
-        if (t + 1 < nt) iter(t + 1, St1, St2, odd);
-        if (t + 2 < nt) iter(t + 2, St2, St0, even);
-        if (t + 3 < nt) iter(t + 3, St0, St1, odd);
-        if (t + 4 < nt) iter(t + 4, St1, St2, even);
-        if (t + 5 < nt) iter(t + 5, St2, St0, odd);
-    }
-
-    // Back to the operands' own scale; then a sum that is not finite (an infinity or a NaN among the operands,
-    // or a sum past the f32 range) is formed again in f32 arithmetic, which says which of them it is.
-    float probe = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int e = __shfl(rs.exponent, (r / 4) * 8 + half * 4 + (r % 4));
-#pragma unroll
-        for (int j = 0; j < CB * NB; j++) {
-            sum[j][r] = __builtin_amdgcn_ldexpf(sum[j][r], -e);
-            probe = fmaf(sum[j][r], 0.0f, probe);
-        }
-    }
-    if (__builtin_amdgcn_ballot_w64(probe != 0.0f) != 0) {  // (NaN compares unequal)
-#pragma unroll
-        for (int j = 0; j < CB * NB; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) sum[j][r] = 0.0f;
-        const int row = m0 + rm0 + l32;
-        for (int tp = t0; tp < nt; tp++) {
-            const int t = KW * tp + grp;
-            int s = 0;
-            if constexpr (NSEG > 1) s = t >= tend[1] ? 2 : (t >= tend[0] ? 1 : 0);
-            const int tl = t - (NSEG > 1 && s > 0 ? (s == 1 ? tend[0] : tend[1]) : 0);
-            const int la = seg_pick<NSEG>(lda_b, s), lb = seg_pick<NSEG>(ldb_b, s);
-            const char* at = seg_pick<NSEG>(abase, s) + (long)tl * 128 + (long)(row < M ? row : M - 1) * la;
-            const char* bt = seg_pick<NSEG>(bbase, s);
-#pragma unroll 1
-            for (int q = 2 * ks; q < 2 * (ks + NS); q++) {
-                const int kq = 8 * q + 4 * half;
-                const float4 af = *reinterpret_cast<const float4*>(at + kq * 4);
-#pragma unroll
-                for (int j = 0; j < CB * NB; j++) {
-                    int n = n0 + (j % CB) * 32 + l32;
-                    n = n < p.N ? n : p.N - 1;
-                    const long k = 32L * tl + kq, step = LAYOUT == 1 ? 2 : lb;
-                    const char* bb = (j < CB ? bt : balt) + (LAYOUT == 1 ? (long)n * lb + k * 2 : k * lb + n * 2);
-                    auto at_k = [&](int e) { return (float)*reinterpret_cast<const _Float16*>(bb + e * step); };
-                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.x, at_k(0), sum[j], 0, 0, 0);
-                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.y, at_k(1), sum[j], 0, 0, 0);
-                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.z, at_k(2), sum[j], 0, 0, 0);
-                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af.w, at_k(3), sum[j], 0, 0, 0);
-                }
-            }
-        }
-    }
-
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    lds_barrier();  // every wave's loads have landed and every wave has left the last stage: the stages are free
-
-    // Epilogue operands (the residual of `out = a@b + add`, gate and up of the SiLU-gate backward, the rotation's
-    // cos and sin): requested here, so that the exchange and the rank-r term run under their latency (in front of the
-    // K loop they would hold 32 registers through it, which costs the SIMD its fourth wave).
+    // Epilogue operands (the residual of `out = a@b + add`, gate and up of the SiLU-gate backward,
+    // the rotation's cos and sin) are requested here, behind the first two tiles and in front of the
+    // K loop: after the last MFMA their latency would be paid when the workgroups of a CU all finish
+    // together. The loop's vmcnt waits cover them (they are older than every later tile request).
     // Out-of-range elements read element 0 instead of branching around the load.
     constexpr bool PRE = BM == 64 && BN == 64 && NSEG == 1 && (EPI == kEpiPlain || EPI == kEpiSiluBwd);
     float2 pre[PRE ? 16 : 1];  // plain: .x = residual, or (cos, sin); SiLU backward: (gate, up)
@@ -1265,58 +1092,45 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
         }
     }
 
-    if constexpr (NSEG > 1) load_ext();
-
-    // The block this wave finishes: rows wm0 .. wm0 + 31 and columns wn0 .. wn0 + WN - 1.
-    floatx16 acc[FM][FN * NB];
-    if constexpr (KS == 1) {
+    // The rank-r products' operands: ordinary loads, consumed last.
+    ExA xa[NSEG];
+    ExB xb[NSEG];
 #pragma unroll
-        for (int j = 0; j < FN * NB; j++) acc[0][j] = sum[j];
-    } else {
-        // Two waves of a row block: each hands the other the sums of the columns that one finishes.
-        static_assert(KS == 1 || 2 * KW * FN * NB * 1024 <= STAGE, "the exchange fits the stages");
-        constexpr int PER = FN * NB * 1024;  // floats a wave hands over
-        const int slot = grp * 4 + wave;
-        auto place = [&](int sl) { return (KW == 2 ? (sl < 4 ? St0 : St1) + (sl & 3) * PER : (sl < 2 ? St0 : St1) + (sl & 1) * PER) + lane; };
-        float* give = place(slot ^ 1);
-        const float* take = place(slot);
-#pragma unroll
-        for (int j = 0; j < FN * NB; j++) {
-            const int c = (j / FN) * CB + j % FN;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                acc[0][j][r] = ks == 0 ? sum[c][r] : sum[c + FN][r];
-                give[(j * 16 + r) * 64] = ks == 0 ? sum[c + FN][r] : sum[c][r];
-            }
+    for (int s = 0; s < NSEG; s++) {
+        if (has_ext[s]) {
+            const AsyncSeg& sg = p.seg[s];
+            xa[s].set_offsets(sg.lda2, m0, M, 4);
+            xb[s].set_offsets(sg.ldb2, n0, p.N, 4);
+            xa[s].template load<float, true>(reinterpret_cast<const char*>(sg.a2), 0, sg.K2);
+            xb[s].template load<float, true>(reinterpret_cast<const char*>(sg.b2), 0, sg.K2);
         }
-        lds_barrier();
-#pragma unroll
-        for (int j = 0; j < FN * NB; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[0][j][r] += take[(j * 16 + r) * 64];
     }
-    auto mfma_step = [&](const float4 (&af)[FM], const float4 (&bf)[FN * NB]) {  // f32 operands: the rank-r term
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN * NB; j++) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].x, bf[j].x, acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].y, bf[j].y, acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].z, bf[j].z, acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i].w, bf[j].w, acc[i][j], 0, 0, 0);
-            }
-    };
+
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (WAIT & 15) | ((WAIT >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(t0 + 2, St2);
+    read_frags(St0 + grp * SUB, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t = t0; t < nt; t += NST) {
+        iter(t, St0, St1);
+        if (t + 1 < nt) iter(t + 1, St1, St2);
+        if (t + 2 < nt) iter(t + 2, St2, St0);
+    }
+
     if constexpr (KW == 2) {
-        // The second wave group hands its sums over through the third stage and retires.
+        // The second wave group hands its sums over through the second stage and retires.
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();  // loads landed, every wave has left the last stage
         static_assert(KW == 1 || FN * NB * 16 * 256 <= STAGE, "the hand-over fits a stage");
-        float* red = St2 + wave * 64 + lane;
+        float* red = St1 + wave * 64 + lane;
         if (grp == 1) {
 #pragma unroll
             for (int j = 0; j < FN * NB; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) red[(j * 16 + r) * 256] = acc[0][j][r];
         }
-        lds_barrier();
+        __syncthreads();
         if (grp == 1) return;
 #pragma unroll
         for (int j = 0; j < FN * NB; j++)
@@ -1326,13 +1140,15 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
 #pragma unroll
     for (int s = 0; s < NSEG; s++) {
         if (has_ext[s]) {  // never with two b matrices
-            lds_barrier();  // every wave has left the exchange (or the previous segment's rank-r tile)
+            // The stage is free when every wave's loads have landed and every wave has left the
+            // last K tile (or the previous segment's rank-r tile).
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
             xa[s].template store<float>(ExAs);
             xb[s].template store<float>(ExBs);
-            lds_barrier();
+            __syncthreads();
 #pragma unroll
             for (int st = 0; st < 2; st++) {
-                if (st == 1 && p.seg[s].K2 <= 8) break;  // ranks up to 8: the second half is all zeros
                 float4 af[FM], bf[FN * NB];
 #pragma unroll
                 for (int i = 0; i < FM; i++) af[i] = ExA::frag(ExAs, st, half, wm0 + i * 32 + l32);
@@ -1342,17 +1158,20 @@ __global__ __launch_bounds__(256 * KW, BM == 64 ? (EPI == kEpiGateUp ? 3 : 4) : 
             }
         }
     }
+    // Nothing may still be landing in LDS when the workgroup retires.
+    __builtin_amdgcn_s_waitcnt(0x0F70);
 
     if constexpr (EPI == kEpiPlain && BM == 64 && BN == 64) {
         if (p.rope) {  // uniform per workgroup; never together with split-K
             // The partner column (+-32) belongs to the neighbouring wave: exchange through the
-            // stage memory (the barrier: every wave has left the rank-r tile).
-            lds_barrier();
+            // stage memory (free now: every wave has waited for its own loads, the barrier makes
+            // that true of all of them).
+            __syncthreads();
             float* mine = (wave < 2 ? St0 : St1) + (wave & 1) * 1024;
             const float* other = (wave < 2 ? St0 : St1) + ((wave & 1) ^ 1) * 1024;
 #pragma unroll
             for (int r = 0; r < 16; r++) mine[r * 64 + lane] = acc[0][0][r];
-            lds_barrier();
+            __syncthreads();
             const int col = n0 + wn0 + l32;
             const bool upper = wn0 != 0;  // this wave holds i + 32
 #pragma unroll
@@ -2008,7 +1827,7 @@ int launch_async(ft_context* ctx, AsyncBatch g, int layout, int epi = kEpiPlain)
 int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout) {
     size_t tiles128 = 0;
     for (int i = 0; i < g.count; i++) tiles128 += (size_t)((g.M + 127) / 128) * (size_t)((g.p[i].N + 127) / 128);
-    if (tiles128 >= 8 * (size_t)ctx->num_cus) return launch_async<128, 128, 32, 128>(ctx, g, layout);
+    if (tiles128 >= 8 * (size_t)ctx->num_cus) return launch_async<128, 128, 64, 64>(ctx, g, layout);
     // A very long K over few tiles (the head's input gradient: K = vocabulary): the large tile with its K
     // tiles shared out runs at the rate of the many-tile case, and the extra pass over the partial tiles is
     // a fraction of a percent of the product.
@@ -2021,7 +1840,7 @@ int launch_async_auto(ft_context* ctx, const AsyncBatch& g, int layout) {
         plain = plain && g.p[i].rope == nullptr && ((size_t)g.M * g.p[i].N) % 4 == 0 && g.p[i].ldc == g.p[i].N;
     }
     if (plain && min_kt >= 512 && tiles128 * 2 <= 2 * (size_t)ctx->num_cus && tiles128 * 8 >= 2 * (size_t)ctx->num_cus)
-        return launch_async<128, 128, 32, 128>(ctx, g, layout);
+        return launch_async<128, 128, 64, 64>(ctx, g, layout);
     return launch_async<64, 64, 32, 32>(ctx, g, layout);
 }
 

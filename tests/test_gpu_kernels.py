@@ -215,84 +215,6 @@ def test_long_k_products_on_eight_waves(g, M, K, N):
     assert_close("matmul_bt_f16b", dx.to_numpy(), f64_mm(gy, cpu.round_f16(w2).T), atol=2e-3, rtol=1e-4)
 
 
-def split_rows(seed, M, K):
-    """Rows as the f16-split products can meet them: magnitudes from 1e-36 to 1e30, zero rows, rows that are zero or
-    tiny in their first K tiles and grow later, one value far above the rest, f32 subnormals."""
-    rng = np.random.default_rng(seed)
-    x = rng.standard_normal((M, K))
-    x *= 10.0 ** rng.uniform(-30, 25, (M, 1))
-    for i in range(M):
-        if i % 7 == 1:
-            x[i] = 0.0
-        elif i % 7 == 2:
-            x[i, :K // 2] = 0.0
-        elif i % 7 == 3:
-            x[i] *= 2.0 ** (np.arange(K) * 40.0 / K)
-        elif i % 7 == 4:
-            x[i, (i * 37) % K] *= 1e5
-        elif i % 7 == 5:
-            x[i] = rng.standard_normal(K) * 1e-39
-    return x.astype(np.float32)
-
-
-@pytest.mark.parametrize("M,K,N", [(31, 32, 64), (64, 64, 64), (130, 288, 136), (70, 1024, 200), (600, 96, 2304), (300, 2048, 960)])
-@pytest.mark.parametrize("layout", [0, 1])
-def test_f16_split_keeps_f32_accuracy_over_the_exponent_range(g, M, K, N, layout):
-    """|err| <= (K/8 + 8) 2^-24 sum|x||w|, the f32 bound of a sum of K/16 partial sums in two halves (before: K/2),
-    plus 2^-36 of the row's largest value times sum|w|, which is what a value far below it may lose, and a subnormal's last place."""
-    from ferrotensor_amd import UnifiedTensor
-    ctx, eng = g
-    x = split_rows(M + K + N, M, K)
-    w = rnd(N + K, K, N, scale=0.05)
-    w[K // 3, :] *= 1e-5      # f16 subnormals among the weights
-    stored = np.ascontiguousarray(w if layout == 0 else w.T)
-    w16 = UnifiedTensor.from_f32_as_f16(ctx, stored, list(stored.shape))
-    wr = cpu.round_f16(w).astype(np.float64)
-    out = empty(ctx, M, N)
-    (eng.matmul_f16b if layout == 0 else eng.matmul_bt_f16b)(ctx, up(ctx, x), w16, out)
-    x64 = x.astype(np.float64)
-    bound = (K / 8 + 8) * 2.0 ** -24 * (np.abs(x64) @ np.abs(wr)) + \
-        2.0 ** -36 * np.abs(x64).max(axis=1, keepdims=True) * np.abs(wr).sum(axis=0) + 2.0 ** -147 * np.abs(wr).sum(axis=0) + 2.0 ** -148
-    err = np.abs(out.to_numpy().reshape(M, N) - x64 @ wr)
-    assert np.all(err <= bound), (np.argwhere(err > bound)[:5], np.max(err / bound))
-
-
-@pytest.mark.parametrize("layout", [0, 1])
-def test_f16_split_products_of_infinities_and_nans(g, layout):
-    """An infinity or NaN among the operands gives what f32 arithmetic gives, in its row or column only; a sum past the
-    f32 range is an infinity; values at the end of the range are kept."""
-    from ferrotensor_amd import UnifiedTensor
-    ctx, eng = g
-    M, K, N = 130, 256, 136
-    x, w = rnd(1, M, K), rnd(2, K, N, scale=0.05)
-    x[3, 7] = np.inf
-    x[40, 200] = -np.inf
-    x[66, 64] = np.nan
-    x[70, 5], x[70, 6] = np.inf, -np.inf
-    x[90] = 3.0e38
-    w[:, 17] = np.abs(w[:, 17]) + 1.0     # row 90 overflows in this column
-    x[100, 31] = np.finfo(np.float32).max
-    w[9, 77] = np.inf
-    stored = np.ascontiguousarray(w if layout == 0 else w.T)
-    w16 = UnifiedTensor.from_f32_as_f16(ctx, stored, list(stored.shape))
-    out = empty(ctx, M, N)
-    (eng.matmul_f16b if layout == 0 else eng.matmul_bt_f16b)(ctx, up(ctx, x), w16, out)
-    got = out.to_numpy().reshape(M, N)
-    with np.errstate(all="ignore"):
-        want = x.astype(np.float64) @ cpu.round_f16(w).astype(np.float64)
-        want = np.where(np.isinf(want.astype(np.float32)), want * np.inf, want)  # past the largest f32
-    sure = np.ones((M, N), bool)
-    sure[90] = False                      # sums near the end of the range: an intermediate sum may overflow
-    sure[90, 17] = True
-    assert np.array_equal(np.isnan(got[sure]), np.isnan(want[sure]))
-    assert np.array_equal(np.isinf(got[sure]), np.isinf(want[sure]))
-    inf = np.isinf(want) & sure
-    assert np.array_equal(np.sign(got[inf]), np.sign(want[inf]))
-    fin = np.isfinite(want) & sure
-    scale = np.abs(np.where(np.isfinite(x), x, 0)).max(axis=1, keepdims=True) * np.ones((1, N))
-    assert np.all(np.abs(got[fin] - want[fin]) <= 1e-5 * np.abs(want[fin]) + 1e-5 * scale[fin])
-
-
 def test_f16_upload_is_bit_exact(g):
     from ferrotensor_amd import DType, UnifiedTensor
     ctx, _ = g
