@@ -716,30 +716,29 @@ __global__ __launch_bounds__(256) void rope_kernel(const float* __restrict__ src
 }
 
 // ---------------------------------------------------------------------------
-// Masked softmax-cross-entropy, one workgroup per row. grad may alias logits (no __restrict__ on
-// either), so the target logit is loaded before the barrier that precedes the gradient stores.
-// A row of up to THREADS * 4 * CACHE floats is held in registers: logits are read once, their
-// exponentials take their place, and the gradient is written once (8 bytes an element).
-// Bound: memory, with the exponentials close behind. 49152 columns as 512 threads x 24 float4, 128
-// registers: two rows share a CU, so one row's loads and stores run under the other's arithmetic
-// (1024 threads x 12 float4 take 93 registers: one row at a time, and a thread's loads waited for
-// each other under `if (i < n4)`). One exponential an element instead of a second one of x - log Z.
-// 1446 x 49152: 134 -> 98 us (5.8 TB/s, what a large copy reaches).
+// Masked softmax-cross-entropy. One 1024-thread workgroup per row. grad may
+// alias logits (no __restrict__ on either), so the target logit is loaded
+// before the barrier that precedes the gradient stores. A row of up
+// to 1024*4*CACHE floats is held in registers between the reduction and the
+// gradient write, so logits are read once and the gradient written once.
 // ---------------------------------------------------------------------------
 
-template <int THREADS, int CACHE>  // float4 per thread kept in registers (0 = stream from memory)
-__global__ __launch_bounds__(THREADS, CACHE > 12 ? 4 : 1) void masked_ce_kernel(
+constexpr int kCeThreads = 1024;
+
+template <int CACHE>  // float4 per thread kept in registers (0 = stream from memory)
+__global__ __launch_bounds__(kCeThreads) void masked_ce_kernel(
     const float* logits, const uint32_t* __restrict__ targets, const float* __restrict__ weights,
     float* grad, float* __restrict__ row_loss, size_t rows, size_t vocab, float grad_scale) {
-    __shared__ float red[THREADS / kWave];
+    __shared__ float red[kCeThreads / kWave];
     const size_t row = blockIdx.x;
     const float* x = logits + row * vocab;
     float* gr = grad + row * vocab;
     const uint32_t tgt = targets[row];
-    const unsigned n4 = (unsigned)(vocab / 4);
+    const size_t n4 = vocab / 4;
     if (tgt == FT_MASKED_CE_SKIP) {
         float4* g4 = reinterpret_cast<float4*>(gr);
-        for (unsigned i = threadIdx.x; i < n4; i += THREADS) g4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) g4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) gr[i] = 0.0f;
         if (threadIdx.x == 0) row_loss[row] = 0.0f;
         return;
     }
@@ -747,64 +746,64 @@ __global__ __launch_bounds__(THREADS, CACHE > 12 ? 4 : 1) void masked_ce_kernel(
     float4 cache[CACHE > 0 ? CACHE : 1];
     float m = -3.4e38f;
     if constexpr (CACHE > 0) {
-        // (a thread past the row's end re-reads its last quad, which changes no maximum and is left out of the sums)
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            const unsigned i = threadIdx.x + j * THREADS;
-            cache[j] = x4[i < n4 ? i : n4 - 1];
+            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
+            if (i < n4) {
+                cache[j] = x4[i];
+                m = fmaxf(m, fmaxf(fmaxf(cache[j].x, cache[j].y), fmaxf(cache[j].z, cache[j].w)));
+            }
         }
-#pragma unroll
-        for (int j = 0; j < CACHE; j++) m = fmaxf(m, fmaxf(fmaxf(cache[j].x, cache[j].y), fmaxf(cache[j].z, cache[j].w)));
     } else {
-        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
+        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
             const float4 v = x4[i];
             m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
         }
     }
-    m = block_max<THREADS>(m, red);
+    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) m = fmaxf(m, x[i]);
+    m = block_max<kCeThreads>(m, red);
     float se = 0.0f;
     if constexpr (CACHE > 0) {
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            cache[j] = make_float4(expf(cache[j].x - m), expf(cache[j].y - m), expf(cache[j].z - m), expf(cache[j].w - m));
-            const float s4 = cache[j].x + cache[j].y + cache[j].z + cache[j].w;
-            if (threadIdx.x + j * THREADS < n4) se += s4;
+            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
+            if (i < n4) se += expf(cache[j].x - m) + expf(cache[j].y - m) + expf(cache[j].z - m) + expf(cache[j].w - m);
         }
     } else {
-        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
+        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
             const float4 v = x4[i];
             se += expf(v.x - m) + expf(v.y - m) + expf(v.z - m) + expf(v.w - m);
         }
     }
-    se = block_sum<THREADS>(se, red);
+    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) se += expf(x[i] - m);
+    se = block_sum<kCeThreads>(se, red);
     const float log_z = m + logf(se);
     const float w = weights[row];
     // The target logit is read before any thread overwrites it (grad may alias logits).
     const float x_t = x[tgt];
     __syncthreads();
     float4* g4 = reinterpret_cast<float4*>(gr);
-    auto grad_of = [&](float prob, unsigned i) {
-        float gv = prob * w;
-        if (i == tgt) gv -= w;
+    auto one = [&](float xv, size_t i) {
+        float gv = expf(xv - log_z) * w;
+        if (i == (size_t)tgt) gv -= w;
         return gv * grad_scale;
     };
-    if (CACHE > 0 && se != 0.0f) {
-        const float inv = 1.0f / se;
+    if constexpr (CACHE > 0) {
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            const unsigned i = threadIdx.x + j * THREADS;
-            const float4 v = cache[j];
-            if (i < n4)
-                g4[i] = make_float4(grad_of(v.x * inv, 4 * i), grad_of(v.y * inv, 4 * i + 1), grad_of(v.z * inv, 4 * i + 2),
-                                    grad_of(v.w * inv, 4 * i + 3));
+            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
+            if (i < n4) {
+                const float4 v = cache[j];
+                g4[i] = make_float4(one(v.x, 4 * i), one(v.y, 4 * i + 1), one(v.z, 4 * i + 2), one(v.w, 4 * i + 3));
+            }
         }
-    } else {  // streamed, or a row whose logits all lie below the maximum's start (no exponential is left)
-        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
+    } else {
+        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
             const float4 v = x4[i];
-            g4[i] = make_float4(grad_of(expf(v.x - log_z), 4 * i), grad_of(expf(v.y - log_z), 4 * i + 1),
-                                grad_of(expf(v.z - log_z), 4 * i + 2), grad_of(expf(v.w - log_z), 4 * i + 3));
+            g4[i] = make_float4(one(v.x, 4 * i), one(v.y, 4 * i + 1), one(v.z, 4 * i + 2), one(v.w, 4 * i + 3));
         }
     }
+    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) gr[i] = one(x[i], i);
     if (threadIdx.x == 0) row_loss[row] = log_z - x_t;
 }
 
@@ -1468,16 +1467,15 @@ int ft_masked_cross_entropy_weighted(ft_context* ctx, const float* logits, const
     if (!vec) {
         hipLaunchKernelGGL(masked_ce_scalar_kernel, grid, dim3(256), 0, ctx->stream, logits, targets, weights, grad,
                            row_loss, rows, vocab, grad_scale);
+    } else if (vocab <= (size_t)kCeThreads * 4 * 4) {
+        hipLaunchKernelGGL((masked_ce_kernel<4>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
+                           grad, row_loss, rows, vocab, grad_scale);
+    } else if (vocab <= (size_t)kCeThreads * 4 * 12) {
+        hipLaunchKernelGGL((masked_ce_kernel<12>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
+                           grad, row_loss, rows, vocab, grad_scale);
     } else {
-#define FT_CE(THREADS, CACHE)                                                                                         \
-    hipLaunchKernelGGL((masked_ce_kernel<THREADS, CACHE>), grid, dim3(THREADS), 0, ctx->stream, logits, targets, weights, \
-                       grad, row_loss, rows, vocab, grad_scale)
-        // the smallest workgroup that holds a row with at most 24 quads a thread; wider rows are streamed
-        if (vocab <= 256 * 4 * 4) FT_CE(256, 4);
-        else if (vocab <= 512 * 4 * 8) FT_CE(512, 8);
-        else if (vocab <= 512 * 4 * 24) FT_CE(512, 24);
-        else FT_CE(1024, 0);
-#undef FT_CE
+        hipLaunchKernelGGL((masked_ce_kernel<0>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
+                           grad, row_loss, rows, vocab, grad_scale);
     }
     FT_LAUNCH_CHECK();
     return FT_OK;
