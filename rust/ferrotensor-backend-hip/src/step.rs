@@ -158,8 +158,9 @@ impl Lfm2Model {
         ok(unsafe { sys::ft_model_read_grad(self.raw, index, out.as_mut_ptr()) })?;
         Ok(out)
     }
-    /// All gradients one after the other, in the order of the parameters (`numel` values in total).
-    pub fn read_grads(&self, numel: usize) -> Result<Vec<f32>, TrainError> {
+    /// All gradients one after the other, in the order of `named_params`, whose sizes add up to the length.
+    pub fn read_grads(&self) -> Result<Vec<f32>, TrainError> {
+        let numel: usize = self.named_params()?.iter().map(|p| p.1).sum();
         let mut out = vec![0.0f32; numel];
         ok(unsafe { sys::ft_model_read_grads(self.raw, out.as_mut_ptr()) })?;
         Ok(out)

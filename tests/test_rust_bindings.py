@@ -78,3 +78,18 @@ def test_step_driver_wrappers_cover_the_model_and_trainer_entry_points():
     fields = re.search(r"pub struct StepStats \{(.*?)\}", text, re.S).group(1)
     for field in ("loss: f32", "tokens: usize", "optimizer_step: bool", "grad_norm: Option<f32>", "lr: Option<f32>"):
         assert field in fields, field
+
+
+def method_body(name):
+    """Signature and body of a method of step.rs."""
+    text = open(SAFE[1]).read()
+    at = text.index("pub fn %s(" % name)
+    return text[at:text.index("\n    }", at)]
+
+
+def test_all_gradients_are_read_into_a_vector_sized_by_the_model():
+    """ft_model_read_grads writes as many values as the model has, so the safe wrapper takes no size from its caller:
+    a smaller one (or one from before an adapter changed its rank) would be written past."""
+    body = method_body("read_grads")
+    assert re.match(r"pub fn read_grads\(&self\) ->", body), body.split("\n")[0]
+    assert body.index("self.named_params()?") < body.index("vec![") < body.index("sys::ft_model_read_grads")
