@@ -85,6 +85,7 @@ pub struct ModelConfig {
 /// `Lfm2Model` for all-attention (Llama / SmolLM2) checkpoints.
 pub struct Lfm2Model {
     ctx: Arc<WgpuContext>,
+    config: ModelConfig,
     raw: *mut sys::FtModel,
 }
 
@@ -111,7 +112,7 @@ impl Lfm2Model {
         };
         let mut raw = std::ptr::null_mut();
         ok(unsafe { sys::ft_model_create(ctx.raw(), &cfg, &mut raw) })?;
-        Ok(Self { ctx, raw })
+        Ok(Self { ctx, config: *config, raw })
     }
     pub fn ctx(&self) -> &Arc<WgpuContext> {
         &self.ctx
@@ -129,8 +130,37 @@ impl Lfm2Model {
     }
     /// An adapter with given factors, `a [in, rank]`, `b [rank, out]` (graph/src/lib.rs:28-56).
     pub fn set_lora(&mut self, prefix: &str, a: &[f32], b: &[f32], rank: usize, alpha: f32) -> Result<(), TrainError> {
+        if let Some((inputs, outputs)) = self.linear_dims(prefix) {
+            if a.len() < inputs.saturating_mul(rank) || b.len() < outputs.saturating_mul(rank) {
+                return Err(TrainError(format!("set_lora: {prefix} of rank {rank} is [{inputs}, {rank}] and \
+                                               [{rank}, {outputs}], given {} and {} values", a.len(), b.len())));
+            }
+        }
         let name = CString::new(prefix).map_err(|e| TrainError(e.to_string()))?;
         ok(unsafe { sys::ft_model_set_lora(self.raw, name.as_ptr(), a.as_ptr(), b.as_ptr(), rank, alpha) })
+    }
+    /// `[in, out]` of a linear by name; a name that is none is the library's to refuse.
+    fn linear_dims(&self, prefix: &str) -> Option<(usize, usize)> {
+        let c = &self.config;
+        let (h, f, v) = (c.hidden_size as usize, c.intermediate_size as usize, c.vocab_size as usize);
+        let kv = h / c.num_attention_heads as usize * c.num_key_value_heads as usize;
+        match prefix.rsplit('.').next()? {
+            "q_proj" | "o_proj" => Some((h, h)),
+            "k_proj" | "v_proj" => Some((h, kv)),
+            "gate_proj" | "up_proj" => Some((h, f)),
+            "down_proj" => Some((f, h)),
+            "lm_head" => Some((h, v)),
+            _ => None,
+        }
+    }
+    /// The library reads and writes whole tensors: refuses a buffer shorter than parameter `index`.
+    fn check_numel(&self, index: usize, numel: usize) -> Result<(), TrainError> {
+        let mut want = 0usize;
+        ok(unsafe { sys::ft_model_param_info(self.raw, index, std::ptr::null_mut(), &mut want) })?;
+        if numel < want {
+            return Err(TrainError(format!("parameter {index} has {want} values, given {numel}")));
+        }
+        Ok(())
     }
     /// `named_lora_params` (lfm.rs:756-770) and, with a trainable base, the weights: name and size.
     pub fn named_params(&self) -> Result<Vec<(String, usize)>, TrainError> {
@@ -146,14 +176,17 @@ impl Lfm2Model {
         Ok(out)
     }
     pub fn read_param(&self, index: usize, numel: usize) -> Result<Vec<f32>, TrainError> {
+        self.check_numel(index, numel)?;
         let mut out = vec![0.0f32; numel];
         ok(unsafe { sys::ft_model_read_param(self.raw, index, out.as_mut_ptr()) })?;
         Ok(out)
     }
     pub fn write_param(&mut self, index: usize, values: &[f32]) -> Result<(), TrainError> {
+        self.check_numel(index, values.len())?;
         ok(unsafe { sys::ft_model_write_param(self.raw, index, values.as_ptr()) })
     }
     pub fn read_grad(&self, index: usize, numel: usize) -> Result<Vec<f32>, TrainError> {
+        self.check_numel(index, numel)?;
         let mut out = vec![0.0f32; numel];
         ok(unsafe { sys::ft_model_read_grad(self.raw, index, out.as_mut_ptr()) })?;
         Ok(out)
@@ -171,6 +204,10 @@ impl Lfm2Model {
         let s = rows.first().map_or(0, |r| r.len());
         assert!(rows.iter().all(|r| r.len() == s), "forward_batch: rows of different lengths");
         let flat: Vec<u32> = rows.iter().flat_map(|r| r.iter().copied()).collect();
+        if vocab_size < self.config.vocab_size as usize {
+            return Err(TrainError(format!("forward_batch: the vocabulary has {} words, given {vocab_size}",
+                                          self.config.vocab_size)));
+        }
         let mut logits = vec![0.0f32; b * s * vocab_size];
         ok(unsafe { sys::ft_model_forward_logits(self.raw, flat.as_ptr(), b, s, logits.as_mut_ptr()) })?;
         Ok(logits)
@@ -411,6 +448,7 @@ impl Trainer {
     /// ferrotensor-autograd/src/lib.rs:1577-1628).
     pub fn read_moments(&mut self, index: usize, numel: usize) -> Result<(Vec<f32>, Vec<f32>), TrainError> {
         let t = self.handle()?;
+        self.model.check_numel(index, numel)?;
         let (mut m, mut v) = (vec![0.0f32; numel], vec![0.0f32; numel]);
         ok(unsafe { sys::ft_trainer_read_moments(t, index, m.as_mut_ptr(), v.as_mut_ptr()) })?;
         Ok((m, v))
@@ -422,6 +460,7 @@ impl Trainer {
         ok(unsafe { sys::ft_trainer_set_adam_hyper(t, saved.lr, saved.beta1, saved.beta2, saved.eps, saved.weight_decay) })?;
         ok(unsafe { sys::ft_trainer_set_adam_t(t, t_steps) })?;
         for (index, m, v) in moments {
+            self.model.check_numel(*index, m.len().min(v.len()))?;
             ok(unsafe { sys::ft_trainer_write_moments(t, *index, m.as_ptr(), v.as_ptr()) })?;
         }
         self.optimizer = *saved;

@@ -83,7 +83,8 @@ def test_step_driver_wrappers_cover_the_model_and_trainer_entry_points():
 def method_body(name):
     """Signature and body of a method of step.rs."""
     text = open(SAFE[1]).read()
-    at = text.index("pub fn %s(" % name)
+    at = text.index("fn %s(" % name)
+    at = text.rindex("\n", 0, at) + 5
     return text[at:text.index("\n    }", at)]
 
 
@@ -93,3 +94,17 @@ def test_all_gradients_are_read_into_a_vector_sized_by_the_model():
     body = method_body("read_grads")
     assert re.match(r"pub fn read_grads\(&self\) ->", body), body.split("\n")[0]
     assert body.index("self.named_params()?") < body.index("vec![") < body.index("sys::ft_model_read_grads")
+
+
+def test_safe_wrappers_check_every_length_the_library_takes_for_granted():
+    """The C side of these calls reads or writes as many values as the tensor has. Each wrapper compares the length it
+    was given with the model's own before the call (longer ones have always been taken)."""
+    for name in ("read_param", "write_param", "read_grad", "read_moments", "load_state"):
+        body = method_body(name)
+        calls = [m.start() for m in re.finditer(r"sys::ft_\w+_(?:read|write)_\w+\(", body)]
+        assert calls and "check_numel(" in body and body.index("check_numel(") < calls[0], name
+    assert "numel < want" in method_body("check_numel")
+    body = method_body("set_lora")
+    assert body.index("self.linear_dims(prefix)") < body.index("sys::ft_model_set_lora")
+    body = method_body("forward_batch")
+    assert body.index("vocab_size < self.config.vocab_size as usize") < body.index("sys::ft_model_forward_logits")
