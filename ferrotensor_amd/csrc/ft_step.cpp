@@ -1181,6 +1181,7 @@ int ft_model_read_grads(ft_model* m, float* out_host) {
             return FT_OK;
         }
         if (!m->grad_segs) {
+            free_grad_gather(m);   // the array of a call that ran out of host memory after it
             FT_HIP(hipHostMalloc((void**)&m->grad_host, total * sizeof(float), hipHostMallocDefault));
             std::vector<ft_segment> segs;
             float* dst = m->grad_host;
