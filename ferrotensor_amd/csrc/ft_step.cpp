@@ -309,6 +309,36 @@ void free_grad_gather(ft_model* m) {
     m->grad_nseg = 0;
 }
 
+// Makes the table and the pinned array; without the memory for both there are neither.
+int make_grad_gather(ft_model* m, size_t total) {
+    free_grad_gather(m);   // the array of a call that ran out of host memory after it
+    if (hipHostMalloc((void**)&m->grad_host, total * sizeof(float), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();   // or the next launch check reports it
+        m->grad_host = nullptr;
+        return FT_ERR_OOM;
+    }
+    std::vector<ft_segment> segs;
+    float* dst = m->grad_host;
+    for (const auto& p : m->params) {
+        for (size_t off = 0; off < p.n; off += FT_SUM_SQUARES_CHUNK) {
+            const size_t n = std::min<size_t>(p.n - off, FT_SUM_SQUARES_CHUNK);
+            segs.push_back(ft_segment{dst + off, p.g + off, nullptr, nullptr, (uint32_t)n});
+        }
+        dst += p.n;
+    }
+    ft_segment* dev = nullptr;
+    int rc = ft_alloc(m->ctx, segs.size() * sizeof(ft_segment), (void**)&dev);
+    if (rc == FT_OK) rc = ft_upload(m->ctx, dev, segs.data(), segs.size() * sizeof(ft_segment));
+    if (rc != FT_OK) {
+        if (dev) (void)ft_free(m->ctx, dev);
+        free_grad_gather(m);
+        return rc;
+    }
+    m->grad_segs = dev;
+    m->grad_nseg = segs.size();
+    return FT_OK;
+}
+
 // The trainable tensors in reporting order. With a trainable base (model_builder.rs:353-357) the
 // linear weights and the norm scales are in it too, and their gradient buffers are made here.
 int rebuild_params(ft_model* m) {
@@ -1173,35 +1203,12 @@ int ft_model_read_grads(ft_model* m, float* out_host) {
         FT_HIP(hipSetDevice(ctx->device));
         // Many small tensors (adapters) are gathered by one kernel into pinned memory; a trainable base is few large
         // ones, which the pinned array would only copy twice.
-        if (total > (size_t)16 << 20) {
+        if (total > (size_t)16 << 20 || (!m->grad_segs && make_grad_gather(m, total) != FT_OK)) {
             for (const auto& p : m->params) {
                 FT_TRY(ft_download(ctx, out_host, p.g, p.n * sizeof(float)));
                 out_host += p.n;
             }
             return FT_OK;
-        }
-        if (!m->grad_segs) {
-            free_grad_gather(m);   // the array of a call that ran out of host memory after it
-            FT_HIP(hipHostMalloc((void**)&m->grad_host, total * sizeof(float), hipHostMallocDefault));
-            std::vector<ft_segment> segs;
-            float* dst = m->grad_host;
-            for (const auto& p : m->params) {
-                for (size_t off = 0; off < p.n; off += FT_SUM_SQUARES_CHUNK) {
-                    const size_t n = std::min<size_t>(p.n - off, FT_SUM_SQUARES_CHUNK);
-                    segs.push_back(ft_segment{dst + off, p.g + off, nullptr, nullptr, (uint32_t)n});
-                }
-                dst += p.n;
-            }
-            ft_segment* dev = nullptr;
-            int rc = ft_alloc(ctx, segs.size() * sizeof(ft_segment), (void**)&dev);
-            if (rc == FT_OK) rc = ft_upload(ctx, dev, segs.data(), segs.size() * sizeof(ft_segment));
-            if (rc != FT_OK) {
-                if (dev) (void)ft_free(ctx, dev);
-                free_grad_gather(m);
-                return rc;
-            }
-            m->grad_segs = dev;
-            m->grad_nseg = segs.size();
         }
         FT_TRY(ft_internal_multi_copy(ctx, m->grad_segs, m->grad_nseg));
         FT_HIP(hipStreamSynchronize(ctx->stream));

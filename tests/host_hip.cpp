@@ -184,6 +184,15 @@ int main(int argc, char** argv) {
         expect(refused > 0, "no allocation was refused");
         check_grads("after the refusals", total);
         expect(g_pinned.size() <= 1, "pinned arrays were lost");
+    } else if (scenario == "no_pinned_memory" || scenario == "no_device_memory") {
+        // the gradients still come, tensor by tensor, and all at once again when there is memory
+        g_refuse_pinned = scenario == "no_pinned_memory";
+        g_refuse_device = !g_refuse_pinned;
+        check_grads("refused", total);
+        expect(g_copies == 8, "one copy per tensor, twice");
+        g_refuse_pinned = g_refuse_device = false;
+        check_grads("with memory again", total);
+        expect(g_copies == 12, "gathered");
     } else {
         printf("no such scenario\n");
         return 2;
