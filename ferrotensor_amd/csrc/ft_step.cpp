@@ -1073,19 +1073,24 @@ int ft_model_set_lora(ft_model* m, const char* prefix, const float* a, const flo
         LinearW* l = find_linear(m, prefix);
         FT_CHECK_ARG(l, "ft_model_set_lora: no linear named %s", prefix);
         if (l->r != rank) {
-            for (float** p : {&l->a, &l->b, &l->ga, &l->gb}) {
-                if (*p) FT_TRY(ft_free(m->ctx, *p));
-                *p = nullptr;
+            // All four new buffers before an old one goes: the parameter list and what was made from it point at the old.
+            const size_t sizes[4] = {l->in * rank, rank * l->out, l->in * rank, rank * l->out};
+            float* fresh[4] = {};
+            int rc = FT_OK;
+            for (int i = 0; i < 4 && rc == FT_OK; i++) rc = alloc_f(m->ctx, sizes[i], &fresh[i]);
+            for (int i = 2; i < 4 && rc == FT_OK; i++) rc = ft_zero(m->ctx, fresh[i], sizes[i] * 4);
+            if (rc != FT_OK) {
+                for (float* p : fresh) (void)ft_free(m->ctx, p);
+                return rc;
             }
-            FT_TRY(alloc_f(m->ctx, l->in * rank, &l->a));
-            FT_TRY(alloc_f(m->ctx, rank * l->out, &l->b));
-            FT_TRY(alloc_f(m->ctx, l->in * rank, &l->ga));
-            FT_TRY(alloc_f(m->ctx, rank * l->out, &l->gb));
-            FT_TRY(ft_zero(m->ctx, l->ga, l->in * rank * 4));
-            FT_TRY(ft_zero(m->ctx, l->gb, rank * l->out * 4));
-            l->r = rank;
             m->params_dirty = true;
             m->param_generation++;
+            float** slots[4] = {&l->a, &l->b, &l->ga, &l->gb};
+            for (int i = 0; i < 4; i++) {
+                (void)ft_free(m->ctx, *slots[i]);
+                *slots[i] = fresh[i];
+            }
+            l->r = rank;
         }
         l->alpha = alpha;
         FT_TRY(ft_upload(m->ctx, l->a, a, l->in * rank * sizeof(float)));

@@ -18,6 +18,7 @@ static std::map<char*, size_t> g_device;
 static std::set<void*> g_pinned;
 static hipError_t g_last = hipSuccess;
 static bool g_refuse_pinned = false, g_refuse_device = false;
+static int g_device_grants = -1;  // device allocations still granted, -1: all
 static long g_news_left = -1;   // operator new throws when this reaches 0
 static int g_failures = 0, g_copies = 0;
 
@@ -47,7 +48,8 @@ static hipError_t fail(hipError_t e) { return g_last = e; }   // stays until hip
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-    if (g_refuse_device) return fail(hipErrorOutOfMemory);
+    if (g_refuse_device || g_device_grants == 0) return fail(hipErrorOutOfMemory);
+    if (g_device_grants > 0) g_device_grants--;
     *p = malloc(n);
     const long news = g_news_left;
     g_news_left = -1;   // the bookkeeping here is not the library's
@@ -193,6 +195,18 @@ int main(int argc, char** argv) {
         g_refuse_pinned = g_refuse_device = false;
         check_grads("with memory again", total);
         expect(g_copies == 12, "gathered");
+    } else if (scenario == "no_memory_for_another_rank") {
+        // each allocation of the new factors is refused in turn (ft_alloc asks twice): the adapter stays what it was
+        check_grads("before", total);
+        for (int granted = 0; granted < 4; granted++) {
+            g_device_grants = granted;
+            expect(set_lora(kLinear[0], 128, 128, 8) == FT_ERR_OOM, "refused");
+            g_device_grants = -1;
+            expect(ft_pool_trim(ctx) == FT_OK, "trim");
+            check_grads("after a refusal", total);
+        }
+        expect(set_lora(kLinear[0], 128, 128, 8) == FT_OK, "another rank");
+        check_grads("after another rank", total + 4 * (128 + 128));
     } else {
         printf("no such scenario\n");
         return 2;

@@ -29,7 +29,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["whole", "no_host_memory_for_the_list", "no_pinned_memory", "no_device_memory"])
+@pytest.mark.parametrize("scenario", ["whole", "no_host_memory_for_the_list", "no_pinned_memory", "no_device_memory",
+                                      "no_memory_for_another_rank"])
 def test_host_half_with_refused_memory(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
