@@ -923,8 +923,8 @@ struct StepControl {
     int apply;       // 0 when the norm is not finite: the update is skipped
 };
 
-// Pieces of many small tensors into one array (w <- g), which may be pinned host memory: 512 gradients of an adapter set
-// one copy and wait each took 4.5 ms of a 20 ms step, this and one wait 0.2 ms.
+// Pieces of many small tensors into one array (w <- g), which may be pinned host memory: the 256 gradients (1.64 M values)
+// of rank-8 adapters on q/k/v/o of the 360M shape take 4.38 ms to read with a copy and a wait each, 0.53 ms this way.
 __global__ __launch_bounds__(256) void multi_copy_kernel(const ft_segment* __restrict__ segs) {
     const ft_segment s = segs[blockIdx.x];
     for (uint32_t i = threadIdx.x; i < s.n; i += 256) s.w[i] = s.g[i];
@@ -1183,6 +1183,7 @@ int ft_internal_multi_grad_norm(ft_context* ctx, const ft_segment* segs_dev, siz
 
 int ft_internal_multi_copy(ft_context* ctx, const ft_segment* segs_dev, size_t nseg) {
     if (nseg == 0) return FT_OK;
+    ft_prof_scope prof(ctx, "multi_copy_kernel", 0.0, 8.0 * (double)nseg * FT_SUM_SQUARES_CHUNK);
     hipLaunchKernelGGL(multi_copy_kernel, dim3((unsigned)nseg), dim3(256), 0, ctx->stream, segs_dev);
     FT_LAUNCH_CHECK();
     return FT_OK;

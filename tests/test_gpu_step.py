@@ -1306,3 +1306,50 @@ def test_all_gradients_at_once_match_single_reads(trainable_base):
             assert any(np.any(v != 0) for v in got.values())
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("trainable_base, H, F, gathers", [(False, 256, 320, 2), (True, 1024, 4352, 0)])
+def test_all_gradients_read_after_each_of_two_steps(trainable_base, H, F, gathers):
+    """The second read goes through the table of the first and brings the second step's gradients; more than 16 Mi
+    values (17.6 M with the trainable base) come one copy per tensor. The library's own profile tells which it was."""
+    import ctypes as C
+    from ferrotensor_amd import HipContext
+    from ferrotensor_amd.trainer import Lfm2Model, ModelConfig, Trainer
+    rng = np.random.default_rng(11)
+    V, heads = 64, H // 64
+    ctx = HipContext(0)
+    try:
+        m = Lfm2Model(ctx, ModelConfig(vocab_size=V, hidden_size=H, intermediate_size=F, num_hidden_layers=1,
+                                       num_attention_heads=heads, num_key_value_heads=heads, tie_word_embeddings=True,
+                                       f16_linears=not trainable_base, trainable_base=trainable_base))
+        m.set_tensor("model.embed_tokens.weight", rng.standard_normal((V, H), dtype=np.float32))
+        for n in ("model.norm", "model.layers.0.input_layernorm", "model.layers.0.post_attention_layernorm"):
+            m.set_tensor(n + ".weight", np.ones(H, np.float32))
+        for name in m.linear_prefixes(["q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj"]):
+            i, o = m.linear_dims(name)
+            m.set_tensor(name + ".weight", rng.standard_normal((o, i), dtype=np.float32) * np.float32(0.05))
+            if not trainable_base:
+                m.set_lora(name, rng.standard_normal((i, 8)) * 0.05, rng.standard_normal((8, o)) * 0.05, 8.0)
+        named = m.named_params()
+        assert (sum(k for _, k in named) > 16 << 20) == (gathers == 0)
+        tr = Trainer(m, lr=1e-3, weight_decay=0.0)
+        lib, last = ctx._lib, None
+        assert lib.ft_profile_begin(ctx.handle) == 0
+        for _ in range(2):
+            rows = rng.integers(0, V, (2, 32)).astype(np.uint32)
+            tr.train_chunk(rows, np.roll(rows, -1, 1), np.ones((2, 32), np.uint8))
+            got = m.grads()
+            for i, (n, k) in enumerate(named):
+                np.testing.assert_array_equal(got[n], m._read(m._lib.ft_model_read_grad, i, k))
+            flat = np.concatenate([got[n] for n, _ in named])
+            assert np.any(flat != 0) and (last is None or np.any(flat != last))
+            last = flat
+        n, launches = C.c_size_t(), {}
+        assert lib.ft_profile_end(ctx.handle, C.byref(n)) == 0
+        for i in range(n.value):
+            name, count = C.c_char_p(), C.c_uint64()
+            assert lib.ft_profile_kernel(ctx.handle, i, C.byref(name), C.byref(count), None, None, None) == 0
+            launches[name.value.decode()] = count.value
+        assert launches["multi_adamw_kernel"] == 2 and launches.get("multi_copy_kernel", 0) == gathers
+    finally:
+        ctx.close()
