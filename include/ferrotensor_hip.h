@@ -427,8 +427,10 @@ int ft_model_read_param(ft_model* m, size_t index, float* out_host);
  * apply_checkpoint does to an existing tensor (ferrotensor-trainer/src/checkpoint.rs:275-283). */
 int ft_model_write_param(ft_model* m, size_t index, const float* host);
 int ft_model_read_grad(ft_model* m, size_t index, float* out_host);
-/* All gradients one after the other, in the order of the parameters, with one wait: out_host holds
- * as many values as the numel of all parameters add up to (ft_model_param_info). */
+/* All gradients one after the other, in the order of the parameters: out_host holds as many values as
+ * the numel of all parameters add up to (ft_model_param_info). Up to 16 Mi values they come through
+ * pinned memory with one wait; the model keeps that memory until its set of parameters changes. Above,
+ * or where that memory is refused, with one wait per tensor. */
 int ft_model_read_grads(ft_model* m, float* out_host);
 /* Lfm2Model::forward_batch (lfm.rs:590-623): logits [B*S, vocab] to the host. */
 int ft_model_forward_logits(ft_model* m, const uint32_t* rows, size_t B, size_t S, float* logits_host);
