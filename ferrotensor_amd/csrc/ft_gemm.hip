@@ -17,6 +17,7 @@
 // and dB products), operands read straight from global memory into MFMA
 // operand registers, the reduction dimension split across the 4 waves.
 #include "ft_common.h"
+#include "ft_split.h"
 #include "ft_thin.h"
 
 #include <cmath>
@@ -1997,6 +1998,8 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     FT_CHECK_ARG(out && (K == 0 || (a && b)), "%s: NULL operand", who);
     FT_CHECK_ARG((a2 == nullptr) == (b2 == nullptr), "%s: a2 and b2 must come together", who);
     FT_CHECK_ARG(!(layout == 2 && (half_b || a2)), "%s: unsupported operand combination", who);
+    if (!ctx->f32_chain && ft_split_gemm_ok(layout, M, K, N, half_b))
+        return ft_split_gemm(ctx, layout, half_b, a, b, out, M, K, N, K2 > 0 ? a2 : nullptr, K2 > 0 ? b2 : nullptr, K2, add);
     GemmArgs p{};
     p.a = a;
     p.b = b;

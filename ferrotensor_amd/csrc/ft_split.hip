@@ -1,0 +1,491 @@
+// f32 matrix products on the bf16 matrix instructions, without giving up f32 operands: every f32 value is the exact
+// sum of three bf16 numbers (8 + 8 + 8 significant bits, f32's own exponent range, so no scaling and no special rows),
+// every f16 weight of two, and a product of two values is the sum of the products of their parts. With an f32 b six of
+// the nine are kept, with an f16 b five of the six: what is left out is below 2^-25 of the product it belongs to, under
+// f32's own rounding of that product. Sums are f32, in the matrix unit. v_mfma_f32_32x32x16_bf16 does eight times the
+// products of v_mfma_f32_32x32x2_f32 in half its cycles: 2.7 (3.2) times the f32 rate after six (five) of them.
+//
+// What the split cannot hold (infinities, and finite values within 2^-8 of the largest f32, whose first part would round
+// to infinity) leaves a sum that is not finite; a wave that ends with one makes its share again with f32 products, so
+// infinities and NaN come out as f32 products give them. The rank-r term and what K leaves after its last whole step of
+// 16 take the f32 instruction too.
+//
+// Bound: VALU and matrix unit together. 8192 x 2048 x 2048 with f16 b: 340 us (202 TFLOP/s; f32 products 518), of them
+// 286 with no operand fetched at all; 2048 x 2560 x 2048 with f32 b: 127 us (160 with f32 products). Relative error
+// against f64 there 3.1e-7 (8.1e-7) and 3.9e-7 (9.1e-7).
+//
+// Work split: the waves of a workgroup share one output tile along K (wave w takes K steps w, w + KW, ...), because an
+// operand is then split into its parts by one wave only: with the usual 2 x 2 waves over the tile every value would be
+// split twice, and the splitting (11 VALU instructions for two values) is as long as the products (64 x 64 x 16: 176
+// VALU instructions of 4 cycles beside 24 MFMAs of 32). A wave fetches its own operand slabs (global -> registers one
+// step ahead -> its own part of LDS -> MFMA operand order), so the K loop has no barrier; the KW sums meet in LDS at the
+// end, in wave order. Nothing depends on alignment but the speed of the loads.
+#include "ft_common.h"
+#include "ft_split.h"
+
+#include <cmath>
+
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+// 16 bytes from any 4-byte (f32) or 2-byte (f16) boundary
+struct __attribute__((packed, aligned(4))) Load16 { uintx4 v; };
+struct __attribute__((packed, aligned(2))) Load16h { uintx4 v; };
+
+struct SplitArgs {
+    const char* a;
+    const char* b;
+    float* out;
+    const float* add;   // optional [M, N] term (may be `out` itself)
+    const float* a2;    // rank-r term: [M, K2] and [K2, N] (b k-major) or [N, K2], or NULL
+    const float* b2;
+    int M, N, K, K2;
+    int lda, ldb;
+    int tiles_m, tiles_n, panel, xcds;
+    int steps;          // K steps of 16 that may be fetched in whole 16-byte groups
+};
+
+// Two values into their three (or two) bf16 parts, packed as the matrix operand wants them.
+__device__ __forceinline__ unsigned pack2(float x, float y) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x, y}, bf16x2));
+}
+// The two halves of a packed pair as f32. (v_dot2_f32_bf16 with (-1, 0) would unpack and subtract in one instruction,
+// but it runs in the matrix unit: measured, an MFMA and eight of them take as long as both apart, with eight of these
+// they take 20 ns where the MFMA alone takes 16.)
+__device__ __forceinline__ float low_half(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float high_half(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
+
+// One operand: F blocks of 32 rows (of a; columns of b) by 16 k per step.
+//   KM = false: element (row, k) at base[row * ld + k];  KM = true: at base[k * ld + row].
+// Tile row of block f, lane l32: KM with two blocks: 2 * l32 + f (one load fetches both), else 32 * f + l32.
+// A lane holds k = 8 * half + e, e = 0..7.
+template <int F, bool KM, bool HALF>
+struct Operand {
+    using Value = typename std::conditional<HALF, _Float16, float>::type;
+    static constexpr int ROWS = 32 * F;
+    static constexpr int ES = HALF ? 2 : 4;
+    static constexpr int LOADS = ROWS * 16 * ES / 1024;            // 16-byte loads per lane and step
+    static constexpr int PAD = HALF && KM && F == 2 ? 128 : 0;     // behind k = 7: the two halves of a wave read k and k + 8
+    static constexpr int BYTES = ROWS * 16 * ES + PAD;
+    uintx4 g[LOADS];
+    unsigned off[LOADS];   // byte offset from the step's base
+
+    __device__ __forceinline__ static int tile_row(int f, int l32) { return KM && F == 2 ? 2 * l32 + f : 32 * f + l32; }
+
+    __device__ __forceinline__ void set_offsets(int row0, int rows, int ld, int lane) {
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            if constexpr (!KM) {
+                constexpr int LPR = HALF ? 2 : 4;                  // lanes per row
+                int row = row0 + (64 / LPR) * i + lane / LPR;
+                row = row < rows ? row : rows - 1;                 // values of rows past the end are never stored
+                off[i] = ((unsigned)row * (unsigned)ld + (unsigned)((lane % LPR) * (16 / ES))) * ES;
+            } else {
+                constexpr int LPK = ROWS * ES / 16;                // lanes per k
+                int row = row0 + (lane % LPK) * (16 / ES);
+                row = row < rows ? row : row0;                     // a group past the end re-reads the tile's first
+                off[i] = ((unsigned)((64 / LPK) * i + lane / LPK) * (unsigned)ld + (unsigned)row) * ES;
+            }
+        }
+    }
+    __device__ __forceinline__ void fetch(const char* base) {
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            if constexpr (HALF) g[i] = reinterpret_cast<const Load16h*>(base + off[i])->v;
+            else g[i] = reinterpret_cast<const Load16*>(base + off[i])->v;
+        }
+    }
+    __device__ __forceinline__ void stash(char* lds, int lane) const {
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            int at;
+            if constexpr (!KM && !HALF) {       // 64-byte rows, 16-byte chunk c at c ^ (row >> 2 & 3): no bank conflicts
+                const int row = 16 * i + lane / 4;
+                at = row * 64 + (((lane % 4) ^ ((row >> 2) & 3)) * 16);
+            } else if constexpr (!KM) {         // 32-byte rows, chunk c at c ^ (row >> 3 & 1)
+                const int row = 32 * i + lane / 2;
+                at = row * 32 + (((lane % 2) ^ ((row >> 3) & 1)) * 16);
+            } else {
+                at = i * 1024 + lane * 16 + (PAD && i > 0 ? PAD : 0);
+            }
+            *reinterpret_cast<uintx4*>(lds + at) = g[i];
+        }
+    }
+    __device__ __forceinline__ static void frags(const char* lds, int l32, int half, Value (&x)[F][8]) {
+        if constexpr (!KM && !HALF) {
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                const int row = 32 * f + l32;
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const floatx4 v = *reinterpret_cast<const floatx4*>(lds + row * 64 + (((2 * half + c) ^ ((row >> 2) & 3)) * 16));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[f][4 * c + e] = v[e];
+                }
+            }
+        } else if constexpr (!KM) {
+#pragma unroll
+            for (int f = 0; f < F; f++) {
+                const int row = 32 * f + l32;
+                const halfx8 v = *reinterpret_cast<const halfx8*>(lds + row * 32 + ((half ^ ((row >> 3) & 1)) * 16));
+#pragma unroll
+                for (int e = 0; e < 8; e++) x[f][e] = v[e];
+            }
+        } else {
+            const char* p = lds + half * (8 * ROWS * ES + PAD);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const char* q = p + e * (ROWS * ES);
+                if constexpr (F == 2 && !HALF) {
+                    const floatx2 v = *reinterpret_cast<const floatx2*>(q + l32 * 8);
+                    x[0][e] = v.x;
+                    x[F - 1][e] = v.y;
+                } else if constexpr (F == 2) {
+                    const halfx2 v = *reinterpret_cast<const halfx2*>(q + l32 * 4);
+                    x[0][e] = v.x;
+                    x[F - 1][e] = v.y;
+                } else if constexpr (!HALF) {
+                    x[0][e] = *reinterpret_cast<const float*>(q + l32 * 4);
+                } else {
+                    x[0][e] = *reinterpret_cast<const _Float16*>(q + l32 * 2);
+                }
+            }
+        }
+    }
+};
+
+// FM x FN blocks of 32 x 32 per wave (and workgroup), KW waves along K.
+template <int FM, int FN, int KW, bool A_KM, bool B_KM, bool B_HALF>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
+    constexpr int TM = 32 * FM, TN = 32 * FN;
+    using OpA = Operand<FM, A_KM, false>;
+    using OpB = Operand<FN, B_KM, B_HALF>;
+    constexpr int SLAB = OpA::BYTES + OpB::BYTES;
+    constexpr int REGION = SLAB > TM * TN * 4 ? SLAB : TM * TN * 4;   // a wave's slab, later its sums
+    __shared__ __attribute__((aligned(16))) char lds[KW * REGION];
+
+    // Tile order as in gemm_async_kernel: XCD x takes the x-th contiguous chunk of a panel order.
+    int bid = (int)blockIdx.x;
+    if (g.xcds == 8) {
+        const int total = (int)gridDim.x, x = bid & 7, q = total >> 3, r = total & 7;
+        bid = x * q + (x < r ? x : r) + (bid >> 3);
+    }
+    const int per_panel = g.tiles_m * g.panel;
+    const int last = (g.tiles_n - 1) / g.panel;
+    int pnl = bid / per_panel;
+    pnl = pnl < last ? pnl : last;
+    const int rem = bid - pnl * per_panel;
+    const int width = pnl == last ? g.tiles_n - last * g.panel : g.panel;
+    const int m0 = (rem / width) * TM, n0 = (pnl * g.panel + rem % width) * TN;
+
+    const int lane = threadIdx.x % 64, l32 = lane % 32, half = lane / 32;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+    char* const slab_a = lds + wave * REGION;
+    char* const slab_b = slab_a + OpA::BYTES;
+
+    OpA oa;
+    OpB ob;
+    oa.set_offsets(m0, g.M, g.lda, lane);
+    ob.set_offsets(n0, g.N, g.ldb, lane);
+    const long a_step = A_KM ? 64L * g.lda : 64L;
+    const long b_step = (B_KM ? 16L * g.ldb : 16L) * OpB::ES;
+    const int steps = g.steps;
+    using BT = typename std::conditional<B_HALF, _Float16, float>::type;
+    if (wave < steps) {
+        oa.fetch(g.a + wave * a_step);
+        ob.fetch(g.b + wave * b_step);
+    }
+
+    floatx16 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+    // Up to 16 k from k0, element by element, on the f32 instruction: what K leaves after its whole steps, and the
+    // rank-r term. The second half of a wave takes the odd k; a k past the end reads as zero.
+    auto f32_rest = [&](const float* pa, bool a_km, int lda, const auto* pb, bool b_km, int ldb, int k0, int k_end) {
+        float xa[FM][8], xb[FN][8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int k = k0 + 2 * e + half;
+            const bool in = k < k_end;
+            const int kc = in ? k : k0;
+#pragma unroll
+            for (int i = 0; i < FM; i++) {
+                int row = m0 + OpA::tile_row(i, l32);
+                row = row < g.M ? row : g.M - 1;
+                const float v = pa[a_km ? (long)kc * lda + row : (long)row * lda + kc];
+                xa[i][e] = in ? v : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                int col = n0 + OpB::tile_row(j, l32);
+                col = col < g.N ? col : g.N - 1;
+                const float v = (float)pb[b_km ? (long)kc * ldb + col : (long)col * ldb + kc];
+                xb[j][e] = in ? v : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (k0 + 2 * e >= k_end) break;
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[i][e], xb[j][e], acc[i][j], 0, 0, 0);
+        }
+    };
+    constexpr int PB = B_HALF ? 2 : 3;
+    constexpr int PRODUCTS = PB == 3 ? 6 : 5, MFMAS = PRODUCTS * FM * FN;
+    constexpr int PAIRS = 4 * (FM + FN);
+    struct Parts {
+        uintx4 a[FM][3], b[FN][PB];
+    };
+    // MFMA n of a step: smallest products first, the blocks of a product in turn (no two neighbours on one accumulator).
+    auto mfma = [&](const Parts& p, int n) {
+        constexpr int U3[6] = {2, 0, 1, 1, 0, 0}, V3[6] = {0, 2, 1, 0, 1, 0};
+        constexpr int U2[6] = {2, 1, 1, 0, 0, 0}, V2[6] = {0, 1, 0, 1, 0, 0};
+        const int q = n / (FM * FN), i = n / FN % FM, j = n % FN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, p.a[i][PB == 3 ? U3[q] : U2[q]]),
+                                                            __builtin_bit_cast(bf16x8, p.b[j][PB == 3 ? V3[q] : V2[q]]),
+                                                            acc[i][j], 0, 0, 0);
+    };
+    auto stash = [&]() {
+        oa.stash(slab_a, lane);
+        ob.stash(slab_b, lane);
+    };
+    auto fetch = [&](int s) {
+        s = s < steps ? s : steps - 1;   // past the end: a step that nobody multiplies
+        oa.fetch(g.a + s * a_step);
+        ob.fetch(g.b + s * b_step);
+    };
+    // The slab of this wave's next step, out of LDS and into parts (`next`), beside the products of the current one
+    // (`p`). A wave issues a VALU instruction every 8 cycles at best, an MFMA keeps the matrix unit for 32: they are
+    // dealt out in turn, a pair of values a slot, its three stages in three slots (a dot product's result may not be
+    // read by the next few instructions).
+    auto split = [&](Parts& next, const Parts& p, int after, auto beside) __attribute__((always_inline)) {
+        constexpr bool BESIDE = decltype(beside)::value;   // false: nothing to multiply yet
+        typename OpA::Value xa[FM][8];
+        typename OpB::Value xb[FN][8];
+        OpA::frags(slab_a, l32, half, xa);
+        OpB::frags(slab_b, l32, half, xb);
+        float u[PAIRS], v[PAIRS];
+        constexpr int SLOTS = PAIRS + 2;
+        constexpr int AHEAD = FM * FN;   // MFMAs over the latency of the LDS reads
+        if constexpr (BESIDE) {
+#pragma unroll
+            for (int n = 0; n < AHEAD; n++) mfma(p, n);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int s = 0; s < SLOTS; s++) {
+            if (s == SLOTS / 3) {   // the slab has been read: the one after it, fetched a step ago, takes its place
+                stash();
+                fetch(after);
+            }
+#pragma unroll
+            for (int ph = 0; ph < 3; ph++) {
+                const int t = s - ph;
+                if (t < 0 || t >= PAIRS) continue;
+                const bool of_a = t < 4 * FM;
+                const int blk = (of_a ? t : t - 4 * FM) / 4, e = t % 4;
+                if (!of_a && ph >= PB) continue;
+                if (ph == 0) {
+                    u[t] = of_a ? xa[of_a ? blk : 0][2 * e] : (float)xb[of_a ? 0 : blk][2 * e];
+                    v[t] = of_a ? xa[of_a ? blk : 0][2 * e + 1] : (float)xb[of_a ? 0 : blk][2 * e + 1];
+                }
+                const unsigned q = pack2(u[t], v[t]);
+                if (of_a) next.a[blk][ph][e] = q;
+                else next.b[blk][ph < PB ? ph : 0][e] = q;
+                if (ph + 1 < (of_a ? 3 : PB)) {
+                    u[t] -= low_half(q);
+                    v[t] -= high_half(q);
+                }
+            }
+            if constexpr (BESIDE) {
+#pragma unroll
+                for (int n = AHEAD + (MFMAS - AHEAD) * s / SLOTS; n < AHEAD + (MFMAS - AHEAD) * (s + 1) / SLOTS; n++) mfma(p, n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    if (wave < steps) {
+        auto finish = [&](const Parts& p) __attribute__((always_inline)) {
+#pragma unroll
+            for (int n = 0; n < MFMAS; n++) mfma(p, n);
+        };
+        Parts p0, p1;   // by turns: copying would be two VALU instructions a slot
+        stash();
+        fetch(wave + KW);
+        split(p0, p0, wave + 2 * KW, std::false_type{});
+        auto step = [&](int s, Parts& next, const Parts& now) __attribute__((always_inline)) {
+            split(next, now, s + 2 * KW, std::true_type{});
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int s = wave + KW;
+#pragma unroll 1
+        for (; s + KW < steps; s += 2 * KW) {
+            step(s, p1, p0);
+            step(s + KW, p0, p1);
+        }
+        if (s < steps) {
+            step(s, p1, p0);
+            finish(p1);
+        } else {
+            finish(p0);
+        }
+    }
+    // The waves with the fewest whole steps are the last ones.
+    auto rest = [&]() {
+        if (g.a2 && wave == KW - 1)
+            for (int k = 0; k < g.K2; k += 16)
+                f32_rest(g.a2, false, g.K2, g.b2, B_KM, B_KM ? g.N : g.K2, k, g.K2);
+        if (steps * 16 < g.K && wave == KW - 2)
+            for (int k = steps * 16; k < g.K; k += 16)
+                f32_rest(reinterpret_cast<const float*>(g.a), A_KM, g.lda, reinterpret_cast<const BT*>(g.b), B_KM, g.ldb, k, g.K);
+    };
+    rest();
+    // A sum that is not finite: an operand was not, or one of its parts, or the sum itself overflowed. This wave's share
+    // is made again with f32 products, which say which.
+    float zero = 0.0f;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) zero = fmaf(acc[i][j][r], 0.0f, zero);
+    if (__builtin_expect(__any(zero != 0.0f), 0)) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+        for (int s = wave; s < steps; s += KW)
+            f32_rest(reinterpret_cast<const float*>(g.a), A_KM, g.lda, reinterpret_cast<const BT*>(g.b), B_KM, g.ldb, 16 * s, 16 * s + 16);
+        rest();
+    }
+
+    // Every wave's sums into its own region, then the tile in wave order.
+    constexpr bool PAIRED = B_KM && FN == 2;   // a lane holds two neighbouring columns
+    auto swz = [](int row) { return TN == 64 && !PAIRED ? (((A_KM && FM == 2 ? row >> 3 : row >> 2) & 1) << 5) : 0; };
+    float* const mine = reinterpret_cast<float*>(slab_a);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = OpA::tile_row(i, (r / 4) * 8 + half * 4 + (r % 4));
+            if constexpr (PAIRED) {
+                *reinterpret_cast<floatx2*>(mine + row * TN + 2 * l32) = floatx2{acc[i][0][r], acc[i][FN - 1][r]};
+            } else {
+#pragma unroll
+                for (int j = 0; j < FN; j++) mine[row * TN + ((32 * j + l32) ^ swz(row))] = acc[i][j][r];
+            }
+        }
+    __syncthreads();
+    const bool vec = g.N % 4 == 0 && ((((uintptr_t)g.out) | ((uintptr_t)g.add)) & 15) == 0;   // uniform
+#pragma unroll 1
+    for (int q = threadIdx.x; q < TM * TN / 4; q += 64 * KW) {
+        const int row = q / (TN / 4), c4 = (q % (TN / 4)) * 4;
+        const float* src = reinterpret_cast<const float*>(lds) + row * TN + (c4 ^ swz(row));
+        floatx4 v = *reinterpret_cast<const floatx4*>(src);
+#pragma unroll
+        for (int w = 1; w < KW; w++) v += *reinterpret_cast<const floatx4*>(src + w * (REGION / 4));
+        const int m = m0 + row, n = n0 + c4;
+        if (m >= g.M || n >= g.N) continue;
+        const long o = (long)m * g.N + n;
+        if (vec) {
+            if (g.add) v += *reinterpret_cast<const floatx4*>(g.add + o);
+            *reinterpret_cast<floatx4*>(g.out + o) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < g.N) g.out[o + e] = g.add ? v[e] + g.add[o + e] : v[e];
+        }
+    }
+}
+
+template <int FM, int FN, int KW>
+void launch(ft_context* ctx, const SplitArgs& g, int layout, bool half_b) {
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n)), block(64 * KW);
+    if (layout == 0 && half_b)
+        hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, false, true, true>), grid, block, 0, ctx->stream, g);
+    else if (layout == 0)
+        hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, false, true, false>), grid, block, 0, ctx->stream, g);
+    else if (layout == 1 && half_b)
+        hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, false, false, true>), grid, block, 0, ctx->stream, g);
+    else if (layout == 1)
+        hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, false, false, false>), grid, block, 0, ctx->stream, g);
+    else
+        hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, true, true, false>), grid, block, 0, ctx->stream, g);
+}
+
+}  // namespace
+
+bool ft_split_gemm_ok(int layout, size_t M, size_t K, size_t N, bool half_b) {
+    if (M < 4 || N < 8 || K < 32) return false;   // whole 16-byte groups in a row of either operand
+    // Per-lane operand offsets are 32-bit byte offsets from a uniform base.
+    const double es = half_b ? 2.0 : 4.0, lim = 4294967296.0;
+    const double a_span = 4.0 * (layout == 2 ? 17.0 * (double)M : ((double)M + 1) * (double)K);
+    const double b_span = es * (layout == 1 ? ((double)N + 1) * (double)K : 17.0 * (double)N);
+    return a_span < lim && b_span < lim;
+}
+
+int ft_split_gemm(ft_context* ctx, int layout, bool half_b, const float* a, const void* b, float* out, size_t M,
+                  size_t K, size_t N, const float* a2, const float* b2, size_t K2, const float* add) {
+    SplitArgs g{};
+    g.a = reinterpret_cast<const char*>(a);
+    g.b = static_cast<const char*>(b);
+    g.out = out;
+    g.add = add;
+    g.a2 = K2 > 0 ? a2 : nullptr;
+    g.b2 = K2 > 0 ? b2 : nullptr;
+    g.M = (int)M;
+    g.N = (int)N;
+    g.K = (int)K;
+    g.K2 = (int)K2;
+    g.lda = layout == 2 ? (int)M : (int)K;
+    g.ldb = layout == 1 ? (int)K : (int)N;
+    // A 16-byte group that runs past its row's end reads the next row's start: not in the last step of a matrix whose
+    // rows are not whole groups (its last row has no next one).
+    const bool whole = (layout != 2 || M % 4 == 0) && (layout == 1 || N % (half_b ? 8 : 4) == 0);
+    g.steps = (int)((whole ? K : K - 1) / 16);
+    g.xcds = ctx->num_cus % 8 == 0 && ctx->num_cus >= 64 ? 8 : 1;
+    const size_t cus = (size_t)ctx->num_cus;
+    // Tile and waves, measured on 256 CUs (us, f16 b unless said; 64 x 64 by 4 / by 8 waves, 32 x 64 by 4, 32 x 32 by 8):
+    //   2048 x 960 x 960  (M x K x N, 480 tiles of 64 x 64)   24.5 / 29.1 / 27.4 / 36.1   with f32 products 35.2
+    //   700 x 1024 x 1024 (176)                               15.0 / 13.6 / 15.2 / 16.0                     27.3
+    //   257 x 733 x 1001  (80, f32 b)                         13.9 / 13.3 / 10.1 / 10.7                     45.5
+    //   96 x 960 x 960    (30)                                13.2 / 12.4 /  9.9 /  6.9                     11.2
+    // Above one tile a CU two workgroups of four waves share a CU; up to there eight waves hide a tile's latencies; with
+    // half the CUs idle smaller tiles reach more of them. With under 8 K steps (8192 x 64 x 5120) two waves: 72 (four
+    // 108, f32 products 76).
+    const size_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64), tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
+    const int tm = tiles64 * 2 > cus ? 64 : 32, tn = tm == 64 || tiles32 > cus ? 64 : 32;
+    g.tiles_m = (int)((M + tm - 1) / tm);
+    g.tiles_n = (int)((N + tn - 1) / tn);
+    int panels = (int)((double)g.tiles_n / 10.0 + 0.5);
+    if (panels < 1) panels = 1;
+    g.panel = (g.tiles_n + panels - 1) / panels;
+    char name[64];
+    snprintf(name, sizeof(name), "gemm_split_kernel<%d, %d, %d, %s>", tm, tn, layout, half_b ? "true" : "false");
+    ft_prof_scope prof(ctx, name, 2.0 * M * (double)N * ((double)K + (double)(g.a2 ? K2 : 0)),
+                       4.0 * M * (double)K + (half_b ? 2.0 : 4.0) * N * (double)K + 4.0 * M * (double)N);
+    if (tm == 64 && tiles64 > cus && g.steps < 8) launch<2, 2, 2>(ctx, g, layout, half_b);
+    else if (tm == 64 && tiles64 > cus) launch<2, 2, 4>(ctx, g, layout, half_b);
+    else if (tm == 64) launch<2, 2, 8>(ctx, g, layout, half_b);
+    else if (tn == 64) launch<1, 2, 4>(ctx, g, layout, half_b);
+    else launch<1, 1, 8>(ctx, g, layout, half_b);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}

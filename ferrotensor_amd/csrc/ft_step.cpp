@@ -449,6 +449,13 @@ struct DeferScope {
 };
 
 // y = x @ W (+ (scale * x @ A) @ B) (+ bias) (+ residual), keeping t = scale * x @ A for backward.
+// A training step's products keep the f32 matrix instruction's rounding (see ft_context::f32_chain).
+struct ChainScope {
+    ft_context* ctx;
+    explicit ChainScope(ft_context* c) : ctx(c) { ctx->f32_chain = true; }
+    ~ChainScope() { ctx->f32_chain = false; }
+};
+
 // `defer` (optional): the product may leave its K shares unadded for the caller's next kernel.
 int linear_forward(ft_context* ctx, LinearW& l, const float* x, float* t, float* y, size_t T,
                    const float* residual = nullptr, ft_deferred_sum* defer = nullptr) {
@@ -1563,6 +1570,7 @@ int ft_trainer_train_chunk(ft_trainer* t, const uint32_t* rows, const uint32_t* 
             if (per_sequence_loss)
                 for (size_t s = 0; s < B; s++) per_sequence_loss[s] = 0.0f;
         } else {
+            ChainScope chain(ctx);
             FT_TRY(stage_chunk(m, rows, B, S, &head, &tg, &wt));
             FT_TRY(model_forward(m, B, S));
             // Loss + d loss / d logits in place, with the backward seed

@@ -1,0 +1,132 @@
+"""Products on bf16 parts (ft_split.hip) at the edges of their tiles, K steps and dispatch, against f64.
+
+Tolerance: the operands are held whole, so an element is off by the roundings of its sum alone: at most n matrix
+instructions follow each other on one accumulator (six per K step of 16, the K steps shared by at least two waves),
+then the waves' sums are added; each may be off by 2^-23 of the sum of the absolute products so far.
+"""
+import numpy as np
+import pytest
+
+from tests.gpu_util import make_ctx
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g():
+    ctx, eng = make_ctx()
+    yield ctx, eng
+    ctx.close()
+
+
+def rnd(seed, *shape, scale=1.0):
+    return (np.random.default_rng(seed).standard_normal(shape) * scale).astype(np.float32)
+
+
+def up(ctx, x):
+    from ferrotensor_amd import UnifiedTensor
+    return UnifiedTensor.new(ctx, np.ascontiguousarray(x), list(x.shape))
+
+
+def up16(ctx, x):
+    from ferrotensor_amd import UnifiedTensor
+    return UnifiedTensor.from_f32_as_f16(ctx, np.ascontiguousarray(x), list(x.shape))
+
+
+def empty(ctx, *shape):
+    from ferrotensor_amd import UnifiedTensor
+    return UnifiedTensor.empty(ctx, list(shape))
+
+
+def check(name, got, terms, K):
+    """terms: (a, b) pairs whose products add up."""
+    want = sum(a.astype(np.float64) @ b.astype(np.float64) for a, b in terms)
+    size = sum(np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64) for a, b in terms)
+    limit = (6 * (K // 16 // 2 + 1) + 32) * 2.0 ** -23 * size
+    got = np.asarray(got, np.float64).reshape(want.shape)
+    assert np.all(np.isfinite(got)), name
+    worst = np.max(np.abs(got - want) / np.maximum(limit, 1e-300))
+    assert worst <= 1.0, "%s: %.3g of the bound" % (name, worst)
+
+
+# Each tile and wave count of the dispatch, one row or column more and less than a tile, K with no whole step left over,
+# 1, 4, 15 left over, and rows of every alignment; K = 32 is the shortest that comes here.
+SHAPES = [(4, 32, 8), (31, 36, 33), (33, 47, 31), (32, 64, 32), (100, 333, 517), (257, 733, 1001), (65, 96, 63),
+          (700, 161, 1024), (1023, 100, 640), (1025, 64, 1100), (1100, 127, 1029), (1088, 576, 1152), (5, 2561, 9)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_f32_layouts(g, M, K, N):
+    ctx, eng = g
+    a, b = rnd(M + K, M, K), rnd(N + K, K, N)
+    out = empty(ctx, M, N)
+    for name, run in (("a@b", lambda: eng.matmul(ctx, up(ctx, a), up(ctx, b), out)),
+                      ("a@bT", lambda: eng.matmul_bt(ctx, up(ctx, a), up(ctx, b.T), out)),
+                      ("aT@b", lambda: eng.matmul_at(ctx, up(ctx, a.T), up(ctx, b), out))):
+        run()
+        check("%s %dx%dx%d" % (name, M, K, N), out.to_vec(), [(a, b)], K)
+
+
+@pytest.mark.parametrize("M,K,N,r", [(4, 32, 8, 4), (33, 64, 40, 8), (17, 96, 1000, 16), (257, 736, 1000, 32), (700, 1024, 1024, 8),
+                                     (1025, 64, 1104, 16), (1100, 352, 1032, 3)])
+def test_adapted_linear_both_ways(g, M, K, N, r):
+    ctx, eng = g
+    x, w, t, b = rnd(M, M, K), rnd(K, K, N, scale=0.05), rnd(r, M, r), rnd(N, r, N)
+    dy, dt, a, res = rnd(M + 1, M, N), rnd(r + 1, M, r), rnd(K + 1, K, r), rnd(M + 2, M, K)
+    w16 = w.astype(np.float16).astype(np.float32)
+    for half in (True, False):
+        W, wv = (up16(ctx, w), w16) if half else (up(ctx, w), w)
+        y, dx = empty(ctx, M, N), empty(ctx, M, K)
+        eng.lora_linear(ctx, up(ctx, x), W, up(ctx, t), up(ctx, b), y)
+        check("y", y.to_vec(), [(x, wv), (t, b)], K)
+        eng.lora_linear_dx(ctx, up(ctx, dy), W, up(ctx, dt), up(ctx, a), dx, residual=up(ctx, res))
+        check("dx", dx.to_vec(), [(dy, wv.T), (dt, a.T), (res, np.eye(K, dtype=np.float32))], N)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_wide_range_of_values_in_one_row(g, half):
+    """Every f32 exponent that f32 products hold: no scale per row, so an outlier costs its neighbours nothing."""
+    ctx, eng = g
+    M, K, N = 96, 192, 96
+    rng = np.random.default_rng(3)
+    a = (rnd(1, M, K) * np.exp2(rng.integers(-60, 40, (M, K)))).astype(np.float32)
+    w = rnd(2, K, N, scale=0.05)
+    w[rng.integers(0, K, 40)] = 0.0   # whole rows of zeros: the outliers that meet them must not show
+    a[:, np.all(w == 0.0, axis=1)] *= np.float32(2.0 ** 60)
+    wv = w.astype(np.float16).astype(np.float32) if half else w
+    out = empty(ctx, M, N)
+    if half:
+        eng.lora_linear(ctx, up(ctx, a), up16(ctx, w), None, None, out)
+    else:
+        eng.matmul(ctx, up(ctx, a), up(ctx, w), out)
+    check("wide", out.to_vec(), [(a, wv)], K)
+
+
+@pytest.mark.parametrize("M,N", [(70, 96), (520, 1100)])
+def test_infinities_and_nan_as_f32_products_give_them(g, M, N):
+    ctx, eng = g
+    K = 80
+    a, b = np.abs(rnd(5, M, K)) + 0.1, np.abs(rnd(6, K, N)) + 0.1
+    a[3, 7], a[9, 20], a[40, 3], a[41, 70] = np.inf, np.nan, 3.4e38, -np.inf
+    b[30, 11], b[70, 50], b[3, 60] = np.inf, 0.0, 1e-30
+    out = empty(ctx, M, N)
+    eng.matmul(ctx, up(ctx, a), up(ctx, b), out)
+    got = np.asarray(out.to_vec(), np.float32).reshape(M, N)
+    with np.errstate(all="ignore"):
+        want = np.zeros((M, N))
+        for k in range(K):
+            want = want + a[:, k:k + 1].astype(np.float64) * b[k:k + 1].astype(np.float64)
+    want[np.abs(want) > 3.4028235e38] = np.sign(want[np.abs(want) > 3.4028235e38]) * np.inf
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
+    fine = np.isfinite(want)
+    np.testing.assert_allclose(got[fine], want[fine], rtol=1e-5)
+
+
+def test_sums_the_same_twice(g):
+    ctx, eng = g
+    a, b = up(ctx, rnd(8, 300, 700)), up(ctx, rnd(9, 700, 500))
+    o1, o2 = empty(ctx, 300, 500), empty(ctx, 300, 500)
+    eng.matmul(ctx, a, b, o1)
+    eng.matmul(ctx, a, b, o2)
+    assert np.array_equal(np.asarray(o1.to_vec()).view(np.uint32), np.asarray(o2.to_vec()).view(np.uint32))
