@@ -716,29 +716,37 @@ __global__ __launch_bounds__(256) void rope_kernel(const float* __restrict__ src
 }
 
 // ---------------------------------------------------------------------------
-// Masked softmax-cross-entropy. One 1024-thread workgroup per row. grad may
-// alias logits (no __restrict__ on either), so the target logit is loaded
-// before the barrier that precedes the gradient stores. A row of up
-// to 1024*4*CACHE floats is held in registers between the reduction and the
-// gradient write, so logits are read once and the gradient written once.
+// Masked softmax-cross-entropy, one workgroup per row. grad may alias logits (no __restrict__ on either), so the
+// target logit is loaded before the barrier that precedes the gradient stores. A row of up to THREADS * 4 * CACHE floats
+// is held in registers between the reduction and the gradient write: logits are read once and the gradient written once.
+//
+// The sum of exponentials is made of kCeLanes = 1024 partial sums whatever the workgroup's size: a thread keeps one for
+// each of the 1024 / THREADS lanes it stands for, and they are added in the order of sixteen waves, so the size is a
+// matter of speed alone. Bound: memory, with the two exponentials an element close behind. 49152 columns as
+// 512 threads x 24 float4: two rows share a CU, and one row's loads and stores run under the other's arithmetic (1024
+// threads x 12 float4 take 93 registers, one row at a time); all loads of a row are issued before the first is used (a
+// load under `if (i < n4)` waits for the one before it). 1446 x 49152: 147 -> 108 us
+// (5.3 TB/s; a large copy reaches 4.7), 1000 x 1024: 8.2 -> 5.1, 2048 x 4096: 21 -> 15.
 // ---------------------------------------------------------------------------
 
-constexpr int kCeThreads = 1024;
+constexpr int kCeLanes = 1024;
 
-template <int CACHE>  // float4 per thread kept in registers (0 = stream from memory)
-__global__ __launch_bounds__(kCeThreads) void masked_ce_kernel(
+template <int THREADS, int CACHE>  // float4 per thread kept in registers (0 = stream from memory)
+__global__ __launch_bounds__(THREADS, CACHE > 12 ? 4 : 1) void masked_ce_kernel(
     const float* logits, const uint32_t* __restrict__ targets, const float* __restrict__ weights,
     float* grad, float* __restrict__ row_loss, size_t rows, size_t vocab, float grad_scale) {
-    __shared__ float red[kCeThreads / kWave];
+    constexpr int V = kCeLanes / THREADS;             // lanes a thread stands for
+    constexpr int WAVES = THREADS / kWave;
+    static_assert(CACHE % V == 0 && (CACHE > 0 || V == 1), "whole rounds of the lanes");
+    __shared__ float red[kCeLanes / kWave];
     const size_t row = blockIdx.x;
     const float* x = logits + row * vocab;
     float* gr = grad + row * vocab;
     const uint32_t tgt = targets[row];
-    const size_t n4 = vocab / 4;
+    const unsigned n4 = (unsigned)(vocab / 4);        // the host sends rows of whole float4 here
     if (tgt == FT_MASKED_CE_SKIP) {
         float4* g4 = reinterpret_cast<float4*>(gr);
-        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) g4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) gr[i] = 0.0f;
+        for (unsigned i = threadIdx.x; i < n4; i += THREADS) g4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (threadIdx.x == 0) row_loss[row] = 0.0f;
         return;
     }
@@ -746,64 +754,72 @@ __global__ __launch_bounds__(kCeThreads) void masked_ce_kernel(
     float4 cache[CACHE > 0 ? CACHE : 1];
     float m = -3.4e38f;
     if constexpr (CACHE > 0) {
+        // (a thread past the row's end re-reads its last quad, which changes no maximum and is left out of the sums)
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
-            if (i < n4) {
-                cache[j] = x4[i];
-                m = fmaxf(m, fmaxf(fmaxf(cache[j].x, cache[j].y), fmaxf(cache[j].z, cache[j].w)));
-            }
+            const unsigned i = threadIdx.x + j * THREADS;
+            cache[j] = x4[i < n4 ? i : n4 - 1];
         }
+#pragma unroll
+        for (int j = 0; j < CACHE; j++) m = fmaxf(m, fmaxf(fmaxf(cache[j].x, cache[j].y), fmaxf(cache[j].z, cache[j].w)));
     } else {
-        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
+        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
             const float4 v = x4[i];
             m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
         }
     }
-    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) m = fmaxf(m, x[i]);
-    m = block_max<kCeThreads>(m, red);
-    float se = 0.0f;
+    m = block_max<THREADS>(m, red);
+    float se[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) se[v] = 0.0f;
     if constexpr (CACHE > 0) {
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
-            if (i < n4) se += expf(cache[j].x - m) + expf(cache[j].y - m) + expf(cache[j].z - m) + expf(cache[j].w - m);
+            const float s4 = expf(cache[j].x - m) + expf(cache[j].y - m) + expf(cache[j].z - m) + expf(cache[j].w - m);
+            if (threadIdx.x + j * THREADS < n4) se[j % V] += s4;
         }
     } else {
-        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
+        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
             const float4 v = x4[i];
-            se += expf(v.x - m) + expf(v.y - m) + expf(v.z - m) + expf(v.w - m);
+            se[0] += expf(v.x - m) + expf(v.y - m) + expf(v.z - m) + expf(v.w - m);
         }
     }
-    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) se += expf(x[i] - m);
-    se = block_sum<kCeThreads>(se, red);
-    const float log_z = m + logf(se);
+    // block_sum of kCeLanes threads: lane t + v * THREADS belongs to wave t / 64 + v * WAVES
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+        const float t = wave_sum(se[v]);
+        if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave + v * WAVES] = t;
+    }
+    __syncthreads();
+    const int l = threadIdx.x % kWave;
+    const float total = wave_sum(l < kCeLanes / kWave ? red[l] : 0.0f);
+    const float log_z = m + logf(total);
     const float w = weights[row];
     // The target logit is read before any thread overwrites it (grad may alias logits).
     const float x_t = x[tgt];
     __syncthreads();
     float4* g4 = reinterpret_cast<float4*>(gr);
-    auto one = [&](float xv, size_t i) {
+    auto one = [&](float xv, unsigned i) {
         float gv = expf(xv - log_z) * w;
-        if (i == (size_t)tgt) gv -= w;
+        if (i == tgt) gv -= w;
         return gv * grad_scale;
     };
     if constexpr (CACHE > 0) {
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
-            const size_t i = threadIdx.x + (size_t)j * kCeThreads;
+            const unsigned i = threadIdx.x + j * THREADS;
             if (i < n4) {
                 const float4 v = cache[j];
                 g4[i] = make_float4(one(v.x, 4 * i), one(v.y, 4 * i + 1), one(v.z, 4 * i + 2), one(v.w, 4 * i + 3));
             }
         }
     } else {
-        for (size_t i = threadIdx.x; i < n4; i += kCeThreads) {
+        for (unsigned i = threadIdx.x; i < n4; i += THREADS) {
             const float4 v = x4[i];
             g4[i] = make_float4(one(v.x, 4 * i), one(v.y, 4 * i + 1), one(v.z, 4 * i + 2), one(v.w, 4 * i + 3));
         }
     }
-    for (size_t i = n4 * 4 + threadIdx.x; i < vocab; i += kCeThreads) gr[i] = one(x[i], i);
     if (threadIdx.x == 0) row_loss[row] = log_z - x_t;
 }
 
@@ -1462,21 +1478,22 @@ int ft_masked_cross_entropy_weighted(ft_context* ctx, const float* logits, const
                  "ft_masked_cross_entropy_weighted: NULL argument");
     FT_CHECK_ARG(vocab > 0, "ft_masked_cross_entropy_weighted: vocab is 0");
     if (rows == 0) return FT_OK;
-    const bool vec = (vocab % 4 == 0) && aligned16(logits) && aligned16(grad);
+    const bool vec = (vocab % 4 == 0) && vocab <= 0xffffffffu && aligned16(logits) && aligned16(grad);
     const dim3 grid((unsigned)rows);
     ft_prof_scope prof(ctx, "masked_ce_kernel", 0.0, 8.0 * (double)rows * vocab);
     if (!vec) {
         hipLaunchKernelGGL(masked_ce_scalar_kernel, grid, dim3(256), 0, ctx->stream, logits, targets, weights, grad,
                            row_loss, rows, vocab, grad_scale);
-    } else if (vocab <= (size_t)kCeThreads * 4 * 4) {
-        hipLaunchKernelGGL((masked_ce_kernel<4>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
-                           grad, row_loss, rows, vocab, grad_scale);
-    } else if (vocab <= (size_t)kCeThreads * 4 * 12) {
-        hipLaunchKernelGGL((masked_ce_kernel<12>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
-                           grad, row_loss, rows, vocab, grad_scale);
     } else {
-        hipLaunchKernelGGL((masked_ce_kernel<0>), grid, dim3(kCeThreads), 0, ctx->stream, logits, targets, weights,
-                           grad, row_loss, rows, vocab, grad_scale);
+#define FT_CE(THREADS, CACHE)                                                                                         \
+    hipLaunchKernelGGL((masked_ce_kernel<THREADS, CACHE>), grid, dim3(THREADS), 0, ctx->stream, logits, targets, weights, \
+                       grad, row_loss, rows, vocab, grad_scale)
+        // the smallest workgroup that holds a row with at most 24 quads a thread; wider rows are streamed
+        if (vocab <= 256 * 4 * 4) FT_CE(256, 4);
+        else if (vocab <= 512 * 4 * 8) FT_CE(512, 8);
+        else if (vocab <= 512 * 4 * 24) FT_CE(512, 24);
+        else FT_CE(1024, 0);
+#undef FT_CE
     }
     FT_LAUNCH_CHECK();
     return FT_OK;

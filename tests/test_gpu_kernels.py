@@ -574,6 +574,11 @@ def test_masked_cross_entropy(g, rows, vocab):
     assert_close("ce loss in place", row_loss.to_numpy(), want_l)
 
 
+@pytest.mark.parametrize("rows,vocab", [(3, 4), (3, 4100), (3, 16384), (2, 49148)])
+def test_masked_cross_entropy_at_the_edges_of_its_workgroup_sizes(g, rows, vocab):
+    test_masked_cross_entropy(g, rows, vocab)
+
+
 def test_sum_squares_and_adamw(g):
     ctx, eng = g
     from ferrotensor_amd import AdamParams, UnifiedTensor
