@@ -2179,6 +2179,13 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
         batch = batch && d.w_dtype == FT_DTYPE_F16 && d.N < (1u << 30) &&
                 async_eligible(0, x, d.w, d.y, d.residual, M, K, d.N, d.t, d.b, d.r);
     }
+    bool split = !ctx->f32_chain && x && M < (1u << 30) && K < (1u << 30) && (count > 1 || any_rope);
+    for (size_t i = 0; i < count && split; i++) {
+        const ft_lora_linear_desc& d = linears[i];
+        split = d.w && d.y && d.N < (1u << 30) && d.r < (1u << 30) && d.w_dtype == linears[0].w_dtype &&
+                ft_split_gemm_ok(0, M, K, d.N, d.w_dtype == FT_DTYPE_F16);
+    }
+    if (split) return ft_split_group(ctx, x, linears, count, M, K, linears[0].w_dtype == FT_DTYPE_F16);
     if (batch && count > 1) {
         AsyncBatch g{};
         g.count = (int)count;
@@ -2250,6 +2257,9 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
     FT_CHECK_ARG(ctx && x && w_gate && w_up && gate && up && act, "ft_mlp_gate_up: NULL argument");
     FT_CHECK_ARG(w_dtype == FT_DTYPE_F32 || w_dtype == FT_DTYPE_F16, "ft_mlp_gate_up: dtype %d", w_dtype);
     if (M == 0 || N == 0) return FT_OK;
+    if (!ctx->f32_chain && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
+        ft_split_gemm_ok(0, M, K, N, w_dtype == FT_DTYPE_F16))
+        return ft_split_gate_up(ctx, x, w_gate, w_up, gate, up, act, M, K, N, w_dtype == FT_DTYPE_F16);
     const bool fused = w_dtype == FT_DTYPE_F16 && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
                        async_eligible(0, x, w_up, up, nullptr, M, K, N, nullptr, nullptr, 0) &&
                        async_eligible(0, x, w_gate, gate, nullptr, M, K, N, nullptr, nullptr, 0) && aligned16p(act);

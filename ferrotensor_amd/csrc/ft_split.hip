@@ -39,18 +39,31 @@ typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 struct __attribute__((packed, aligned(4))) Load16 { uintx4 v; };
 struct __attribute__((packed, aligned(2))) Load16h { uintx4 v; };
 
-struct SplitArgs {
-    const char* a;
+// Products that share a (q, k and v of one input) form one row of column tiles, as in gemm_async_kernel.
+constexpr int kSplitProducts = 3;
+struct SplitProduct {
     const char* b;
     float* out;
-    const float* add;   // optional [M, N] term (may be `out` itself)
-    const float* a2;    // rank-r term: [M, K2] and [K2, N] (b k-major) or [N, K2], or NULL
+    const float* add;     // optional [M, N] term (may be `out` itself)
+    const float* a2;      // rank-r term: [M, K2] and [K2, N] (b k-major) or [N, K2], or NULL
     const float* b2;
-    int M, N, K, K2;
-    int lda, ldb;
-    int tiles_m, tiles_n, panel, xcds;
-    int steps;          // K steps of 16 that may be fetched in whole 16-byte groups
+    const float2* rope;   // RoPE on the output, heads of 64 columns: (cos, sin) of [position][32], or NULL
+    int rope_seq;         // position = row % rope_seq
+    int N, ldb, K2;
+    int tile_begin;       // its first column tile
 };
+struct SplitArgs {
+    const char* a;
+    int M, K, lda;
+    int steps;            // K steps of 16 that may be fetched in whole 16-byte groups
+    int tiles_m, tiles_n, panel, xcds, count;
+    SplitProduct p[kSplitProducts];
+    // EPI = kSplitGateUp: a second b of the same shape; out = a @ b, out2 = a @ b_alt, out3 = silu(out2) * out
+    const char* b_alt;
+    float* out2;
+    float* out3;
+};
+constexpr int kSplitPlain = 0, kSplitGroup = 1, kSplitGateUp = 2;
 
 // Two values into their three (or two) bf16 parts, packed as the matrix operand wants them.
 __device__ __forceinline__ unsigned pack2(float x, float y) {
@@ -161,13 +174,17 @@ struct Operand {
     }
 };
 
-// FM x FN blocks of 32 x 32 per wave (and workgroup), KW waves along K.
-template <int FM, int FN, int KW, bool A_KM, bool B_KM, bool B_HALF>
+// FM x FN blocks of 32 x 32 per wave (and workgroup), KW waves along K. EPI: kSplitGroup takes up to three products and
+// rotates heads (64 columns wide); kSplitGateUp multiplies the same 32 columns of two matrices, side by side in the tile.
+template <int FM, int FN, int KW, bool A_KM, bool B_KM, bool B_HALF, int EPI = kSplitPlain>
 __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
+    constexpr bool DUAL = EPI == kSplitGateUp;
+    static_assert(!DUAL || FN == 2, "one block of columns of each matrix");
     constexpr int TM = 32 * FM, TN = 32 * FN;
     using OpA = Operand<FM, A_KM, false>;
-    using OpB = Operand<FN, B_KM, B_HALF>;
-    constexpr int SLAB = OpA::BYTES + OpB::BYTES;
+    using OpB = Operand<DUAL ? 1 : FN, B_KM, B_HALF>;
+    constexpr int NB = DUAL ? 2 : 1;
+    constexpr int SLAB = OpA::BYTES + NB * OpB::BYTES;
     constexpr int REGION = SLAB > TM * TN * 4 ? SLAB : TM * TN * 4;   // a wave's slab, later its sums
     __shared__ __attribute__((aligned(16))) char lds[KW * REGION];
 
@@ -183,7 +200,14 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
     pnl = pnl < last ? pnl : last;
     const int rem = bid - pnl * per_panel;
     const int width = pnl == last ? g.tiles_n - last * g.panel : g.panel;
-    const int m0 = (rem / width) * TM, n0 = (pnl * g.panel + rem % width) * TN;
+    int tn = pnl * g.panel + rem % width;
+    SplitProduct p = g.p[0];
+    if constexpr (EPI == kSplitGroup) {
+        if (g.count > 2 && tn >= g.p[2].tile_begin) p = g.p[2];
+        else if (g.count > 1 && tn >= g.p[1].tile_begin) p = g.p[1];
+        tn -= p.tile_begin;
+    }
+    const int m0 = (rem / width) * TM, n0 = tn * (DUAL ? 32 : TN);
 
     const int lane = threadIdx.x % 64, l32 = lane % 32, half = lane / 32;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
@@ -191,16 +215,19 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
     char* const slab_b = slab_a + OpA::BYTES;
 
     OpA oa;
-    OpB ob;
+    OpB ob[NB];
     oa.set_offsets(m0, g.M, g.lda, lane);
-    ob.set_offsets(n0, g.N, g.ldb, lane);
+#pragma unroll
+    for (int t = 0; t < NB; t++) ob[t].set_offsets(n0, p.N, p.ldb, lane);
+    const char* const bases[2] = {p.b, g.b_alt};
     const long a_step = A_KM ? 64L * g.lda : 64L;
-    const long b_step = (B_KM ? 16L * g.ldb : 16L) * OpB::ES;
+    const long b_step = (B_KM ? 16L * p.ldb : 16L) * OpB::ES;
     const int steps = g.steps;
     using BT = typename std::conditional<B_HALF, _Float16, float>::type;
     if (wave < steps) {
         oa.fetch(g.a + wave * a_step);
-        ob.fetch(g.b + wave * b_step);
+#pragma unroll
+        for (int t = 0; t < NB; t++) ob[t].fetch(bases[t] + wave * b_step);
     }
 
     floatx16 acc[FM][FN];
@@ -213,7 +240,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
 
     // Up to 16 k from k0, element by element, on the f32 instruction: what K leaves after its whole steps, and the
     // rank-r term. The second half of a wave takes the odd k; a k past the end reads as zero.
-    auto f32_rest = [&](const float* pa, bool a_km, int lda, const auto* pb, bool b_km, int ldb, int k0, int k_end) {
+    auto f32_rest = [&](const float* pa, bool a_km, int lda, const auto* pb, const auto* pb1, bool b_km, int ldb, int k0, int k_end) {
         float xa[FM][8], xb[FN][8];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
@@ -229,9 +256,9 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
             }
 #pragma unroll
             for (int j = 0; j < FN; j++) {
-                int col = n0 + OpB::tile_row(j, l32);
-                col = col < g.N ? col : g.N - 1;
-                const float v = (float)pb[b_km ? (long)kc * ldb + col : (long)col * ldb + kc];
+                int col = n0 + (DUAL ? l32 : OpB::tile_row(j, l32));
+                col = col < p.N ? col : p.N - 1;
+                const float v = (float)(DUAL && j == 1 ? pb1 : pb)[b_km ? (long)kc * ldb + col : (long)col * ldb + kc];
                 xb[j][e] = in ? v : 0.0f;
             }
         }
@@ -262,12 +289,14 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
     };
     auto stash = [&]() {
         oa.stash(slab_a, lane);
-        ob.stash(slab_b, lane);
+#pragma unroll
+        for (int t = 0; t < NB; t++) ob[t].stash(slab_b + t * OpB::BYTES, lane);
     };
     auto fetch = [&](int s) {
         s = s < steps ? s : steps - 1;   // past the end: a step that nobody multiplies
         oa.fetch(g.a + s * a_step);
-        ob.fetch(g.b + s * b_step);
+#pragma unroll
+        for (int t = 0; t < NB; t++) ob[t].fetch(bases[t] + s * b_step);
     };
     // The slab of this wave's next step, out of LDS and into parts (`next`), beside the products of the current one
     // (`p`). A wave issues a VALU instruction every 8 cycles at best, an MFMA keeps the matrix unit for 32: they are
@@ -278,7 +307,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
         typename OpA::Value xa[FM][8];
         typename OpB::Value xb[FN][8];
         OpA::frags(slab_a, l32, half, xa);
-        OpB::frags(slab_b, l32, half, xb);
+        if constexpr (DUAL) {
+#pragma unroll
+            for (int t = 0; t < NB; t++)
+                OpB::frags(slab_b + t * OpB::BYTES, l32, half, *reinterpret_cast<typename OpB::Value(*)[1][8]>(&xb[t]));
+        } else {
+            OpB::frags(slab_b, l32, half, xb);
+        }
         float u[PAIRS], v[PAIRS];
         constexpr int SLOTS = PAIRS + 2;
         constexpr int AHEAD = FM * FN;   // MFMAs over the latency of the LDS reads
@@ -345,14 +380,16 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
             finish(p0);
         }
     }
+    const float* const af = reinterpret_cast<const float*>(g.a);
+    const BT* const b0 = reinterpret_cast<const BT*>(p.b);
+    const BT* const b1 = reinterpret_cast<const BT*>(g.b_alt);
     // The waves with the fewest whole steps are the last ones.
     auto rest = [&]() {
-        if (g.a2 && wave == KW - 1)
-            for (int k = 0; k < g.K2; k += 16)
-                f32_rest(g.a2, false, g.K2, g.b2, B_KM, B_KM ? g.N : g.K2, k, g.K2);
+        if (!DUAL && p.a2 && wave == KW - 1)
+            for (int k = 0; k < p.K2; k += 16)
+                f32_rest(p.a2, false, p.K2, p.b2, p.b2, B_KM, B_KM ? p.N : p.K2, k, p.K2);
         if (steps * 16 < g.K && wave == KW - 2)
-            for (int k = steps * 16; k < g.K; k += 16)
-                f32_rest(reinterpret_cast<const float*>(g.a), A_KM, g.lda, reinterpret_cast<const BT*>(g.b), B_KM, g.ldb, k, g.K);
+            for (int k = steps * 16; k < g.K; k += 16) f32_rest(af, A_KM, g.lda, b0, b1, B_KM, p.ldb, k, g.K);
     };
     rest();
     // A sum that is not finite: an operand was not, or one of its parts, or the sum itself overflowed. This wave's share
@@ -371,13 +408,12 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
             for (int j = 0; j < FN; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-        for (int s = wave; s < steps; s += KW)
-            f32_rest(reinterpret_cast<const float*>(g.a), A_KM, g.lda, reinterpret_cast<const BT*>(g.b), B_KM, g.ldb, 16 * s, 16 * s + 16);
+        for (int s = wave; s < steps; s += KW) f32_rest(af, A_KM, g.lda, b0, b1, B_KM, p.ldb, 16 * s, 16 * s + 16);
         rest();
     }
 
     // Every wave's sums into its own region, then the tile in wave order.
-    constexpr bool PAIRED = B_KM && FN == 2;   // a lane holds two neighbouring columns
+    constexpr bool PAIRED = B_KM && FN == 2 && !DUAL;   // a lane holds two neighbouring columns
     auto swz = [](int row) { return TN == 64 && !PAIRED ? (((A_KM && FM == 2 ? row >> 3 : row >> 2) & 1) << 5) : 0; };
     float* const mine = reinterpret_cast<float*>(slab_a);
 #pragma unroll
@@ -393,25 +429,76 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
             }
         }
     __syncthreads();
-    const bool vec = g.N % 4 == 0 && ((((uintptr_t)g.out) | ((uintptr_t)g.add)) & 15) == 0;   // uniform
-#pragma unroll 1
-    for (int q = threadIdx.x; q < TM * TN / 4; q += 64 * KW) {
-        const int row = q / (TN / 4), c4 = (q % (TN / 4)) * 4;
+    auto sum4 = [&](int row, int c4) {
         const float* src = reinterpret_cast<const float*>(lds) + row * TN + (c4 ^ swz(row));
         floatx4 v = *reinterpret_cast<const floatx4*>(src);
 #pragma unroll
         for (int w = 1; w < KW; w++) v += *reinterpret_cast<const floatx4*>(src + w * (REGION / 4));
-        const int m = m0 + row, n = n0 + c4;
-        if (m >= g.M || n >= g.N) continue;
-        const long o = (long)m * g.N + n;
+        return v;
+    };
+    auto store4 = [&](float* out, long o, int n, bool vec, floatx4 v) {
         if (vec) {
-            if (g.add) v += *reinterpret_cast<const floatx4*>(g.add + o);
-            *reinterpret_cast<floatx4*>(g.out + o) = v;
+            *reinterpret_cast<floatx4*>(out + o) = v;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (n + e < g.N) g.out[o + e] = g.add ? v[e] + g.add[o + e] : v[e];
+                if (n + e < p.N) out[o + e] = v[e];
         }
+    };
+    if constexpr (EPI != kSplitPlain) {
+        // Two groups of four columns, 32 apart, per thread: the halves of a head, or the up and gate of a column.
+        bool both = EPI == kSplitGateUp;
+        if constexpr (EPI == kSplitGroup) both = p.rope != nullptr;
+        if (both) {
+            const bool vec = p.N % 4 == 0 && ((((uintptr_t)p.out) | ((uintptr_t)g.out2) | ((uintptr_t)g.out3)) & 15) == 0;
+#pragma unroll 1
+            for (int q = threadIdx.x; q < TM * 8; q += 64 * KW) {
+                const int row = q / 8, c4 = (q % 8) * 4;
+                const floatx4 x = sum4(row, c4), y = sum4(row, c4 + 32);
+                const int m = m0 + row, n = n0 + c4;
+                if (m >= g.M || n >= p.N) continue;
+                const long o = (long)m * p.N + n;
+                if constexpr (EPI == kSplitGateUp) {
+                    floatx4 act;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) act[e] = y[e] * (1.0f / (1.0f + __expf(-y[e]))) * x[e];
+                    store4(p.out, o, n, vec, x);
+                    store4(g.out2, o, n, vec, y);
+                    store4(g.out3, o, n, vec, act);
+                } else {
+                    // whole heads (the host checks): x holds columns i, y columns i + 32
+                    const float2* cs = p.rope + (long)(m % p.rope_seq) * 32 + c4;
+                    floatx4 lo, hi;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        lo[e] = x[e] * cs[e].x - y[e] * cs[e].y;
+                        hi[e] = x[e] * cs[e].y + y[e] * cs[e].x;
+                    }
+                    store4(p.out, o, n, vec, lo);
+                    store4(p.out, o + 32, n + 32, vec, hi);
+                }
+            }
+            return;
+        }
+    }
+    const bool vec = p.N % 4 == 0 && ((((uintptr_t)p.out) | ((uintptr_t)p.add)) & 15) == 0;   // uniform
+#pragma unroll 1
+    for (int q = threadIdx.x; q < TM * TN / 4; q += 64 * KW) {
+        const int row = q / (TN / 4), c4 = (q % (TN / 4)) * 4;
+        floatx4 v = sum4(row, c4);
+        const int m = m0 + row, n = n0 + c4;
+        if (m >= g.M || n >= p.N) continue;
+        const long o = (long)m * p.N + n;
+        if (p.add) {
+            if (vec) {
+                v += *reinterpret_cast<const floatx4*>(p.add + o);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < p.N) v[e] += p.add[o + e];
+            }
+        }
+        store4(p.out, o, n, vec, v);
     }
 }
 
@@ -430,6 +517,53 @@ void launch(ft_context* ctx, const SplitArgs& g, int layout, bool half_b) {
         hipLaunchKernelGGL((gemm_split_kernel<FM, FN, KW, true, true, false>), grid, block, 0, ctx->stream, g);
 }
 
+// Groups and gate + up: a[M, K] @ b[K, N].
+template <int FM, int KW, int EPI>
+void launch_fused(ft_context* ctx, const SplitArgs& g, bool half_b) {
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n)), block(64 * KW);
+    if (half_b)
+        hipLaunchKernelGGL((gemm_split_kernel<FM, 2, KW, false, true, true, EPI>), grid, block, 0, ctx->stream, g);
+    else
+        hipLaunchKernelGGL((gemm_split_kernel<FM, 2, KW, false, true, false, EPI>), grid, block, 0, ctx->stream, g);
+}
+
+// What the products of a launch share. `whole`: see SplitArgs::steps.
+SplitArgs split_args(ft_context* ctx, const float* a, size_t M, size_t K, size_t lda, bool whole) {
+    SplitArgs g{};
+    g.a = reinterpret_cast<const char*>(a);
+    g.M = (int)M;
+    g.K = (int)K;
+    g.lda = (int)lda;
+    // A 16-byte group that runs past its row's end reads the next row's start: not in the last step of a matrix whose
+    // rows are not whole groups (its last row has no next one).
+    g.steps = (int)((whole ? K : K - 1) / 16);
+    g.xcds = ctx->num_cus % 8 == 0 && ctx->num_cus >= 64 ? 8 : 1;
+    g.count = 1;
+    return g;
+}
+
+void set_tiles(SplitArgs& g, int tm, int tiles_n) {
+    g.tiles_m = (g.M + tm - 1) / tm;
+    g.tiles_n = tiles_n;
+    int panels = (int)((double)tiles_n / 10.0 + 0.5);
+    if (panels < 1) panels = 1;
+    g.panel = (tiles_n + panels - 1) / panels;
+}
+
+// Groups and gate + up, tiles 64 columns wide (32 of each matrix): as the plain products, half as high where whole
+// tiles leave half of the CUs idle. 96 x 960: q/k/v of 960 + 320 + 320 columns 22 -> 10.5 us, gate + up + SiLU-gate of
+// 2560 37 -> 16.6 (f32 products before).
+template <int EPI>
+int launch_group(ft_context* ctx, SplitArgs& g, int tiles_n, bool half_b) {
+    const size_t cus = (size_t)ctx->num_cus, tiles64 = (size_t)((g.M + 63) / 64) * tiles_n;
+    set_tiles(g, tiles64 * 2 > cus ? 64 : 32, tiles_n);
+    if (tiles64 > cus) launch_fused<2, 4, EPI>(ctx, g, half_b);
+    else if (tiles64 * 2 > cus) launch_fused<2, 8, EPI>(ctx, g, half_b);
+    else launch_fused<1, 8, EPI>(ctx, g, half_b);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}
+
 }  // namespace
 
 bool ft_split_gemm_ok(int layout, size_t M, size_t K, size_t N, bool half_b) {
@@ -443,24 +577,10 @@ bool ft_split_gemm_ok(int layout, size_t M, size_t K, size_t N, bool half_b) {
 
 int ft_split_gemm(ft_context* ctx, int layout, bool half_b, const float* a, const void* b, float* out, size_t M,
                   size_t K, size_t N, const float* a2, const float* b2, size_t K2, const float* add) {
-    SplitArgs g{};
-    g.a = reinterpret_cast<const char*>(a);
-    g.b = static_cast<const char*>(b);
-    g.out = out;
-    g.add = add;
-    g.a2 = K2 > 0 ? a2 : nullptr;
-    g.b2 = K2 > 0 ? b2 : nullptr;
-    g.M = (int)M;
-    g.N = (int)N;
-    g.K = (int)K;
-    g.K2 = (int)K2;
-    g.lda = layout == 2 ? (int)M : (int)K;
-    g.ldb = layout == 1 ? (int)K : (int)N;
-    // A 16-byte group that runs past its row's end reads the next row's start: not in the last step of a matrix whose
-    // rows are not whole groups (its last row has no next one).
     const bool whole = (layout != 2 || M % 4 == 0) && (layout == 1 || N % (half_b ? 8 : 4) == 0);
-    g.steps = (int)((whole ? K : K - 1) / 16);
-    g.xcds = ctx->num_cus % 8 == 0 && ctx->num_cus >= 64 ? 8 : 1;
+    SplitArgs g = split_args(ctx, a, M, K, layout == 2 ? M : K, whole);
+    g.p[0] = SplitProduct{static_cast<const char*>(b), out, add, K2 > 0 ? a2 : nullptr, K2 > 0 ? b2 : nullptr, nullptr, 1,
+                          (int)N, layout == 1 ? (int)K : (int)N, (int)K2, 0};
     const size_t cus = (size_t)ctx->num_cus;
     // Tile and waves, measured on 256 CUs (us, f16 b unless said; 64 x 64 by 4 / by 8 waves, 32 x 64 by 4, 32 x 32 by 8):
     //   2048 x 960 x 960  (M x K x N, 480 tiles of 64 x 64)   24.5 / 29.1 / 27.4 / 36.1   with f32 products 35.2
@@ -472,14 +592,10 @@ int ft_split_gemm(ft_context* ctx, int layout, bool half_b, const float* a, cons
     // 108, f32 products 76).
     const size_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64), tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
     const int tm = tiles64 * 2 > cus ? 64 : 32, tn = tm == 64 || tiles32 > cus ? 64 : 32;
-    g.tiles_m = (int)((M + tm - 1) / tm);
-    g.tiles_n = (int)((N + tn - 1) / tn);
-    int panels = (int)((double)g.tiles_n / 10.0 + 0.5);
-    if (panels < 1) panels = 1;
-    g.panel = (g.tiles_n + panels - 1) / panels;
+    set_tiles(g, tm, (int)((N + tn - 1) / tn));
     char name[64];
     snprintf(name, sizeof(name), "gemm_split_kernel<%d, %d, %d, %s>", tm, tn, layout, half_b ? "true" : "false");
-    ft_prof_scope prof(ctx, name, 2.0 * M * (double)N * ((double)K + (double)(g.a2 ? K2 : 0)),
+    ft_prof_scope prof(ctx, name, 2.0 * M * (double)N * ((double)K + (double)(g.p[0].a2 ? K2 : 0)),
                        4.0 * M * (double)K + (half_b ? 2.0 : 4.0) * N * (double)K + 4.0 * M * (double)N);
     if (tm == 64 && tiles64 > cus && g.steps < 8) launch<2, 2, 2>(ctx, g, layout, half_b);
     else if (tm == 64 && tiles64 > cus) launch<2, 2, 4>(ctx, g, layout, half_b);
@@ -488,4 +604,37 @@ int ft_split_gemm(ft_context* ctx, int layout, bool half_b, const float* a, cons
     else launch<1, 1, 8>(ctx, g, layout, half_b);
     FT_LAUNCH_CHECK();
     return FT_OK;
+}
+
+int ft_split_group(ft_context* ctx, const float* x, const ft_lora_linear_desc* d, size_t count, size_t M, size_t K,
+                   bool half_b) {
+    bool whole = true;
+    for (size_t i = 0; i < count; i++) whole = whole && d[i].N % (half_b ? 8 : 4) == 0;
+    SplitArgs g = split_args(ctx, x, M, K, K, whole);
+    g.count = (int)count;
+    int tiles = 0;
+    double flops = 0.0, bytes = 4.0 * M * (double)K;
+    for (size_t i = 0; i < count; i++) {
+        const bool ranked = d[i].r > 0;
+        g.p[i] = SplitProduct{static_cast<const char*>(d[i].w), d[i].y, d[i].residual, ranked ? d[i].t : nullptr,
+                              ranked ? d[i].b : nullptr, reinterpret_cast<const float2*>(d[i].rope_table), (int)d[i].rope_seq,
+                              (int)d[i].N, (int)d[i].N, (int)d[i].r, tiles};
+        tiles += (int)((d[i].N + 63) / 64);
+        flops += 2.0 * M * (double)d[i].N * (double)(K + d[i].r);
+        bytes += (half_b ? 2.0 : 4.0) * d[i].N * (double)K + 4.0 * M * (double)d[i].N;
+    }
+    ft_prof_scope prof(ctx, "gemm_split_kernel<group>", flops, bytes);
+    return launch_group<kSplitGroup>(ctx, g, tiles, half_b);
+}
+
+int ft_split_gate_up(ft_context* ctx, const float* x, const void* w_gate, const void* w_up, float* gate, float* up,
+                     float* act, size_t M, size_t K, size_t N, bool half_b) {
+    SplitArgs g = split_args(ctx, x, M, K, K, N % (half_b ? 8 : 4) == 0);
+    g.p[0] = SplitProduct{static_cast<const char*>(w_up), up, nullptr, nullptr, nullptr, nullptr, 1, (int)N, (int)N, 0, 0};
+    g.b_alt = static_cast<const char*>(w_gate);
+    g.out2 = gate;
+    g.out3 = act;
+    ft_prof_scope prof(ctx, "gemm_split_kernel<gate_up>", 4.0 * M * (double)N * (double)K,
+                       4.0 * M * (double)K + (half_b ? 4.0 : 8.0) * N * (double)K + 12.0 * M * (double)N);
+    return launch_group<kSplitGateUp>(ctx, g, (int)((N + 31) / 32), half_b);
 }

@@ -130,3 +130,55 @@ def test_sums_the_same_twice(g):
     eng.matmul(ctx, a, b, o1)
     eng.matmul(ctx, a, b, o2)
     assert np.array_equal(np.asarray(o1.to_vec()).view(np.uint32), np.asarray(o2.to_vec()).view(np.uint32))
+
+
+def rope_table(ctx, seq, theta=10000.0):
+    pos, i = np.arange(seq)[:, None], np.arange(32)[None, :]
+    angle = pos * theta ** (-2.0 * i / 64)
+    t = np.stack([np.cos(angle), np.sin(angle)], axis=-1).astype(np.float32)
+    return up(ctx, t.reshape(seq, 64)), t
+
+
+@pytest.mark.parametrize("M,K,widths,half", [(4, 32, (64, 64, 64), True), (33, 100, (128, 64, 72), False), (96, 960, (960, 320, 320), True),
+                                             (520, 250, (1088, 64, 64), True), (1040, 64, (1024, 128, 8), False)])
+def test_group_with_rotation_and_residual(g, M, K, widths, half):
+    """Two rotated products and one with a residual and a rank-r term, every tile height and wave count."""
+    ctx, eng = g
+    x, seq = rnd(M, M, K), M // 4 if M % 4 == 0 else M
+    table, t = rope_table(ctx, seq)
+    linears, want = [], []
+    for i, n in enumerate(widths):
+        w, f, b = rnd(n + i, K, n, scale=0.05), rnd(i, M, 8), rnd(i + 9, 8, n)
+        wv = w.astype(np.float16).astype(np.float32) if half else w
+        res = rnd(i + 20, M, n) if i == 2 else None
+        y = empty(ctx, M, n)
+        linears.append((up16(ctx, w) if half else up(ctx, w), up(ctx, f), up(ctx, b), y, up(ctx, res) if i == 2 else None))
+        terms = [(x, wv), (f, b)] + ([(res, np.eye(n, dtype=np.float32))] if i == 2 else [])
+        plain = sum(p.astype(np.float64) @ q.astype(np.float64) for p, q in terms)
+        size = sum(np.abs(p).astype(np.float64) @ np.abs(q).astype(np.float64) for p, q in terms)
+        if i < 2:
+            c, s = (np.tile(t[..., k].astype(np.float64), (M // seq, 1))[:, None, :] for k in (0, 1))
+            h, hs = plain.reshape(M, n // 64, 2, 32), size.reshape(M, n // 64, 2, 32)
+            plain = np.stack([h[:, :, 0] * c - h[:, :, 1] * s, h[:, :, 0] * s + h[:, :, 1] * c], 2).reshape(M, n)
+            size = np.stack([hs[:, :, 0] + hs[:, :, 1]] * 2, 2).reshape(M, n)
+        want.append((plain, size))
+    eng.lora_linear_group(ctx, up(ctx, x), linears, rope_table=table, rope_seq=seq, n_rope=2)
+    for (w, f, b, y, r), (plain, size) in zip(linears, want):
+        limit = (6 * (K // 16 // 4 + 1) + 36) * 2.0 ** -23 * size
+        got = np.asarray(y.to_vec(), np.float64).reshape(plain.shape)
+        assert np.all(np.abs(got - plain) <= limit), (y.shape, np.max(np.abs(got - plain) / limit))
+
+
+@pytest.mark.parametrize("M,K,N,half", [(4, 32, 8, True), (33, 100, 41, False), (96, 960, 2560, True), (300, 200, 1000, True), (1040, 64, 1024, False)])
+def test_gate_up(g, M, K, N, half):
+    ctx, eng = g
+    x, wg, wu = rnd(M, M, K), rnd(N, K, N, scale=0.05), rnd(N + 1, K, N, scale=0.05)
+    gv, uv = (w.astype(np.float16).astype(np.float32) if half else w for w in (wg, wu))
+    make = up16 if half else up
+    gate, u, act = (empty(ctx, M, N) for _ in range(3))
+    eng.mlp_gate_up(ctx, up(ctx, x), make(ctx, wg), make(ctx, wu), gate, u, act)
+    check("gate", gate.to_vec(), [(x, gv)], K)
+    check("up", u.to_vec(), [(x, uv)], K)
+    gt, ut = (np.asarray(o.to_vec(), np.float64) for o in (gate, u))
+    want = gt / (1.0 + np.exp(-gt)) * ut
+    np.testing.assert_allclose(np.asarray(act.to_vec(), np.float64), want, rtol=2e-6, atol=1e-30)
