@@ -1,0 +1,316 @@
+// Attention forward outside a training step, head dim 64: the work decomposition of the 16-row kernels
+// (ft_attention16.hip) on v_mfma_f32_16x16x32_bf16. Every operand, the probabilities too, is the exact sum
+// of three bf16 parts and a product is six products of parts, as in ft_split.hip: f32 operands and f32 sums at 2.7 times
+// the rate of the f32 instruction.
+//
+// K and V are split once per workgroup, on their way into LDS, as three planes each: rows of a key for the products over
+// the head dim, rows of a head-dim index (32 keys of a wave's half, in the order in which the probabilities leave the
+// score product's registers: 16 u + 4 g + i at 8 g + 4 u + i) for the products over the keys. The probabilities then
+// are the second operand of their product without leaving their lane.
+//
+// A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends the workgroup through
+// the f32 kernel's code, which says what it is.
+//
+// Bound: a tile of 64 keys costs a workgroup about 3000 cycles each of matrix unit, VALU (softmax and splitting) and LDS
+// reads, and the barrier per tile keeps its waves in step, so they overlap little. us by HIP events, f32 kernel -> this:
+// 4 x 1024 tokens, 15 heads on 5: 93 -> 63; 8 x 1024, 32 heads: 363 -> 256; 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and
+// not kept: one query tile of 64 rows per workgroup, two workgroups a CU (64, 272, 15.5); 32 rows a wave (61, 248, 17.5);
+// dQ the same way (128 registers spill: 132 against 130).
+#include "ft_attention16.h"
+
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int PLANE = KT * D64 * 2;   // bytes of one part of a 64-key tile
+
+__device__ __forceinline__ unsigned pack2(float x, float y) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x, y}, bf16x2));
+}
+// Two values into the packed halves of their three parts.
+__device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3]) {
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        const unsigned q = pack2(x, y);
+        part[t] = q;
+        if (t < 2) {
+            x -= __uint_as_float(q << 16);
+            y -= __uint_as_float(q & 0xffff0000u);
+        }
+    }
+}
+// Eight values of a lane into the operand registers of their parts.
+__device__ __forceinline__ void split8(const float (&x)[8], uintx4 (&part)[3]) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        unsigned q[3];
+        split2(x[2 * e], x[2 * e + 1], q);
+#pragma unroll
+        for (int t = 0; t < 3; t++) part[t][e] = q[t];
+    }
+}
+
+// acc += a b over 32 k, smallest products first
+__device__ __forceinline__ floatx4 mfma_parts(const uintx4 (&a)[3], const uintx4 (&b)[3], floatx4 acc) {
+    constexpr int U[6] = {2, 0, 1, 1, 0, 0}, V[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int t = 0; t < 6; t++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[U[t]]), __builtin_bit_cast(bf16x8, b[V[t]]),
+                                                      acc, 0, 0, 0);
+    return acc;
+}
+
+// Chunk swizzles (16 bytes) that spread the 16 lanes served together over all banks, see ft_attention16.h: rows of 128
+// bytes (a key's 64 head-dim values) and of 64 bytes (a head-dim index's 32 keys).
+__device__ __forceinline__ int sw_key(int row, int chunk) { return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4); }
+__device__ __forceinline__ int sw_dim(int row, int chunk) {
+    const int x = (row >> 2) & 3;
+    return row * 64 + ((chunk ^ (((x << 1) ^ ((x >> 1) * 3)) & 3)) << 4);
+}
+
+// One operand's tile of 64 keys on its way from global memory to LDS: four values a thread and round.
+template <int NT>
+struct KeyRows {       // planes [key][64]
+    static constexpr int N = KT * 16 / NT;
+    float4 pre[N];
+    __device__ __forceinline__ void fetch(const float* src, const AttnArgs& p, int b, int kvh, int t, int tid) {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int e = tid + NT * u;
+            int key = t * KT + e / 16;
+            key = key < p.Sk ? key : p.Sk - 1;
+            pre[u] = *reinterpret_cast<const float4*>(src + (((long)b * p.Sk + key) * p.Hkv + kvh) * D64 + 4 * (e % 16));
+        }
+    }
+    __device__ __forceinline__ void store(char* planes, int tid) const {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int e = tid + NT * u, c = e % 16;
+            unsigned lo[3], hi[3];
+            split2(pre[u].x, pre[u].y, lo);
+            split2(pre[u].z, pre[u].w, hi);
+            char* at = planes + sw_key(e / 16, c >> 1) + (c & 1) * 8;
+#pragma unroll
+            for (int q = 0; q < 3; q++) *reinterpret_cast<uintx2*>(at + q * PLANE) = uintx2{lo[q], hi[q]};
+        }
+    }
+};
+template <int NT>
+struct KeyColumns {    // planes [key half][64][32 keys]
+    static constexpr int N = KT * 16 / NT;
+    float pre[N][4];
+    __device__ __forceinline__ void fetch(const float* src, const AttnArgs& p, int b, int kvh, int t, int tid) {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int e = tid + NT * u, d = e % 64, kg = e / 64;   // keys 4 kg .. 4 kg + 3
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                int key = t * KT + 4 * kg + i;
+                key = key < p.Sk ? key : p.Sk - 1;
+                pre[u][i] = src[(((long)b * p.Sk + key) * p.Hkv + kvh) * D64 + d];
+            }
+        }
+    }
+    __device__ __forceinline__ void store(char* planes, int tid) const {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int e = tid + NT * u, d = e % 64, kg = e / 64;
+            unsigned lo[3], hi[3];
+            split2(pre[u][0], pre[u][1], lo);
+            split2(pre[u][2], pre[u][3], hi);
+            char* at = planes + (kg >> 3) * (PLANE / 2) + sw_dim(d, kg & 3) + ((kg >> 2) & 1) * 8;
+#pragma unroll
+            for (int q = 0; q < 3; q++) *reinterpret_cast<uintx2*>(at + q * PLANE) = uintx2{lo[q], hi[q]};
+        }
+    }
+};
+
+__device__ __forceinline__ void read_parts(const char* at, uintx4 (&part)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) part[q] = *reinterpret_cast<const uintx4*>(at + q * PLANE);
+}
+
+// A row's 64 values (this lane's 16 of them) as the two k steps' operand registers, scaled.
+__device__ __forceinline__ void row_parts(const float* row, int g, float scale, uintx4 (&part)[2][3]) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        const float4 a = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g);
+        const float4 b = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g + 4);
+        const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
+        split8(x, part[ks]);
+    }
+}
+
+__device__ __forceinline__ bool not_finite(floatx4 v) {
+    const float z = v[0] * 0.0f + v[1] * 0.0f + v[2] * 0.0f + v[3] * 0.0f;
+    return !(z == 0.0f);
+}
+
+template <int NG>
+__global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p) {
+    constexpr int NT = 4 * NG * 64, STAGE = 6 * PLANE;   // K rows, V columns
+    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    QueryWave<NG> w;
+    w.init(p, wave, l16);
+    KeyRows<NT> kl;
+    KeyColumns<NT> vl;
+    if (w.nkt > 0) {
+        kl.fetch(p.k, p, w.b, w.kvh, 0, tid);
+        vl.fetch(p.v, p, w.b, w.kvh, 0, tid);
+    }
+    // scores are kept in base 2: log2(e) / sqrt(D) goes into Q
+    uintx4 qp[2][3];
+    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, p.scale * kLog2e, qp);
+    floatx4 o[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = zero4();
+    float m_run = kAttnMasked, l_lane = 0.0f;
+    bool bad = false;   // something here is for the f32 code
+    // the last key this lane's query may see
+    const int key_lim = (p.causal && w.q + p.causal_offset < p.Sk - 1) ? w.q + p.causal_offset : p.Sk - 1;
+
+    if (w.nkt > 0) {
+        kl.store(smem, tid);
+        vl.store(smem + 3 * PLANE, tid);
+    }
+    __syncthreads();
+
+    auto tile = [&](auto nsb_tag, auto mask_tag, const char* ks, const char* vs, int kb) {
+        constexpr int NSB = decltype(nsb_tag)::value;
+        constexpr bool MASK = decltype(mask_tag)::value;
+        floatx4 s[2] = {zero4(), zero4()};
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            uintx4 kp[NSB][3];
+#pragma unroll
+            for (int u = 0; u < NSB; u++) read_parts(ks + sw_key(32 * w.kh + 16 * u + l16, 4 * t + g), kp[u]);
+#pragma unroll
+            for (int u = 0; u < NSB; u++) s[u] = mfma_parts(kp[u], qp[t], s[u]);
+        }
+        float tmax = kAttnMasked;
+#pragma unroll
+        for (int u = 0; u < NSB; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if constexpr (MASK) {
+                    const int key = kb + 32 * w.kh + 16 * u + 4 * g + i;
+                    s[u][i] = key <= key_lim ? s[u][i] : kAttnMasked;
+                    bad = bad || s[u][i] != s[u][i];   // below, a NaN score counts as a masked one
+                }
+                tmax = fmaxf(tmax, s[u][i]);
+            }
+        tmax = group_max(tmax);
+        const float m_new = fmaxf(m_run, tmax);
+        const float corr = exp2_fast(m_run - m_new);
+        float psum = 0.0f;
+        float pr[8];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float pj = 0.0f;
+                if (u < NSB) {
+                    pj = exp2_fast(s[u][i] - m_new);
+                    if constexpr (MASK) pj = s[u][i] > kAttnMasked ? pj : 0.0f;
+                    psum += pj;
+                }
+                pr[4 * u + i] = pj;
+            }
+        l_lane = l_lane * corr + psum;  // this lane's keys only; the lanes of a query meet at the end
+        m_run = m_new;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] *= corr;
+        uintx4 pp[3];
+        split8(pr, pp);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            uintx4 vp[3];
+            read_parts(vs + w.kh * (PLANE / 2) + sw_dim(16 * e + l16, g), vp);
+            o[e] = mfma_parts(vp, pp, o[e]);
+        }
+    };
+    using std::integral_constant;
+    for (int t = 0; t < w.nkt; t++) {
+        const bool more = t + 1 < w.nkt;
+        if (more) {
+            kl.fetch(p.k, p, w.b, w.kvh, t + 1, tid);
+            vl.fetch(p.v, p, w.b, w.kvh, t + 1, tid);
+        }
+        const char* ks = smem + (t & 1) * STAGE;
+        const char* vs = ks + 3 * PLANE;
+        const int kb = t * KT;
+        const int nsb = w.visible_subblocks(kb);
+        if (nsb > 0) {
+            if (w.half_unmasked(kb))
+                tile(integral_constant<int, 2>{}, std::false_type{}, ks, vs, kb);
+            else if (nsb == 2)
+                tile(integral_constant<int, 2>{}, std::true_type{}, ks, vs, kb);
+            else
+                tile(integral_constant<int, 1>{}, std::true_type{}, ks, vs, kb);
+        }
+        if (more) {
+            char* next = smem + ((t + 1) & 1) * STAGE;
+            kl.store(next, tid);
+            vl.store(next + 3 * PLANE, tid);
+        }
+        __syncthreads();
+    }
+
+    // The two key halves of a row block meet through LDS, lane for lane.
+    float* mrg = reinterpret_cast<float*>(smem) + (w.w2 * 18) * 64 + lane;
+    if (w.kh == 1) {
+        mrg[0] = m_run;
+        mrg[64] = l_lane;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) mrg[(2 + 4 * e + r) * 64] = o[e][r];
+    }
+    __syncthreads();
+    if (w.kh == 0) {
+        const float m_o = mrg[0], l_o = mrg[64];
+        const float m_new = fmaxf(m_run, m_o);
+        const float c0 = exp2_fast(m_run - m_new), c1 = exp2_fast(m_o - m_new);
+        l_lane = l_lane * c0 + l_o * c1;
+        m_run = m_new;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[e][r] = o[e][r] * c0 + mrg[(2 + 4 * e + r) * 64] * c1;
+        const float l_run = group_sum(l_lane);
+        const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+        const float lse = l_run > 0.0f ? (m_run + log2_fast(l_run)) * kLn2 : kAttnLseEmpty;
+        bad = bad || !(fabsf(lse) <= 3.0e38f) || !(l_run >= 0.0f);
+        // register r of accumulator e is head-dim index 16 e + 4 g + r
+        float* orow = p.o + (((long)w.b * p.Sq + w.q) * p.H + w.h) * D64;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const floatx4 v = o[e] * inv;
+            bad = bad || not_finite(v);
+            if (w.q_ok) *reinterpret_cast<floatx4*>(orow + 16 * e + 4 * g) = v;
+        }
+        if (w.q_ok && p.stats && g == 0) p.stats[2 * (((long)w.b * p.H + w.h) * p.Sq + w.q) + 1] = lse;
+    }
+    if (__syncthreads_or(bad && w.q_ok)) attn16_fwd<NG>(p, reinterpret_cast<float*>(smem));
+}
+
+template <int NG>
+dim3 query_grid(const AttnArgs& a) {
+    const size_t nT = ft_div_up(a.Sq, 16 * NG);
+    return dim3((unsigned)(((nT + 1) / 2) * (size_t)a.B * a.H));
+}
+
+}  // namespace
+
+int ft_attn_split_forward(ft_context* ctx, const AttnArgs& a, int groups) {
+    if (groups == 2) hipLaunchKernelGGL(attn_split_fwd_kernel<2>, query_grid<2>(a), dim3(512), 0, ctx->stream, a);
+    else hipLaunchKernelGGL(attn_split_fwd_kernel<4>, query_grid<4>(a), dim3(1024), 0, ctx->stream, a);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}

@@ -182,3 +182,56 @@ def test_gate_up(g, M, K, N, half):
     gt, ut = (np.asarray(o.to_vec(), np.float64) for o in (gate, u))
     want = gt / (1.0 + np.exp(-gt)) * ut
     np.testing.assert_allclose(np.asarray(act.to_vec(), np.float64), want, rtol=2e-6, atol=1e-30)
+
+
+def attention64(q, k, v, causal, offset):
+    """f64 attention of [B, Sq, H, D] over [B, Sk, Hkv, D]; log-sum-exp too."""
+    B, Sq, H, D = q.shape
+    rep = H // k.shape[2]
+    k, v = np.repeat(k, rep, axis=2).astype(np.float64), np.repeat(v, rep, axis=2).astype(np.float64)
+    s = np.matmul(q.astype(np.float64).transpose(0, 2, 1, 3), k.transpose(0, 2, 3, 1)) / np.sqrt(D)
+    if causal:
+        s = np.where(np.arange(k.shape[1])[None, :] <= np.arange(Sq)[:, None] + offset, s, -np.inf)
+    m = s.max(-1, keepdims=True)
+    e = np.exp(s - m)
+    z = e.sum(-1, keepdims=True)
+    return np.matmul(e / z, v.transpose(0, 2, 1, 3)).transpose(0, 2, 1, 3), (m + np.log(z))[..., 0]
+
+
+# The two tile heights (from 64 and 128 workgroups of 64-row pairs on), ragged queries and keys, one and several tiles,
+# grouped heads, an offset, no mask.
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(8, 33, 33, 8, 8, True, 0), (8, 128, 128, 16, 4, True, 0), (3, 200, 200, 15, 5, True, 0),
+                                                         (4, 190, 257, 15, 5, True, 67), (2, 130, 77, 32, 8, False, 0), (16, 1, 100, 16, 16, False, 0)])
+def test_attention_forward(g, B, Sq, Sk, H, Hkv, causal, offset):
+    from ferrotensor_amd import AttentionOptions
+    ctx, eng = g
+    q, k, v = rnd(1, B, Sq, H, 64), rnd(2, B, Sk, Hkv, 64), rnd(3, B, Sk, Hkv, 64)
+    o, stats = empty(ctx, B, Sq, H, 64), empty(ctx, B * H * Sq, 2)
+    eng.flash_attention_v2_with_stats(ctx, up(ctx, q), up(ctx, k), up(ctx, v), o, stats, AttentionOptions(causal=causal, causal_offset=offset))
+    want, lse = attention64(q, k, v, causal, offset)
+    # probabilities to 2^-18 of themselves (scores of a few units, exp2 in f32), then averages of values near 1
+    np.testing.assert_allclose(np.asarray(o.to_vec(), np.float64).reshape(want.shape), want, atol=2e-5)
+    np.testing.assert_allclose(np.asarray(stats.to_vec(), np.float64).reshape(B, H, Sq, 2)[..., 1], lse, atol=1e-5)
+
+
+def test_attention_with_infinite_and_nan_values_as_the_f32_kernel(g):
+    """V and K of some heads hold an infinity, a NaN, a value at the top of f32: the queries that see them come out as from
+    the f32 kernel (where a tile crosses the diagonal, a NaN score counts as masked), the others as ever."""
+    from ferrotensor_amd import AttentionOptions
+    ctx, eng = g
+    B, S, H = 4, 160, 16
+    q, k, v = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64)
+    v[0, 50, 3, 7], v[1, 100, 5, 9], k[2, 70, 1, 4] = np.inf, np.nan, np.nan
+    v[3, 20, 2, 11] = 3.4e38   # finite, but its first bf16 part is not
+    o, stats = empty(ctx, B, S, H, 64), empty(ctx, B * H * S, 2)
+    eng.flash_attention_v2_with_stats(ctx, up(ctx, q), up(ctx, k), up(ctx, v), o, stats, AttentionOptions(causal=True))
+    got = np.asarray(o.to_vec(), np.float64).reshape(B, S, H, 64)
+    fine = np.isfinite(got)
+    assert not fine[0, 50:, 3, 7].any() and not fine[1, 100:, 5, 9].any() and not fine[2, 128:, 1].any()
+    with np.errstate(all="ignore"):
+        want, _ = attention64(q, k, np.where(np.isfinite(v), v, 0.0), True, 0)
+    ok = fine & np.isfinite(want)
+    ok[3, :, 2, 11] = False
+    np.testing.assert_allclose(got[ok], want[ok], atol=2e-5)
+    np.testing.assert_allclose(got[3, :, 2, 11], want[3, :, 2, 11], rtol=1e-4, atol=2e-5)
+    assert fine[[0, 1, 3]][:, :, [0, 4, 6]].all()   # the other heads
