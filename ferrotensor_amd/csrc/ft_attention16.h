@@ -1,6 +1,5 @@
-// The query-row parts of the 16-row attention kernels (see ft_attention16.hip): what a workgroup does in the forward and
-// dQ kernels, for the kernels themselves and for those on bf16 parts (ft_attention_split.hip), which share the work
-// decomposition and come back to these where a result is not finite.
+// What a workgroup of the 16-row attention kernels does (see ft_attention16.hip), for the kernels themselves and for those
+// on bf16 parts (ft_attention_split.hip), which come back to this where a result is not finite.
 #pragma once
 
 #include "ft_attention.h"
@@ -109,7 +108,7 @@ constexpr int HALF = 32 * D64;   // floats of one key half of a tile
 
 template <int NG>
 struct QueryWave {
-    static constexpr int TQ = 16 * NG;
+    static constexpr int TQ = 16 * NG, WAVES = 4 * NG;
     int b, h, kvh;
     int kh;        // key half of every tile this wave multiplies
     int w2;        // index among the waves of its half
@@ -121,7 +120,7 @@ struct QueryWave {
     int kfull_w;   // keys below this are visible to every row of the wave
     int nkt;       // K/V tiles the workgroup walks
 
-    __device__ __forceinline__ void init(const AttnArgs& p, int wave, int l16) {
+    __device__ __forceinline__ void init(const AttnArgs& p, int wave, int l16, int = 0, int = 0) {
         const int nbh = p.B * p.H;
         const int nT = (p.Sq + TQ - 1) / TQ;
         const int pi = blockIdx.x / nbh, bh = blockIdx.x % nbh;
@@ -162,6 +161,30 @@ struct QueryWave {
     }
     // is every key of this wave's half of that tile visible to every row?
     __device__ __forceinline__ bool half_unmasked(int kb) const { return kb + 32 * (kh + 1) <= kfull_w; }
+};
+
+// The same for a workgroup of 2 * NG waves on the one query tile `tile` of (batch, head) `bh`; a wave owns QB blocks of
+// 16 rows, and `q`, `qc`, `q_ok` are those of its first.
+template <int NG, int QB = 1>
+struct QueryTile : QueryWave<NG> {
+    static constexpr int TQ = 16 * NG * QB, WAVES = 2 * NG;
+    __device__ __forceinline__ void init(const AttnArgs& p, int wave, int l16, int tile, int bh) {
+        this->b = bh / p.H;
+        this->h = bh % p.H;
+        this->kvh = this->h / (p.H / p.Hkv);
+        this->kh = wave / NG;
+        this->w2 = wave % NG;
+        this->q0w = tile * TQ + 16 * QB * this->w2;
+        this->q = this->q0w + l16;
+        this->q_ok = this->q < p.Sq;
+        this->qc = this->q_ok ? this->q : p.Sq - 1;
+        const int end_w = this->q0w + 16 * QB;
+        this->kend_w = this->q0w < p.Sq ? this->key_end(p, (end_w < p.Sq ? end_w : p.Sq) - 1) : 0;
+        this->kfull_w = p.causal ? this->q0w + p.causal_offset + 1 : p.Sk;
+        if (this->kfull_w > p.Sk) this->kfull_w = p.Sk;
+        const int qlast_wg = ((tile + 1) * TQ < p.Sq ? (tile + 1) * TQ : p.Sq) - 1;
+        this->nkt = (this->key_end(p, qlast_wg) + KT - 1) / KT;
+    }
 };
 
 // The K/V tile of 64 keys: global -> registers (the next tile's while the current one multiplies)
@@ -360,14 +383,14 @@ __device__ __forceinline__ void attn16_fwd(const AttnArgs& p, float* smem) {   /
 // dS = P (dO.V - Delta), P = exp(S - LSE). Same decomposition as the forward; the
 // two key halves of a row block add their partial dQ through LDS at the end.
 // ---------------------------------------------------------------------------
-template <int NG>
-__device__ __forceinline__ void attn16_dq(const AttnArgs& p, float* smem) {
-    constexpr int NT = 4 * NG * 64;
+template <int NG, typename Waves = QueryWave<NG>>
+__device__ __forceinline__ void attn16_dq(const AttnArgs& p, float* smem, int qtile = 0, int qbh = 0) {
+    constexpr int NT = Waves::WAVES * 64;
     const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
 
-    QueryWave<NG> w;
-    w.init(p, wave, l16);
+    Waves w;
+    w.init(p, wave, l16, qtile, qbh);
     FT_ATTN16_KV_LOADER(p, w, tid, smem);
     if (w.nkt > 0) kv_fetch(0);
 
@@ -529,6 +552,207 @@ __device__ __forceinline__ void attn16_dq(const AttnArgs& p, float* smem) {
     for (int r = 0; r < 4; r++)
         *reinterpret_cast<float4*>(drow + 4 * (4 * g + r)) =
             make_float4(acc[0][r] * p.scale, acc[1][r] * p.scale, acc[2][r] * p.scale, acc[3][r] * p.scale);
+}
+
+// ---------------------------------------------------------------------------
+// Backward, pass 2: dK and dV of 16 keys of one (batch, kv head), summed over the
+// query heads of the group and over the 16-query blocks that can see them. The
+// key block (K pre-scaled for the base-2 scores, V) sits in LDS for all eight
+// waves; the (head, query block) items are dealt round-robin to the waves, which
+// run without a barrier until the end: an item's Q and dO rows come from global
+// memory as 16-byte quads straight into the A operands of S = Q K^T and
+// dP = dO V^T (the next item's while the current one multiplies), pass through a
+// wave-private LDS tile, and are read back with the head dim as the row for
+// dV^T += dO^T P and dK^T += Q^T dS. The waves' partial sums are added in wave
+// order through LDS (no atomics). One workgroup per (key block, batch * kv head),
+// key block 0 (the most items under the causal mask) first.
+// ---------------------------------------------------------------------------
+template <int DP>
+__device__ __forceinline__ void attn16_dkdv(AttnArgs p, float* smem, int unit) {
+    constexpr int NB = DP / 16, EV = DP / 16, PITCH = DP, NW = 8, C4 = DP / 4;
+    constexpr int BLK = 16 * PITCH;
+    // smem: K block, V block, 8 x (Q tile, dO tile)
+    const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // wave-uniform: keeps the tile bookkeeping in SGPRs
+    float* ks = smem;
+    float* vs = smem + BLK;
+    float* qs = smem + 2 * BLK + wave * 2 * BLK;
+    float* dos = qs + BLK;
+
+    const int nhu = p.B * (p.split_g ? p.H : p.Hkv);
+    const int kbi = unit / nhu, bh = unit % nhu;
+    const int Gfull = p.H / p.Hkv;
+    const int b = bh / (p.split_g ? p.H : p.Hkv);
+    const int hsel = bh % (p.split_g ? p.H : p.Hkv);
+    const int kvh = p.split_g ? hsel / Gfull : hsel;
+    const int g0 = p.split_g ? hsel % Gfull : 0;  // first query head of this workgroup within the group
+    const int G = p.split_g ? 1 : Gfull;          // and how many it covers
+    const int kb0 = kbi * 16;
+    const int key = kb0 + l16;
+    const int key_m = key < p.Sk ? key : 0x7fffffff;  // a key past the end is visible to nobody
+
+    const float kscale = p.scale * kLog2e;
+    for (int e = tid; e < 2 * 16 * C4; e += NW * 64) {
+        const int which = e / (16 * C4), r = (e / C4) % 16, c = e % C4;
+        int kr = kb0 + r;
+        kr = kr < p.Sk ? kr : p.Sk - 1;
+        const long o = (((long)b * p.Sk + kr) * p.Hkv + kvh) * DP + 4 * c;
+        if (which == 0) {
+            const float4 t = *reinterpret_cast<const float4*>(p.k + o);
+            *reinterpret_cast<float4*>(ks + sw(r, c)) =
+                make_float4(t.x * kscale, t.y * kscale, t.z * kscale, t.w * kscale);
+        } else {
+            *reinterpret_cast<float4*>(vs + sw(r, c)) = *reinterpret_cast<const float4*>(p.v + o);
+        }
+    }
+
+    // 16-query blocks that can see this key block
+    const int nqb = (p.Sq + 15) / 16;
+    int qb_start = 0;
+    if (p.causal) {
+        const int first_q = kb0 - p.causal_offset;  // smallest i with i + offset >= kb0
+        qb_start = first_q > 0 ? first_q / 16 : 0;
+    }
+    const int per_head = nqb > qb_start ? nqb - qb_start : 0;
+    const int items = per_head * G;
+
+    float4 qa[NB], da[NB];
+    float2 st[4];
+    auto fetch = [&](int item) {
+        const int gi = item / per_head;
+        const int q0 = (qb_start + item % per_head) * 16;
+        const int h = kvh * Gfull + g0 + gi;
+        int qr = q0 + l16;
+        qr = qr < p.Sq ? qr : p.Sq - 1;
+        const long ro = (((long)b * p.Sq + qr) * p.H + h) * DP;
+#pragma unroll
+        for (int blk = 0; blk < NB; blk++) {
+            qa[blk] = *reinterpret_cast<const float4*>(p.q + ro + 16 * blk + 4 * g);
+            da[blk] = *reinterpret_cast<const float4*>(p.d_out + ro + 16 * blk + 4 * g);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            int qi = q0 + 4 * g + i;
+            qi = qi < p.Sq ? qi : p.Sq - 1;
+            st[i] = *reinterpret_cast<const float2*>(p.stats + 2 * (((long)b * p.H + h) * p.Sq + qi));
+        }
+    };
+    if (wave < items) fetch(wave);
+    __syncthreads();  // K/V block complete
+
+    floatx4 dk[EV], dv[EV];
+#pragma unroll
+    for (int e = 0; e < EV; e++) {
+        dk[e] = zero4();
+        dv[e] = zero4();
+    }
+
+    for (int item = wave; item < items; item += NW) {
+        const int q0 = (qb_start + item % per_head) * 16;
+        // this item's rows -> the wave's LDS tile (for the transposed reads further down)
+#pragma unroll
+        for (int blk = 0; blk < NB; blk++) {
+            *reinterpret_cast<float4*>(qs + sw(l16, 4 * blk + g)) = qa[blk];
+            *reinterpret_cast<float4*>(dos + sw(l16, 4 * blk + g)) = da[blk];
+        }
+        floatx4 s = zero4(), dp = zero4();
+#pragma unroll
+        for (int blk = 0; blk < NB; blk++) {
+            const float4 kq = *reinterpret_cast<const float4*>(ks + sw(l16, 4 * blk + g));
+            const float4 vq = *reinterpret_cast<const float4*>(vs + sw(l16, 4 * blk + g));
+            s = MFMA16(qa[blk].x, kq.x, s);
+            dp = MFMA16(da[blk].x, vq.x, dp);
+            s = MFMA16(qa[blk].y, kq.y, s);
+            dp = MFMA16(da[blk].y, vq.y, dp);
+            s = MFMA16(qa[blk].z, kq.z, s);
+            dp = MFMA16(da[blk].z, vq.z, dp);
+            s = MFMA16(qa[blk].w, kq.w, s);
+            dp = MFMA16(da[blk].w, vq.w, dp);
+        }
+        // register i of this lane is query q0 + 4 g + i against key `key`
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // visible: a real key, a real query, and not above the diagonal; written without
+            // short-circuit operators so that it stays a select (exp2(-inf) = 0)
+            const int qi = q0 + 4 * g + i;
+            const int lim = qi < p.Sq ? (p.causal ? qi + p.causal_offset : 0x7ffffffe) : -1;
+            const float pij = exp2_fast(key_m <= lim ? s[i] - st[i].y * kLog2e : -INFINITY);
+            s[i] = pij;                        // P
+            dp[i] = pij * (dp[i] - st[i].x);   // dS
+        }
+        // the next item's rows travel while the rest of this one is computed
+        fetch(item + NW < items ? item + NW : item);  // (the last item is fetched again: no branch, no copies)
+        wave_lds_fence();
+        float ao[4][EV], aq[4][EV];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lds_vec<EV>(dos + sw(4 * g + i, l16), ao[i]);
+            lds_vec<EV>(qs + sw(4 * g + i, l16), aq[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int e = 0; e < EV; e++) {
+                dv[e] = MFMA16(ao[i][e], s[i], dv[e]);
+                dk[e] = MFMA16(aq[i][e], dp[i], dk[e]);
+            }
+        wave_lds_fence();  // the tile is rewritten by the next item
+    }
+
+    // Cross-wave sum in wave order. A wave's tile pair takes its partial dK (Q tile) and dV (dO tile)
+    // as [key][head dim]; register r of accumulator e is head-dim index EV * (4 g + r) + e.
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float a[EV], c[EV];
+#pragma unroll
+        for (int e = 0; e < EV; e++) {
+            a[e] = dk[e][r];
+            c[e] = dv[e][r];
+        }
+        store_vec<EV>(qs + sw(l16, 4 * g + r), a);
+        store_vec<EV>(dos + sw(l16, 4 * g + r), c);
+    }
+    __syncthreads();
+    const float* red = smem + 2 * BLK;
+    for (int e = tid; e < 2 * 16 * C4; e += NW * 64) {
+        const int which = e / (16 * C4), kk = (e / C4) % 16, c = e % C4;
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int wv = 0; wv < NW; wv++) {
+            const float4 t = *reinterpret_cast<const float4*>(red + (wv * 2 + which) * BLK + sw(kk, c));
+            sum.x += t.x; sum.y += t.y; sum.z += t.z; sum.w += t.w;
+        }
+        const int krow = kb0 + kk;
+        const long o = (((long)b * p.Sk + krow) * p.Hkv + kvh) * DP + 4 * c;
+        if (p.split_g) {
+            if (krow < p.Sk) {
+                const long n_all = (long)p.B * p.Sk * p.Hkv * DP;
+                *reinterpret_cast<float4*>(p.part + (2 * g0 + which) * n_all + o) = sum;
+            }
+            continue;
+        }
+        if (which == 1) {
+            if (krow < p.Sk) *reinterpret_cast<float4*>(p.dv + o) = sum;
+            continue;
+        }
+        // dK = scale * sum dS Q (Q is read unscaled)
+        sum.x *= p.scale; sum.y *= p.scale; sum.z *= p.scale; sum.w *= p.scale;
+        if (DP == 64 && p.rope) {
+            // rotated back: the partner chunk (head-dim index +- 32) is held by lane ^ 8 of this wave
+            float4 oth;
+            oth.x = __shfl_xor(sum.x, 8, 64);
+            oth.y = __shfl_xor(sum.y, 8, 64);
+            oth.z = __shfl_xor(sum.z, 8, 64);
+            oth.w = __shfl_xor(sum.w, 8, 64);
+            const int kc = krow < p.Sk ? krow : p.Sk - 1;
+            const float2* tb = p.rope + (long)kc * 32 + ((4 * c) & 31);
+            const float2 c0 = tb[0], c1 = tb[1], c2 = tb[2], c3 = tb[3];
+            const float sg = c < 8 ? 1.0f : -1.0f;
+            sum = make_float4(sum.x * c0.x + sg * oth.x * c0.y, sum.y * c1.x + sg * oth.y * c1.y,
+                              sum.z * c2.x + sg * oth.z * c2.y, sum.w * c3.x + sg * oth.w * c3.y);
+        }
+        if (krow < p.Sk) *reinterpret_cast<float4*>(p.dk + o) = sum;
+    }
 }
 
 }  // namespace

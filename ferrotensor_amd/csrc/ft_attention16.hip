@@ -35,205 +35,10 @@ __global__ __launch_bounds__(4 * NG * 64) void attn16_dq_kernel(AttnArgs p) {
     attn16_dq<NG>(p, smem);
 }
 
-// ---------------------------------------------------------------------------
-// Backward, pass 2: dK and dV of 16 keys of one (batch, kv head), summed over the
-// query heads of the group and over the 16-query blocks that can see them. The
-// key block (K pre-scaled for the base-2 scores, V) sits in LDS for all eight
-// waves; the (head, query block) items are dealt round-robin to the waves, which
-// run without a barrier until the end: an item's Q and dO rows come from global
-// memory as 16-byte quads straight into the A operands of S = Q K^T and
-// dP = dO V^T (the next item's while the current one multiplies), pass through a
-// wave-private LDS tile, and are read back with the head dim as the row for
-// dV^T += dO^T P and dK^T += Q^T dS. The waves' partial sums are added in wave
-// order through LDS (no atomics). One workgroup per (key block, batch * kv head),
-// key block 0 (the most items under the causal mask) first.
-// ---------------------------------------------------------------------------
 template <int DP>
 __global__ __launch_bounds__(512, 4) void attn16_dkdv_kernel(AttnArgs p) {
-    constexpr int NB = DP / 16, EV = DP / 16, PITCH = DP, NW = 8, C4 = DP / 4;
-    constexpr int BLK = 16 * PITCH;
-    extern __shared__ __attribute__((aligned(16))) float smem[];  // K block, V block, 8 x (Q tile, dO tile)
-    const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // wave-uniform: keeps the tile bookkeeping in SGPRs
-    float* ks = smem;
-    float* vs = smem + BLK;
-    float* qs = smem + 2 * BLK + wave * 2 * BLK;
-    float* dos = qs + BLK;
-
-    const int nhu = p.B * (p.split_g ? p.H : p.Hkv);
-    const int kbi = blockIdx.x / nhu, bh = blockIdx.x % nhu;
-    const int Gfull = p.H / p.Hkv;
-    const int b = bh / (p.split_g ? p.H : p.Hkv);
-    const int hsel = bh % (p.split_g ? p.H : p.Hkv);
-    const int kvh = p.split_g ? hsel / Gfull : hsel;
-    const int g0 = p.split_g ? hsel % Gfull : 0;  // first query head of this workgroup within the group
-    const int G = p.split_g ? 1 : Gfull;          // and how many it covers
-    const int kb0 = kbi * 16;
-    const int key = kb0 + l16;
-    const int key_m = key < p.Sk ? key : 0x7fffffff;  // a key past the end is visible to nobody
-
-    const float kscale = p.scale * kLog2e;
-    for (int e = tid; e < 2 * 16 * C4; e += NW * 64) {
-        const int which = e / (16 * C4), r = (e / C4) % 16, c = e % C4;
-        int kr = kb0 + r;
-        kr = kr < p.Sk ? kr : p.Sk - 1;
-        const long o = (((long)b * p.Sk + kr) * p.Hkv + kvh) * DP + 4 * c;
-        if (which == 0) {
-            const float4 t = *reinterpret_cast<const float4*>(p.k + o);
-            *reinterpret_cast<float4*>(ks + sw(r, c)) =
-                make_float4(t.x * kscale, t.y * kscale, t.z * kscale, t.w * kscale);
-        } else {
-            *reinterpret_cast<float4*>(vs + sw(r, c)) = *reinterpret_cast<const float4*>(p.v + o);
-        }
-    }
-
-    // 16-query blocks that can see this key block
-    const int nqb = (p.Sq + 15) / 16;
-    int qb_start = 0;
-    if (p.causal) {
-        const int first_q = kb0 - p.causal_offset;  // smallest i with i + offset >= kb0
-        qb_start = first_q > 0 ? first_q / 16 : 0;
-    }
-    const int per_head = nqb > qb_start ? nqb - qb_start : 0;
-    const int items = per_head * G;
-
-    float4 qa[NB], da[NB];
-    float2 st[4];
-    auto fetch = [&](int item) {
-        const int gi = item / per_head;
-        const int q0 = (qb_start + item % per_head) * 16;
-        const int h = kvh * Gfull + g0 + gi;
-        int qr = q0 + l16;
-        qr = qr < p.Sq ? qr : p.Sq - 1;
-        const long ro = (((long)b * p.Sq + qr) * p.H + h) * DP;
-#pragma unroll
-        for (int blk = 0; blk < NB; blk++) {
-            qa[blk] = *reinterpret_cast<const float4*>(p.q + ro + 16 * blk + 4 * g);
-            da[blk] = *reinterpret_cast<const float4*>(p.d_out + ro + 16 * blk + 4 * g);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            int qi = q0 + 4 * g + i;
-            qi = qi < p.Sq ? qi : p.Sq - 1;
-            st[i] = *reinterpret_cast<const float2*>(p.stats + 2 * (((long)b * p.H + h) * p.Sq + qi));
-        }
-    };
-    if (wave < items) fetch(wave);
-    __syncthreads();  // K/V block complete
-
-    floatx4 dk[EV], dv[EV];
-#pragma unroll
-    for (int e = 0; e < EV; e++) {
-        dk[e] = zero4();
-        dv[e] = zero4();
-    }
-
-    for (int item = wave; item < items; item += NW) {
-        const int q0 = (qb_start + item % per_head) * 16;
-        // this item's rows -> the wave's LDS tile (for the transposed reads further down)
-#pragma unroll
-        for (int blk = 0; blk < NB; blk++) {
-            *reinterpret_cast<float4*>(qs + sw(l16, 4 * blk + g)) = qa[blk];
-            *reinterpret_cast<float4*>(dos + sw(l16, 4 * blk + g)) = da[blk];
-        }
-        floatx4 s = zero4(), dp = zero4();
-#pragma unroll
-        for (int blk = 0; blk < NB; blk++) {
-            const float4 kq = *reinterpret_cast<const float4*>(ks + sw(l16, 4 * blk + g));
-            const float4 vq = *reinterpret_cast<const float4*>(vs + sw(l16, 4 * blk + g));
-            s = MFMA16(qa[blk].x, kq.x, s);
-            dp = MFMA16(da[blk].x, vq.x, dp);
-            s = MFMA16(qa[blk].y, kq.y, s);
-            dp = MFMA16(da[blk].y, vq.y, dp);
-            s = MFMA16(qa[blk].z, kq.z, s);
-            dp = MFMA16(da[blk].z, vq.z, dp);
-            s = MFMA16(qa[blk].w, kq.w, s);
-            dp = MFMA16(da[blk].w, vq.w, dp);
-        }
-        // register i of this lane is query q0 + 4 g + i against key `key`
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            // visible: a real key, a real query, and not above the diagonal; written without
-            // short-circuit operators so that it stays a select (exp2(-inf) = 0)
-            const int qi = q0 + 4 * g + i;
-            const int lim = qi < p.Sq ? (p.causal ? qi + p.causal_offset : 0x7ffffffe) : -1;
-            const float pij = exp2_fast(key_m <= lim ? s[i] - st[i].y * kLog2e : -INFINITY);
-            s[i] = pij;                        // P
-            dp[i] = pij * (dp[i] - st[i].x);   // dS
-        }
-        // the next item's rows travel while the rest of this one is computed
-        fetch(item + NW < items ? item + NW : item);  // (the last item is fetched again: no branch, no copies)
-        wave_lds_fence();
-        float ao[4][EV], aq[4][EV];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            lds_vec<EV>(dos + sw(4 * g + i, l16), ao[i]);
-            lds_vec<EV>(qs + sw(4 * g + i, l16), aq[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int e = 0; e < EV; e++) {
-                dv[e] = MFMA16(ao[i][e], s[i], dv[e]);
-                dk[e] = MFMA16(aq[i][e], dp[i], dk[e]);
-            }
-        wave_lds_fence();  // the tile is rewritten by the next item
-    }
-
-    // Cross-wave sum in wave order. A wave's tile pair takes its partial dK (Q tile) and dV (dO tile)
-    // as [key][head dim]; register r of accumulator e is head-dim index EV * (4 g + r) + e.
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float a[EV], c[EV];
-#pragma unroll
-        for (int e = 0; e < EV; e++) {
-            a[e] = dk[e][r];
-            c[e] = dv[e][r];
-        }
-        store_vec<EV>(qs + sw(l16, 4 * g + r), a);
-        store_vec<EV>(dos + sw(l16, 4 * g + r), c);
-    }
-    __syncthreads();
-    const float* red = smem + 2 * BLK;
-    for (int e = tid; e < 2 * 16 * C4; e += NW * 64) {
-        const int which = e / (16 * C4), kk = (e / C4) % 16, c = e % C4;
-        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int wv = 0; wv < NW; wv++) {
-            const float4 t = *reinterpret_cast<const float4*>(red + (wv * 2 + which) * BLK + sw(kk, c));
-            sum.x += t.x; sum.y += t.y; sum.z += t.z; sum.w += t.w;
-        }
-        const int krow = kb0 + kk;
-        const long o = (((long)b * p.Sk + krow) * p.Hkv + kvh) * DP + 4 * c;
-        if (p.split_g) {
-            if (krow < p.Sk) {
-                const long n_all = (long)p.B * p.Sk * p.Hkv * DP;
-                *reinterpret_cast<float4*>(p.part + (2 * g0 + which) * n_all + o) = sum;
-            }
-            continue;
-        }
-        if (which == 1) {
-            if (krow < p.Sk) *reinterpret_cast<float4*>(p.dv + o) = sum;
-            continue;
-        }
-        // dK = scale * sum dS Q (Q is read unscaled)
-        sum.x *= p.scale; sum.y *= p.scale; sum.z *= p.scale; sum.w *= p.scale;
-        if (DP == 64 && p.rope) {
-            // rotated back: the partner chunk (head-dim index +- 32) is held by lane ^ 8 of this wave
-            float4 oth;
-            oth.x = __shfl_xor(sum.x, 8, 64);
-            oth.y = __shfl_xor(sum.y, 8, 64);
-            oth.z = __shfl_xor(sum.z, 8, 64);
-            oth.w = __shfl_xor(sum.w, 8, 64);
-            const int kc = krow < p.Sk ? krow : p.Sk - 1;
-            const float2* tb = p.rope + (long)kc * 32 + ((4 * c) & 31);
-            const float2 c0 = tb[0], c1 = tb[1], c2 = tb[2], c3 = tb[3];
-            const float sg = c < 8 ? 1.0f : -1.0f;
-            sum = make_float4(sum.x * c0.x + sg * oth.x * c0.y, sum.y * c1.x + sg * oth.y * c1.y,
-                              sum.z * c2.x + sg * oth.z * c2.y, sum.w * c3.x + sg * oth.w * c3.y);
-        }
-        if (krow < p.Sk) *reinterpret_cast<float4*>(p.dk + o) = sum;
-    }
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    attn16_dkdv<DP>(p, smem, blockIdx.x);
 }
 
 template <typename K>
@@ -279,6 +84,34 @@ int query_tile_groups(const ft_context* ctx, const AttnArgs& a, bool backward) {
     if (wgs64 * 2 >= cus) return 4;
     if (wgs64 * 4 >= cus) return 2;
     return 0;
+}
+
+// The kernels on bf16 parts hold one workgroup of 8 waves per CU and want a few rounds of them. dQ, 480 workgroups
+// (4 x 1024 tokens, 15 heads on 5): 89 us against 128; 120 (one sequence): 13 us longer. dK/dV, time of the whole
+// backward beside the f32 kernel's: 8 x 1024, 32 heads (4096 workgroups) 924 against 1154, 4 x 1024, 15 on 5 (960) 232
+// against 246, 8 x 256, 15 on 5 (480) 61.9 against 60.0.
+bool split_dq_pays(const ft_context* ctx, const AttnArgs& a) {
+    return ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 >= 3 * (size_t)ctx->num_cus;
+}
+bool split_dkdv_pays(const ft_context* ctx, const AttnArgs& a) {
+    return ft_div_up(a.Sk, 64) * (size_t)a.B * a.H >= 3 * (size_t)ctx->num_cus;
+}
+
+// One workgroup per 64 keys and query head, then the ordered sum over the group where there is one (and room for its
+// shares; otherwise per kv head).
+int launch_split_dkdv(ft_context* ctx, const AttnArgs& a) {
+    const size_t G = (size_t)a.H / a.Hkv, n_all = (size_t)a.B * a.Sk * a.Hkv * a.D;
+    AttnArgs s = a;
+    if (G > 1 && 2 * G * n_all <= kAttnScratchFloats) {
+        if (!ctx->attn_scratch) {
+            FT_HIP(hipSetDevice(ctx->device));
+            FT_HIP(hipMalloc((void**)&ctx->attn_scratch, kAttnScratchFloats * sizeof(float)));
+        }
+        s.part = ctx->attn_scratch;
+        s.split_g = 1;
+    }
+    FT_TRY(ft_attn_split_dkdv(ctx, s));
+    return s.split_g ? ft_attn_dkdv_combine(ctx, s, 64) : FT_OK;
 }
 
 template <int DP>
@@ -329,8 +162,12 @@ int ft_attn16_forward(ft_context* ctx, const AttnArgs& a) {
 }
 
 int ft_attn16_backward_dq(ft_context* ctx, const AttnArgs& a) {
+    if (!ctx->f32_chain && !a.rope && split_dq_pays(ctx, a)) return ft_attn_split_dq(ctx, a);
     return query_tile_groups(ctx, a, true) == 2 ? launch_query_kernels<2>(ctx, a, true)
                                                 : launch_query_kernels<4>(ctx, a, true);
 }
 
-int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a) { return launch_dkdv<64>(ctx, a); }
+int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a) {
+    if (!ctx->f32_chain && !a.rope && split_dkdv_pays(ctx, a)) return launch_split_dkdv(ctx, a);
+    return launch_dkdv<64>(ctx, a);
+}

@@ -1,21 +1,20 @@
-// Attention forward outside a training step, head dim 64: the work decomposition of the 16-row kernels
-// (ft_attention16.hip) on v_mfma_f32_16x16x32_bf16. Every operand, the probabilities too, is the exact sum
-// of three bf16 parts and a product is six products of parts, as in ft_split.hip: f32 operands and f32 sums at 2.7 times
-// the rate of the f32 instruction.
+// Attention outside a training step, head dim 64: the work of the 16-row kernels (ft_attention16.hip) on
+// v_mfma_f32_16x16x32_bf16. Every operand, probabilities and dS too, is the exact sum of three bf16 parts and a product is
+// six products of parts, as in ft_split.hip: f32 operands and f32 sums at 2.7 times the rate of the f32 instruction.
 //
 // K and V are split once per workgroup, on their way into LDS, as three planes each: rows of a key for the products over
 // the head dim, rows of a head-dim index (32 keys of a wave's half, in the order in which the probabilities leave the
 // score product's registers: 16 u + 4 g + i at 8 g + 4 u + i) for the products over the keys. The probabilities then
 // are the second operand of their product without leaving their lane.
 //
-// A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends the workgroup through
-// the f32 kernel's code, which says what it is.
+// A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends
+// the workgroup through the f32 kernel's code, which says what it is.
 //
 // Bound: a tile of 64 keys costs a workgroup about 3000 cycles each of matrix unit, VALU (softmax and splitting) and LDS
 // reads, and the barrier per tile keeps its waves in step, so they overlap little. us by HIP events, f32 kernel -> this:
-// 4 x 1024 tokens, 15 heads on 5: 93 -> 63; 8 x 1024, 32 heads: 363 -> 256; 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and
-// not kept: one query tile of 64 rows per workgroup, two workgroups a CU (64, 272, 15.5); 32 rows a wave (61, 248, 17.5);
-// dQ the same way (128 registers spill: 132 against 130).
+// forward of 4 x 1024 tokens, 15 heads on 5: 93 -> 63, backward 285 -> 239; 8 x 1024, 32 heads: 363 -> 256 and 1264 ->
+// 951; forward of 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and not kept for the forward: one query tile of 64 rows per
+// workgroup, two workgroups a CU (64, 272, 15.5); 32 rows a wave (61, 248, 17.5).
 #include "ft_attention16.h"
 
 namespace {
@@ -72,18 +71,19 @@ __device__ __forceinline__ int sw_dim(int row, int chunk) {
     return row * 64 + ((chunk ^ (((x << 1) ^ ((x >> 1) * 3)) & 3)) << 4);
 }
 
-// One operand's tile of 64 keys on its way from global memory to LDS: four values a thread and round.
+// One operand's tile of 64 rows (keys; queries in the dK/dV kernel) of one head on its way from global memory to LDS:
+// four values a thread and round; rows past the end repeat the last.
 template <int NT>
-struct KeyRows {       // planes [key][64]
+struct TileRows {       // planes [key][64]
     static constexpr int N = KT * 16 / NT;
     float4 pre[N];
-    __device__ __forceinline__ void fetch(const float* src, const AttnArgs& p, int b, int kvh, int t, int tid) {
+    __device__ __forceinline__ void fetch(const float* src, int stride, int rows, int t, int tid) {
 #pragma unroll
         for (int u = 0; u < N; u++) {
             const int e = tid + NT * u;
-            int key = t * KT + e / 16;
-            key = key < p.Sk ? key : p.Sk - 1;
-            pre[u] = *reinterpret_cast<const float4*>(src + (((long)b * p.Sk + key) * p.Hkv + kvh) * D64 + 4 * (e % 16));
+            int row = t * KT + e / 16;
+            row = row < rows ? row : rows - 1;
+            pre[u] = *reinterpret_cast<const float4*>(src + (long)row * stride + 4 * (e % 16));
         }
     }
     __device__ __forceinline__ void store(char* planes, int tid) const {
@@ -100,18 +100,18 @@ struct KeyRows {       // planes [key][64]
     }
 };
 template <int NT>
-struct KeyColumns {    // planes [key half][64][32 keys]
+struct TileColumns {    // planes [key half][64][32 keys]
     static constexpr int N = KT * 16 / NT;
     float pre[N][4];
-    __device__ __forceinline__ void fetch(const float* src, const AttnArgs& p, int b, int kvh, int t, int tid) {
+    __device__ __forceinline__ void fetch(const float* src, int stride, int rows, int t, int tid) {
 #pragma unroll
         for (int u = 0; u < N; u++) {
             const int e = tid + NT * u, d = e % 64, kg = e / 64;   // keys 4 kg .. 4 kg + 3
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                int key = t * KT + 4 * kg + i;
-                key = key < p.Sk ? key : p.Sk - 1;
-                pre[u][i] = src[(((long)b * p.Sk + key) * p.Hkv + kvh) * D64 + d];
+                int row = t * KT + 4 * kg + i;
+                row = row < rows ? row : rows - 1;
+                pre[u][i] = src[(long)row * stride + d];
             }
         }
     }
@@ -158,11 +158,14 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     QueryWave<NG> w;
     w.init(p, wave, l16);
-    KeyRows<NT> kl;
-    KeyColumns<NT> vl;
+    const int kv_stride = p.Hkv * D64;
+    const float* const k_head = p.k + ((long)w.b * p.Sk * p.Hkv + w.kvh) * D64;
+    const float* const v_head = p.v + ((long)w.b * p.Sk * p.Hkv + w.kvh) * D64;
+    TileRows<NT> kl;
+    TileColumns<NT> vl;
     if (w.nkt > 0) {
-        kl.fetch(p.k, p, w.b, w.kvh, 0, tid);
-        vl.fetch(p.v, p, w.b, w.kvh, 0, tid);
+        kl.fetch(k_head, kv_stride, p.Sk, 0, tid);
+        vl.fetch(v_head, kv_stride, p.Sk, 0, tid);
     }
     // scores are kept in base 2: log2(e) / sqrt(D) goes into Q
     uintx4 qp[2][3];
@@ -239,8 +242,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
     for (int t = 0; t < w.nkt; t++) {
         const bool more = t + 1 < w.nkt;
         if (more) {
-            kl.fetch(p.k, p, w.b, w.kvh, t + 1, tid);
-            vl.fetch(p.v, p, w.b, w.kvh, t + 1, tid);
+            kl.fetch(k_head, kv_stride, p.Sk, t + 1, tid);
+            vl.fetch(v_head, kv_stride, p.Sk, t + 1, tid);
         }
         const char* ks = smem + (t & 1) * STAGE;
         const char* vs = ks + 3 * PLANE;
@@ -300,10 +303,330 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
     if (__syncthreads_or(bad && w.q_ok)) attn16_fwd<NG>(p, reinterpret_cast<float*>(smem));
 }
 
+// dQ = scale * sum_j dS_ij K_j and Delta = dO.O (stats slot 0), dS = P (dO.V - Delta), P = exp(S - LSE). A workgroup
+// takes one query tile of 128 rows, the last (under the causal mask the longest) first; a wave 32 of them, against one
+// half of every 64-key tile: 16 rows a wave on the forward's 16 waves need more than their 128 registers, and an operand
+// read from LDS serves two blocks of rows.
+__global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
+    constexpr int QB = 2;
+    using Waves = QueryTile<4, QB>;
+    constexpr int NT = Waves::WAVES * 64, STAGE = 9 * PLANE;   // K rows, V rows, K columns
+    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int nbh = p.B * p.H, qtile = (p.Sq + Waves::TQ - 1) / Waves::TQ - 1 - (int)blockIdx.x / nbh, qbh = (int)blockIdx.x % nbh;
+    Waves w;
+    w.init(p, wave, l16, qtile, qbh);
+    const int kv_stride = p.Hkv * D64;
+    const float* const k_head = p.k + ((long)w.b * p.Sk * p.Hkv + w.kvh) * D64;
+    const float* const v_head = p.v + ((long)w.b * p.Sk * p.Hkv + w.kvh) * D64;
+    TileRows<NT> kl, vl;
+    TileColumns<NT> kc;
+    auto fetch = [&](int t) {
+        kl.fetch(k_head, kv_stride, p.Sk, t, tid);
+        vl.fetch(v_head, kv_stride, p.Sk, t, tid);
+        kc.fetch(k_head, kv_stride, p.Sk, t, tid);
+    };
+    auto store = [&](char* stage) {
+        kl.store(stage, tid);
+        vl.store(stage + 3 * PLANE, tid);
+        kc.store(stage + 6 * PLANE, tid);
+    };
+    if (w.nkt > 0) fetch(0);
+    uintx4 qp[QB][2][3], dop[QB][2][3];
+    float delta[QB], lse2[QB];
+    int key_lim[QB];
+    floatx4 acc[QB][4];
+#pragma unroll
+    for (int c = 0; c < QB; c++) {
+        const int q = w.q + 16 * c, qc = q < p.Sq ? q : p.Sq - 1;
+        const long qoff = (((long)w.b * p.Sq + qc) * p.H + w.h) * D64;
+        const long srow = ((long)w.b * p.H + w.h) * p.Sq + qc;
+        row_parts(p.q + qoff, g, p.scale * kLog2e, qp[c]);
+        row_parts(p.d_out + qoff, g, 1.0f, dop[c]);
+        delta[c] = 0.0f;
+#pragma unroll
+        for (int blk = 0; blk < 4; blk++) {   // dO.O as the f32 kernel adds it
+            const int d = 16 * blk + 4 * g;
+            const float4 dv = *reinterpret_cast<const float4*>(p.d_out + qoff + d);
+            const float4 ov = *reinterpret_cast<const float4*>(p.out + qoff + d);
+            delta[c] += dv.x * ov.x + dv.y * ov.y + dv.z * ov.z + dv.w * ov.w;
+        }
+        delta[c] = group_sum(delta[c]);
+        lse2[c] = (q < p.Sq ? p.stats[2 * srow + 1] : kAttnLseEmpty) * kLog2e;
+        if (q < p.Sq && g == 0 && w.kh == 0) p.stats[2 * srow] = delta[c];
+        key_lim[c] = (p.causal && q + p.causal_offset < p.Sk - 1) ? q + p.causal_offset : p.Sk - 1;
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[c][e] = zero4();
+    }
+    if (w.nkt > 0) store(smem);
+    __syncthreads();
+
+    bool bad = false;   // something here is for the f32 code
+    auto tile = [&](auto nsb_tag, auto mask_tag, const char* stage, int kb) {
+        constexpr int NSB = decltype(nsb_tag)::value;
+        constexpr bool MASK = decltype(mask_tag)::value;
+        float ds[QB][8];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            floatx4 s[QB], dp[QB];
+#pragma unroll
+            for (int c = 0; c < QB; c++) s[c] = dp[c] = zero4();
+            if (u < NSB) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const int at = sw_key(32 * w.kh + 16 * u + l16, 4 * t + g);
+                    uintx4 kp[3], vp[3];
+                    read_parts(stage + at, kp);
+                    read_parts(stage + 3 * PLANE + at, vp);
+#pragma unroll
+                    for (int c = 0; c < QB; c++) s[c] = mfma_parts(kp, qp[c][t], s[c]);
+#pragma unroll
+                    for (int c = 0; c < QB; c++) dp[c] = mfma_parts(vp, dop[c][t], dp[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < QB; c++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float pij = u < NSB ? exp2_fast(s[c][i] - lse2[c]) : 0.0f;
+                    if constexpr (MASK) {
+                        const int key = kb + 32 * w.kh + 16 * u + 4 * g + i;
+                        pij = key <= key_lim[c] ? pij : 0.0f;
+                    }
+                    ds[c][4 * u + i] = u < NSB ? pij * (dp[c][i] - delta[c]) : 0.0f;
+                }
+        }
+        uintx4 sp[QB][3];
+#pragma unroll
+        for (int c = 0; c < QB; c++) split8(ds[c], sp[c]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            uintx4 kp[3];
+            read_parts(stage + 6 * PLANE + w.kh * (PLANE / 2) + sw_dim(16 * e + l16, g), kp);
+#pragma unroll
+            for (int c = 0; c < QB; c++) acc[c][e] = mfma_parts(kp, sp[c], acc[c][e]);
+        }
+    };
+    using std::integral_constant;
+    for (int t = 0; t < w.nkt; t++) {
+        const bool more = t + 1 < w.nkt;
+        if (more) fetch(t + 1);
+        const char* stage = smem + (t & 1) * STAGE;
+        const int kb = t * KT;
+        const int nsb = w.visible_subblocks(kb);
+        if (nsb > 0) {
+            if (w.half_unmasked(kb))
+                tile(integral_constant<int, 2>{}, std::false_type{}, stage, kb);
+            else if (nsb == 2)
+                tile(integral_constant<int, 2>{}, std::true_type{}, stage, kb);
+            else
+                tile(integral_constant<int, 1>{}, std::true_type{}, stage, kb);
+        }
+        if (more) store(smem + ((t + 1) & 1) * STAGE);
+        __syncthreads();
+    }
+
+    // the second key half's partial dQ joins the first's, lane for lane
+    float* mrg = reinterpret_cast<float*>(smem) + (w.w2 * 16 * QB) * 64 + lane;
+    if (w.kh == 1) {
+#pragma unroll
+        for (int c = 0; c < QB; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) mrg[(16 * c + 4 * e + r) * 64] = acc[c][e][r];
+    }
+    __syncthreads();
+    if (w.kh == 0) {
+        // K in LDS carries no scale (only Q does, for the scores): dQ = scale * dS K
+#pragma unroll
+        for (int c = 0; c < QB; c++) {
+            const int q = w.q + 16 * c;
+            float* drow = p.dq + (((long)w.b * p.Sq + q) * p.H + w.h) * D64;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                floatx4 v;
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[r] = (acc[c][e][r] + mrg[(16 * c + 4 * e + r) * 64]) * p.scale;
+                if (q < p.Sq) {
+                    bad = bad || not_finite(v);
+                    *reinterpret_cast<floatx4*>(drow + 16 * e + 4 * g) = v;
+                }
+            }
+        }
+    }
+    if (__syncthreads_or(bad)) {
+#pragma unroll 1
+        for (int c = 0; c < QB; c++) {
+            if ((qtile * QB + c) * 64 < p.Sq)
+                attn16_dq<4, QueryTile<4>>(p, reinterpret_cast<float*>(smem), qtile * QB + c, qbh);
+            __syncthreads();
+        }
+    }
+}
+
 template <int NG>
 dim3 query_grid(const AttnArgs& a) {
     const size_t nT = ft_div_up(a.Sq, 16 * NG);
     return dim3((unsigned)(((nT + 1) / 2) * (size_t)a.B * a.H));
+}
+
+// dK and dV of 64 keys, of one query head (split_g) or summed over a kv head's group: a wave owns 16 keys (their K, scaled
+// for base-2 scores, and V in registers) against one half of every 64-query tile, whose Q and dO lie in LDS as rows and
+// as columns. P and dS leave the score products as second operands of dV^T += dO^T P and dK^T += Q^T dS. Key tile 0
+// (under the causal mask the most queries) first.
+__global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
+    constexpr int NT = 512;
+    __shared__ __attribute__((aligned(16))) char smem[12 * PLANE + KT * 8];   // Q rows, dO rows, Q columns, dO columns; stats
+    float2* const st = reinterpret_cast<float2*>(smem + 12 * PLANE);           // (Delta, LSE in base 2) of the tile's queries
+    const int tid = threadIdx.x, lane = tid % 64, l16 = lane % 16, g = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64), qh = wave / 4;
+    const int nhu = p.B * (p.split_g ? p.H : p.Hkv);
+    const int kt = (int)blockIdx.x / nhu, bh = (int)blockIdx.x % nhu;
+    const int Gfull = p.H / p.Hkv;
+    const int b = bh / (p.split_g ? p.H : p.Hkv), hsel = bh % (p.split_g ? p.H : p.Hkv);
+    const int kvh = p.split_g ? hsel / Gfull : hsel, g0 = p.split_g ? hsel % Gfull : 0, G = p.split_g ? 1 : Gfull;
+    const int kb0 = kt * KT + 16 * (wave % 4);
+    const int key = kb0 + l16;
+    const int key_m = key < p.Sk ? key : 0x7fffffff;   // a key past the end is visible to nobody
+    const long krow = (((long)b * p.Sk + (key < p.Sk ? key : p.Sk - 1)) * p.Hkv + kvh) * D64;
+    uintx4 kp[2][3], vp[2][3];
+    row_parts(p.k + krow, g, p.scale * kLog2e, kp);
+    row_parts(p.v + krow, g, 1.0f, vp);
+
+    const int nqt = (p.Sq + KT - 1) / KT;
+    int qt0 = 0;
+    if (p.causal) {
+        const int first_q = kt * KT - p.causal_offset;   // the first query that sees the tile's first key
+        qt0 = first_q > 0 ? first_q / KT : 0;
+    }
+    const int per_head = nqt > qt0 ? nqt - qt0 : 0, items = per_head * G;
+    TileRows<NT> ql, dl;
+    TileColumns<NT> qc, dc;
+    float2 stat = make_float2(0.f, 0.f);
+    auto fetch = [&](int item) {
+        const int h = kvh * Gfull + g0 + item / per_head, t = qt0 + item % per_head;
+        const long head = ((long)b * p.Sq * p.H + h) * D64;
+        const int stride = p.H * D64;
+        ql.fetch(p.q + head, stride, p.Sq, t, tid);
+        dl.fetch(p.d_out + head, stride, p.Sq, t, tid);
+        qc.fetch(p.q + head, stride, p.Sq, t, tid);
+        dc.fetch(p.d_out + head, stride, p.Sq, t, tid);
+        if (tid < KT) {
+            int q = t * KT + tid;
+            q = q < p.Sq ? q : p.Sq - 1;
+            stat = *reinterpret_cast<const float2*>(p.stats + 2 * (((long)b * p.H + h) * p.Sq + q));
+        }
+    };
+    auto store = [&]() {
+        ql.store(smem, tid);
+        dl.store(smem + 3 * PLANE, tid);
+        qc.store(smem + 6 * PLANE, tid);
+        dc.store(smem + 9 * PLANE, tid);
+        if (tid < KT) st[tid] = make_float2(stat.x, stat.y * kLog2e);
+    };
+    floatx4 dk[4], dv[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) dk[e] = dv[e] = zero4();
+    if (items > 0) {
+        fetch(0);
+        store();
+    }
+    __syncthreads();
+    for (int item = 0; item < items; item++) {
+        const bool more = item + 1 < items;
+        if (more) fetch(item + 1);
+        const int q0 = (qt0 + item % per_head) * KT + 32 * qh;
+        // queries of this half that see some key of the wave: all of them, or none of the first ones
+        const bool some = !p.causal || q0 + 31 + p.causal_offset >= kb0;
+        if (some && q0 < p.Sq) {
+            float pr[8], ds[8];
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                floatx4 s = zero4(), dp = zero4();
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const int at = sw_key(32 * qh + 16 * u + l16, 4 * t + g);
+                    uintx4 qp[3], dop[3];
+                    read_parts(smem + at, qp);
+                    read_parts(smem + 3 * PLANE + at, dop);
+                    s = mfma_parts(qp, kp[t], s);
+                    dp = mfma_parts(dop, vp[t], dp);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    // visible: a real key, a real query, and not above the diagonal (a select: exp2(-inf) = 0)
+                    const int qi = q0 + 16 * u + 4 * g + i;
+                    const float2 c = st[32 * qh + 16 * u + 4 * g + i];
+                    const int lim = qi < p.Sq ? (p.causal ? qi + p.causal_offset : 0x7ffffffe) : -1;
+                    const float pij = exp2_fast(key_m <= lim ? s[i] - c.y : -INFINITY);
+                    pr[4 * u + i] = pij;
+                    ds[4 * u + i] = pij * (dp[i] - c.x);
+                }
+            }
+            uintx4 pp[3], sp[3];
+            split8(pr, pp);
+            split8(ds, sp);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int at = 6 * PLANE + qh * (PLANE / 2) + sw_dim(16 * e + l16, g);
+                uintx4 qp[3], dop[3];
+                read_parts(smem + at, qp);
+                read_parts(smem + 3 * PLANE + at, dop);
+                dk[e] = mfma_parts(qp, sp, dk[e]);
+                dv[e] = mfma_parts(dop, pp, dv[e]);
+            }
+        }
+        __syncthreads();
+        if (more) {
+            store();
+            __syncthreads();
+        }
+    }
+
+    // The two query halves of a key block meet through LDS, lane for lane.
+    float* mrg = reinterpret_cast<float*>(smem) + (wave % 4) * 32 * 64 + lane;
+    if (qh == 1) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                mrg[(4 * e + r) * 64] = dk[e][r];
+                mrg[(16 + 4 * e + r) * 64] = dv[e][r];
+            }
+    }
+    __syncthreads();
+    bool bad = false;
+    if (qh == 0) {
+        // register r of accumulator e is head-dim index 16 e + 4 g + r; dK = scale * sum dS Q (here, or where the heads
+        // of the group are added)
+        const long n_all = (long)p.B * p.Sk * p.Hkv * D64;
+        float* const dk_out = p.split_g ? p.part + 2 * g0 * n_all : p.dk;
+        float* const dv_out = p.split_g ? p.part + (2 * g0 + 1) * n_all : p.dv;
+        const float scale = p.split_g ? 1.0f : p.scale;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            floatx4 x, y;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                x[r] = (dk[e][r] + mrg[(4 * e + r) * 64]) * scale;
+                y[r] = dv[e][r] + mrg[(16 + 4 * e + r) * 64];
+            }
+            if (key < p.Sk) {
+                bad = bad || not_finite(x) || not_finite(y);
+                *reinterpret_cast<floatx4*>(dk_out + krow + 16 * e + 4 * g) = x;
+                *reinterpret_cast<floatx4*>(dv_out + krow + 16 * e + 4 * g) = y;
+            }
+        }
+    }
+    if (__syncthreads_or(bad)) {
+#pragma unroll 1
+        for (int c = 0; c < 4; c++) {
+            if (kt * KT + 16 * c < p.Sk) attn16_dkdv<64>(p, reinterpret_cast<float*>(smem), (4 * kt + c) * nhu + bh);
+            __syncthreads();
+        }
+    }
 }
 
 }  // namespace
@@ -311,6 +634,19 @@ dim3 query_grid(const AttnArgs& a) {
 int ft_attn_split_forward(ft_context* ctx, const AttnArgs& a, int groups) {
     if (groups == 2) hipLaunchKernelGGL(attn_split_fwd_kernel<2>, query_grid<2>(a), dim3(512), 0, ctx->stream, a);
     else hipLaunchKernelGGL(attn_split_fwd_kernel<4>, query_grid<4>(a), dim3(1024), 0, ctx->stream, a);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}
+
+int ft_attn_split_dq(ft_context* ctx, const AttnArgs& a) {
+    hipLaunchKernelGGL(attn_split_dq_kernel, dim3((unsigned)(ft_div_up(a.Sq, 128) * (size_t)a.B * a.H)), dim3(512), 0, ctx->stream, a);
+    FT_LAUNCH_CHECK();
+    return FT_OK;
+}
+
+int ft_attn_split_dkdv(ft_context* ctx, const AttnArgs& a) {
+    const size_t heads = (size_t)a.B * (a.split_g ? a.H : a.Hkv);
+    hipLaunchKernelGGL(attn_split_dkdv_kernel, dim3((unsigned)(ft_div_up(a.Sk, 64) * heads)), dim3(512), 0, ctx->stream, a);
     FT_LAUNCH_CHECK();
     return FT_OK;
 }

@@ -235,3 +235,60 @@ def test_attention_with_infinite_and_nan_values_as_the_f32_kernel(g):
     np.testing.assert_allclose(got[ok], want[ok], atol=2e-5)
     np.testing.assert_allclose(got[3, :, 2, 11], want[3, :, 2, 11], rtol=1e-4, atol=2e-5)
     assert fine[[0, 1, 3]][:, :, [0, 4, 6]].all()   # the other heads
+
+
+def backward64(q, k, v, do, causal, offset):
+    B, Sq, H, D = q.shape
+    Hkv = k.shape[2]
+    rep = H // Hkv
+    qt, dt = (x.astype(np.float64).transpose(0, 2, 1, 3) for x in (q, do))
+    kt, vt = (np.repeat(x, rep, axis=2).astype(np.float64).transpose(0, 2, 1, 3) for x in (k, v))
+    s = np.matmul(qt, kt.transpose(0, 1, 3, 2)) / np.sqrt(D)
+    if causal:
+        s = np.where(np.arange(k.shape[1])[None, :] <= np.arange(Sq)[:, None] + offset, s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    dp = np.matmul(dt, vt.transpose(0, 1, 3, 2))
+    ds = p * (dp - (p * dp).sum(-1, keepdims=True)) / np.sqrt(D)
+    back = lambda x: x.transpose(0, 2, 1, 3)
+    group = lambda x: back(x).reshape(B, -1, Hkv, rep, D).sum(3)
+    return back(np.matmul(ds, kt)), group(np.matmul(ds.transpose(0, 1, 3, 2), qt)), group(np.matmul(p.transpose(0, 1, 3, 2), dt))
+
+
+def run_attention(ctx, eng, q, k, v, do, causal, offset):
+    from ferrotensor_amd import AttentionOptions
+    B, Sq, H, D = q.shape
+    t = [up(ctx, x) for x in (q, k, v)]
+    o, stats = empty(ctx, *q.shape), empty(ctx, B * H * Sq, 2)
+    dq, dk, dv = empty(ctx, *q.shape), empty(ctx, *k.shape), empty(ctx, *k.shape)
+    opts = AttentionOptions(causal=causal, causal_offset=offset)
+    eng.flash_attention_v2_with_stats(ctx, *t, o, stats, opts)
+    eng.flash_attention_v2_backward_with_stats(ctx, *t, o, up(ctx, do), dq, dk, dv, stats, opts)
+    return [np.asarray(x.to_vec(), np.float32).reshape(y.shape) for x, y in ((dq, q), (dk, k), (dv, k))]
+
+
+# From 384 workgroups of 128 queries (dQ) and 768 of 64 keys (dK/dV) on: ragged tiles, heads without a group, a group added
+# by the second kernel, a group too large for its scratch, an offset, no mask.
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(8, 200, 200, 32, 32, True, 0), (8, 129, 193, 32, 16, True, 64), (7, 140, 190, 32, 32, False, 0),
+                                                         (8, 300, 300, 32, 8, True, 0), (8, 65, 200, 48, 48, True, 0)])
+def test_attention_backward(g, B, Sq, Sk, H, Hkv, causal, offset):
+    ctx, eng = g
+    q, k, v, do = rnd(1, B, Sq, H, 64), rnd(2, B, Sk, Hkv, 64), rnd(3, B, Sk, Hkv, 64), rnd(4, B, Sq, H, 64, scale=1e-2)
+    for name, got, want in zip(("dq", "dk", "dv"), run_attention(ctx, eng, q, k, v, do, causal, offset), backward64(q, k, v, do, causal, offset)):
+        # probabilities to 2^-18 of themselves, sums of at most a few hundred rounded terms
+        assert np.max(np.abs(got - want)) <= 2e-5 * np.max(np.abs(want)), name
+
+
+def test_attention_backward_with_infinite_and_nan_values_as_the_f32_kernels(g):
+    """The batch takes the kernels on bf16 parts; its sequences one at a time do not: the same values are not finite."""
+    ctx, eng = g
+    B, S, H = 8, 200, 32
+    q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
+    v[0, 50, 3, 7], do[1, 100, 5, 9], k[2, 70, 1, 4], q[3, 190, 2, 1], do[4, 3, 7, 0] = np.inf, np.nan, np.nan, np.inf, 3.4e38
+    batch = run_attention(ctx, eng, q, k, v, do, True, 0)
+    for i in range(5):
+        one = run_attention(ctx, eng, *(x[i:i + 1] for x in (q, k, v, do)), True, 0)
+        for name, a, b in zip(("dq", "dk", "dv"), batch, one):
+            assert np.array_equal(np.isfinite(a[i]), np.isfinite(b[0])), (i, name)
+            fine = np.isfinite(b[0])
+            np.testing.assert_allclose(a[i][fine], b[0][fine], rtol=2e-4, atol=2e-6)
