@@ -279,6 +279,20 @@ def test_fused_lora_linear_forward_and_backward(g, M, K, N, r, f16):
     assert_close("dA", da.to_numpy(), grads["l.lora_a"], atol=2e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("r", [4, 8, 16])
+@pytest.mark.parametrize("M", [1, 127, 128, 129])
+def test_lora_factor_gradients_at_the_edge_of_one_slice(g, M, r):
+    ctx, eng = g
+    x, t = rnd(M, M, 100), rnd(r, M, r)
+    da, db = empty(ctx, 100, r), empty(ctx, r, 100)
+    eng.lora_grad_a(ctx, up(ctx, x), up(ctx, t), da)
+    eng.lora_grad_b(ctx, up(ctx, t), up(ctx, x), db)
+    want = f64_mm(x.T, t)
+    # at most M roundings of sums of at most sum |x||t|
+    limit = (M + 2) * 2.0 ** -24 * f64_mm(np.abs(x.T), np.abs(t)) + 1e-30
+    assert np.all(np.abs(da.to_numpy() - want) <= limit) and np.all(np.abs(db.to_numpy() - want.T) <= limit.T)
+
+
 @pytest.mark.parametrize("M,K,Ns,r,f16", [(256, 960, (960, 320, 320), 8, True), (100, 64, (64, 32, 96), 4, True),
                                           (192, 128, (320, 256), 0, True), (64, 32, (48, 40), 8, False),
                                           (130, 96, (40, 72, 8), 16, True),
