@@ -1039,6 +1039,32 @@ def test_135m_width_step_matches_oracle(ctx, checkpoint):
         assert np.all(np.abs(params[n] - before[n]).reshape(-1)[~firm] <= 1.001e-3), n
 
 
+@pytest.mark.parametrize("rank", [4, 16])
+def test_f32_weights_step_matches_oracle(ctx, rank):
+    """f32 weights, adapters on all seven projections, ragged rows: products with a rank-r term, a residual or both on the
+    DMA-fed f32 kernel, forward (a @ b) and input gradient (a @ b^T)."""
+    from ferrotensor_amd.trainer import ModelConfig, Trainer
+    cfg = ModelConfig(vocab_size=256, hidden_size=192, intermediate_size=416, num_hidden_layers=2,
+                      num_attention_heads=3, num_key_value_heads=1, rms_norm_eps=1e-5, rope_theta=100000.0,
+                      tie_word_embeddings=True, f16_linears=False)
+    hip, orc = build_pair(ctx, cfg, ["q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj"], rank=rank,
+                          alpha=16.0, seed=78)
+    rng = np.random.default_rng(9)
+    rows = rng.integers(0, 256, (3, 101)).astype(np.uint32)
+    targets = np.concatenate([rows[:, 1:], rows[:, :1]], axis=1)
+    masks = np.ones((3, 101), np.uint8)
+    masks[:, :20] = 0
+    tr = Trainer(hip, lr=1e-3, weight_decay=0.0, clip_grad_norm=1.0)
+    tr.train_chunk(rows, targets, masks, apply=False)
+    grads = hip.grads()
+    want_stats, _, want_grads = rs.train_chunk(orc, rs.AdamW(lr=1e-3, weight_decay=0.0), rows, targets, masks, clip_grad_norm=1.0,
+                                               return_grads=True)
+    cs = want_stats.clip_scale or 1.0
+    for n in grads:
+        assert_close(f"grad {n}", grads[n], want_grads[n] / np.float32(cs))
+    assert_close("loss", [tr.train_chunk(rows, targets, masks).loss], [want_stats.loss])
+
+
 def _with_biases(tensors, which, seed):
     rng = np.random.default_rng(seed)
     out = dict(tensors)
