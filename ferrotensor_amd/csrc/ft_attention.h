@@ -31,6 +31,7 @@ struct AttnArgs {
     // adds the group in head order.
     float* part;
     int split_g;
+    int forward_only;   // no backward will ask for this forward's statistics
 };
 
 constexpr size_t kAttnScratchFloats = (size_t)8 << 20;  // 32 MiB of per-head partial dK/dV

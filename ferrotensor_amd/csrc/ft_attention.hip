@@ -1273,6 +1273,18 @@ int ft_flash_attention_v2_backward_with_stats(ft_context* ctx, const float* q, c
 
 }  // extern "C"
 
+// ft_flash_attention_v2_with_stats for a pass that no backward follows.
+int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
+                                       size_t Sq, size_t Sk, size_t H, size_t Hkv, size_t D, const ft_attention_options* opts) {
+    FT_TRY(check_common("attention forward", ctx, B, Sq, Sk, H, Hkv, D, opts));
+    AttnArgs a = make_args(B, Sq, Sk, H, Hkv, D, opts);
+    a.q = q; a.k = k; a.v = v; a.o = out;
+    a.forward_only = 1;
+    if (D <= 32) return launch_fwd<32>(ctx, a);
+    if (D <= 64) return launch_fwd<64>(ctx, a);
+    return launch_fwd<128>(ctx, a);
+}
+
 // Can the backward kernels rotate dQ and dK back through RoPE themselves (self-attention over
 // whole rows from position 0, head_dim 64, aligned tensors)?
 bool ft_internal_attention_rope_fusable(const float* q, const float* k, const float* v, const float* out,

@@ -86,15 +86,17 @@ int query_tile_groups(const ft_context* ctx, const AttnArgs& a, bool backward) {
     return 0;
 }
 
-// The kernels on bf16 parts hold one workgroup of 8 waves per CU and want a few rounds of them. dQ, 480 workgroups
-// (4 x 1024 tokens, 15 heads on 5): 89 us against 128; 120 (one sequence): 13 us longer. dK/dV, time of the whole
-// backward beside the f32 kernel's: 8 x 1024, 32 heads (4096 workgroups) 924 against 1154, 4 x 1024, 15 on 5 (960) 232
-// against 246, 8 x 256, 15 on 5 (480) 61.9 against 60.0.
-bool split_dq_pays(const ft_context* ctx, const AttnArgs& a) {
-    return ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 >= 3 * (size_t)ctx->num_cus;
+// The backward on bf16 parts: its kernels hold one workgroup of 8 waves per CU and want a few rounds of them. dQ, 480
+// workgroups (4 x 1024 tokens, 15 heads on 5): 89 us against 128; 120 (one sequence): 13 us longer. dK/dV, time of the
+// whole backward beside the f32 kernel's: 8 x 1024, 32 heads (4096 workgroups) 924 against 1154, 4 x 1024, 15 on 5 (960)
+// 232 against 246, 8 x 256, 15 on 5 (480) 61.9 against 60.0. Both or neither, and the forward with them: kernels that form
+// the same scores with the same rounding lose less in the probabilities.
+bool split_backward_pays(const ft_context* ctx, const AttnArgs& a) {
+    return !ctx->f32_chain && ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 >= 3 * (size_t)ctx->num_cus &&
+           ft_div_up(a.Sk, 64) * (size_t)a.B * a.H >= 3 * (size_t)ctx->num_cus;
 }
-bool split_dkdv_pays(const ft_context* ctx, const AttnArgs& a) {
-    return ft_div_up(a.Sk, 64) * (size_t)a.B * a.H >= 3 * (size_t)ctx->num_cus;
+bool split_forward_pays(const ft_context* ctx, const AttnArgs& a) {
+    return !ctx->f32_chain && (a.forward_only || split_backward_pays(ctx, a));
 }
 
 // One workgroup per 64 keys and query head, then the ordered sum over the group where there is one (and room for its
@@ -152,15 +154,17 @@ bool ft_attn16_usable(const AttnArgs& a) {
            al(a.o) && al(a.dq) && al(a.dk) && al(a.dv) && (((uintptr_t)a.stats) & 7) == 0;
 }
 
-// (The forward on bf16 parts beats the 32-row kernels at every size: 1 x 96 tokens, 15 heads, 7.0 us against 8.0;
-// 2 x 160, 9 heads 8.7 against 11.4; 1 x 40, 9 heads 5.5 against 7.1.)
+// (Alone the forward on bf16 parts beats the f32 kernels at every size, the 32-row ones too: 1 x 96 tokens, 15 heads, 7.0 us
+// against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 40, 9 heads 5.5 against 7.1.)
 bool ft_attn16_forward_pays(const ft_context* ctx, const AttnArgs& a) {
-    return !ctx->f32_chain || query_tile_groups(ctx, a, false) != 0;
+    return split_forward_pays(ctx, a) || query_tile_groups(ctx, a, false) != 0;
 }
-bool ft_attn16_backward_dq_pays(const ft_context* ctx, const AttnArgs& a) { return query_tile_groups(ctx, a, true) != 0; }
+bool ft_attn16_backward_dq_pays(const ft_context* ctx, const AttnArgs& a) {
+    return (!a.rope && split_backward_pays(ctx, a)) || query_tile_groups(ctx, a, true) != 0;
+}
 
 int ft_attn16_forward(ft_context* ctx, const AttnArgs& a) {
-    if (!ctx->f32_chain) {
+    if (split_forward_pays(ctx, a)) {
         const int groups = query_tile_groups(ctx, a, false);
         return ft_attn_split_forward(ctx, a, groups ? groups : 2);
     }
@@ -169,12 +173,12 @@ int ft_attn16_forward(ft_context* ctx, const AttnArgs& a) {
 }
 
 int ft_attn16_backward_dq(ft_context* ctx, const AttnArgs& a) {
-    if (!ctx->f32_chain && !a.rope && split_dq_pays(ctx, a)) return ft_attn_split_dq(ctx, a);
+    if (!a.rope && split_backward_pays(ctx, a)) return ft_attn_split_dq(ctx, a);
     return query_tile_groups(ctx, a, true) == 2 ? launch_query_kernels<2>(ctx, a, true)
                                                 : launch_query_kernels<4>(ctx, a, true);
 }
 
 int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a) {
-    if (!ctx->f32_chain && !a.rope && split_dkdv_pays(ctx, a)) return launch_split_dkdv(ctx, a);
+    if (!a.rope && split_backward_pays(ctx, a)) return launch_split_dkdv(ctx, a);
     return launch_dkdv<64>(ctx, a);
 }

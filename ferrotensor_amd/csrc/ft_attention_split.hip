@@ -10,10 +10,14 @@
 // A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends
 // the workgroup through the f32 kernel's code, which says what it is.
 //
+// Relative error against f64 (2-norm), f32 kernels -> these, 4 x 1024 tokens, 15 heads on 5, normal values: o 2.8e-7 -> 2.1e-7,
+// dq 4.4e-7 -> 3.6e-7, dk 5.6e-7 -> 3.4e-7, dv 5.1e-7 -> 3.0e-7; scores nine times as large (4 x 512, 32 heads): 9.3e-7 ->
+// 6.0e-7, 2.1e-6 -> 1.5e-6, 2.5e-6 -> 1.5e-6, 2.0e-6 -> 1.1e-6.
+//
 // Bound: a tile of 64 keys costs a workgroup about 3000 cycles each of matrix unit, VALU (softmax and splitting) and LDS
 // reads, and the barrier per tile keeps its waves in step, so they overlap little. us by HIP events, f32 kernel -> this:
-// forward of 4 x 1024 tokens, 15 heads on 5: 93 -> 63, backward 285 -> 239; 8 x 1024, 32 heads: 363 -> 256 and 1264 ->
-// 951; forward of 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and not kept for the forward: one query tile of 64 rows per
+// forward of 4 x 1024 tokens, 15 heads on 5: 93 -> 63, backward 285 -> 240; 8 x 1024, 32 heads: 363 -> 260 and 1264 ->
+// 965; forward alone of 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and not kept for the forward: one query tile of 64 rows per
 // workgroup, two workgroups a CU (64, 272, 15.5); 32 rows a wave (61, 248, 17.5).
 #include "ft_attention16.h"
 
@@ -53,14 +57,23 @@ __device__ __forceinline__ void split8(const float (&x)[8], uintx4 (&part)[3]) {
     }
 }
 
-// acc += a b over 32 k, smallest products first
+// acc += a b over 32 k, smallest products first. SWAPPED: in the order that mfma_parts(b, a) takes.
+template <bool SWAPPED = false>
 __device__ __forceinline__ floatx4 mfma_parts(const uintx4 (&a)[3], const uintx4 (&b)[3], floatx4 acc) {
     constexpr int U[6] = {2, 0, 1, 1, 0, 0}, V[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
     for (int t = 0; t < 6; t++)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[U[t]]), __builtin_bit_cast(bf16x8, b[V[t]]),
-                                                      acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[SWAPPED ? V[t] : U[t]]),
+                                                      __builtin_bit_cast(bf16x8, b[SWAPPED ? U[t] : V[t]]), acc, 0, 0, 0);
     return acc;
+}
+
+// A score in base 2, rounded here and nowhere else: the three kernels take the same products in the same order and
+// exponentiate the same number, so what a score is off by leaves the probabilities with the log-sum-exp. (A fused
+// multiply-add with what is subtracted from it would round elsewhere.)
+__device__ __forceinline__ float scaled_score(float s, float scale) {
+#pragma clang fp contract(off)
+    return s * scale;
 }
 
 // Chunk swizzles (16 bytes) that spread the 16 lanes served together over all banks, see ft_attention16.h: rows of 128
@@ -134,13 +147,13 @@ __device__ __forceinline__ void read_parts(const char* at, uintx4 (&part)[3]) {
     for (int q = 0; q < 3; q++) part[q] = *reinterpret_cast<const uintx4*>(at + q * PLANE);
 }
 
-// A row's 64 values (this lane's 16 of them) as the two k steps' operand registers, scaled.
-__device__ __forceinline__ void row_parts(const float* row, int g, float scale, uintx4 (&part)[2][3]) {
+// A row's 64 values (this lane's 16 of them) as the two k steps' operand registers.
+__device__ __forceinline__ void row_parts(const float* row, int g, uintx4 (&part)[2][3]) {
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
         const float4 a = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g);
         const float4 b = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g + 4);
-        const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale, b.x * scale, b.y * scale, b.z * scale, b.w * scale};
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         split8(x, part[ks]);
     }
 }
@@ -167,9 +180,9 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         kl.fetch(k_head, kv_stride, p.Sk, 0, tid);
         vl.fetch(v_head, kv_stride, p.Sk, 0, tid);
     }
-    // scores are kept in base 2: log2(e) / sqrt(D) goes into Q
+    const float sscale = p.scale * kLog2e;   // scores are kept in base 2
     uintx4 qp[2][3];
-    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, p.scale * kLog2e, qp);
+    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, qp);
     floatx4 o[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = zero4();
@@ -201,6 +214,7 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         for (int u = 0; u < NSB; u++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
+                s[u][i] = scaled_score(s[u][i], sscale);
                 if constexpr (MASK) {
                     const int key = kb + 32 * w.kh + 16 * u + 4 * g + i;
                     s[u][i] = key <= key_lim ? s[u][i] : kAttnMasked;
@@ -333,6 +347,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         kc.store(stage + 6 * PLANE, tid);
     };
     if (w.nkt > 0) fetch(0);
+    const float sscale = p.scale * kLog2e;
     uintx4 qp[QB][2][3], dop[QB][2][3];
     float delta[QB], lse2[QB];
     int key_lim[QB];
@@ -342,8 +357,8 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         const int q = w.q + 16 * c, qc = q < p.Sq ? q : p.Sq - 1;
         const long qoff = (((long)w.b * p.Sq + qc) * p.H + w.h) * D64;
         const long srow = ((long)w.b * p.H + w.h) * p.Sq + qc;
-        row_parts(p.q + qoff, g, p.scale * kLog2e, qp[c]);
-        row_parts(p.d_out + qoff, g, 1.0f, dop[c]);
+        row_parts(p.q + qoff, g, qp[c]);
+        row_parts(p.d_out + qoff, g, dop[c]);
         delta[c] = 0.0f;
 #pragma unroll
         for (int blk = 0; blk < 4; blk++) {   // dO.O as the f32 kernel adds it
@@ -389,7 +404,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
             for (int c = 0; c < QB; c++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    float pij = u < NSB ? exp2_fast(s[c][i] - lse2[c]) : 0.0f;
+                    float pij = u < NSB ? exp2_fast(scaled_score(s[c][i], sscale) - lse2[c]) : 0.0f;
                     if constexpr (MASK) {
                         const int key = kb + 32 * w.kh + 16 * u + 4 * g + i;
                         pij = key <= key_lim[c] ? pij : 0.0f;
@@ -439,7 +454,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
     }
     __syncthreads();
     if (w.kh == 0) {
-        // K in LDS carries no scale (only Q does, for the scores): dQ = scale * dS K
+        // dQ = scale * dS K
 #pragma unroll
         for (int c = 0; c < QB; c++) {
             const int q = w.q + 16 * c;
@@ -472,8 +487,8 @@ dim3 query_grid(const AttnArgs& a) {
     return dim3((unsigned)(((nT + 1) / 2) * (size_t)a.B * a.H));
 }
 
-// dK and dV of 64 keys, of one query head (split_g) or summed over a kv head's group: a wave owns 16 keys (their K, scaled
-// for base-2 scores, and V in registers) against one half of every 64-query tile, whose Q and dO lie in LDS as rows and
+// dK and dV of 64 keys, of one query head (split_g) or summed over a kv head's group: a wave owns 16 keys (their K and V
+// in registers) against one half of every 64-query tile, whose Q and dO lie in LDS as rows and
 // as columns. P and dS leave the score products as second operands of dV^T += dO^T P and dK^T += Q^T dS. Key tile 0
 // (under the causal mask the most queries) first.
 __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
@@ -491,9 +506,10 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
     const int key = kb0 + l16;
     const int key_m = key < p.Sk ? key : 0x7fffffff;   // a key past the end is visible to nobody
     const long krow = (((long)b * p.Sk + (key < p.Sk ? key : p.Sk - 1)) * p.Hkv + kvh) * D64;
+    const float sscale = p.scale * kLog2e;
     uintx4 kp[2][3], vp[2][3];
-    row_parts(p.k + krow, g, p.scale * kLog2e, kp);
-    row_parts(p.v + krow, g, 1.0f, vp);
+    row_parts(p.k + krow, g, kp);
+    row_parts(p.v + krow, g, vp);
 
     const int nqt = (p.Sq + KT - 1) / KT;
     int qt0 = 0;
@@ -551,8 +567,8 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
                     uintx4 qp[3], dop[3];
                     read_parts(smem + at, qp);
                     read_parts(smem + 3 * PLANE + at, dop);
-                    s = mfma_parts(qp, kp[t], s);
-                    dp = mfma_parts(dop, vp[t], dp);
+                    s = mfma_parts<true>(qp, kp[t], s);
+                    dp = mfma_parts<true>(dop, vp[t], dp);
                 }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
@@ -560,7 +576,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
                     const int qi = q0 + 16 * u + 4 * g + i;
                     const float2 c = st[32 * qh + 16 * u + 4 * g + i];
                     const int lim = qi < p.Sq ? (p.causal ? qi + p.causal_offset : 0x7ffffffe) : -1;
-                    const float pij = exp2_fast(key_m <= lim ? s[i] - c.y : -INFINITY);
+                    const float pij = exp2_fast(key_m <= lim ? scaled_score(s[i], sscale) - c.y : -INFINITY);
                     pr[4 * u + i] = pij;
                     ds[4 * u + i] = pij * (dp[i] - c.x);
                 }
@@ -574,8 +590,9 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
                 uintx4 qp[3], dop[3];
                 read_parts(smem + at, qp);
                 read_parts(smem + 3 * PLANE + at, dop);
-                dk[e] = mfma_parts(qp, sp, dk[e]);
-                dv[e] = mfma_parts(dop, pp, dv[e]);
+                // (a tile's sum of its own first: one rounding of the running sum a tile, not six)
+                dk[e] += mfma_parts(qp, sp, zero4());
+                dv[e] += mfma_parts(dop, pp, zero4());
             }
         }
         __syncthreads();

@@ -52,6 +52,8 @@ int ft_internal_row_bias_add(ft_context* ctx, float* y, const float* bias, size_
 int ft_internal_col_sum(ft_context* ctx, const float* g, float* out, size_t rows, size_t cols, int accumulate);
 bool ft_internal_attention_rope_fusable(const float* q, const float* k, const float* v, const float* out,
                                         const float* d_out, size_t Sq, size_t Sk, size_t D);
+int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
+                                       size_t Sq, size_t Sk, size_t H, size_t Hkv, size_t D, const ft_attention_options* opts);
 int ft_internal_attention_backward_rope(ft_context* ctx, const float* q, const float* k, const float* v,
                                         const float* out, const float* d_out, float* dq, float* dk, float* dv,
                                         float* stats, size_t B, size_t S, size_t H, size_t Hkv,
@@ -659,7 +661,10 @@ int layer_forward(ft_model* m, size_t l, size_t B, size_t S, bool defer_tail = f
             FT_TRY(ft_rope_theta(ctx, a.q, B, S, nh * D, D, 0, c.rope_theta));
             FT_TRY(ft_rope_theta(ctx, a.k, B, S, nkv * D, D, 0, c.rope_theta));
         }
-        FT_TRY(ft_flash_attention_v2_with_stats(ctx, a.q, a.k, a.v, a.attn, a.stats, B, S, S, nh, nkv, D, &opts));
+        if (ctx->f32_chain)
+            FT_TRY(ft_flash_attention_v2_with_stats(ctx, a.q, a.k, a.v, a.attn, a.stats, B, S, S, nh, nkv, D, &opts));
+        else
+            FT_TRY(ft_internal_attention_forward_only(ctx, a.q, a.k, a.v, a.attn, B, S, S, nh, nkv, D, &opts));
         // h = x + o_proj(attn): the residual is added in the GEMM epilogue, or, when the product's K is shared
         // out over workgroups, by the norm kernel that reads h next
         const bool can_sum = ft_internal_norm_can_sum(T, H);
