@@ -128,4 +128,10 @@ __device__ __forceinline__ T ft_pinned(T v) {
     return v;
 }
 
+// Do the `na` bytes at a and the `nb` bytes at b meet?
+static inline bool ft_overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return na > 0 && nb > 0 && x < y + nb && y < x + na;
+}
+
 static inline unsigned ft_div_up(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }

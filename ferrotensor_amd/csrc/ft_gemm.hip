@@ -2107,6 +2107,24 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     return launch_cfg<64, 64, 32, 32>(ctx, p, layout, half_b, fast);
 }
 
+// May the linears of a group share a launch? Not when one of them writes what another reads or writes (t_1 = y_0, or
+// residual_1 = y_0): one by one, in order, they give what a caller who chains them means.
+bool group_apart(const ft_lora_linear_desc* d, size_t count, size_t M, size_t K) {
+    for (size_t i = 0; i < count; i++) {
+        const size_t out = 4 * M * d[i].N;
+        for (size_t j = 0; j < count; j++) {
+            if (j == i) continue;
+            const ft_lora_linear_desc& o = d[j];
+            auto meets = [&](const void* p, size_t bytes) { return p && ft_overlap(d[i].y, out, p, bytes); };
+            if (meets(o.y, 4 * M * o.N) || meets(o.w, (o.w_dtype == FT_DTYPE_F16 ? 2 : 4) * K * o.N) ||
+                meets(o.residual, 4 * M * o.N) || meets(o.rope_table, 4 * 64 * o.rope_seq) ||
+                (o.r > 0 && (meets(o.t, 4 * M * o.r) || meets(o.b, 4 * o.r * o.N))))
+                return false;
+        }
+    }
+    return true;
+}
+
 template <bool XT, bool YT, bool OT>
 int skinny_launch(ft_context* ctx, const float* x, const float* y, float* out, size_t R, size_t Kr, size_t C,
                   long ldx, long ldy, long ldo, float scale) {
@@ -2124,6 +2142,11 @@ int skinny_launch(ft_context* ctx, const float* x, const float* y, float* out, s
 }  // namespace
 
 extern "C" {
+
+// The rule above for callers that have no device (its test).
+int ft_internal_group_apart(const ft_lora_linear_desc* linears, size_t count, size_t M, size_t K) {
+    return group_apart(linears, count, M, K) ? 1 : 0;
+}
 
 int ft_mfma_probe(ft_context* ctx, size_t rounds, size_t waves_per_simd, size_t chains, int random_operands,
                   double* seconds, double* flops) {
@@ -2233,7 +2256,9 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
         batch = batch && d.w_dtype == FT_DTYPE_F16 && d.N < (1u << 30) &&
                 async_eligible(0, x, d.w, d.y, d.residual, M, K, d.N, d.t, d.b, d.r);
     }
-    bool split = !ctx->f32_chain && x && M < (1u << 30) && K < (1u << 30) && (count > 1 || any_rope);
+    const bool apart = group_apart(linears, count, M, K);
+    batch = batch && apart;
+    bool split = !ctx->f32_chain && apart && x && M < (1u << 30) && K < (1u << 30) && (count > 1 || any_rope);
     for (size_t i = 0; i < count && split; i++) {
         const ft_lora_linear_desc& d = linears[i];
         split = d.w && d.y && d.N < (1u << 30) && d.r < (1u << 30) && d.w_dtype == linears[0].w_dtype &&
@@ -2311,10 +2336,14 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
     FT_CHECK_ARG(ctx && x && w_gate && w_up && gate && up && act, "ft_mlp_gate_up: NULL argument");
     FT_CHECK_ARG(w_dtype == FT_DTYPE_F32 || w_dtype == FT_DTYPE_F16, "ft_mlp_gate_up: dtype %d", w_dtype);
     if (M == 0 || N == 0) return FT_OK;
-    if (!ctx->f32_chain && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
+    // One by one (up, gate, then the activation) act may take the place of x, and gate that of w_up.
+    const size_t wide = w_dtype == FT_DTYPE_F16 ? 2 : 4;
+    const bool apart = !ft_overlap(act, 4 * M * N, x, 4 * M * K) && !ft_overlap(act, 4 * M * N, w_gate, wide * K * N) &&
+                       !ft_overlap(act, 4 * M * N, w_up, wide * K * N) && !ft_overlap(gate, 4 * M * N, w_up, wide * K * N);
+    if (!ctx->f32_chain && apart && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
         ft_split_gemm_ok(0, M, K, N, w_dtype == FT_DTYPE_F16))
         return ft_split_gate_up(ctx, x, w_gate, w_up, gate, up, act, M, K, N, w_dtype == FT_DTYPE_F16);
-    const bool fused = w_dtype == FT_DTYPE_F16 && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
+    const bool fused = w_dtype == FT_DTYPE_F16 && apart && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
                        async_eligible(0, x, w_up, up, nullptr, M, K, N, nullptr, nullptr, 0) &&
                        async_eligible(0, x, w_gate, gate, nullptr, M, K, N, nullptr, nullptr, 0) && aligned16p(act);
     if (fused) {

@@ -442,9 +442,18 @@ int ft_thin_colwise(ft_context* ctx, const ft_thin_problem* probs, int count) {
     }
     const dim3 fgrid(ft_div_up(fmax, 256), (unsigned)b.count);
     ft_prof_scope prof(ctx, "thin_colwise+finish", 0.0, bytes);
-    // M == 0 (no slice at all) is the finish kernel's: it writes zeros
+    // M == 0 (no slice at all) is the finish kernel's: it writes zeros. So are results in the place of an operand, which
+    // other workgroups still read.
     bool direct = true;
     for (int i = 0; i < b.count; i++) direct = direct && b.p[i].slices == 1;
+    for (int i = 0; i < count && direct; i++)
+        for (int j = 0; j < count && direct; j++) {
+            const ft_thin_problem &o = probs[i], &q = probs[j];
+            if (o.M <= 0 || o.R <= 0 || q.M <= 0 || q.R <= 0) continue;
+            const size_t out = 4 * ((size_t)((o.out_transposed ? o.C : o.R) - 1) * o.ldo + (o.out_transposed ? o.R : o.C));
+            direct = !ft_overlap(o.out, out, q.x, 4 * ((size_t)(q.M - 1) * q.ldx + q.R)) &&
+                     !ft_overlap(o.out, out, q.y, 4 * ((size_t)(q.M - 1) * q.ldy + q.C));
+        }
 #define FT_COL(NSET)                                                                                                    \
     do {                                                                                                                \
         if (direct)                                                                                                     \

@@ -147,7 +147,9 @@ int ft_matmul_bt_f16b(ft_context* ctx, const float* a, const uint16_t* b, float*
  * y_i[M,N_i] = x[M,K] @ w_i[K,N_i] (+ t_i[M,r_i] @ b_i[r_i,N_i]) (+ residual_i),
  * exactly as ft_lora_linear does. The tiles of all of them share one grid, so a
  * narrow projection no longer leaves most of the chip idle. Linears that cannot
- * take the batched path (f32 weights, unaligned operands) run one by one. */
+ * take the batched path (weights of two types, in a training step f32 weights or
+ * unaligned operands) run one by one, and so do linears that feed each other (an
+ * output that another one reads or writes): in order, as the separate calls. */
 typedef struct ft_lora_linear_desc {
     const void* w;
     int32_t w_dtype;       /* FT_DTYPE_F32 or FT_DTYPE_F16 */

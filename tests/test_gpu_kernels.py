@@ -293,6 +293,22 @@ def test_lora_factor_gradients_at_the_edge_of_one_slice(g, M, r):
     assert np.all(np.abs(da.to_numpy() - want) <= limit) and np.all(np.abs(db.to_numpy() - want.T) <= limit.T)
 
 
+@pytest.mark.parametrize("M", [64, 128, 300])
+def test_lora_factor_gradients_in_the_place_of_an_operand(g, M):
+    """dA over dt and dB over t (several column tiles read the operand that the result overwrites)."""
+    ctx, eng = g
+    x, t = rnd(M, M, M), rnd(8, M, 8)
+    tt, da = up(ctx, t), empty(ctx, M, 8)
+    eng.lora_grad_a(ctx, up(ctx, x), tt, da)
+    eng.lora_grad_a(ctx, up(ctx, x), tt, tt)
+    assert np.array_equal(tt.to_numpy().view(np.uint32), da.to_numpy().view(np.uint32))
+    db = empty(ctx, 8, M)
+    eng.lora_grad_b(ctx, up(ctx, t), up(ctx, x), db)
+    same = up(ctx, t)
+    eng.lora_grad_b(ctx, same, up(ctx, x), same)
+    assert np.array_equal(same.to_numpy().reshape(-1).view(np.uint32), db.to_numpy().reshape(-1).view(np.uint32))
+
+
 @pytest.mark.parametrize("M,K,Ns,r,f16", [(256, 960, (960, 320, 320), 8, True), (100, 64, (64, 32, 96), 4, True),
                                           (192, 128, (320, 256), 0, True), (64, 32, (48, 40), 8, False),
                                           (130, 96, (40, 72, 8), 16, True),

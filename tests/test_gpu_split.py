@@ -184,6 +184,39 @@ def test_gate_up(g, M, K, N, half):
     np.testing.assert_allclose(np.asarray(act.to_vec(), np.float64), want, rtol=2e-6, atol=1e-30)
 
 
+@pytest.mark.parametrize("half", [False, True])
+def test_group_whose_linears_feed_each_other(g, half):
+    """Down to the rank, up again with it as the factor, and a third that adds to the second's output: in order, as three calls."""
+    ctx, eng = g
+    M, K, N, r = 300, 96, 640, 8
+    x, a, w, b, v = rnd(1, M, K), rnd(2, K, r), rnd(3, K, N, scale=0.05), rnd(4, r, N), rnd(5, K, N, scale=0.05)
+    make = up16 if half else up
+    seen = (lambda m: m.astype(np.float16).astype(np.float32)) if half else (lambda m: m)
+    t, y, z = empty(ctx, M, r), empty(ctx, M, N), empty(ctx, M, N)
+    eng.lora_linear_group(ctx, up(ctx, x), [(make(ctx, a), None, None, t, None), (make(ctx, w), t, up(ctx, b), y, None),
+                                            (make(ctx, v), None, None, z, y)])
+    got = np.asarray(t.to_vec(), np.float32).reshape(M, r)
+    check("t", got, [(x, seen(a))], K)
+    check("y", y.to_vec(), [(x, seen(w)), (got, b)], K)
+    check("z", z.to_vec(), [(x, seen(v)), (np.asarray(y.to_vec(), np.float32).reshape(M, N), np.eye(N, dtype=np.float32))], K)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_gate_up_with_the_activation_in_the_place_of_its_input(g, half):
+    ctx, eng = g
+    M, K = 300, 192
+    x, wg, wu = rnd(1, M, K), rnd(2, K, K, scale=0.05), rnd(3, K, K, scale=0.05)
+    make = up16 if half else up
+    outs = []
+    for inplace in (False, True):
+        X, gate, u = up(ctx, x), empty(ctx, M, K), empty(ctx, M, K)
+        act = X if inplace else empty(ctx, M, K)
+        eng.mlp_gate_up(ctx, X, make(ctx, wg), make(ctx, wu), gate, u, act)
+        outs.append([np.asarray(o.to_vec(), np.float32) for o in (gate, u, act)])
+    for a, b in zip(*outs):
+        np.testing.assert_allclose(b, a, rtol=2e-6, atol=2e-6)   # one launch or three: sums in another order
+
+
 def attention64(q, k, v, causal, offset):
     """f64 attention of [B, Sq, H, D] over [B, Sk, Hkv, D]; log-sum-exp too."""
     B, Sq, H, D = q.shape
