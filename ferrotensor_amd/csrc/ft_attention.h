@@ -32,6 +32,7 @@ struct AttnArgs {
     float* part;
     int split_g;
     int forward_only;   // no backward will ask for this forward's statistics
+    int in_place;       // set by the launch of a kernel on bf16 parts: a result lies where an operand of its rows does
 };
 
 constexpr size_t kAttnScratchFloats = (size_t)8 << 20;  // 32 MiB of per-head partial dK/dV

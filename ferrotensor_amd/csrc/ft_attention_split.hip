@@ -8,7 +8,9 @@
 // are the second operand of their product without leaving their lane.
 //
 // A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends
-// the workgroup through the f32 kernel's code, which says what it is.
+// the workgroup through the f32 kernel's code, which says what it is. That reads the operands again: where a result takes
+// the place of one (o over q, dq over out, dk or dv over k or v: AttnArgs::in_place) the workgroup settles this before it
+// writes, otherwise after (the vote first costs every call 1 to 4 %: 4 x 512 tokens, 32 heads, forward 41.0 -> 42.6 us).
 //
 // Relative error against f64 (2-norm), f32 kernels -> these, 4 x 1024 tokens, 15 heads on 5, normal values: o 2.8e-7 -> 2.1e-7,
 // dq 4.4e-7 -> 3.6e-7, dk 5.6e-7 -> 3.4e-7, dv 5.1e-7 -> 3.0e-7; scores nine times as large (4 x 512, 32 heads): 9.3e-7 ->
@@ -290,6 +292,7 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
             for (int r = 0; r < 4; r++) mrg[(2 + 4 * e + r) * 64] = o[e][r];
     }
     __syncthreads();
+    float lse = kAttnLseEmpty;
     if (w.kh == 0) {
         const float m_o = mrg[0], l_o = mrg[64];
         const float m_new = fmaxf(m_run, m_o);
@@ -302,19 +305,24 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
             for (int r = 0; r < 4; r++) o[e][r] = o[e][r] * c0 + mrg[(2 + 4 * e + r) * 64] * c1;
         const float l_run = group_sum(l_lane);
         const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-        const float lse = l_run > 0.0f ? (m_run + log2_fast(l_run)) * kLn2 : kAttnLseEmpty;
+        if (l_run > 0.0f) lse = (m_run + log2_fast(l_run)) * kLn2;
         bad = bad || !(fabsf(lse) <= 3.0e38f) || !(l_run >= 0.0f);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            o[e] *= inv;
+            bad = bad || not_finite(o[e]);
+        }
+    }
+    bool again = p.in_place && __syncthreads_or(bad && w.q_ok);
+    if (w.kh == 0 && w.q_ok && !again) {
         // register r of accumulator e is head-dim index 16 e + 4 g + r
         float* orow = p.o + (((long)w.b * p.Sq + w.q) * p.H + w.h) * D64;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const floatx4 v = o[e] * inv;
-            bad = bad || not_finite(v);
-            if (w.q_ok) *reinterpret_cast<floatx4*>(orow + 16 * e + 4 * g) = v;
-        }
-        if (w.q_ok && p.stats && g == 0) p.stats[2 * (((long)w.b * p.H + w.h) * p.Sq + w.q) + 1] = lse;
+        for (int e = 0; e < 4; e++) *reinterpret_cast<floatx4*>(orow + 16 * e + 4 * g) = o[e];
+        if (p.stats && g == 0) p.stats[2 * (((long)w.b * p.H + w.h) * p.Sq + w.q) + 1] = lse;
     }
-    if (__syncthreads_or(bad && w.q_ok)) attn16_fwd<NG>(p, reinterpret_cast<float*>(smem));
+    if (!p.in_place) again = __syncthreads_or(bad && w.q_ok);
+    if (again) attn16_fwd<NG>(p, reinterpret_cast<float*>(smem));
 }
 
 // dQ = scale * sum_j dS_ij K_j and Delta = dO.O (stats slot 0), dS = P (dO.V - Delta), P = exp(S - LSE). A workgroup
@@ -453,8 +461,8 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
                 for (int r = 0; r < 4; r++) mrg[(16 * c + 4 * e + r) * 64] = acc[c][e][r];
     }
     __syncthreads();
-    if (w.kh == 0) {
-        // dQ = scale * dS K
+    // dQ = scale * dS K
+    auto results = [&](auto write) {
 #pragma unroll
         for (int c = 0; c < QB; c++) {
             const int q = w.q + 16 * c;
@@ -466,12 +474,19 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
                 for (int r = 0; r < 4; r++) v[r] = (acc[c][e][r] + mrg[(16 * c + 4 * e + r) * 64]) * p.scale;
                 if (q < p.Sq) {
                     bad = bad || not_finite(v);
-                    *reinterpret_cast<floatx4*>(drow + 16 * e + 4 * g) = v;
+                    if constexpr (decltype(write)::value) *reinterpret_cast<floatx4*>(drow + 16 * e + 4 * g) = v;
                 }
             }
         }
+    };
+    bool again = false;
+    if (p.in_place) {
+        if (w.kh == 0) results(std::false_type{});
+        again = __syncthreads_or(bad);
     }
-    if (__syncthreads_or(bad)) {
+    if (w.kh == 0 && !again) results(std::true_type{});
+    if (!p.in_place) again = __syncthreads_or(bad);
+    if (again) {
 #pragma unroll 1
         for (int c = 0; c < QB; c++) {
             if ((qtile * QB + c) * 64 < p.Sq)
@@ -614,10 +629,10 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
             }
     }
     __syncthreads();
+    // register r of accumulator e is head-dim index 16 e + 4 g + r; dK = scale * sum dS Q (here, or where the heads
+    // of the group are added)
     bool bad = false;
-    if (qh == 0) {
-        // register r of accumulator e is head-dim index 16 e + 4 g + r; dK = scale * sum dS Q (here, or where the heads
-        // of the group are added)
+    auto results = [&](auto write) {
         const long n_all = (long)p.B * p.Sk * p.Hkv * D64;
         float* const dk_out = p.split_g ? p.part + 2 * g0 * n_all : p.dk;
         float* const dv_out = p.split_g ? p.part + (2 * g0 + 1) * n_all : p.dv;
@@ -632,12 +647,21 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
             }
             if (key < p.Sk) {
                 bad = bad || not_finite(x) || not_finite(y);
-                *reinterpret_cast<floatx4*>(dk_out + krow + 16 * e + 4 * g) = x;
-                *reinterpret_cast<floatx4*>(dv_out + krow + 16 * e + 4 * g) = y;
+                if constexpr (decltype(write)::value) {
+                    *reinterpret_cast<floatx4*>(dk_out + krow + 16 * e + 4 * g) = x;
+                    *reinterpret_cast<floatx4*>(dv_out + krow + 16 * e + 4 * g) = y;
+                }
             }
         }
+    };
+    bool again = false;
+    if (p.in_place) {
+        if (qh == 0) results(std::false_type{});
+        again = __syncthreads_or(bad);
     }
-    if (__syncthreads_or(bad)) {
+    if (qh == 0 && !again) results(std::true_type{});
+    if (!p.in_place) again = __syncthreads_or(bad);
+    if (again) {
 #pragma unroll 1
         for (int c = 0; c < 4; c++) {
             if (kt * KT + 16 * c < p.Sk) attn16_dkdv<64>(p, reinterpret_cast<float*>(smem), (4 * kt + c) * nhu + bh);
@@ -648,21 +672,30 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
 
 }  // namespace
 
-int ft_attn_split_forward(ft_context* ctx, const AttnArgs& a, int groups) {
+int ft_attn_split_forward(ft_context* ctx, const AttnArgs& args, int groups) {
+    AttnArgs a = args;
+    const size_t rows = (size_t)a.B * a.Sq * a.H * D64 * sizeof(float);
+    a.in_place = ft_overlap(a.o, rows, a.q, rows);
     if (groups == 2) hipLaunchKernelGGL(attn_split_fwd_kernel<2>, query_grid<2>(a), dim3(512), 0, ctx->stream, a);
     else hipLaunchKernelGGL(attn_split_fwd_kernel<4>, query_grid<4>(a), dim3(1024), 0, ctx->stream, a);
     FT_LAUNCH_CHECK();
     return FT_OK;
 }
 
-int ft_attn_split_dq(ft_context* ctx, const AttnArgs& a) {
+int ft_attn_split_dq(ft_context* ctx, const AttnArgs& args) {
+    AttnArgs a = args;
+    const size_t rows = (size_t)a.B * a.Sq * a.H * D64 * sizeof(float);
+    a.in_place = ft_overlap(a.dq, rows, a.out, rows);
     hipLaunchKernelGGL(attn_split_dq_kernel, dim3((unsigned)(ft_div_up(a.Sq, 128) * (size_t)a.B * a.H)), dim3(512), 0, ctx->stream, a);
     FT_LAUNCH_CHECK();
     return FT_OK;
 }
 
-int ft_attn_split_dkdv(ft_context* ctx, const AttnArgs& a) {
-    const size_t heads = (size_t)a.B * (a.split_g ? a.H : a.Hkv);
+int ft_attn_split_dkdv(ft_context* ctx, const AttnArgs& args) {
+    AttnArgs a = args;
+    const size_t heads = (size_t)a.B * (a.split_g ? a.H : a.Hkv), rows = (size_t)a.B * a.Sk * a.Hkv * D64 * sizeof(float);
+    a.in_place = !a.split_g && (ft_overlap(a.dk, rows, a.k, rows) || ft_overlap(a.dk, rows, a.v, rows) ||
+                                ft_overlap(a.dv, rows, a.k, rows) || ft_overlap(a.dv, rows, a.v, rows));
     hipLaunchKernelGGL(attn_split_dkdv_kernel, dim3((unsigned)(ft_div_up(a.Sk, 64) * heads)), dim3(512), 0, ctx->stream, a);
     FT_LAUNCH_CHECK();
     return FT_OK;

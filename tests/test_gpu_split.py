@@ -355,3 +355,27 @@ def test_model_forward_attention_at_small_sizes(B, S, heads, kv):
     want = np.asarray(want).reshape(-1)
     assert np.all(np.abs(got.reshape(-1) - want) <= 1e-4 * np.sqrt(np.mean(want ** 2)) + 1e-3 * np.abs(want))
     ctx.close()
+
+
+def test_attention_results_in_the_place_of_an_operand(g):
+    """o over q, dq over out, dk over k and dv over v, with values that send some workgroups back to the f32 code (which reads
+    the operands again): the same bits as with buffers of their own."""
+    from ferrotensor_amd import AttentionOptions
+    ctx, eng = g
+    B, S, H = 3, 512, 32
+    q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
+    v[0, 50, 3, 7], k[1, 100, 5, 9], do[2, 70, 1, 4] = np.inf, np.nan, 3.4e38
+    opts = AttentionOptions(causal=True)
+    results = []
+    for inplace in (False, True):
+        Q, K, V, DO = (up(ctx, x) for x in (q, k, v, do))
+        stats, o = empty(ctx, B * H * S, 2), Q if inplace else empty(ctx, *q.shape)
+        eng.flash_attention_v2_with_stats(ctx, Q, K, V, o, stats, opts)
+        out = o.to_vec()
+        if inplace:   # the backward needs q
+            Q, o = up(ctx, q), up(ctx, np.asarray(out, np.float32).reshape(q.shape))
+        dq, dk, dv = (o, K, V) if inplace else (empty(ctx, *q.shape), empty(ctx, *k.shape), empty(ctx, *v.shape))
+        eng.flash_attention_v2_backward_with_stats(ctx, Q, K, V, o, DO, dq, dk, dv, stats, opts)
+        results.append([np.asarray(x, np.float32) for x in (out, dq.to_vec(), dk.to_vec(), dv.to_vec())])
+    for name, a, b in zip(("o", "dq", "dk", "dv"), *results):
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)]), name
