@@ -1,14 +1,17 @@
-// f32 matrix products on the bf16 matrix instructions, without giving up f32 operands: every f32 value is the exact
-// sum of three bf16 numbers (8 + 8 + 8 significant bits, f32's own exponent range, so no scaling and no special rows),
+// f32 matrix products on the bf16 matrix instructions, without giving up f32 operands: an f32 value from 2^-110 up is the
+// exact sum of three bf16 numbers (8 + 8 + 8 significant bits, f32's own exponents, so no scaling and no special rows),
 // every f16 weight of two, and a product of two values is the sum of the products of their parts. With an f32 b six of
-// the nine are kept, with an f16 b five of the six: what is left out is below 2^-25 of the product it belongs to, under
-// f32's own rounding of that product. Sums are f32, in the matrix unit. v_mfma_f32_32x32x16_bf16 does eight times the
-// products of v_mfma_f32_32x32x2_f32 in half its cycles: 2.7 (3.2) times the f32 rate after six (five) of them.
+// the nine are kept, with an f16 b five of the six: what is left out is at most 2^-24 (2^-25) of the product it belongs to,
+// as much as f32 may round a sum of that size by. Sums are f32, in the matrix unit, subnormals included.
+// v_mfma_f32_32x32x16_bf16 does eight times the products of v_mfma_f32_32x32x2_f32 in half its cycles: 2.7 (3.2) times the
+// f32 rate after six (five) of them.
 //
-// What the split cannot hold (infinities, and finite values within 2^-8 of the largest f32, whose first part would round
-// to infinity) leaves a sum that is not finite; a wave that ends with one makes its share again with f32 products, so
-// infinities and NaN come out as f32 products give them. The rank-r term and what K leaves after its last whole step of
-// 16 take the f32 instruction too.
+// What the split cannot hold makes a wave do its share again with f32 products: infinities and finite values within 2^-8 of
+// the largest f32, whose first part would round to infinity, leave a sum that is not finite; a value below 2^-110 (bf16
+// ends at 2^-133) leaves something over after its third part, which one v_or3_b32 for two values collects. So infinities
+// and NaN come out as f32 products give them, and tiny values count in full. With every wave's share made twice a product
+// takes 1.7 to 2.8 times as long (8192 x 2048 x 2048, f16 b: 830 us for 328); looking for it costs 1 to 3 % (f16 b: 1 %).
+// The rank-r term and what K leaves after its last whole step of 16 take the f32 instruction too.
 //
 // Bound: VALU and matrix unit together. 8192 x 2048 x 2048 with f16 b: 340 us (202 TFLOP/s; f32 products 518), of them
 // 286 with no operand fetched at all; 2048 x 2560 x 2048 with f32 b: 127 us (160 with f32 products). Relative error
@@ -292,20 +295,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
 #pragma unroll
         for (int t = 0; t < NB; t++) ob[t].stash(slab_b + t * OpB::BYTES, lane);
     };
-    auto fetch = [&](int s) {
-        s = s < steps ? s : steps - 1;   // past the end: a step that nobody multiplies
-        oa.fetch(g.a + s * a_step);
-#pragma unroll
-        for (int t = 0; t < NB; t++) ob[t].fetch(bases[t] + s * b_step);
-    };
-    // The slab of this wave's next step, out of LDS and into parts (`next`), beside the products of the current one
-    // (`p`). A wave issues a VALU instruction every 8 cycles at best, an MFMA keeps the matrix unit for 32: they are
-    // dealt out in turn, a pair of values a slot, its three stages in three slots (a dot product's result may not be
-    // read by the next few instructions).
-    auto split = [&](Parts& next, const Parts& p, int after, auto beside) __attribute__((always_inline)) {
-        constexpr bool BESIDE = decltype(beside)::value;   // false: nothing to multiply yet
-        typename OpA::Value xa[FM][8];
-        typename OpB::Value xb[FN][8];
+    auto frags = [&](typename OpA::Value (&xa)[FM][8], typename OpB::Value (&xb)[FN][8]) {
         OpA::frags(slab_a, l32, half, xa);
         if constexpr (DUAL) {
 #pragma unroll
@@ -314,6 +304,24 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
         } else {
             OpB::frags(slab_b, l32, half, xb);
         }
+    };
+    auto fetch = [&](int s) {
+        s = s < steps ? s : steps - 1;   // past the end: a step that nobody multiplies
+        oa.fetch(g.a + s * a_step);
+#pragma unroll
+        for (int t = 0; t < NB; t++) ob[t].fetch(bases[t] + s * b_step);
+    };
+    // What third parts leave over, as bits: a third part holds its value when the low half of that value is zero.
+    unsigned left = 0;
+    // The slab of this wave's next step, out of LDS and into parts (`next`), beside the products of the current one
+    // (`p`). A wave issues a VALU instruction every 8 cycles at best, an MFMA keeps the matrix unit for 32: they are
+    // dealt out in turn, a pair of values a slot, its three stages in three slots, so that no stage waits for the one
+    // before it.
+    auto split = [&](Parts& next, const Parts& p, int after, auto beside) __attribute__((always_inline)) {
+        constexpr bool BESIDE = decltype(beside)::value;   // false: nothing to multiply yet
+        typename OpA::Value xa[FM][8];
+        typename OpB::Value xb[FN][8];
+        frags(xa, xb);
         float u[PAIRS], v[PAIRS];
         constexpr int SLOTS = PAIRS + 2;
         constexpr int AHEAD = FM * FN;   // MFMAs over the latency of the LDS reads
@@ -335,6 +343,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
                 const bool of_a = t < 4 * FM;
                 const int blk = (of_a ? t : t - 4 * FM) / 4, e = t % 4;
                 if (!of_a && ph >= PB) continue;
+                if (ph == 2) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(left) : "v"(u[t]), "v"(v[t]));   // (in C it waits for the end of the step, with all its registers)
                 if (ph == 0) {
                     u[t] = of_a ? xa[of_a ? blk : 0][2 * e] : (float)xb[of_a ? 0 : blk][2 * e];
                     v[t] = of_a ? xa[of_a ? blk : 0][2 * e + 1] : (float)xb[of_a ? 0 : blk][2 * e + 1];
@@ -392,8 +401,8 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
             for (int k = steps * 16; k < g.K; k += 16) f32_rest(af, A_KM, g.lda, b0, b1, B_KM, p.ldb, k, g.K);
     };
     rest();
-    // A sum that is not finite: an operand was not, or one of its parts, or the sum itself overflowed. This wave's share
-    // is made again with f32 products, which say which.
+    // A sum that is not finite (an operand was not, or one of its parts, or the sum itself overflowed), or a value that its
+    // parts do not hold: this wave's share is made again with f32 products.
     float zero = 0.0f;
 #pragma unroll
     for (int i = 0; i < FM; i++)
@@ -401,14 +410,29 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
         for (int j = 0; j < FN; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) zero = fmaf(acc[i][j][r], 0.0f, zero);
-    if (__builtin_expect(__any(zero != 0.0f), 0)) {
+    if (__builtin_expect(__any(zero != 0.0f || (left & 0xffffu) != 0), 0)) {
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int j = 0; j < FN; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-        for (int s = wave; s < steps; s += KW) f32_rest(af, A_KM, g.lda, b0, b1, B_KM, p.ldb, 16 * s, 16 * s + 16);
+        if (wave < steps) fetch(wave);
+#pragma unroll 1
+        for (int s = wave; s < steps; s += KW) {
+            stash();
+            fetch(s + KW);
+            typename OpA::Value xa[FM][8];
+            typename OpB::Value xb[FN][8];
+            frags(xa, xb);
+#pragma unroll
+            for (int e = 0; e < 8; e++)   // k = e of the first half of a wave, 8 + e of the second
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[i][e], (float)xb[j][e], acc[i][j], 0, 0, 0);
+        }
         rest();
     }
 

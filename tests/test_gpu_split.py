@@ -2,7 +2,8 @@
 
 Tolerance: the operands are held whole, so an element is off by the roundings of its sum alone: at most n matrix
 instructions follow each other on one accumulator (six per K step of 16, the K steps shared by at least two waves),
-then the waves' sums are added; each may be off by 2^-23 of the sum of the absolute products so far.
+then the waves' sums are added; each may be off by 2^-23 of the sum of the absolute products so far, or, among subnormal
+numbers, by their distance 2^-149.
 """
 import numpy as np
 import pytest
@@ -42,7 +43,7 @@ def check(name, got, terms, K):
     """terms: (a, b) pairs whose products add up."""
     want = sum(a.astype(np.float64) @ b.astype(np.float64) for a, b in terms)
     size = sum(np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64) for a, b in terms)
-    limit = (6 * (K // 16 // 2 + 1) + 32) * 2.0 ** -23 * size
+    limit = (6 * (K // 16 // 2 + 1) + 32) * (2.0 ** -23 * size + 2.0 ** -149)
     got = np.asarray(got, np.float64).reshape(want.shape)
     assert np.all(np.isfinite(got)), name
     worst = np.max(np.abs(got - want) / np.maximum(limit, 1e-300))
@@ -85,7 +86,8 @@ def test_adapted_linear_both_ways(g, M, K, N, r):
 
 @pytest.mark.parametrize("half", [False, True])
 def test_wide_range_of_values_in_one_row(g, half):
-    """Every f32 exponent that f32 products hold: no scale per row, so an outlier costs its neighbours nothing."""
+    """Exponents from -60 to 40, and 100 on columns that meet zeros: no scale per row, so an outlier costs its neighbours
+    nothing."""
     ctx, eng = g
     M, K, N = 96, 192, 96
     rng = np.random.default_rng(3)
@@ -100,6 +102,56 @@ def test_wide_range_of_values_in_one_row(g, half):
     else:
         eng.matmul(ctx, up(ctx, a), up(ctx, w), out)
     check("wide", out.to_vec(), [(a, wv)], K)
+
+
+# Tiles of every shape; K with whole steps only, and with a rest.
+@pytest.mark.parametrize("M,K,N", [(40, 64, 48), (96, 200, 960), (300, 192, 1100), (1025, 100, 1104)])
+@pytest.mark.parametrize("kind", ["all", "few", "products"])
+def test_values_below_what_three_bf16_parts_hold(g, M, K, N, kind):
+    """Values down to the last subnormal against large ones: all of an operand, single ones that alone decide a result (the
+    others meet zeros), and ordinary values whose products are subnormal."""
+    ctx, eng = g
+    rng = np.random.default_rng(K)
+    a, b = rnd(1, M, K), rnd(2, K, N)
+    if kind == "all":
+        a, b = np.ldexp(a, rng.integers(-149, -108, a.shape)), np.ldexp(b, 100)
+    elif kind == "few":
+        b[K // 2] = 0.0
+        a[1:, K // 2] = np.ldexp(a[1:, K // 2], 60)
+        a[M // 2, :] = 0.0
+        a[M // 2, K // 2 - 1] = np.ldexp(np.float32(1.2345678), -121)   # this row's only value
+        b[K // 2 - 1] = np.ldexp(b[K // 2 - 1], 90)
+        a[M // 2 + 1 :, K // 2 - 1] = 0.0
+    else:
+        a, b = np.ldexp(a, -70), np.ldexp(b, -68)
+    a, b = a.astype(np.float32), b.astype(np.float32)
+    out, w = empty(ctx, M, N), up(ctx, b)
+    for name, run in (("a@b", lambda: eng.matmul(ctx, up(ctx, a), w, out)), ("a@bT", lambda: eng.matmul_bt(ctx, up(ctx, a), up(ctx, b.T), out)),
+                      ("aT@b", lambda: eng.matmul_at(ctx, up(ctx, a.T), w, out))):
+        run()
+        check("%s %s" % (kind, name), out.to_vec(), [(a, b)], K)
+    out = empty(ctx, N, M)   # as the second operand
+    eng.matmul(ctx, up(ctx, b.T), up(ctx, a.T), out)
+    check("%s second" % kind, out.to_vec(), [(b.T, a.T)], K)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_values_below_what_three_bf16_parts_hold_in_the_fused_launches(g, half):
+    ctx, eng = g
+    M, K, N = 100, 144, 128
+    x = np.ldexp(rnd(1, M, K), np.random.default_rng(1).integers(-149, -108, (M, K))).astype(np.float32)
+    w1, w2 = rnd(2, K, N), rnd(3, K, N)
+    make = up16 if half else up
+    w1, w2 = (w.astype(np.float16).astype(np.float32) if half else w for w in (w1, w2))
+    y1, y2 = empty(ctx, M, N), empty(ctx, M, N)
+    scale = np.float32(1.0) if half else np.ldexp(np.float32(1.0), 100)
+    eng.lora_linear_group(ctx, up(ctx, x), [(make(ctx, w1 * scale), None, None, y1, None), (make(ctx, w2 * scale), None, None, y2, None)])
+    check("group 1", y1.to_vec(), [(x, w1 * scale)], K)
+    check("group 2", y2.to_vec(), [(x, w2 * scale)], K)
+    gate, u, act = (empty(ctx, M, N) for _ in range(3))
+    eng.mlp_gate_up(ctx, up(ctx, x), make(ctx, w1 * scale), make(ctx, w2 * scale), gate, u, act)
+    check("gate", gate.to_vec(), [(x, w1 * scale)], K)
+    check("up", u.to_vec(), [(x, w2 * scale)], K)
 
 
 @pytest.mark.parametrize("M,N", [(70, 96), (520, 1100)])
