@@ -1,16 +1,19 @@
 // Attention outside a training step, head dim 64: the work of the 16-row kernels (ft_attention16.hip) on
-// v_mfma_f32_16x16x32_bf16. Every operand, probabilities and dS too, is the exact sum of three bf16 parts and a product is
-// six products of parts, as in ft_split.hip: f32 operands and f32 sums at 2.7 times the rate of the f32 instruction.
+// v_mfma_f32_16x16x32_bf16. Every operand, probabilities and dS too, is the sum of three bf16 parts and a product is six
+// products of parts, as in ft_split.hip: f32 operands and f32 sums at 2.7 times the rate of the f32 instruction.
 //
 // K and V are split once per workgroup, on their way into LDS, as three planes each: rows of a key for the products over
 // the head dim, rows of a head-dim index (32 keys of a wave's half, in the order in which the probabilities leave the
 // score product's registers: 16 u + 4 g + i at 8 g + 4 u + i) for the products over the keys. The probabilities then
 // are the second operand of their product without leaving their lane.
 //
-// A score that is NaN or a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16) sends
-// the workgroup through the f32 kernel's code, which says what it is. That reads the operands again: where a result takes
-// the place of one (o over q, dq over out, dk or dv over k or v: AttnArgs::in_place) the workgroup settles this before it
-// writes, otherwise after (the vote first costs every call 1 to 4 %: 4 x 512 tokens, 32 heads, forward 41.0 -> 42.6 us).
+// A score that is NaN, a result that is not finite (infinite or NaN inputs, values that round to an infinite bf16), an operand
+// that three parts do not hold (below 2^-110) or a row of dQ or dK so small that its dS may be among those sends the workgroup
+// through the f32 kernel's code, which says what it is. (Probabilities need no such look: their parts hold them to 2^-134,
+// and exp2 makes zero of what is below 2^-126.) Looking for small ones costs the backward 3 to 5 %. The f32 code reads the
+// operands again: where a result takes the place of one (o over q, dq over out, dk or dv over k or v: AttnArgs::in_place)
+// the workgroup settles this before it writes, otherwise after (the vote first costs every call 1 to 4 %: 4 x 512 tokens,
+// 32 heads, forward 41.0 -> 42.6 us).
 //
 // Relative error against f64 (2-norm), f32 kernels -> these, 4 x 1024 tokens, 15 heads on 5, normal values: o 2.8e-7 -> 2.1e-7,
 // dq 4.4e-7 -> 3.6e-7, dk 5.6e-7 -> 3.4e-7, dv 5.1e-7 -> 3.0e-7; scores nine times as large (4 x 512, 32 heads): 9.3e-7 ->
@@ -36,10 +39,12 @@ constexpr int PLANE = KT * D64 * 2;   // bytes of one part of a 64-key tile
 __device__ __forceinline__ unsigned pack2(float x, float y) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x, y}, bf16x2));
 }
-// Two values into the packed halves of their three parts.
-__device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3]) {
+// Two values into the packed halves of their three parts. `left` collects what the third parts leave over, as bits: a
+// third part holds its value when the low half of that value is zero (from 2^-110 up, always).
+__device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3], unsigned* left = nullptr) {
 #pragma unroll
     for (int t = 0; t < 3; t++) {
+        if (t == 2 && left) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(*left) : "v"(x), "v"(y));
         const unsigned q = pack2(x, y);
         part[t] = q;
         if (t < 2) {
@@ -49,11 +54,11 @@ __device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3]) {
     }
 }
 // Eight values of a lane into the operand registers of their parts.
-__device__ __forceinline__ void split8(const float (&x)[8], uintx4 (&part)[3]) {
+__device__ __forceinline__ void split8(const float (&x)[8], uintx4 (&part)[3], unsigned* left = nullptr) {
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         unsigned q[3];
-        split2(x[2 * e], x[2 * e + 1], q);
+        split2(x[2 * e], x[2 * e + 1], q, left);
 #pragma unroll
         for (int t = 0; t < 3; t++) part[t][e] = q[t];
     }
@@ -92,6 +97,13 @@ template <int NT>
 struct TileRows {       // planes [key][64]
     static constexpr int N = KT * 16 / NT;
     float4 pre[N];
+    __device__ __forceinline__ float largest() const {   // of the tile's values of this thread
+        float m = 0.0f;
+#pragma unroll
+        for (int u = 0; u < N; u++)
+            m = fmaxf(fmaxf(fmaxf(fabsf(pre[u].x), fabsf(pre[u].y)), fmaxf(fabsf(pre[u].z), fabsf(pre[u].w))), m);
+        return m;
+    }
     __device__ __forceinline__ void fetch(const float* src, int stride, int rows, int t, int tid) {
 #pragma unroll
         for (int u = 0; u < N; u++) {
@@ -101,13 +113,13 @@ struct TileRows {       // planes [key][64]
             pre[u] = *reinterpret_cast<const float4*>(src + (long)row * stride + 4 * (e % 16));
         }
     }
-    __device__ __forceinline__ void store(char* planes, int tid) const {
+    __device__ __forceinline__ void store(char* planes, int tid, unsigned* left) const {
 #pragma unroll
         for (int u = 0; u < N; u++) {
             const int e = tid + NT * u, c = e % 16;
             unsigned lo[3], hi[3];
-            split2(pre[u].x, pre[u].y, lo);
-            split2(pre[u].z, pre[u].w, hi);
+            split2(pre[u].x, pre[u].y, lo, left);
+            split2(pre[u].z, pre[u].w, hi, left);
             char* at = planes + sw_key(e / 16, c >> 1) + (c & 1) * 8;
 #pragma unroll
             for (int q = 0; q < 3; q++) *reinterpret_cast<uintx2*>(at + q * PLANE) = uintx2{lo[q], hi[q]};
@@ -130,13 +142,13 @@ struct TileColumns {    // planes [key half][64][32 keys]
             }
         }
     }
-    __device__ __forceinline__ void store(char* planes, int tid) const {
+    __device__ __forceinline__ void store(char* planes, int tid, unsigned* left = nullptr) const {
 #pragma unroll
         for (int u = 0; u < N; u++) {
             const int e = tid + NT * u, d = e % 64, kg = e / 64;
             unsigned lo[3], hi[3];
-            split2(pre[u][0], pre[u][1], lo);
-            split2(pre[u][2], pre[u][3], hi);
+            split2(pre[u][0], pre[u][1], lo, left);
+            split2(pre[u][2], pre[u][3], hi, left);
             char* at = planes + (kg >> 3) * (PLANE / 2) + sw_dim(d, kg & 3) + ((kg >> 2) & 1) * 8;
 #pragma unroll
             for (int q = 0; q < 3; q++) *reinterpret_cast<uintx2*>(at + q * PLANE) = uintx2{lo[q], hi[q]};
@@ -150,14 +162,47 @@ __device__ __forceinline__ void read_parts(const char* at, uintx4 (&part)[3]) {
 }
 
 // A row's 64 values (this lane's 16 of them) as the two k steps' operand registers.
-__device__ __forceinline__ void row_parts(const float* row, int g, uintx4 (&part)[2][3]) {
+__device__ __forceinline__ void row_parts(const float* row, int g, uintx4 (&part)[2][3], unsigned* left) {
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
         const float4 a = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g);
         const float4 b = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g + 4);
         const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        split8(x, part[ks]);
+        split8(x, part[ks], left);
     }
+}
+
+// What the backward kernels look out for, in LDS (a slot of its own per thread, so nobody waits) where their loops have no
+// register to spare: what third parts leave over (split2), and the largest operand that dS is multiplied with.
+struct Watch {
+    unsigned left[512], most[512], all;
+    __device__ __forceinline__ void start(int tid) {   // a barrier follows before join()
+        left[tid] = most[tid] = 0;
+        if (tid == 0) all = 0;
+    }
+    __device__ __forceinline__ void add(int tid, unsigned l, float m) {   // (non-negative floats compare as whole numbers)
+        atomicOr(&left[tid], l);
+        atomicMax(&most[tid], __float_as_uint(m));
+    }
+    __device__ __forceinline__ void join(int tid) {    // a barrier follows before largest()
+        float m = __uint_as_float(most[tid]);
+#pragma unroll
+        for (int x = 1; x < 64; x *= 2) m = fmaxf(m, __shfl_xor(m, x));
+        if (tid % 64 == 0) atomicMax(&all, __float_as_uint(m));
+    }
+    __device__ __forceinline__ float largest() const { return __uint_as_float(all); }
+    __device__ __forceinline__ bool left_over(int tid) const { return (left[tid] & 0xffffu) != 0; }
+};
+// dS is a product and may be any small: its parts hold it to 2^-134 (half of bf16's smallest step). A row of a result that is
+// a sum over `terms` of them times operands of at most `largest`, and that small, may be off by more than a rounding.
+__device__ __forceinline__ bool too_small(const floatx4 (&row)[4], float terms, float largest, float scale) {
+    float m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) m = fmaxf(m, fabsf(row[e][r]));
+    m = group_max(m);
+    return m > 0.0f && m < terms * largest * (scale * 0x1p-110f);
 }
 
 __device__ __forceinline__ bool not_finite(floatx4 v) {
@@ -184,7 +229,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
     }
     const float sscale = p.scale * kLog2e;   // scores are kept in base 2
     uintx4 qp[2][3];
-    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, qp);
+    unsigned left = 0;
+    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, qp, &left);
     floatx4 o[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = zero4();
@@ -194,8 +240,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
     const int key_lim = (p.causal && w.q + p.causal_offset < p.Sk - 1) ? w.q + p.causal_offset : p.Sk - 1;
 
     if (w.nkt > 0) {
-        kl.store(smem, tid);
-        vl.store(smem + 3 * PLANE, tid);
+        kl.store(smem, tid, &left);
+        vl.store(smem + 3 * PLANE, tid, &left);
     }
     __syncthreads();
 
@@ -275,8 +321,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         }
         if (more) {
             char* next = smem + ((t + 1) & 1) * STAGE;
-            kl.store(next, tid);
-            vl.store(next + 3 * PLANE, tid);
+            kl.store(next, tid, &left);
+            vl.store(next + 3 * PLANE, tid, &left);
         }
         __syncthreads();
     }
@@ -313,7 +359,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
             bad = bad || not_finite(o[e]);
         }
     }
-    bool again = p.in_place && __syncthreads_or(bad && w.q_ok);
+    bad = (bad && w.q_ok) || (left & 0xffffu);
+    bool again = p.in_place && __syncthreads_or(bad);
     if (w.kh == 0 && w.q_ok && !again) {
         // register r of accumulator e is head-dim index 16 e + 4 g + r
         float* orow = p.o + (((long)w.b * p.Sq + w.q) * p.H + w.h) * D64;
@@ -321,7 +368,7 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         for (int e = 0; e < 4; e++) *reinterpret_cast<floatx4*>(orow + 16 * e + 4 * g) = o[e];
         if (p.stats && g == 0) p.stats[2 * (((long)w.b * p.H + w.h) * p.Sq + w.q) + 1] = lse;
     }
-    if (!p.in_place) again = __syncthreads_or(bad && w.q_ok);
+    if (!p.in_place) again = __syncthreads_or(bad);
     if (again) attn16_fwd<NG>(p, reinterpret_cast<float*>(smem));
 }
 
@@ -349,11 +396,16 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         vl.fetch(v_head, kv_stride, p.Sk, t, tid);
         kc.fetch(k_head, kv_stride, p.Sk, t, tid);
     };
+    __shared__ Watch watch;
+    watch.start(tid);
     auto store = [&](char* stage) {
-        kl.store(stage, tid);
-        vl.store(stage + 3 * PLANE, tid);
+        unsigned left = 0;
+        kl.store(stage, tid, &left);
+        vl.store(stage + 3 * PLANE, tid, &left);
         kc.store(stage + 6 * PLANE, tid);
+        watch.add(tid, left, kl.largest());
     };
+    unsigned left = 0;
     if (w.nkt > 0) fetch(0);
     const float sscale = p.scale * kLog2e;
     uintx4 qp[QB][2][3], dop[QB][2][3];
@@ -365,8 +417,8 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         const int q = w.q + 16 * c, qc = q < p.Sq ? q : p.Sq - 1;
         const long qoff = (((long)w.b * p.Sq + qc) * p.H + w.h) * D64;
         const long srow = ((long)w.b * p.H + w.h) * p.Sq + qc;
-        row_parts(p.q + qoff, g, qp[c]);
-        row_parts(p.d_out + qoff, g, dop[c]);
+        row_parts(p.q + qoff, g, qp[c], &left);
+        row_parts(p.d_out + qoff, g, dop[c], &left);
         delta[c] = 0.0f;
 #pragma unroll
         for (int blk = 0; blk < 4; blk++) {   // dO.O as the f32 kernel adds it
@@ -382,6 +434,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[c][e] = zero4();
     }
+    watch.add(tid, left, 0.0f);
     if (w.nkt > 0) store(smem);
     __syncthreads();
 
@@ -450,6 +503,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         __syncthreads();
     }
 
+    watch.join(tid);
     // the second key half's partial dQ joins the first's, lane for lane
     float* mrg = reinterpret_cast<float*>(smem) + (w.w2 * 16 * QB) * 64 + lane;
     if (w.kh == 1) {
@@ -467,18 +521,21 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         for (int c = 0; c < QB; c++) {
             const int q = w.q + 16 * c;
             float* drow = p.dq + (((long)w.b * p.Sq + q) * p.H + w.h) * D64;
+            floatx4 v[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                floatx4 v;
 #pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = (acc[c][e][r] + mrg[(16 * c + 4 * e + r) * 64]) * p.scale;
+                for (int r = 0; r < 4; r++) v[e][r] = (acc[c][e][r] + mrg[(16 * c + 4 * e + r) * 64]) * p.scale;
                 if (q < p.Sq) {
-                    bad = bad || not_finite(v);
-                    if constexpr (decltype(write)::value) *reinterpret_cast<floatx4*>(drow + 16 * e + 4 * g) = v;
+                    bad = bad || not_finite(v[e]);
+                    if constexpr (decltype(write)::value) *reinterpret_cast<floatx4*>(drow + 16 * e + 4 * g) = v[e];
                 }
             }
+            const bool small = too_small(v, (float)p.Sk, watch.largest(), p.scale);
+            bad = bad || (small && q < p.Sq);
         }
     };
+    bad = watch.left_over(tid);
     bool again = false;
     if (p.in_place) {
         if (w.kh == 0) results(std::false_type{});
@@ -523,8 +580,9 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
     const long krow = (((long)b * p.Sk + (key < p.Sk ? key : p.Sk - 1)) * p.Hkv + kvh) * D64;
     const float sscale = p.scale * kLog2e;
     uintx4 kp[2][3], vp[2][3];
-    row_parts(p.k + krow, g, kp);
-    row_parts(p.v + krow, g, vp);
+    unsigned left = 0;
+    row_parts(p.k + krow, g, kp, &left);
+    row_parts(p.v + krow, g, vp, &left);
 
     const int nqt = (p.Sq + KT - 1) / KT;
     int qt0 = 0;
@@ -550,9 +608,14 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
             stat = *reinterpret_cast<const float2*>(p.stats + 2 * (((long)b * p.H + h) * p.Sq + q));
         }
     };
+    __shared__ Watch watch;
+    watch.start(tid);
+    watch.add(tid, left, 0.0f);
     auto store = [&]() {
-        ql.store(smem, tid);
-        dl.store(smem + 3 * PLANE, tid);
+        unsigned left = 0;
+        ql.store(smem, tid, &left);
+        dl.store(smem + 3 * PLANE, tid, &left);
+        watch.add(tid, left, ql.largest());
         qc.store(smem + 6 * PLANE, tid);
         dc.store(smem + 9 * PLANE, tid);
         if (tid < KT) st[tid] = make_float2(stat.x, stat.y * kLog2e);
@@ -617,6 +680,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
         }
     }
 
+    watch.join(tid);
     // The two query halves of a key block meet through LDS, lane for lane.
     float* mrg = reinterpret_cast<float*>(smem) + (wave % 4) * 32 * 64 + lane;
     if (qh == 1) {
@@ -631,28 +695,31 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
     __syncthreads();
     // register r of accumulator e is head-dim index 16 e + 4 g + r; dK = scale * sum dS Q (here, or where the heads
     // of the group are added)
-    bool bad = false;
+    bool bad = watch.left_over(tid);
     auto results = [&](auto write) {
         const long n_all = (long)p.B * p.Sk * p.Hkv * D64;
         float* const dk_out = p.split_g ? p.part + 2 * g0 * n_all : p.dk;
         float* const dv_out = p.split_g ? p.part + (2 * g0 + 1) * n_all : p.dv;
         const float scale = p.split_g ? 1.0f : p.scale;
+        floatx4 x[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            floatx4 x, y;
+            floatx4 y;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                x[r] = (dk[e][r] + mrg[(4 * e + r) * 64]) * scale;
+                x[e][r] = (dk[e][r] + mrg[(4 * e + r) * 64]) * scale;
                 y[r] = dv[e][r] + mrg[(16 + 4 * e + r) * 64];
             }
             if (key < p.Sk) {
-                bad = bad || not_finite(x) || not_finite(y);
+                bad = bad || not_finite(x[e]) || not_finite(y);
                 if constexpr (decltype(write)::value) {
-                    *reinterpret_cast<floatx4*>(dk_out + krow + 16 * e + 4 * g) = x;
+                    *reinterpret_cast<floatx4*>(dk_out + krow + 16 * e + 4 * g) = x[e];
                     *reinterpret_cast<floatx4*>(dv_out + krow + 16 * e + 4 * g) = y;
                 }
             }
         }
+        const bool small = too_small(x, (float)p.Sq * (float)G, watch.largest(), scale);
+        bad = bad || (small && key < p.Sk);
     };
     bool again = false;
     if (p.in_place) {

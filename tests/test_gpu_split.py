@@ -431,3 +431,50 @@ def test_attention_results_in_the_place_of_an_operand(g):
         results.append([np.asarray(x, np.float32) for x in (out, dq.to_vec(), dk.to_vec(), dv.to_vec())])
     for name, a, b in zip(("o", "dq", "dk", "dv"), *results):
         assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)]), name
+
+
+# (which operand is scaled by which power of two, and what else)
+@pytest.mark.parametrize("case", ["v", "k", "q", "one v", "one do", "do", "ds", "none"])
+def test_attention_with_values_below_what_three_bf16_parts_hold(g, case):
+    """Operands below 2^-110 (all of one, against a large other one; a single value that decides a result), and dO and V whose
+    product is: relative to the largest of a head's results, as ordinary values. Also against the f32 kernels (the batch's
+    first sequence alone)."""
+    from ferrotensor_amd import AttentionOptions
+    ctx, eng = g
+    B, S, H = 3, 512, 32
+    q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
+    ld = lambda x, e: np.ldexp(x, e).astype(np.float32)
+    if case == "v":
+        v = ld(v, -124)
+    elif case == "k":
+        k, q = ld(k, -120), ld(q, 119)
+    elif case == "q":
+        q, k = ld(q, -124), ld(k, 123)
+    elif case == "one v":
+        v[0, :, 3, 7] = 0.0
+        v[0, 5, 3, 7] = np.ldexp(1.2345678, -121)
+    elif case == "one do":
+        do[0, :, 3] = 0.0
+        do[0, 300, 3, 7] = np.ldexp(1.2345678, -121)
+        v[0, :, 3] = ld(v[0, :, 3], 60)
+    elif case == "do":
+        do = ld(do, -112)
+    elif case == "ds":
+        do, v, k = ld(do, -60), ld(v, -60), ld(k, 60)
+        q = ld(q, -60)
+    opts = AttentionOptions(causal=True)
+    o, stats = empty(ctx, *q.shape), empty(ctx, B * H * S, 2)
+    eng.flash_attention_v2_with_stats(ctx, up(ctx, q), up(ctx, k), up(ctx, v), o, stats, opts)
+    got = [np.asarray(o.to_vec(), np.float32).reshape(q.shape), *run_attention(ctx, eng, q, k, v, do, True, 0)]
+    want = [attention64(q, k, v, True, 0)[0], *backward64(q, k, v, do, True, 0)]
+    alone = [x[:1] for x in (q, k, v, do)]
+    o1, s1 = empty(ctx, 1, S, H, 64), empty(ctx, H * S, 2)
+    eng.flash_attention_v2_with_stats(ctx, *(up(ctx, x) for x in alone[:3]), o1, s1, opts)
+    f32 = [np.asarray(o1.to_vec(), np.float32).reshape(1, S, H, 64), *run_attention(ctx, eng, *alone, True, 0)]
+    for name, a, b, c in zip(("o", "dq", "dk", "dv"), got, want, f32):
+        for h in (0, 3, 31):
+            scale = np.max(np.abs(b[0, :, h]))
+            err, err32 = (np.max(np.abs(x[0, :, h] - b[0, :, h])) for x in (a, c))
+            # as test_attention_backward, or among subnormal results their distance; where cancellation is all there is
+            # (dS of a head with hardly any dP), as far off as the f32 kernels
+            assert err <= max(2e-5 * scale, 64 * 2.0 ** -149, 2 * err32), (name, h, err, scale, err32)
