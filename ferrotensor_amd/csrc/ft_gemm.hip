@@ -1969,6 +1969,14 @@ bool f32_async_eligible(int layout, const float* a, const void* b, const float* 
     return a_span < lim && b_span < lim;
 }
 
+// Workgroups along K of a plain product on gemm_f32_async_kernel with `tiles` tiles of 64 x 64, for at most 2 per CU.
+int f32_async_shares(size_t cus, size_t tiles, size_t K) {
+    int want = (int)((2 * cus + tiles - 1) / tiles);
+    if (want > 8) want = 8;
+    if (want > (int)(K / 32) / 4) want = (int)(K / 32) / 4;
+    return want;
+}
+
 int launch_f32_async(ft_context* ctx, int layout, const float* a, const float* b, float* out, size_t M, size_t K,
                      size_t N, const float* a2 = nullptr, const float* b2 = nullptr, size_t K2 = 0,
                      const float* add = nullptr) {
@@ -2001,9 +2009,7 @@ int launch_f32_async(ft_context* ctx, int layout, const float* a, const float* b
     g.lda2 = (int)K2;
     g.ldb2 = layout == 1 ? (int)K2 : (int)N;
     if (!a2 && !add && tiles * 2 <= (size_t)ctx->num_cus && (M * N) % 4 == 0) {
-        int want = (int)((2 * (size_t)ctx->num_cus + tiles - 1) / tiles);
-        if (want > 8) want = 8;
-        if (want > g.nt / 4) want = g.nt / 4;
+        const int want = f32_async_shares((size_t)ctx->num_cus, tiles, K);
         if (want >= 2 && M * N * (size_t)want <= kSplitScratchFloats) {
             if (!ctx->gemm_scratch) {
                 FT_HIP(hipSetDevice(ctx->device));
@@ -2037,6 +2043,49 @@ int launch_f32_async(ft_context* ctx, int layout, const float* a, const float* b
     return FT_OK;
 }
 
+// Does a product outside a training step gain by bf16 parts (ft_split.hip) where the f32 instruction's vector kernels can
+// take it? Nearly everywhere. Not so, by measurements on 256 CUs (us, f32 instruction -> parts; T: tiles of 64 x 64):
+//  * below three K steps of 16: 4096 x 32 x 576 (M x K x N) 5.9 -> 7.1;
+//  * few steps on tiles that just fill the CUs once or twice (f16 b: twice; with four steps five and six times too): 2048 x
+//    64 x 576 6.3 -> 7.4, with f16 b 6.3 -> 6.9; once, up to ten steps: 1024 x 128 x 576 5.5 -> 5.9 (twice gains: 7.3 -> 6.8);
+//  * an f16 b with a rank-r term, which the other kernel's K loop takes along: 1024 x 64 x 5120 13 -> 15.5, 4096 x 128 x 576
+//    12 -> 13.2; with a residual, which the parts' kernels read last, up to ten steps, from three tiles a CU on twelve: 2048 x 64 x 5120
+//    25 -> 32, 2048 x 192 x 1536 16 -> 18;
+//  * an f32 b, long K and few tiles, which gemm_f32_async_kernel shares out over the CUs: 128 x 2560 x 960 12.9 -> 14.4, 256 x
+//    4096 x 512 15.5 -> 19.6, 64 x 16384 x 2048 42.8 -> 73.0; with more tiles where its shares fill the CUs evenly: 128 x
+//    16384 x 2048 78 -> 86.
+bool split_pays(size_t cus, bool half_b, bool ranked, bool residual, size_t M, size_t K, size_t N) {
+    const size_t T = ((M + 63) / 64) * ((N + 63) / 64), rounds = (T + cus - 1) / cus;
+    const bool one = rounds == 1 && T * 2 > cus;   // one tile a CU, on most of them
+    if (K < 48) return false;
+    if (half_b) {
+        if (residual && (K <= 160 ? T * 2 > cus : K <= 192 && rounds >= 3)) return false;
+        if (K <= 64 && (rounds == 5 || rounds == 6)) return false;
+        if (K <= 96 && rounds == 2) return false;
+        if (ranked && K <= 128 && (one || (rounds >= (K <= 96 ? 5 : 3) && rounds <= 6))) return false;
+        return true;
+    }
+    if (K <= 96 && (one || rounds == 2)) return false;
+    if (K <= 160 && one) return false;
+    if (K > 2048 && !ranked && !residual) {
+        if (T * (K < 2560 ? 16 : 8) <= cus) return false;
+        if (K >= 8192 && T * 2 <= cus && T * (size_t)f32_async_shares(cus, T, K) <= 2 * cus) return false;
+    }
+    return true;
+}
+
+// The same for the fused launches of ft_lora_linear_group (T: tiles of all its linears) and ft_mlp_gate_up, where the other
+// path can take them: with f16 weights in one launch too, with few K steps the faster one (group of 2048 + 512 + 512 columns,
+// 1024 x 64: 8.9 -> 13.1 us; x 128: 11.9 -> 14.1; x 160: 13.5 -> 14.1, not held against it; gate + up of 5120 columns, 512 x 32: 10.1 -> 13.1,
+// 512 x 64: 13.4 -> 14.5, 2048 x 96: 48.5 -> 52.5); with f32 weights gate and up apart, each with its K shared out (64 x
+// 8192 x 1024: 48 -> 57; 256 x 4096 x 512 gains).
+bool split_group_pays(size_t cus, size_t T, size_t K) { return !((K <= 64 && T > cus) || (K <= 128 && T > 2 * cus)); }
+bool split_gate_up_pays(size_t cus, bool half_b, size_t M, size_t K, size_t N) {
+    const size_t T = ((M + 63) / 64) * ((N + 63) / 64);
+    if (!half_b) return K < 6144 || T * 8 > cus;
+    return !((K < 48 && T * 2 > cus) || (K <= 64 && T > cus) || (K <= 96 && T > 2 * cus));
+}
+
 int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, const float* a, const void* b,
                   float* out, size_t M, size_t K, size_t N, const float* a2, const float* b2, size_t K2,
                   const float* add = nullptr) {
@@ -2046,8 +2095,6 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     FT_CHECK_ARG(out && (K == 0 || (a && b)), "%s: NULL operand", who);
     FT_CHECK_ARG((a2 == nullptr) == (b2 == nullptr), "%s: a2 and b2 must come together", who);
     FT_CHECK_ARG(!(layout == 2 && (half_b || a2)), "%s: unsupported operand combination", who);
-    if (!ctx->f32_chain && ft_split_gemm_ok(layout, M, K, N, half_b))
-        return ft_split_gemm(ctx, layout, half_b, a, b, out, M, K, N, K2 > 0 ? a2 : nullptr, K2 > 0 ? b2 : nullptr, K2, add);
     GemmArgs p{};
     p.a = a;
     p.b = b;
@@ -2064,33 +2111,6 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     p.ldc = (long)N;
     p.lda2 = (long)K2;
     p.ldb2 = layout == 1 ? (long)K2 : (long)N;
-    if (half_b && K > 0 && async_eligible(layout, a, b, out, add, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0)) {
-        AsyncBatch g{};
-        g.count = 1;
-        g.M = (int)M;
-        g.p[0].seg[0] = make_seg(layout, a, b, K, N, p.a2, p.b2, p.a2 ? K2 : 0);
-        g.p[0].nseg = 1;
-        g.p[0].out = out;
-        g.p[0].add = add;
-        g.p[0].N = (int)N;
-        g.p[0].ldc = (int)N;
-        return launch_async_auto(ctx, g, layout);
-    }
-    if (!half_b && !p.a2 && !add && f32_async_eligible(layout, a, b, out, M, K, N))
-        return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N);
-    // With a rank-r term or a residual: the same pipeline, the K chain in one piece. 135M-width step on f32 weights, 2912
-    // rows: 10.45 -> 9.73 ms (117 of these products a step, on the register-staged kernel 32 us each on average).
-    if (!half_b && layout != 2 && (p.a2 || add) && f32_async_eligible(layout, a, b, out, M, K, N) &&
-        (!p.a2 || (K2 <= 16 && K2 % 4 == 0 && aligned16p(a2) && aligned16p(b2) && (layout == 1 || N % 4 == 0))) &&
-        ((M + 127) / 128) * ((N + 127) / 128) < 8 * (size_t)ctx->num_cus)
-        return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0, add);
-    // Tile choice for the register-staged kernels, from measurements on MI355X at
-    // M = 2048: 128x128 tiles when there are many per CU, else 64x64; a deep K
-    // loop on few tiles prefers BK = 64 (half the barriers per MFMA).
-    const size_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-    const size_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
-    int best = tiles128 >= 8 * (size_t)ctx->num_cus ? 0 : 2;
-    if (best == 2 && K >= 4096 && tiles64 <= 2 * (size_t)ctx->num_cus) best = 3;
     // The branch-free kernel needs aligned operands and whole float4 groups.
     auto al16 = [](const void* q) { return (((uintptr_t)q) & 15) == 0; };
     bool fast = al16(a) && al16(b) && al16(out) && K % 4 == 0 && K >= 4 && (p.lda % 4 == 0) && (p.ldb % 4 == 0);
@@ -2102,6 +2122,38 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     const double lim = 4294967296.0;
     fast = fast && 4.0 * (double)M * (double)(layout == 2 ? 1 : K) + 4.0 * 64 * (double)p.lda < lim &&
            4.0 * (double)N * (double)(layout == 1 ? K : 1) + 4.0 * 64 * (double)p.ldb < lim;
+    const bool half_async = half_b && K > 0 && async_eligible(layout, a, b, out, add, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0);
+    const bool f32_async = !half_b && f32_async_eligible(layout, a, b, out, M, K, N);
+    if (!ctx->f32_chain && ft_split_gemm_ok(layout, M, K, N, half_b) &&
+        (!(half_async || f32_async || (fast && K <= 160)) || split_pays((size_t)ctx->num_cus, half_b, p.a2 != nullptr, add != nullptr, M, K, N)))
+        return ft_split_gemm(ctx, layout, half_b, a, b, out, M, K, N, p.a2, p.b2, K2, add);
+    if (half_async) {
+        AsyncBatch g{};
+        g.count = 1;
+        g.M = (int)M;
+        g.p[0].seg[0] = make_seg(layout, a, b, K, N, p.a2, p.b2, p.a2 ? K2 : 0);
+        g.p[0].nseg = 1;
+        g.p[0].out = out;
+        g.p[0].add = add;
+        g.p[0].N = (int)N;
+        g.p[0].ldc = (int)N;
+        return launch_async_auto(ctx, g, layout);
+    }
+    if (f32_async && !p.a2 && !add)
+        return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N);
+    // With a rank-r term or a residual: the same pipeline, the K chain in one piece. 135M-width step on f32 weights, 2912
+    // rows: 10.45 -> 9.73 ms (117 of these products a step, on the register-staged kernel 32 us each on average).
+    if (f32_async && layout != 2 && (p.a2 || add) &&
+        (!p.a2 || (K2 <= 16 && K2 % 4 == 0 && aligned16p(a2) && aligned16p(b2) && (layout == 1 || N % 4 == 0))) &&
+        ((M + 127) / 128) * ((N + 127) / 128) < 8 * (size_t)ctx->num_cus)
+        return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0, add);
+    // Tile choice for the register-staged kernels, from measurements on MI355X at
+    // M = 2048: 128x128 tiles when there are many per CU, else 64x64; a deep K
+    // loop on few tiles prefers BK = 64 (half the barriers per MFMA).
+    const size_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+    const size_t tiles64 = ((M + 63) / 64) * ((N + 63) / 64);
+    int best = tiles128 >= 8 * (size_t)ctx->num_cus ? 0 : 2;
+    if (best == 2 && K >= 4096 && tiles64 <= 2 * (size_t)ctx->num_cus) best = 3;
     if (best == 0) return launch_cfg<128, 128, 64, 64>(ctx, p, layout, half_b, fast);
     if (best == 3) return launch_cfg<64, 64, 32, 32, 64>(ctx, p, layout, half_b, fast);
     return launch_cfg<64, 64, 32, 32>(ctx, p, layout, half_b, fast);
@@ -2143,7 +2195,13 @@ int skinny_launch(ft_context* ctx, const float* x, const float* y, float* out, s
 
 extern "C" {
 
-// The rule above for callers that have no device (its test).
+// Rules above for callers that have no device (their tests).
+int ft_internal_split_pays(size_t cus, int half_b, int ranked, int residual, size_t M, size_t K, size_t N) {
+    return split_pays(cus, half_b != 0, ranked != 0, residual != 0, M, K, N) ? 1 : 0;
+}
+int ft_internal_split_fused_pays(size_t cus, int gate_up, int half_b, size_t M, size_t K, size_t N) {
+    return gate_up ? split_gate_up_pays(cus, half_b != 0, M, K, N) : split_group_pays(cus, ((M + 63) / 64) * ((N + 63) / 64), K);
+}
 int ft_internal_group_apart(const ft_lora_linear_desc* linears, size_t count, size_t M, size_t K) {
     return group_apart(linears, count, M, K) ? 1 : 0;
 }
@@ -2259,12 +2317,15 @@ int ft_lora_linear_group(ft_context* ctx, const float* x, const ft_lora_linear_d
     const bool apart = group_apart(linears, count, M, K);
     batch = batch && apart;
     bool split = !ctx->f32_chain && apart && x && M < (1u << 30) && K < (1u << 30) && (count > 1 || any_rope);
+    size_t tiles = 0;
     for (size_t i = 0; i < count && split; i++) {
         const ft_lora_linear_desc& d = linears[i];
+        tiles += ((M + 63) / 64) * ((d.N + 63) / 64);
         split = d.w && d.y && d.N < (1u << 30) && d.r < (1u << 30) && d.w_dtype == linears[0].w_dtype &&
                 ft_split_gemm_ok(0, M, K, d.N, d.w_dtype == FT_DTYPE_F16);
     }
-    if (split) return ft_split_group(ctx, x, linears, count, M, K, linears[0].w_dtype == FT_DTYPE_F16);
+    if (split && (!batch || count == 1 || split_group_pays((size_t)ctx->num_cus, tiles, K)))
+        return ft_split_group(ctx, x, linears, count, M, K, linears[0].w_dtype == FT_DTYPE_F16);
     if (batch && count > 1) {
         AsyncBatch g{};
         g.count = (int)count;
@@ -2340,12 +2401,14 @@ int ft_mlp_gate_up(ft_context* ctx, const float* x, const void* w_gate, const vo
     const size_t wide = w_dtype == FT_DTYPE_F16 ? 2 : 4;
     const bool apart = !ft_overlap(act, 4 * M * N, x, 4 * M * K) && !ft_overlap(act, 4 * M * N, w_gate, wide * K * N) &&
                        !ft_overlap(act, 4 * M * N, w_up, wide * K * N) && !ft_overlap(gate, 4 * M * N, w_up, wide * K * N);
-    if (!ctx->f32_chain && apart && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
-        ft_split_gemm_ok(0, M, K, N, w_dtype == FT_DTYPE_F16))
-        return ft_split_gate_up(ctx, x, w_gate, w_up, gate, up, act, M, K, N, w_dtype == FT_DTYPE_F16);
     const bool fused = w_dtype == FT_DTYPE_F16 && apart && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
                        async_eligible(0, x, w_up, up, nullptr, M, K, N, nullptr, nullptr, 0) &&
                        async_eligible(0, x, w_gate, gate, nullptr, M, K, N, nullptr, nullptr, 0) && aligned16p(act);
+    const bool other = w_dtype == FT_DTYPE_F16 ? fused : f32_async_eligible(0, x, w_up, up, M, K, N) && aligned16p(w_gate);
+    if (!ctx->f32_chain && apart && M < (1u << 30) && K < (1u << 30) && N < (1u << 30) &&
+        ft_split_gemm_ok(0, M, K, N, w_dtype == FT_DTYPE_F16) &&
+        (!other || split_gate_up_pays((size_t)ctx->num_cus, w_dtype == FT_DTYPE_F16, M, K, N)))
+        return ft_split_gate_up(ctx, x, w_gate, w_up, gate, up, act, M, K, N, w_dtype == FT_DTYPE_F16);
     if (fused) {
         AsyncBatch g{};
         g.count = 1;

@@ -47,3 +47,34 @@ def test_linears_that_feed_each_other_do_not_share_a_launch(lib, change, togethe
     for order in ((first, second), (second, first)):
         assert lib.ft_internal_group_apart(group(*order), C.c_size_t(2), M, K) == together, order
     assert lib.ft_internal_group_apart(group(second), C.c_size_t(1), M, K) == 1
+
+
+AB, RANKED, RESIDUAL = (0, 0), (1, 0), (1, 1)
+
+
+@pytest.mark.parametrize("half,terms,M,K,N,pays", [
+    # where the f32 instruction was measured faster (256 CUs): short K
+    (0, AB, 4096, 32, 576, 0), (1, AB, 4096, 32, 576, 0), (0, AB, 2048, 64, 576, 0), (1, AB, 2048, 64, 576, 0),
+    (0, AB, 640, 64, 1536, 0), (0, AB, 1024, 128, 576, 0), (1, AB, 4096, 64, 1536, 0),
+    (1, RANKED, 640, 128, 1536, 0), (1, RANKED, 1024, 64, 5120, 0), (1, RANKED, 2048, 128, 1536, 0),
+    (1, RESIDUAL, 2048, 64, 5120, 0), (1, RESIDUAL, 4096, 128, 5120, 0), (1, RESIDUAL, 2048, 192, 1536, 0),
+    # long K on few tiles
+    (0, AB, 64, 4096, 256, 0), (0, AB, 128, 2560, 960, 0), (0, AB, 64, 16384, 2048, 0), (0, AB, 128, 16384, 2048, 0),
+    # where the parts are: the same sizes with another b or more K or tiles, and the usual ones
+    (1, AB, 640, 64, 1536, 1), (0, AB, 2048, 128, 576, 1), (1, AB, 1024, 128, 576, 1), (0, AB, 1024, 192, 576, 1),
+    (1, AB, 8192, 64, 5120, 1), (0, AB, 8192, 64, 5120, 1), (1, RESIDUAL, 2048, 256, 1536, 1), (1, RANKED, 2048, 160, 1536, 1),
+    (1, AB, 64, 16384, 2048, 1), (0, RANKED, 128, 2560, 960, 1), (0, AB, 192, 2560, 960, 1), (0, AB, 64, 2048, 2048, 1),
+    (0, AB, 512, 16384, 2048, 1), (0, AB, 256, 2304, 512, 1), (1, RANKED, 2048, 960, 960, 1), (1, RESIDUAL, 2048, 576, 1536, 1),
+    (0, AB, 1000, 960, 2560, 1), (0, AB, 17, 64, 64, 1), (1, AB, 17, 64, 64, 1),
+])
+def test_products_take_bf16_parts_where_those_are_faster(lib, half, terms, M, K, N, pays):
+    assert lib.ft_internal_split_pays(C.c_size_t(256), half, *terms, C.c_size_t(M), C.c_size_t(K), C.c_size_t(N)) == pays
+
+
+@pytest.mark.parametrize("gate_up,half,M,K,N,pays", [
+    (0, 1, 1024, 64, 3072, 0), (0, 1, 1024, 128, 3072, 0), (0, 1, 2048, 64, 960, 0), (0, 1, 2048, 960, 1600, 1), (0, 1, 96, 64, 960, 1),
+    (1, 1, 512, 32, 1536, 0), (1, 1, 512, 64, 5120, 0), (1, 1, 2048, 96, 5120, 0), (1, 0, 64, 8192, 1024, 0),
+    (1, 1, 2048, 128, 5120, 1), (1, 1, 96, 960, 2560, 1), (1, 0, 256, 4096, 512, 1), (1, 0, 1024, 8192, 1024, 1),
+])
+def test_fused_launches_take_bf16_parts_where_those_are_faster(lib, gate_up, half, M, K, N, pays):
+    assert lib.ft_internal_split_fused_pays(C.c_size_t(256), gate_up, half, C.c_size_t(M), C.c_size_t(K), C.c_size_t(N)) == pays
