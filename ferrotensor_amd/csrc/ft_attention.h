@@ -47,7 +47,7 @@ int ft_attn16_forward(ft_context* ctx, const AttnArgs& a);
 int ft_attn16_backward_dq(ft_context* ctx, const AttnArgs& a);
 int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a);
 
-// ft_attention_split.hip: the forward on bf16 matrix instructions, outside a training step (ft_context::f32_chain);
+// ft_attention_split.hip: the same three on bf16 matrix instructions, outside a training step (ft_context::f32_chain).
 // groups: 4 or 2, the height of a query tile in 16-row blocks.
 int ft_attn_split_forward(ft_context* ctx, const AttnArgs& a, int groups);
 int ft_attn_split_dq(ft_context* ctx, const AttnArgs& a);

@@ -1274,7 +1274,7 @@ int ft_flash_attention_v2_backward_with_stats(ft_context* ctx, const float* q, c
 }  // extern "C"
 
 // ft_flash_attention_v2_with_stats for a pass that no backward follows.
-int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
+extern "C" int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
                                        size_t Sq, size_t Sk, size_t H, size_t Hkv, size_t D, const ft_attention_options* opts) {
     FT_TRY(check_common("attention forward", ctx, B, Sq, Sk, H, Hkv, D, opts));
     AttnArgs a = make_args(B, Sq, Sk, H, Hkv, D, opts);

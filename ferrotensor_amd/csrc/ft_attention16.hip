@@ -86,25 +86,52 @@ int query_tile_groups(const ft_context* ctx, const AttnArgs& a, bool backward) {
     return 0;
 }
 
-// The backward on bf16 parts: its kernels hold one workgroup of 8 waves per CU and want a few rounds of them. dQ, 480
-// workgroups (4 x 1024 tokens, 15 heads on 5): 89 us against 128; 120 (one sequence): 13 us longer. dK/dV, time of the
-// whole backward beside the f32 kernel's: 8 x 1024, 32 heads (4096 workgroups) 924 against 1154, 4 x 1024, 15 on 5 (960)
-// 232 against 246, 8 x 256, 15 on 5 (480) 61.9 against 60.0. Both or neither, and the forward with them: kernels that form
-// the same scores with the same rounding lose less in the probabilities.
-bool split_backward_pays(const ft_context* ctx, const AttnArgs& a) {
-    return !ctx->f32_chain && ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 >= 3 * (size_t)ctx->num_cus &&
-           ft_div_up(a.Sk, 64) * (size_t)a.B * a.H >= 3 * (size_t)ctx->num_cus;
+// dK/dV on bf16 parts: one workgroup per 64 keys and query head where the shares of a group fit their scratch, else per kv
+// head.
+struct DkdvUnits {
+    bool per_head;
+    size_t workgroups;
+};
+DkdvUnits split_dkdv_units(const AttnArgs& a) {
+    const size_t G = (size_t)a.H / a.Hkv, n_all = (size_t)a.B * a.Sk * a.Hkv * a.D;
+    const bool per_head = G == 1 || 2 * G * n_all <= kAttnScratchFloats;
+    return {per_head, ft_div_up(a.Sk, 64) * (size_t)a.B * (per_head ? a.H : a.Hkv)};
 }
+
+// The backward on bf16 parts: its kernels hold one workgroup of 8 waves per CU and want a few rounds of them, of tiles that
+// are not mostly empty. Time of the whole backward, f32 kernels -> these (us, causal):
+//  * dQ, 480 workgroups of 128 queries (4 x 1024 tokens, 15 heads on 5) 128 -> 89, 120 (one sequence) 13 us longer;
+//  * dK/dV per head: 4096 workgroups (8 x 1024, 32 heads) 1266 -> 928, 960 (4 x 1024, 15 on 5) 284 -> 236, 480 (8 x 256, 15 on
+//    5) 60 -> 62. With a group's shares to add it takes longer queries: 4 x 384, 32 on 8 120 -> 107; 24 x 300, 9 on 3
+//    139 -> 148; 16 x 128, 32 on 8 78 -> 93; without a mask 16 x 256, 15 on 5 156 -> 143, 24 x 200, 9 on 3 116 -> 126;
+//  * dK/dV per kv head, workgroups as long as the group is large: 352 (4 x 700, 32 on 8) 299 -> 273, 512 561 -> 436; 264 (3 x
+//    700) 241 -> 257, 88 (4 x 700, 32 on 2) 396 -> 752;
+//  * tiles a quarter empty and more: 24 x 17, 32 heads 36 -> 43, 13 x 65 54 -> 57; 12 x 100 gains.
+// All or none, and the forward with them: kernels that form the same scores with the same rounding lose less in the
+// probabilities.
+bool split_backward_pays(const ft_context* ctx, const AttnArgs& a) {
+    const size_t cus = (size_t)ctx->num_cus, G = (size_t)a.H / a.Hkv;
+    auto full = [](int rows) { return 4 * (size_t)rows >= 3 * 64 * (size_t)ft_div_up(rows, 64); };
+    if (ctx->f32_chain || !full(a.Sq) || !full(a.Sk) || ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 < 3 * cus) return false;
+    const DkdvUnits u = split_dkdv_units(a);
+    if (!u.per_head) return u.workgroups * 3 >= 4 * cus;
+    return u.workgroups >= 3 * cus && (G == 1 || a.Sq >= (a.causal ? 384 : 256));
+}
+// Alone the forward on bf16 parts beats the f32 kernels nearly everywhere, the 32-row ones too (1 x 96 tokens, 15 heads, 7.0
+// us against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 40, 9 heads 5.5 against 7.1), but not with half a tile of queries
+// (4 x 8, 32 heads 5.4 against 4.7) and not where so few workgroups have so long a row of keys that four waves sharing it are
+// worth more (1 x 1024, 3 heads 31.4 against 29.2; 1 x 384 15.0 against 14.6).
 bool split_forward_pays(const ft_context* ctx, const AttnArgs& a) {
-    return !ctx->f32_chain && (a.forward_only || split_backward_pays(ctx, a));
+    if (ctx->f32_chain) return false;
+    if (a.forward_only) return a.Sq >= 32 && (a.Sk <= 256 || query_tile_groups(ctx, a, false) != 0);
+    return split_backward_pays(ctx, a);
 }
 
 // One workgroup per 64 keys and query head, then the ordered sum over the group where there is one (and room for its
 // shares; otherwise per kv head).
 int launch_split_dkdv(ft_context* ctx, const AttnArgs& a) {
-    const size_t G = (size_t)a.H / a.Hkv, n_all = (size_t)a.B * a.Sk * a.Hkv * a.D;
     AttnArgs s = a;
-    if (G > 1 && 2 * G * n_all <= kAttnScratchFloats) {
+    if (a.H > a.Hkv && split_dkdv_units(a).per_head) {
         if (!ctx->attn_scratch) {
             FT_HIP(hipSetDevice(ctx->device));
             FT_HIP(hipMalloc((void**)&ctx->attn_scratch, kAttnScratchFloats * sizeof(float)));
@@ -154,8 +181,6 @@ bool ft_attn16_usable(const AttnArgs& a) {
            al(a.o) && al(a.dq) && al(a.dk) && al(a.dv) && (((uintptr_t)a.stats) & 7) == 0;
 }
 
-// (Alone the forward on bf16 parts beats the f32 kernels at every size, the 32-row ones too: 1 x 96 tokens, 15 heads, 7.0 us
-// against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 40, 9 heads 5.5 against 7.1.)
 bool ft_attn16_forward_pays(const ft_context* ctx, const AttnArgs& a) {
     return split_forward_pays(ctx, a) || query_tile_groups(ctx, a, false) != 0;
 }
@@ -181,4 +206,17 @@ int ft_attn16_backward_dq(ft_context* ctx, const AttnArgs& a) {
 int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a) {
     if (!a.rope && split_backward_pays(ctx, a)) return launch_split_dkdv(ctx, a);
     return launch_dkdv<64>(ctx, a);
+}
+
+// For tests. The second: which call takes the kernels on bf16 parts (outside a training step, operands aligned) on a device
+// of so many CUs: the backward with the forward before it, or a forward alone.
+extern "C" size_t ft_internal_num_cus(const ft_context* ctx) { return (size_t)ctx->num_cus; }
+extern "C" int ft_internal_attention_split(size_t cus, size_t B, size_t Sq, size_t Sk, size_t H, size_t Hkv, int causal,
+                                           int forward_only) {
+    ft_context ctx;
+    ctx.num_cus = (int)cus;
+    AttnArgs a{};
+    a.B = (int)B, a.Sq = (int)Sq, a.Sk = (int)Sk, a.H = (int)H, a.Hkv = (int)Hkv, a.D = 64, a.causal = causal;
+    a.forward_only = forward_only;
+    return split_forward_pays(&ctx, a) ? 1 : 0;
 }

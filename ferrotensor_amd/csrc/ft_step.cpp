@@ -52,7 +52,7 @@ int ft_internal_row_bias_add(ft_context* ctx, float* y, const float* bias, size_
 int ft_internal_col_sum(ft_context* ctx, const float* g, float* out, size_t rows, size_t cols, int accumulate);
 bool ft_internal_attention_rope_fusable(const float* q, const float* k, const float* v, const float* out,
                                         const float* d_out, size_t Sq, size_t Sk, size_t D);
-int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
+extern "C" int ft_internal_attention_forward_only(ft_context* ctx, const float* q, const float* k, const float* v, float* out, size_t B,
                                        size_t Sq, size_t Sk, size_t H, size_t Hkv, size_t D, const ft_attention_options* opts);
 int ft_internal_attention_backward_rope(ft_context* ctx, const float* q, const float* k, const float* v,
                                         const float* out, const float* d_out, float* dq, float* dk, float* dv,

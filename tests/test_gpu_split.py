@@ -5,6 +5,8 @@ instructions follow each other on one accumulator (six per K step of 16, the K s
 then the waves' sums are added; each may be off by 2^-23 of the sum of the absolute products so far, or, among subnormal
 numbers, by their distance 2^-149.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -283,13 +285,25 @@ def attention64(q, k, v, causal, offset):
     return np.matmul(e / z, v.transpose(0, 2, 1, 3)).transpose(0, 2, 1, 3), (m + np.log(z))[..., 0]
 
 
-# From 384 workgroups of 128 queries and 768 of 64 keys on: ragged queries and keys, one and several tiles, grouped heads, an
-# offset, no mask. (Shorter forwards on bf16 parts, tiles of 32 rows among them, come from a model's forward pass.)
-@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(8, 200, 200, 32, 32, True, 0), (8, 129, 193, 32, 16, True, 64), (7, 140, 190, 32, 32, False, 0),
-                                                         (8, 65, 200, 48, 48, True, 0), (16, 33, 129, 32, 8, True, 96)])
+def on_parts(ctx, B, Sq, Sk, H, Hkv, causal, forward_only=0):
+    """Do these sizes take the kernels on bf16 parts on this device?"""
+    from ferrotensor_amd import _lib
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    return lib.ft_internal_attention_split(*(ctypes.c_size_t(x) for x in (lib.ft_internal_num_cus(ctx.handle), B, Sq, Sk, H, Hkv)),
+                                           int(causal), forward_only)
+
+
+# Ragged queries and keys, heads without a group, a group added by the second kernel, a group too large for its scratch,
+# fewer queries than keys with an offset, no mask.
+ATTENTION = [(8, 200, 200, 32, 32, True, 0), (4, 397, 461, 32, 16, True, 64), (8, 150, 190, 32, 32, False, 0), (4, 300, 333, 32, 16, False, 0),
+             (8, 400, 400, 32, 8, True, 0), (12, 96, 200, 32, 32, True, 104), (8, 385, 400, 32, 8, False, 0)]
+
+
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", ATTENTION)
 def test_attention_forward(g, B, Sq, Sk, H, Hkv, causal, offset):
     from ferrotensor_amd import AttentionOptions
     ctx, eng = g
+    assert on_parts(ctx, B, Sq, Sk, H, Hkv, causal)
     q, k, v = rnd(1, B, Sq, H, 64), rnd(2, B, Sk, Hkv, 64), rnd(3, B, Sk, Hkv, 64)
     o, stats = empty(ctx, B, Sq, H, 64), empty(ctx, B * H * Sq, 2)
     eng.flash_attention_v2_with_stats(ctx, up(ctx, q), up(ctx, k), up(ctx, v), o, stats, AttentionOptions(causal=causal, causal_offset=offset))
@@ -299,12 +313,30 @@ def test_attention_forward(g, B, Sq, Sk, H, Hkv, causal, offset):
     np.testing.assert_allclose(np.asarray(stats.to_vec(), np.float64).reshape(B, H, Sq, 2)[..., 1], lse, atol=1e-5)
 
 
+# Tiles of 32 rows (few workgroups) and of 64, ragged, an offset, no mask.
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(1, 40, 40, 3, 1, True, 0), (2, 65, 129, 4, 2, True, 64), (1, 200, 200, 9, 3, False, 0),
+                                                         (1, 256, 256, 3, 1, True, 0), (8, 130, 130, 16, 4, True, 0), (8, 127, 200, 16, 16, False, 0)])
+def test_attention_forward_alone(g, B, Sq, Sk, H, Hkv, causal, offset):
+    """The entry that a model's forward pass takes, which no operator call reaches at these sizes."""
+    from ferrotensor_amd import _lib
+    ctx, eng = g
+    assert on_parts(ctx, B, Sq, Sk, H, Hkv, causal, 1)
+    q, k, v = rnd(1, B, Sq, H, 64), rnd(2, B, Sk, Hkv, 64), rnd(3, B, Sk, Hkv, 64)
+    o, t = empty(ctx, B, Sq, H, 64), [up(ctx, x) for x in (q, k, v)]
+    opts = _lib.AttentionOptionsC(int(causal), offset, 0, 0.0, 0)
+    run = ctypes.CDLL(_lib.LIB_PATH).ft_internal_attention_forward_only
+    assert run(ctx.handle, *(ctypes.c_void_p(x.ptr) for x in (*t, o)), *(ctypes.c_size_t(x) for x in (B, Sq, Sk, H, Hkv, 64)), ctypes.byref(opts)) == 0
+    want, _ = attention64(q, k, v, causal, offset)
+    np.testing.assert_allclose(np.asarray(o.to_vec(), np.float64).reshape(want.shape), want, atol=2e-5)
+
+
 def test_attention_with_infinite_and_nan_values_as_the_f32_kernel(g):
     """V and K of some heads hold an infinity, a NaN, a value at the top of f32: the queries that see them come out as from
     the f32 kernel (where a tile crosses the diagonal, a NaN score counts as masked), the others as ever."""
     from ferrotensor_amd import AttentionOptions
     ctx, eng = g
     B, S, H = 8, 160, 32
+    assert on_parts(ctx, B, S, S, H, H, True)
     q, k, v = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64)
     v[0, 50, 3, 7], v[1, 100, 5, 9], k[2, 70, 1, 4] = np.inf, np.nan, np.nan
     v[3, 20, 2, 11] = 3.4e38   # finite, but its first bf16 part is not
@@ -352,12 +384,10 @@ def run_attention(ctx, eng, q, k, v, do, causal, offset):
     return [np.asarray(x.to_vec(), np.float32).reshape(y.shape) for x, y in ((dq, q), (dk, k), (dv, k))]
 
 
-# From 384 workgroups of 128 queries (dQ) and 768 of 64 keys (dK/dV) on: ragged tiles, heads without a group, a group added
-# by the second kernel, a group too large for its scratch, an offset, no mask.
-@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(8, 200, 200, 32, 32, True, 0), (8, 129, 193, 32, 16, True, 64), (7, 140, 190, 32, 32, False, 0),
-                                                         (8, 300, 300, 32, 8, True, 0), (8, 65, 200, 48, 48, True, 0)])
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", ATTENTION)
 def test_attention_backward(g, B, Sq, Sk, H, Hkv, causal, offset):
     ctx, eng = g
+    assert on_parts(ctx, B, Sq, Sk, H, Hkv, causal)
     q, k, v, do = rnd(1, B, Sq, H, 64), rnd(2, B, Sk, Hkv, 64), rnd(3, B, Sk, Hkv, 64), rnd(4, B, Sq, H, 64, scale=1e-2)
     for name, got, want in zip(("dq", "dk", "dv"), run_attention(ctx, eng, q, k, v, do, causal, offset), backward64(q, k, v, do, causal, offset)):
         # probabilities to 2^-18 of themselves, sums of at most a few hundred rounded terms
@@ -368,6 +398,7 @@ def test_attention_backward_with_infinite_and_nan_values_as_the_f32_kernels(g):
     """The batch takes the kernels on bf16 parts; its sequences one at a time do not: the same values are not finite."""
     ctx, eng = g
     B, S, H = 8, 200, 32
+    assert on_parts(ctx, B, S, S, H, H, True) and not on_parts(ctx, 1, S, S, H, H, True)
     q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
     v[0, 50, 3, 7], do[1, 100, 5, 9], k[2, 70, 1, 4], q[3, 190, 2, 1], do[4, 3, 7, 0] = np.inf, np.nan, np.nan, np.inf, 3.4e38
     batch = run_attention(ctx, eng, q, k, v, do, True, 0)
@@ -381,7 +412,7 @@ def test_attention_backward_with_infinite_and_nan_values_as_the_f32_kernels(g):
 
 @pytest.mark.parametrize("B,S,heads,kv", [(1, 8, 3, 1), (2, 50, 4, 2), (2, 70, 16, 8), (3, 150, 12, 4)])
 def test_model_forward_attention_at_small_sizes(B, S, heads, kv):
-    """A forward pass takes attention on bf16 parts at every size (32- and 64-row tiles): logits against the oracle's."""
+    """A forward pass takes attention on bf16 parts from 32 tokens on (32- and 64-row tiles): logits against the oracle's."""
     from ferrotensor_amd import HipContext
     from ferrotensor_amd.trainer import Lfm2Model, ModelConfig
     from oracle import reference_step as rs
@@ -415,6 +446,7 @@ def test_attention_results_in_the_place_of_an_operand(g):
     from ferrotensor_amd import AttentionOptions
     ctx, eng = g
     B, S, H = 3, 512, 32
+    assert on_parts(ctx, B, S, S, H, H, True)
     q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
     v[0, 50, 3, 7], k[1, 100, 5, 9], do[2, 70, 1, 4] = np.inf, np.nan, 3.4e38
     opts = AttentionOptions(causal=True)
@@ -442,6 +474,7 @@ def test_attention_with_values_below_what_three_bf16_parts_hold(g, case):
     from ferrotensor_amd import AttentionOptions
     ctx, eng = g
     B, S, H = 3, 512, 32
+    assert on_parts(ctx, B, S, S, H, H, True)
     q, k, v, do = rnd(1, B, S, H, 64), rnd(2, B, S, H, 64), rnd(3, B, S, H, 64), rnd(4, B, S, H, 64, scale=1e-2)
     ld = lambda x, e: np.ldexp(x, e).astype(np.float32)
     if case == "v":

@@ -78,3 +78,26 @@ def test_products_take_bf16_parts_where_those_are_faster(lib, half, terms, M, K,
 ])
 def test_fused_launches_take_bf16_parts_where_those_are_faster(lib, gate_up, half, M, K, N, pays):
     assert lib.ft_internal_split_fused_pays(C.c_size_t(256), gate_up, half, C.c_size_t(M), C.c_size_t(K), C.c_size_t(N)) == pays
+
+
+def on_parts(lib, B, Sq, Sk, H, Hkv, causal, forward_only=0):
+    return lib.ft_internal_attention_split(*(C.c_size_t(x) for x in (256, B, Sq, Sk, H, Hkv)), causal, forward_only)
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,causal,pays", [
+    # where the f32 kernels were measured faster (256 CUs): large groups, short queries of grouped heads, tiles mostly empty
+    (4, 700, 32, 2, 1, 0), (3, 700, 32, 4, 1, 0), (8, 512, 32, 4, 1, 0), (3, 700, 32, 8, 1, 0), (24, 700, 8, 1, 0, 0),
+    (16, 128, 32, 8, 1, 0), (8, 200, 32, 8, 1, 0), (8, 256, 32, 8, 1, 0), (24, 300, 9, 3, 1, 0), (24, 200, 9, 3, 0, 0),
+    (24, 17, 32, 32, 1, 0), (24, 40, 32, 32, 1, 0), (13, 65, 32, 32, 0, 0), (1, 1024, 15, 5, 1, 0), (8, 256, 15, 5, 1, 0),
+    # where the parts are
+    (4, 1024, 15, 5, 1, 1), (8, 1024, 9, 3, 1, 1), (5, 1024, 15, 5, 1, 1), (8, 1024, 32, 32, 1, 1), (4, 384, 32, 8, 1, 1),
+    (4, 700, 32, 8, 1, 1), (8, 1024, 32, 4, 1, 1), (8, 200, 32, 32, 1, 1), (16, 256, 15, 5, 0, 1), (12, 100, 32, 32, 1, 1),
+])
+def test_attention_backward_takes_bf16_parts_where_those_are_faster(lib, B, S, H, Hkv, causal, pays):
+    assert on_parts(lib, B, S, S, H, Hkv, causal) == pays
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,pays", [(4, 8, 32, 32, 0), (1, 1024, 3, 1, 0), (1, 4096, 1, 1, 0), (1, 768, 9, 3, 0),
+                                            (1, 40, 9, 3, 1), (1, 96, 15, 5, 1), (1, 384, 3, 1, 0), (1, 256, 3, 1, 1), (1, 1024, 15, 5, 1), (1, 2048, 15, 5, 1)])
+def test_attention_forward_alone_takes_bf16_parts_where_those_are_faster(lib, B, S, H, Hkv, pays):
+    assert on_parts(lib, B, S, S, H, Hkv, 1, 1) == pays
