@@ -722,9 +722,9 @@ __global__ __launch_bounds__(256) void rope_kernel(const float* __restrict__ src
 //
 // The sum of exponentials is made of kCeLanes = 1024 partial sums whatever the workgroup's size: a thread keeps one for
 // each of the 1024 / THREADS lanes it stands for, and they are added in the order of sixteen waves, so the size is a
-// matter of speed alone. Bound: memory, with the two exponentials an element close behind. 49152 columns as
+// matter of speed alone. Bound: memory, with the two exponentials an element close behind. 49152 columns of many rows as
 // 512 threads x 24 float4: two rows share a CU, and one row's loads and stores run under the other's arithmetic (1024
-// threads x 12 float4 take 93 registers, one row at a time); all loads of a row are issued before the first is used (a
+// threads x 12 float4 take 93 registers, one row at a time: for at most a row a CU); all loads of a row are issued before the first is used (a
 // load under `if (i < n4)` waits for the one before it). 1446 x 49152: 147 -> 108 us
 // (5.3 TB/s; a large copy reaches 4.7), 1000 x 1024: 8.2 -> 5.1, 2048 x 4096: 21 -> 15.
 // ---------------------------------------------------------------------------
@@ -775,6 +775,7 @@ __global__ __launch_bounds__(THREADS, CACHE > 12 ? 4 : 1) void masked_ce_kernel(
     if constexpr (CACHE > 0) {
 #pragma unroll
         for (int j = 0; j < CACHE; j++) {
+            if (V == 1 && j * THREADS >= n4) break;   // nobody has a quad left
             const float s4 = expf(cache[j].x - m) + expf(cache[j].y - m) + expf(cache[j].z - m) + expf(cache[j].w - m);
             if (threadIdx.x + j * THREADS < n4) se[j % V] += s4;
         }
@@ -1488,8 +1489,15 @@ int ft_masked_cross_entropy_weighted(ft_context* ctx, const float* logits, const
 #define FT_CE(THREADS, CACHE)                                                                                         \
     hipLaunchKernelGGL((masked_ce_kernel<THREADS, CACHE>), grid, dim3(THREADS), 0, ctx->stream, logits, targets, weights, \
                        grad, row_loss, rows, vocab, grad_scale)
-        // the smallest workgroup that holds a row with at most 24 quads a thread; wider rows are streamed
-        if (vocab <= 256 * 4 * 4) FT_CE(256, 4);
+        // The smallest workgroup that holds a row with at most 24 quads a thread; wider rows are streamed. With at most one
+        // row a CU there is no other row to run beside, and a row gets the largest workgroup, which leaves out
+        // the rounds past its end (in the others that costs more than it saves) (us, the smallest workgroup -> the largest: 256 x 4096 5.4 -> 4.9, 1 x 32000 11.8 -> 10.9, 64 x 49152 17.6 ->
+        // 16.4; 257 x 4096 5.5, was 6.0 with the largest).
+        const bool alone = rows <= (size_t)ctx->num_cus && vocab > 1024;
+        if (alone && vocab <= 1024 * 4 * 4) FT_CE(1024, 4);
+        else if (alone && vocab <= 1024 * 4 * 8) FT_CE(1024, 8);
+        else if (alone && vocab <= 1024 * 4 * 12) FT_CE(1024, 12);
+        else if (vocab <= 256 * 4 * 4) FT_CE(256, 4);
         else if (vocab <= 512 * 4 * 8) FT_CE(512, 8);
         else if (vocab <= 512 * 4 * 24) FT_CE(512, 24);
         else FT_CE(1024, 0);

@@ -609,6 +609,31 @@ def test_masked_cross_entropy_at_the_edges_of_its_workgroup_sizes(g, rows, vocab
     test_masked_cross_entropy(g, rows, vocab)
 
 
+@pytest.mark.parametrize("vocab", [1028, 4096, 4100, 16384, 16388, 32768, 32772, 49152])
+def test_masked_cross_entropy_of_few_and_of_many_rows_is_the_same(g, vocab):
+    """At most a row a CU takes other workgroup sizes than more rows: against f64 at both, and bit for bit alike."""
+    from ferrotensor_amd import UnifiedTensor
+    ctx, eng = g
+    few, many = 5, 1030   # more than one row per CU of any of these chips
+    logits, weights = rnd(7, few, vocab, scale=4.0), np.linspace(0.1, 2.0, few, dtype=np.float32)
+    targets = np.array([0, vocab - 1, vocab // 2, rs.MASKED_CE_SKIP, 3], np.uint32)
+    want_g, want_l = cpu.masked_cross_entropy(logits, targets, weights)
+    results = []
+    for rows in (few, many):
+        rep = -(-rows // few)
+        grad, row_loss = empty(ctx, rows, vocab), empty(ctx, rows)
+        eng.masked_cross_entropy_weighted(ctx, up(ctx, np.tile(logits, (rep, 1))[:rows]),
+                                          UnifiedTensor.from_bytes(ctx, np.tile(targets, rep)[:rows], [rows]),
+                                          up(ctx, np.tile(weights, rep)[:rows]), grad, row_loss)
+        got = grad.to_numpy().reshape(rows, vocab)
+        results.append((got[:few], row_loss.to_numpy()[:few]))
+        assert np.array_equal(got[rows - few:].view(np.uint32), np.roll(got[:few], -(rows % few), 0).view(np.uint32))
+    assert_close("ce grad", results[0][0], want_g, atol=1e-6)
+    assert_close("ce loss", results[0][1], want_l)
+    for a, b in zip(*results):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_sum_squares_and_adamw(g):
     ctx, eng = g
     from ferrotensor_amd import AdamParams, UnifiedTensor
