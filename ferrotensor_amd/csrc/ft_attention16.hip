@@ -208,9 +208,8 @@ int ft_attn16_backward_dkdv(ft_context* ctx, const AttnArgs& a) {
     return launch_dkdv<64>(ctx, a);
 }
 
-// For tests. The second: which call takes the kernels on bf16 parts (outside a training step, operands aligned) on a device
-// of so many CUs: the backward with the forward before it, or a forward alone.
-extern "C" size_t ft_internal_num_cus(const ft_context* ctx) { return (size_t)ctx->num_cus; }
+// Which call takes the kernels on bf16 parts (outside a training step, operands aligned), for callers that have no device (its
+// test): the backward with the forward before it, or a forward alone.
 extern "C" int ft_internal_attention_split(size_t cus, size_t B, size_t Sq, size_t Sk, size_t H, size_t Hkv, int causal,
                                            int forward_only) {
     ft_context ctx;

@@ -305,3 +305,8 @@ int ft_copy_tensor(ft_context* ctx, const void* src_dev, size_t bytes, void* dst
 }
 
 }  // extern "C"
+
+// For tests, not in the header: the CUs that the dispatch rules count with, and operator calls on the kernels that a training
+// step runs (ft_context::f32_chain), which outside of one they no longer reach.
+extern "C" size_t ft_internal_num_cus(const ft_context* ctx) { return (size_t)ctx->num_cus; }
+extern "C" void ft_internal_step_kernels(ft_context* ctx, int on) { ctx->f32_chain = on != 0; }

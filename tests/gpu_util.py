@@ -20,6 +20,13 @@ def make_ctx():
     return ctx, ComputeEngine(ctx)
 
 
+def step_kernels(ctx, on=True):
+    """Operator calls of this context on the kernels of a training step (the f32 matrix instruction throughout)."""
+    import ctypes
+    from ferrotensor_amd import _lib
+    ctypes.CDLL(_lib.LIB_PATH).ft_internal_step_kernels(ctx.handle, int(on))
+
+
 def assert_close(name, got, want, atol=ATOL, rtol=RTOL):
     got = np.asarray(got, np.float64).reshape(-1)
     want = np.asarray(want, np.float64).reshape(-1)

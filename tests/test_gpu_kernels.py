@@ -10,16 +10,22 @@ import pytest
 
 from oracle import cpu
 from oracle import reference_step as rs
-from tests.gpu_util import assert_close, make_ctx
+from tests.gpu_util import assert_close, make_ctx, step_kernels
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
-def g():
+def g(request):
     ctx, eng = make_ctx()
+    step_kernels(ctx, getattr(request, "param", None) == "in_a_step")
     yield ctx, eng
     ctx.close()
+
+
+# Products of a training step and of any other call run on different kernels: the f32 matrix instruction's (what the comments
+# below say of tiles, K shares and epilogues is about those) and those on bf16 parts (whose own edges test_gpu_split.py has).
+both_routes = pytest.mark.parametrize("g", ["outside", "in_a_step"], indirect=True)
 
 
 def rnd(seed, *shape, scale=1.0):
@@ -52,6 +58,7 @@ def f64_mm(a, b):
 
 
 @pytest.mark.parametrize("M,K,N", MATMUL_SHAPES)
+@both_routes
 def test_matmul_layouts_match_cpu(g, M, K, N):
     ctx, eng = g
     a, b = rnd(M * 7 + K, M, K), rnd(N * 3 + K, K, N)
@@ -79,6 +86,7 @@ SMOLLM2_PROJECTIONS = [("135M q/o", 576, 576), ("135M k/v", 576, 192), ("135M fu
 
 @pytest.mark.parametrize("name,K,N", SMOLLM2_PROJECTIONS)
 @pytest.mark.parametrize("M", [31, 256])
+@both_routes
 def test_f16_weight_projections(g, name, K, N, M):
     from ferrotensor_amd import UnifiedTensor
     ctx, eng = g
@@ -98,6 +106,7 @@ def test_f16_weight_projections(g, name, K, N, M):
 @pytest.mark.parametrize("name,M,K,N", [("1.7B gate/up, 8 x 1024 rows", 8192, 2048, 8192),
                                         ("1.7B down, 8 x 1024 rows", 8192, 8192, 2048),
                                         ("360M lm_head on the supervised rows of the headline batch", 1446, 960, 49152)])
+@both_routes
 def test_projections_at_the_row_counts_of_the_full_batches(g, name, M, K, N):
     """The GEMMs of the 1.7B-shaped step at its real row count (M = 8192: thousands of tiles per launch) and
     the vocabulary head (the 128x128 tile): forward and input gradient, sampled rows against f64 (the full
@@ -131,6 +140,7 @@ SMALLEST_SHARES_K = [256, 288, 512, 832]
 
 @pytest.mark.parametrize("K", SHORT_K + SMALLEST_SHARES_K)
 @pytest.mark.parametrize("M,N", [(256, 192), (31, 960), (130, 128)])
+@both_routes
 def test_f16_weight_products_with_short_k_and_smallest_split_shares(g, M, N, K):
     """(256, 192) and (130, 128) are a dozen 64x64 tiles or fewer, so K >= 256 is split over workgroups;
     (31, 960) is one ragged row block."""
@@ -152,6 +162,7 @@ def test_f16_weight_products_with_short_k_and_smallest_split_shares(g, M, N, K):
 
 @pytest.mark.parametrize("K", [64, 96, 256, 288, 512])
 @pytest.mark.parametrize("M,N", [(256, 128), (132, 260)])
+@both_routes
 def test_f32_products_with_short_k_and_smallest_split_shares(g, M, N, K):
     """The DMA-fed f32 kernel takes K >= 64 (two tiles); (256, 128) is 8 tiles of 64x64, so K >= 256 is split
     into shares of 4 and 5 tiles; (132, 260) has ragged last tiles both ways. All three operand layouts."""
@@ -170,6 +181,7 @@ def test_f32_products_with_short_k_and_smallest_split_shares(g, M, N, K):
 
 
 @pytest.mark.parametrize("M,K,N", [(2048, 960, 1600), (2000, 512, 1600), (2048, 960, 1664)])
+@both_routes
 def test_tile_counts_just_above_a_multiple_of_the_cu_count(g, M, K, N):
     """800 (or 832) tiles of 64x64 on 256 CUs: the last 32 (64) tiles of the order are shared out along K over
     8 or 4 workgroups each and added by a second kernel. Plain product, product with residual and rank-8 term,
@@ -195,6 +207,7 @@ def test_tile_counts_just_above_a_multiple_of_the_cu_count(g, M, K, N):
 
 
 @pytest.mark.parametrize("M,K,N", [(1536, 2560, 960), (2048, 1024, 960), (1472, 2048, 896)])
+@both_routes
 def test_long_k_products_on_eight_waves(g, M, K, N):
     """320 to 512 output tiles of 64x64 and K >= 1024: the workgroup's eight waves share the K loop
     in pairs of tiles (both operand layouts; 1472 rows: a ragged last row block)."""
@@ -236,6 +249,7 @@ def test_f16_upload_is_bit_exact(g):
                                      (96, 64, 40, 2), (256, 576, 1536, 32), (70, 96, 200, 1), (128, 192, 64, 12),
                                      (2048, 576, 1536, 8)])  # the last: the kernel-microbench GEMM, full size
 @pytest.mark.parametrize("f16", [False, True])
+@both_routes
 def test_fused_lora_linear_forward_and_backward(g, M, K, N, r, f16):
     """Linear::project_2d and its backward (graph/src/lib.rs:112-126; autograd MatMulNode/ScaleNode)."""
     from ferrotensor_amd import UnifiedTensor
@@ -279,6 +293,34 @@ def test_fused_lora_linear_forward_and_backward(g, M, K, N, r, f16):
     assert_close("dA", da.to_numpy(), grads["l.lora_a"], atol=2e-3, rtol=1e-4)
 
 
+@pytest.mark.parametrize("M,K,N", [(4099, 64, 4), (2050, 96, 8), (129, 64, 132), (127, 96, 260), (257, 64, 68), (65, 256, 256),
+                                   (193, 64, 124), (1025, 288, 64)])
+@pytest.mark.parametrize("r", [0, 4, 8, 12, 16])
+@pytest.mark.parametrize("g", ["in_a_step"], indirect=True)
+def test_f32_products_with_a_rank_r_term_or_a_residual(g, M, K, N, r):
+    """The DMA-fed f32 kernel's tail: every rank it takes, none with a residual, rows and columns just off a tile, fewer columns
+    than a tile (b2 runs along them), the fewest K tiles; x @ w and dy @ w^T, the residual in place too."""
+    ctx, eng = g
+    x, w, wt, res = rnd(M, M, K), rnd(K, K, N), rnd(K + 1, N, K), rnd(M + 1, M, N)
+    t, b, bt = rnd(r, M, max(r, 1)), rnd(r + 1, max(r, 1), N), rnd(r + 2, N, max(r, 1))
+    T, Bk, Bt = (up(ctx, t), up(ctx, b), up(ctx, bt)) if r else (None, None, None)
+    for name, run, terms in (("x@w", lambda out, add: eng.lora_linear(ctx, up(ctx, x), up(ctx, w), T, Bk, out, add), [(x, w), (t, b)]),
+                             ("dy@wT", lambda out, add: eng.lora_linear_dx(ctx, up(ctx, x), up(ctx, wt), T, Bt, out, residual=add),
+                              [(x, wt.T), (t, bt.T)])):
+        for residual in (None, "apart", "in place"):
+            if r == 0 and residual is None:
+                continue
+            add = up(ctx, res) if residual else None
+            out = add if residual == "in place" else empty(ctx, M, N)
+            run(out, add)
+            pairs = terms[:2 if r else 1]
+            want = sum(f64_mm(p, q) for p, q in pairs) + (res if residual else 0.0)
+            # K + r fused multiply-adds and the residual, each off by at most 2^-24 of the sum of absolute products so far
+            size = sum(f64_mm(np.abs(p), np.abs(q)) for p, q in pairs) + (np.abs(res) if residual else 0.0)
+            got = out.to_numpy().reshape(M, N)
+            assert np.all(np.abs(got - want) <= (K + r + 2) * 2.0 ** -24 * size), (name, residual)
+
+
 @pytest.mark.parametrize("r", [4, 8, 16])
 @pytest.mark.parametrize("M", [1, 127, 128, 129])
 def test_lora_factor_gradients_at_the_edge_of_one_slice(g, M, r):
@@ -314,6 +356,7 @@ def test_lora_factor_gradients_in_the_place_of_an_operand(g, M):
                                           (130, 96, (40, 72, 8), 16, True),
                                           # the step's own shapes: the summed input gradient runs its K segments on eight waves
                                           (2048, 960, (960, 320, 320), 8, True), (2048, 960, (2560, 2560), 0, True)])
+@both_routes
 def test_grouped_linears_match_single_calls(g, M, K, Ns, r, f16):
     """q/k/v (gate/up) of one input in one launch, and their summed input gradient in one launch."""
     from ferrotensor_amd import UnifiedTensor
@@ -357,6 +400,7 @@ def test_grouped_linears_match_single_calls(g, M, K, Ns, r, f16):
 
 @pytest.mark.parametrize("B,S,K,heads,kv,r,f16", [(2, 64, 192, 3, 1, 8, True), (1, 32, 64, 2, 2, 0, True),
                                                   (2, 24, 96, 2, 1, 4, False)])
+@both_routes
 def test_grouped_projections_with_rope_in_the_epilogue(g, B, S, K, heads, kv, r, f16):
     """q and k rotated inside the projection launch (heads of 64) == projection followed by rope."""
     from ferrotensor_amd import UnifiedTensor
@@ -394,6 +438,7 @@ def test_grouped_projections_with_rope_in_the_epilogue(g, B, S, K, heads, kv, r,
 
 @pytest.mark.parametrize("M,H,F,f16", [(256, 960, 2560, True), (100, 64, 96, True), (70, 32, 40, True),
                                        (64, 32, 48, False)])
+@both_routes
 def test_fused_gated_mlp_halves(g, M, H, F, f16):
     """gate/up projections + silu_gate in one launch; down-projection backward + silu_gate backward in one."""
     from ferrotensor_amd import UnifiedTensor

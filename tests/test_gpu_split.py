@@ -5,6 +5,7 @@ instructions follow each other on one accumulator (six per K step of 16, the K s
 then the waves' sums are added; each may be off by 2^-23 of the sum of the absolute products so far, or, among subnormal
 numbers, by their distance 2^-149.
 """
+import contextlib
 import ctypes
 
 import numpy as np
@@ -41,6 +42,24 @@ def empty(ctx, *shape):
     return UnifiedTensor.empty(ctx, list(shape))
 
 
+@contextlib.contextmanager
+def on_bf16_parts(ctx):
+    """What runs inside is here to test gemm_split_kernel: sizes that take another one say so."""
+    from ferrotensor_amd import _lib
+    lib = _lib.load()
+    assert lib.ft_profile_begin(ctx.handle) == 0
+    yield
+    n = ctypes.c_size_t()
+    assert lib.ft_profile_end(ctx.handle, ctypes.byref(n)) == 0
+    names = []
+    for i in range(n.value):
+        name, launches, x = ctypes.c_char_p(), ctypes.c_uint64(), [ctypes.c_double() for _ in range(3)]
+        assert lib.ft_profile_kernel(ctx.handle, i, ctypes.byref(name), ctypes.byref(launches), *(ctypes.byref(v) for v in x)) == 0
+        names.append(name.value.decode())
+    products = [x for x in names if x.startswith(("gemm", "splitk"))]
+    assert products and all(x.startswith("gemm_split_kernel") for x in products), names
+
+
 def check(name, got, terms, K):
     """terms: (a, b) pairs whose products add up."""
     want = sum(a.astype(np.float64) @ b.astype(np.float64) for a, b in terms)
@@ -53,9 +72,9 @@ def check(name, got, terms, K):
 
 
 # Each tile and wave count of the dispatch, one row or column more and less than a tile, K with no whole step left over,
-# 1, 4, 15 left over, and rows of every alignment; K = 32 is the shortest that comes here.
-SHAPES = [(4, 32, 8), (31, 36, 33), (33, 47, 31), (32, 64, 32), (100, 333, 517), (257, 733, 1001), (65, 96, 63),
-          (700, 161, 1024), (1023, 100, 640), (1025, 64, 1100), (1100, 127, 1029), (1088, 576, 1152), (5, 2561, 9)]
+# 1, 4, 15 left over, and rows of every alignment, K of two steps and a rest on.
+SHAPES = [(4, 48, 8), (4, 33, 9), (31, 52, 33), (33, 47, 31), (32, 64, 32), (100, 333, 517), (257, 733, 1001), (65, 96, 63),
+          (700, 161, 1024), (1023, 101, 641), (1025, 66, 1101), (2113, 64, 1100), (1100, 127, 1029), (1088, 576, 1152), (5, 2561, 9)]
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
@@ -66,12 +85,17 @@ def test_f32_layouts(g, M, K, N):
     for name, run in (("a@b", lambda: eng.matmul(ctx, up(ctx, a), up(ctx, b), out)),
                       ("a@bT", lambda: eng.matmul_bt(ctx, up(ctx, a), up(ctx, b.T), out)),
                       ("aT@b", lambda: eng.matmul_at(ctx, up(ctx, a.T), up(ctx, b), out))):
-        run()
+        with on_bf16_parts(ctx):
+            run()
         check("%s %dx%dx%d" % (name, M, K, N), out.to_vec(), [(a, b)], K)
 
 
-@pytest.mark.parametrize("M,K,N,r", [(4, 32, 8, 4), (33, 64, 40, 8), (17, 96, 1000, 16), (257, 736, 1000, 32), (700, 1024, 1024, 8),
-                                     (1025, 64, 1104, 16), (1100, 352, 1032, 3)])
+@pytest.mark.parametrize("M,K,N,r", [(4, 48, 8, 4), (33, 64, 40, 8), (17, 96, 1000, 16), (257, 736, 1000, 32), (700, 1024, 1024, 8),
+                                     (2113, 64, 1104, 16), (1100, 352, 1032, 3),
+                                     # widths that are no multiple of 8 (f16) or 4: loads from 2- and 4-byte boundaries, a last
+                                     # K step (dx: of N) element by element, every tile size
+                                     (5, 33, 9, 4), (33, 70, 41, 8), (100, 100, 333, 8), (257, 733, 1001, 16), (700, 161, 1023, 8),
+                                     (1100, 127, 1029, 8), (1090, 577, 1150, 4)])
 def test_adapted_linear_both_ways(g, M, K, N, r):
     ctx, eng = g
     x, w, t, b = rnd(M, M, K), rnd(K, K, N, scale=0.05), rnd(r, M, r), rnd(N, r, N)
@@ -80,9 +104,11 @@ def test_adapted_linear_both_ways(g, M, K, N, r):
     for half in (True, False):
         W, wv = (up16(ctx, w), w16) if half else (up(ctx, w), w)
         y, dx = empty(ctx, M, N), empty(ctx, M, K)
-        eng.lora_linear(ctx, up(ctx, x), W, up(ctx, t), up(ctx, b), y)
+        with on_bf16_parts(ctx):
+            eng.lora_linear(ctx, up(ctx, x), W, up(ctx, t), up(ctx, b), y)
         check("y", y.to_vec(), [(x, wv), (t, b)], K)
-        eng.lora_linear_dx(ctx, up(ctx, dy), W, up(ctx, dt), up(ctx, a), dx, residual=up(ctx, res))
+        with on_bf16_parts(ctx) if N >= 48 else contextlib.nullcontext():   # (a sum over N)
+            eng.lora_linear_dx(ctx, up(ctx, dy), W, up(ctx, dt), up(ctx, a), dx, residual=up(ctx, res))
         check("dx", dx.to_vec(), [(dy, wv.T), (dt, a.T), (res, np.eye(K, dtype=np.float32))], N)
 
 
@@ -130,7 +156,8 @@ def test_values_below_what_three_bf16_parts_hold(g, M, K, N, kind):
     out, w = empty(ctx, M, N), up(ctx, b)
     for name, run in (("a@b", lambda: eng.matmul(ctx, up(ctx, a), w, out)), ("a@bT", lambda: eng.matmul_bt(ctx, up(ctx, a), up(ctx, b.T), out)),
                       ("aT@b", lambda: eng.matmul_at(ctx, up(ctx, a.T), w, out))):
-        run()
+        with on_bf16_parts(ctx):
+            run()
         check("%s %s" % (kind, name), out.to_vec(), [(a, b)], K)
     out = empty(ctx, N, M)   # as the second operand
     eng.matmul(ctx, up(ctx, b.T), up(ctx, a.T), out)
@@ -159,12 +186,13 @@ def test_values_below_what_three_bf16_parts_hold_in_the_fused_launches(g, half):
 @pytest.mark.parametrize("M,N", [(70, 96), (520, 1100)])
 def test_infinities_and_nan_as_f32_products_give_them(g, M, N):
     ctx, eng = g
-    K = 80
+    K = 81
     a, b = np.abs(rnd(5, M, K)) + 0.1, np.abs(rnd(6, K, N)) + 0.1
     a[3, 7], a[9, 20], a[40, 3], a[41, 70] = np.inf, np.nan, 3.4e38, -np.inf
     b[30, 11], b[70, 50], b[3, 60] = np.inf, 0.0, 1e-30
     out = empty(ctx, M, N)
-    eng.matmul(ctx, up(ctx, a), up(ctx, b), out)
+    with on_bf16_parts(ctx):
+        eng.matmul(ctx, up(ctx, a), up(ctx, b), out)
     got = np.asarray(out.to_vec(), np.float32).reshape(M, N)
     with np.errstate(all="ignore"):
         want = np.zeros((M, N))
@@ -194,7 +222,8 @@ def rope_table(ctx, seq, theta=10000.0):
 
 
 @pytest.mark.parametrize("M,K,widths,half", [(4, 32, (64, 64, 64), True), (33, 100, (128, 64, 72), False), (96, 960, (960, 320, 320), True),
-                                             (520, 250, (1088, 64, 64), True), (1040, 64, (1024, 128, 8), False)])
+                                             (520, 250, (1088, 64, 64), True), (1040, 64, (1024, 128, 8), False),
+                                             (33, 100, (64, 64, 73), True), (520, 251, (1024, 64, 70), True), (1040, 193, (1024, 128, 9), False)])
 def test_group_with_rotation_and_residual(g, M, K, widths, half):
     """Two rotated products and one with a residual and a rank-r term, every tile height and wave count."""
     ctx, eng = g
@@ -216,21 +245,24 @@ def test_group_with_rotation_and_residual(g, M, K, widths, half):
             plain = np.stack([h[:, :, 0] * c - h[:, :, 1] * s, h[:, :, 0] * s + h[:, :, 1] * c], 2).reshape(M, n)
             size = np.stack([hs[:, :, 0] + hs[:, :, 1]] * 2, 2).reshape(M, n)
         want.append((plain, size))
-    eng.lora_linear_group(ctx, up(ctx, x), linears, rope_table=table, rope_seq=seq, n_rope=2)
+    with on_bf16_parts(ctx):
+        eng.lora_linear_group(ctx, up(ctx, x), linears, rope_table=table, rope_seq=seq, n_rope=2)
     for (w, f, b, y, r), (plain, size) in zip(linears, want):
         limit = (6 * (K // 16 // 4 + 1) + 36) * 2.0 ** -23 * size
         got = np.asarray(y.to_vec(), np.float64).reshape(plain.shape)
         assert np.all(np.abs(got - plain) <= limit), (y.shape, np.max(np.abs(got - plain) / limit))
 
 
-@pytest.mark.parametrize("M,K,N,half", [(4, 32, 8, True), (33, 100, 41, False), (96, 960, 2560, True), (300, 200, 1000, True), (1040, 64, 1024, False)])
+@pytest.mark.parametrize("M,K,N,half", [(4, 32, 8, True), (33, 100, 41, False), (96, 960, 2560, True), (300, 200, 1000, True), (1040, 64, 1024, False), (33, 101, 41, True),
+                                        (520, 205, 1003, True)])
 def test_gate_up(g, M, K, N, half):
     ctx, eng = g
     x, wg, wu = rnd(M, M, K), rnd(N, K, N, scale=0.05), rnd(N + 1, K, N, scale=0.05)
     gv, uv = (w.astype(np.float16).astype(np.float32) if half else w for w in (wg, wu))
     make = up16 if half else up
     gate, u, act = (empty(ctx, M, N) for _ in range(3))
-    eng.mlp_gate_up(ctx, up(ctx, x), make(ctx, wg), make(ctx, wu), gate, u, act)
+    with on_bf16_parts(ctx):
+        eng.mlp_gate_up(ctx, up(ctx, x), make(ctx, wg), make(ctx, wu), gate, u, act)
     check("gate", gate.to_vec(), [(x, gv)], K)
     check("up", u.to_vec(), [(x, uv)], K)
     gt, ut = (np.asarray(o.to_vec(), np.float64) for o in (gate, u))
