@@ -2142,8 +2142,10 @@ int gemm_dispatch(ft_context* ctx, const char* who, int layout, bool half_b, con
     if (f32_async && !p.a2 && !add)
         return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N);
     // With a rank-r term or a residual: the same pipeline, the K chain in one piece. 135M-width step on f32 weights, 2912
-    // rows: 10.45 -> 9.73 ms (117 of these products a step, on the register-staged kernel 32 us each on average).
-    if (f32_async && layout != 2 && (p.a2 || add) &&
+    // rows: 10.45 -> 9.73 ms (117 of these products a step, on the register-staged kernel 32 us each on average). Not a @ b
+    // with a rank-r term over two or three K tiles, where loading that term's tiles apart shows: 2048 x 64 x 576 6.95 -> 7.23,
+    // 512 x 96 x 8192 14.6 -> 15.5.
+    if (f32_async && layout != 2 && (p.a2 || add) && (layout == 1 || !p.a2 || K >= 128) &&
         (!p.a2 || (K2 <= 16 && K2 % 4 == 0 && aligned16p(a2) && aligned16p(b2) && (layout == 1 || N % 4 == 0))) &&
         ((M + 127) / 128) * ((N + 127) / 128) < 8 * (size_t)ctx->num_cus)
         return launch_f32_async(ctx, layout, a, static_cast<const float*>(b), out, M, K, N, p.a2, p.b2, p.a2 ? K2 : 0, add);
