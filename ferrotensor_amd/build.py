@@ -43,7 +43,7 @@ def _compile(src):
 
 def build(force=True, sources=None):
     srcs = [s for s in (sources or SOURCES) if os.path.exists(os.path.join(CSRC, s))]
-    headers = [os.path.join(CSRC, "ft_common.h"), os.path.join(CSRC, "ft_split.h"), os.path.join(CSRC, "ft_thin.h"), os.path.join(CSRC, "ft_attention.h"), os.path.join(CSRC, "ft_attention16.h"), os.path.join(ROOT, "include", "ferrotensor_hip.h")]
+    headers = [os.path.join(CSRC, "ft_common.h"), os.path.join(CSRC, "ft_split.h"), os.path.join(CSRC, "ft_parts.h"), os.path.join(CSRC, "ft_thin.h"), os.path.join(CSRC, "ft_attention.h"), os.path.join(CSRC, "ft_attention16.h"), os.path.join(ROOT, "include", "ferrotensor_hip.h")]
     deps = [os.path.join(CSRC, s) for s in srcs] + headers
     if not force and not _stale(LIB, deps):
         return LIB

@@ -25,31 +25,25 @@
 // 965; forward alone of 8 x 256, 15 on 5: 19.8 -> 14.8. Measured and not kept for the forward: one query tile of 64 rows per
 // workgroup, two workgroups a CU (64, 272, 15.5); 32 rows a wave (61, 248, 17.5).
 #include "ft_attention16.h"
+#include "ft_parts.h"
 
 namespace {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 constexpr int PLANE = KT * D64 * 2;   // bytes of one part of a 64-key tile
 
-__device__ __forceinline__ unsigned pack2(float x, float y) {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x, y}, bf16x2));
-}
-// Two values into the packed halves of their three parts. `left` collects what the third parts leave over, as bits: a
-// third part holds its value when the low half of that value is zero (from 2^-110 up, always).
+// Two values into the packed halves of their three parts.
 __device__ __forceinline__ void split2(float x, float y, unsigned (&part)[3], unsigned* left = nullptr) {
 #pragma unroll
     for (int t = 0; t < 3; t++) {
-        if (t == 2 && left) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(*left) : "v"(x), "v"(y));
+        if (t == 2 && left) collect_left(*left, x, y);
         const unsigned q = pack2(x, y);
         part[t] = q;
         if (t < 2) {
-            x -= __uint_as_float(q << 16);
-            y -= __uint_as_float(q & 0xffff0000u);
+            x -= low_half(q);
+            y -= high_half(q);
         }
     }
 }
@@ -191,7 +185,7 @@ struct Watch {
         if (tid % 64 == 0) atomicMax(&all, __float_as_uint(m));
     }
     __device__ __forceinline__ float largest() const { return __uint_as_float(all); }
-    __device__ __forceinline__ bool left_over(int tid) const { return (left[tid] & 0xffffu) != 0; }
+    __device__ __forceinline__ bool left_over(int tid) const { return ::left_over(left[tid]); }
 };
 // dS is a product and may be any small: its parts hold it to 2^-134 (half of bf16's smallest step). A row of a result that is
 // a sum over `terms` of them times operands of at most `largest`, and that small, may be off by more than a rounding.
@@ -359,7 +353,7 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
             bad = bad || not_finite(o[e]);
         }
     }
-    bad = (bad && w.q_ok) || (left & 0xffffu);
+    bad = (bad && w.q_ok) || left_over(left);
     bool again = p.in_place && __syncthreads_or(bad);
     if (w.kh == 0 && w.q_ok && !again) {
         // register r of accumulator e is head-dim index 16 e + 4 g + r

@@ -24,6 +24,7 @@
 // step ahead -> its own part of LDS -> MFMA operand order), so the K loop has no barrier; the KW sums meet in LDS at the
 // end, in wave order. Nothing depends on alignment but the speed of the loads.
 #include "ft_common.h"
+#include "ft_parts.h"
 #include "ft_split.h"
 
 #include <cmath>
@@ -31,10 +32,7 @@
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
@@ -67,16 +65,6 @@ struct SplitArgs {
     float* out3;
 };
 constexpr int kSplitPlain = 0, kSplitGroup = 1, kSplitGateUp = 2;
-
-// Two values into their three (or two) bf16 parts, packed as the matrix operand wants them.
-__device__ __forceinline__ unsigned pack2(float x, float y) {
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{x, y}, bf16x2));
-}
-// The two halves of a packed pair as f32. (v_dot2_f32_bf16 with (-1, 0) would unpack and subtract in one instruction,
-// but it runs in the matrix unit: measured, an MFMA and eight of them take as long as both apart, with eight of these
-// they take 20 ns where the MFMA alone takes 16.)
-__device__ __forceinline__ float low_half(unsigned p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float high_half(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 
 // One operand: F blocks of 32 rows (of a; columns of b) by 16 k per step.
 //   KM = false: element (row, k) at base[row * ld + k];  KM = true: at base[k * ld + row].
@@ -311,8 +299,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
 #pragma unroll
         for (int t = 0; t < NB; t++) ob[t].fetch(bases[t] + s * b_step);
     };
-    // What third parts leave over, as bits: a third part holds its value when the low half of that value is zero.
-    unsigned left = 0;
+    unsigned left = 0;   // what third parts leave over
     // The slab of this wave's next step, out of LDS and into parts (`next`), beside the products of the current one
     // (`p`). A wave issues a VALU instruction every 8 cycles at best, an MFMA keeps the matrix unit for 32: they are
     // dealt out in turn, a pair of values a slot, its three stages in three slots, so that no stage waits for the one
@@ -343,7 +330,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
                 const bool of_a = t < 4 * FM;
                 const int blk = (of_a ? t : t - 4 * FM) / 4, e = t % 4;
                 if (!of_a && ph >= PB) continue;
-                if (ph == 2) asm("v_or3_b32 %0, %0, %1, %2" : "+v"(left) : "v"(u[t]), "v"(v[t]));   // (in C it waits for the end of the step, with all its registers)
+                if (ph == 2) collect_left(left, u[t], v[t]);
                 if (ph == 0) {
                     u[t] = of_a ? xa[of_a ? blk : 0][2 * e] : (float)xb[of_a ? 0 : blk][2 * e];
                     v[t] = of_a ? xa[of_a ? blk : 0][2 * e + 1] : (float)xb[of_a ? 0 : blk][2 * e + 1];
@@ -410,7 +397,7 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_split_kernel(SplitArgs g) {
         for (int j = 0; j < FN; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) zero = fmaf(acc[i][j][r], 0.0f, zero);
-    if (__builtin_expect(__any(zero != 0.0f || (left & 0xffffu) != 0), 0)) {
+    if (__builtin_expect(__any(zero != 0.0f || left_over(left)), 0)) {
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll

@@ -450,7 +450,6 @@ struct DeferScope {
     ~DeferScope() { ctx->defer = nullptr; }
 };
 
-// y = x @ W (+ (scale * x @ A) @ B) (+ bias) (+ residual), keeping t = scale * x @ A for backward.
 // A training step's products keep the f32 matrix instruction's rounding (see ft_context::f32_chain).
 struct ChainScope {
     ft_context* ctx;
@@ -458,6 +457,7 @@ struct ChainScope {
     ~ChainScope() { ctx->f32_chain = false; }
 };
 
+// y = x @ W (+ (scale * x @ A) @ B) (+ bias) (+ residual), keeping t = scale * x @ A for backward.
 // `defer` (optional): the product may leave its K shares unadded for the caller's next kernel.
 int linear_forward(ft_context* ctx, LinearW& l, const float* x, float* t, float* y, size_t T,
                    const float* residual = nullptr, ft_deferred_sum* defer = nullptr) {

@@ -293,13 +293,14 @@ def test_fused_lora_linear_forward_and_backward(g, M, K, N, r, f16):
     assert_close("dA", da.to_numpy(), grads["l.lora_a"], atol=2e-3, rtol=1e-4)
 
 
-@pytest.mark.parametrize("M,K,N", [(4099, 64, 4), (2050, 96, 8), (129, 64, 132), (127, 96, 260), (257, 64, 68), (65, 256, 256),
-                                   (193, 64, 124), (1025, 288, 64)])
+@pytest.mark.parametrize("M,K,N", [(4099, 128, 4), (2050, 160, 8), (129, 128, 132), (127, 96, 260), (257, 64, 68), (65, 256, 256),
+                                   (193, 128, 124), (1025, 288, 64)])
 @pytest.mark.parametrize("r", [0, 4, 8, 12, 16])
 @pytest.mark.parametrize("g", ["in_a_step"], indirect=True)
 def test_f32_products_with_a_rank_r_term_or_a_residual(g, M, K, N, r):
     """The DMA-fed f32 kernel's tail: every rank it takes, none with a residual, rows and columns just off a tile, fewer columns
-    than a tile (b2 runs along them), the fewest K tiles; x @ w and dy @ w^T, the residual in place too."""
+    than a tile (b2 runs along them), the fewest K tiles (four for x @ w with a rank, else two; below, the register-staged
+    kernel); x @ w and dy @ w^T, the residual in place too."""
     ctx, eng = g
     x, w, wt, res = rnd(M, M, K), rnd(K, K, N), rnd(K + 1, N, K), rnd(M + 1, M, N)
     t, b, bt = rnd(r, M, max(r, 1)), rnd(r + 1, max(r, 1), N), rnd(r + 2, N, max(r, 1))
