@@ -118,12 +118,12 @@ bool split_backward_pays(const ft_context* ctx, const AttnArgs& a) {
     return u.workgroups >= 3 * cus && (G == 1 || a.Sq >= (a.causal ? 384 : 256));
 }
 // Alone the forward on bf16 parts beats the f32 kernels nearly everywhere, the 32-row ones too (1 x 96 tokens, 15 heads, 7.0
-// us against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 40, 9 heads 5.5 against 7.1), but not with half a tile of queries
-// (4 x 8, 32 heads 5.4 against 4.7) and not where so few workgroups have so long a row of keys that four waves sharing it are
-// worth more (1 x 1024, 3 heads 31.4 against 29.2; 1 x 384 15.0 against 14.6).
+// us against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 8, 9 heads 4.6 against 6.5), but not the 16-row ones with half a tile
+// of queries (4 x 8, 32 heads 5.4 against 4.7) and not where so few workgroups have so long a row of keys that four waves
+// sharing it are worth more (1 x 1024, 3 heads 31.4 against 29.2; 1 x 384 15.0 against 14.6).
 bool split_forward_pays(const ft_context* ctx, const AttnArgs& a) {
     if (ctx->f32_chain) return false;
-    if (a.forward_only) return a.Sq >= 32 && (a.Sk <= 256 || query_tile_groups(ctx, a, false) != 0);
+    if (a.forward_only) return query_tile_groups(ctx, a, false) != 0 ? a.Sq >= 32 : a.Sk <= 256;
     return split_backward_pays(ctx, a);
 }
 

@@ -155,16 +155,24 @@ __device__ __forceinline__ void read_parts(const char* at, uintx4 (&part)[3]) {
     for (int q = 0; q < 3; q++) part[q] = *reinterpret_cast<const uintx4*>(at + q * PLANE);
 }
 
-// A row's 64 values (this lane's 16 of them) as the two k steps' operand registers.
-__device__ __forceinline__ void row_parts(const float* row, int g, uintx4 (&part)[2][3], unsigned* left) {
+// A row's 64 values (this lane's 16 of them) on their way to the two k steps' operand registers. The forward splits them
+// behind its first tile and the barrier after it (before, the wait for these loads, the last ones, comes ahead of the tile:
+// 33 tokens 5.6 us for 5.3); in the backward, which has no register to spare, that is slower.
+struct Row {
+    float4 pre[4];
+    __device__ __forceinline__ void fetch(const float* row, int g) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-        const float4 a = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g);
-        const float4 b = *reinterpret_cast<const float4*>(row + 32 * ks + 8 * g + 4);
-        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        split8(x, part[ks], left);
+        for (int e = 0; e < 4; e++) pre[e] = *reinterpret_cast<const float4*>(row + 32 * (e / 2) + 8 * g + 4 * (e % 2));
     }
-}
+    __device__ __forceinline__ void parts(uintx4 (&part)[2][3], unsigned* left) const {
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            const float4 a = pre[2 * ks], b = pre[2 * ks + 1];
+            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            split8(x, part[ks], left);
+        }
+    }
+};
 
 // What the backward kernels look out for, in LDS (a slot of its own per thread, so nobody waits) where their loops have no
 // register to spare: what third parts leave over (split2), and the largest operand that dS is multiplied with.
@@ -222,9 +230,9 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         vl.fetch(v_head, kv_stride, p.Sk, 0, tid);
     }
     const float sscale = p.scale * kLog2e;   // scores are kept in base 2
-    uintx4 qp[2][3];
+    Row q_row;
+    q_row.fetch(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g);
     unsigned left = 0;
-    row_parts(p.q + (((long)w.b * p.Sq + w.qc) * p.H + w.h) * D64, g, qp, &left);
     floatx4 o[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) o[e] = zero4();
@@ -238,6 +246,8 @@ __global__ __launch_bounds__(4 * NG * 64) void attn_split_fwd_kernel(AttnArgs p)
         vl.store(smem + 3 * PLANE, tid, &left);
     }
     __syncthreads();
+    uintx4 qp[2][3];
+    q_row.parts(qp, &left);
 
     auto tile = [&](auto nsb_tag, auto mask_tag, const char* ks, const char* vs, int kb) {
         constexpr int NSB = decltype(nsb_tag)::value;
@@ -411,8 +421,11 @@ __global__ __launch_bounds__(512, 2) void attn_split_dq_kernel(AttnArgs p) {
         const int q = w.q + 16 * c, qc = q < p.Sq ? q : p.Sq - 1;
         const long qoff = (((long)w.b * p.Sq + qc) * p.H + w.h) * D64;
         const long srow = ((long)w.b * p.H + w.h) * p.Sq + qc;
-        row_parts(p.q + qoff, g, qp[c], &left);
-        row_parts(p.d_out + qoff, g, dop[c], &left);
+        Row q_row, do_row;
+        q_row.fetch(p.q + qoff, g);
+        q_row.parts(qp[c], &left);
+        do_row.fetch(p.d_out + qoff, g);
+        do_row.parts(dop[c], &left);
         delta[c] = 0.0f;
 #pragma unroll
         for (int blk = 0; blk < 4; blk++) {   // dO.O as the f32 kernel adds it
@@ -575,8 +588,11 @@ __global__ __launch_bounds__(512, 2) void attn_split_dkdv_kernel(AttnArgs p) {
     const float sscale = p.scale * kLog2e;
     uintx4 kp[2][3], vp[2][3];
     unsigned left = 0;
-    row_parts(p.k + krow, g, kp, &left);
-    row_parts(p.v + krow, g, vp, &left);
+    Row k_row, v_row;
+    k_row.fetch(p.k + krow, g);
+    k_row.parts(kp, &left);
+    v_row.fetch(p.v + krow, g);
+    v_row.parts(vp, &left);
 
     const int nqt = (p.Sq + KT - 1) / KT;
     int qt0 = 0;

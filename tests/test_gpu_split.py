@@ -346,7 +346,7 @@ def test_attention_forward(g, B, Sq, Sk, H, Hkv, causal, offset):
 
 
 # Tiles of 32 rows (few workgroups) and of 64, ragged, an offset, no mask.
-@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(1, 40, 40, 3, 1, True, 0), (2, 65, 129, 4, 2, True, 64), (1, 200, 200, 9, 3, False, 0),
+@pytest.mark.parametrize("B,Sq,Sk,H,Hkv,causal,offset", [(1, 40, 40, 3, 1, True, 0), (1, 7, 9, 3, 1, True, 2), (2, 65, 129, 4, 2, True, 64), (1, 200, 200, 9, 3, False, 0),
                                                          (1, 256, 256, 3, 1, True, 0), (8, 130, 130, 16, 4, True, 0), (8, 127, 200, 16, 16, False, 0)])
 def test_attention_forward_alone(g, B, Sq, Sk, H, Hkv, causal, offset):
     """The entry that a model's forward pass takes, which no operator call reaches at these sizes."""
@@ -444,7 +444,7 @@ def test_attention_backward_with_infinite_and_nan_values_as_the_f32_kernels(g):
 
 @pytest.mark.parametrize("B,S,heads,kv", [(1, 8, 3, 1), (2, 50, 4, 2), (2, 70, 16, 8), (3, 150, 12, 4)])
 def test_model_forward_attention_at_small_sizes(B, S, heads, kv):
-    """A forward pass takes attention on bf16 parts from 32 tokens on (32- and 64-row tiles): logits against the oracle's."""
+    """A forward pass takes attention on bf16 parts at these sizes (32- and 64-row tiles): logits against the oracle's."""
     from ferrotensor_amd import HipContext
     from ferrotensor_amd.trainer import Lfm2Model, ModelConfig
     from oracle import reference_step as rs

@@ -97,7 +97,7 @@ def test_attention_backward_takes_bf16_parts_where_those_are_faster(lib, B, S, H
     assert on_parts(lib, B, S, S, H, Hkv, causal) == pays
 
 
-@pytest.mark.parametrize("B,S,H,Hkv,pays", [(4, 8, 32, 32, 0), (1, 1024, 3, 1, 0), (1, 4096, 1, 1, 0), (1, 768, 9, 3, 0),
+@pytest.mark.parametrize("B,S,H,Hkv,pays", [(4, 8, 32, 32, 0), (1, 8, 9, 3, 1), (1, 23, 6, 2, 1), (1, 1024, 3, 1, 0), (1, 4096, 1, 1, 0), (1, 768, 9, 3, 0),
                                             (1, 40, 9, 3, 1), (1, 96, 15, 5, 1), (1, 384, 3, 1, 0), (1, 256, 3, 1, 1), (1, 1024, 15, 5, 1), (1, 2048, 15, 5, 1)])
 def test_attention_forward_alone_takes_bf16_parts_where_those_are_faster(lib, B, S, H, Hkv, pays):
     assert on_parts(lib, B, S, S, H, Hkv, 1, 1) == pays
