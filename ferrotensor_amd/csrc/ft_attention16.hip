@@ -132,12 +132,8 @@ bool split_forward_pays(const ft_context* ctx, const AttnArgs& a) {
 int launch_split_dkdv(ft_context* ctx, const AttnArgs& a) {
     AttnArgs s = a;
     if (a.H > a.Hkv && split_dkdv_units(a).per_head) {
-        if (!ctx->attn_scratch) {
-            FT_HIP(hipSetDevice(ctx->device));
-            FT_HIP(hipMalloc((void**)&ctx->attn_scratch, kAttnScratchFloats * sizeof(float)));
-        }
-        s.part = ctx->attn_scratch;
-        s.split_g = 1;
+        s.part = ft_scratch_or_none(ctx, &ctx->attn_scratch, kAttnScratchFloats);   // (the f32 kernels need none here)
+        s.split_g = s.part != nullptr;
     }
     FT_TRY(ft_attn_split_dkdv(ctx, s));
     return s.split_g ? ft_attn_dkdv_combine(ctx, s, 64) : FT_OK;

@@ -89,6 +89,10 @@ struct ft_prof_scope {
 
 int ft_set_error(int code, const char* fmt, ...);
 
+// One of the context's scratch buffers, allocated on first use, or NULL where that cannot be had (under stream capture, or
+// memory is short): for launches that can do without it.
+float* ft_scratch_or_none(ft_context* ctx, float** slot, size_t floats);
+
 // Looks up, once per device, the device address of the fixed scratch array behind
 // ft_rms_norm_backward_noalloc (ft_rowops.hip). `device` must be the current device.
 int ft_internal_noalloc_init(int device);

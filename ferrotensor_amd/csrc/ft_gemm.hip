@@ -2011,12 +2011,12 @@ int launch_f32_async(ft_context* ctx, int layout, const float* a, const float* b
     if (!a2 && !add && tiles * 2 <= (size_t)ctx->num_cus && (M * N) % 4 == 0) {
         const int want = f32_async_shares((size_t)ctx->num_cus, tiles, K);
         if (want >= 2 && M * N * (size_t)want <= kSplitScratchFloats) {
-            if (!ctx->gemm_scratch) {
+            if (!ctx->gemm_scratch && ctx->f32_chain) {   // a step's order of sums does not depend on memory
                 FT_HIP(hipSetDevice(ctx->device));
                 FT_HIP(hipMalloc((void**)&ctx->gemm_scratch, kSplitScratchFloats * sizeof(float)));
             }
-            g.splits = want;
-            g.partial = ctx->gemm_scratch;
+            g.partial = ft_scratch_or_none(ctx, &ctx->gemm_scratch, kSplitScratchFloats);
+            if (g.partial) g.splits = want;
         }
     }
     const dim3 grid((unsigned)tiles, (unsigned)g.splits);
@@ -2194,6 +2194,17 @@ int skinny_launch(ft_context* ctx, const float* x, const float* y, float* out, s
 }
 
 }  // namespace
+
+float* ft_scratch_or_none(ft_context* ctx, float** slot, size_t floats) {
+    if (*slot) return *slot;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone ||
+        hipSetDevice(ctx->device) != hipSuccess || hipMalloc((void**)slot, floats * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();   // not the next launch's error
+        *slot = nullptr;
+    }
+    return *slot;
+}
 
 extern "C" {
 

@@ -543,3 +543,53 @@ def test_attention_with_values_below_what_three_bf16_parts_hold(g, case):
             # as test_attention_backward, or among subnormal results their distance; where cancellation is all there is
             # (dS of a head with hardly any dP), as far off as the f32 kernels
             assert err <= max(2e-5 * scale, 64 * 2.0 ** -149, 2 * err32), (name, h, err, scale, err32)
+
+
+def replays_match(ctx, call, outputs, eager_call, eager_outputs, bound):
+    """Captures `call` on the context's stream, then replays it three times, with the eager call between the replays."""
+    from ferrotensor_amd import _lib
+    hip, lib = ctypes.CDLL("libamdhip64.so.7"), _lib.load()
+    stream, graph, run = ctypes.c_void_p(lib.ft_context_stream(ctx.handle)), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    call()
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for i in range(3):
+        assert hip.hipGraphLaunch(run, stream) == 0
+        ctx.synchronize()
+        eager_call()
+        for n, (a, b) in enumerate(zip(outputs, eager_outputs)):
+            x, y = (np.asarray(t.to_vec(), np.float32) for t in (a, b))
+            assert np.max(np.abs(x - y)) <= bound * np.max(np.abs(y)), (i, n)
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
+def test_attention_backward_is_captured_without_a_warm_up():
+    """A context that has run nothing yet: the group's shares have no scratch, and under capture none can be allocated; the f32
+    kernels need none at these sizes."""
+    from ferrotensor_amd import AttentionOptions
+    B, S, H, Hkv = 3, 512, 32, 8
+    host = [rnd(1, B, S, H, 64), rnd(2, B, S, Hkv, 64), rnd(3, B, S, Hkv, 64), rnd(4, B, S, H, 64, scale=1e-2)]
+    opts = AttentionOptions(causal=True)
+    ctx, eng = make_ctx()
+    assert on_parts(ctx, B, S, S, H, Hkv, True)
+    q, k, v, do = (up(ctx, x) for x in host)
+    o, stats = empty(ctx, *host[0].shape), empty(ctx, B * H * S, 2)
+    out, eager = ([empty(ctx, *x.shape) for x in host[:3]] for _ in range(2))
+    eng.flash_attention_v2_with_stats(ctx, q, k, v, o, stats, opts)
+    ctx.synchronize()
+    back = lambda to: eng.flash_attention_v2_backward_with_stats(ctx, q, k, v, o, do, *to, stats, opts)
+    # heads added in another order: sums of at most a few thousand rounded terms
+    replays_match(ctx, lambda: back(out), out, lambda: back(eager), eager, 2e-5)
+    ctx.close()
+
+
+def test_f32_product_with_long_k_is_captured_without_a_warm_up():
+    """The same for a product whose K the f32 kernel shares out over workgroups, which add through scratch memory."""
+    ctx, eng = make_ctx()
+    a, b = up(ctx, rnd(1, 64, 4096)), up(ctx, rnd(2, 4096, 256))
+    out, eager = empty(ctx, 64, 256), empty(ctx, 64, 256)
+    ctx.synchronize()
+    # 4096 fused multiply-adds in one chain or in eight
+    replays_match(ctx, lambda: eng.matmul(ctx, a, b, out), [out], lambda: eng.matmul(ctx, a, b, eager), [eager], 4096 * 2.0 ** -24)
+    ctx.close()
