@@ -52,10 +52,11 @@ struct ft_context {
     // shares itself; the launch fills it in (and leaves out splitk_reduce_kernel) when it splits K,
     // and clears the pointer either way.
     ft_deferred_sum* defer = nullptr;
-    // Set by the step driver for the length of a training step: its products keep the rounding of the f32 matrix
-    // instruction (one chain of fused multiply-adds per K share), so that a run goes on with the bits it began with.
-    // AdamW's first updates divide a gradient by its own size, which makes whole steps of the rounding noise in the
-    // smallest ones. Products outside a step take the faster split ones (ft_split.hip).
+    // Set by the step driver for the length of a training step: its products and attention stay on the f32 matrix
+    // instruction (one chain of fused multiply-adds per K share), outside a step they take the faster bf16 parts
+    // (ft_split.hip). AdamW's first updates divide a gradient by its own size, which makes whole steps of the rounding noise
+    // in the smallest ones: after one update two equally exact orders of summation differ by 3e-3 of a gradient's rms (5e-4
+    // is what a step is held to). Parts have not been measured in a step.
     bool f32_chain = false;
     // Per-query-head partial dK/dV of the attention backward at small batch; allocated on first use.
     float* attn_scratch = nullptr;

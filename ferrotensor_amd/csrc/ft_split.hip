@@ -13,14 +13,14 @@
 // takes 1.7 to 2.8 times as long (8192 x 2048 x 2048, f16 b: 830 us for 328); looking for it costs 1 to 3 % (f16 b: 1 %).
 // The rank-r term and what K leaves after its last whole step of 16 take the f32 instruction too.
 //
-// Bound: VALU and matrix unit together. 8192 x 2048 x 2048 with f16 b: 340 us (202 TFLOP/s; f32 products 518), of them
-// 286 with no operand fetched at all; 2048 x 2560 x 2048 with f32 b: 127 us (160 with f32 products). Relative error
+// Bound: VALU and matrix unit together. 8192 x 2048 x 2048 with f16 b: 329 to 342 us (204 TFLOP/s; f32 products 518), of them
+// 286 with no operand fetched at all; 2048 x 2560 x 2048 with f32 b: 129 to 134 us (160 with f32 products). Relative error
 // against f64 there 3.1e-7 (8.1e-7) and 3.9e-7 (9.1e-7).
 //
 // Work split: the waves of a workgroup share one output tile along K (wave w takes K steps w, w + KW, ...), because an
 // operand is then split into its parts by one wave only: with the usual 2 x 2 waves over the tile every value would be
-// split twice, and the splitting (11 VALU instructions for two values) is as long as the products (64 x 64 x 16: 176
-// VALU instructions of 4 cycles beside 24 MFMAs of 32). A wave fetches its own operand slabs (global -> registers one
+// split twice, and the splitting (11 VALU instructions for two values, and one to look after them) is as long as the products
+// (64 x 64 x 16: 192 VALU instructions of 4 cycles beside 24 MFMAs of 32). A wave fetches its own operand slabs (global -> registers one
 // step ahead -> its own part of LDS -> MFMA operand order), so the K loop has no barrier; the KW sums meet in LDS at the
 // end, in wave order. Nothing depends on alignment but the speed of the loads.
 #include "ft_common.h"
@@ -593,7 +593,8 @@ int ft_split_gemm(ft_context* ctx, int layout, bool half_b, const float* a, cons
     g.p[0] = SplitProduct{static_cast<const char*>(b), out, add, K2 > 0 ? a2 : nullptr, K2 > 0 ? b2 : nullptr, nullptr, 1,
                           (int)N, layout == 1 ? (int)K : (int)N, (int)K2, 0};
     const size_t cus = (size_t)ctx->num_cus;
-    // Tile and waves, measured on 256 CUs (us, f16 b unless said; 64 x 64 by 4 / by 8 waves, 32 x 64 by 4, 32 x 32 by 8):
+    // Tile and waves, measured on 256 CUs (us, f16 b unless said; 64 x 64 by 4 / by 8 waves, 32 x 64 by 4, 32 x 32 by 8;
+    // without the look for small values, which adds 1 % with an f16 b and 3 % with an f32 one):
     //   2048 x 960 x 960  (M x K x N, 480 tiles of 64 x 64)   24.5 / 29.1 / 27.4 / 36.1   with f32 products 35.2
     //   700 x 1024 x 1024 (176)                               15.0 / 13.6 / 15.2 / 16.0                     27.3
     //   257 x 733 x 1001  (80, f32 b)                         13.9 / 13.3 / 10.1 / 10.7                     45.5
