@@ -99,23 +99,27 @@ DkdvUnits split_dkdv_units(const AttnArgs& a) {
 }
 
 // The backward on bf16 parts: its kernels hold one workgroup of 8 waves per CU and want a few rounds of them, of tiles that
-// are not mostly empty. Time of the whole backward, f32 kernels -> these (us, causal):
+// are not half empty. All three run this way or none: kernels that form the same scores with the same rounding lose less in
+// the probabilities. So a line lies where forward and backward together break even (us, f32 kernels -> these, forward +
+// backward, causal unless said):
 //  * dQ, 480 workgroups of 128 queries (4 x 1024 tokens, 15 heads on 5) 128 -> 89, 120 (one sequence) 13 us longer;
-//  * dK/dV per head: 4096 workgroups (8 x 1024, 32 heads) 1266 -> 928, 960 (4 x 1024, 15 on 5) 284 -> 236, 480 (8 x 256, 15 on
-//    5) 60 -> 62. With a group's shares to add it takes longer queries: 4 x 384, 32 on 8 120 -> 107; 24 x 300, 9 on 3
-//    139 -> 148; 16 x 128, 32 on 8 78 -> 93; without a mask 16 x 256, 15 on 5 156 -> 143, 24 x 200, 9 on 3 116 -> 126;
-//  * dK/dV per kv head, workgroups as long as the group is large: 352 (4 x 700, 32 on 8) 299 -> 273, 512 561 -> 436; 264 (3 x
-//    700) 241 -> 257, 88 (4 x 700, 32 on 2) 396 -> 752;
-//  * tiles a quarter empty and more: 24 x 17, 32 heads 36 -> 43, 13 x 65 54 -> 57; 12 x 100 gains.
-// All or none, and the forward with them: kernels that form the same scores with the same rounding lose less in the
-// probabilities.
+//  * dK/dV per head: 4096 workgroups (8 x 1024, 32 heads) 360 + 1266 -> 252 + 963, 960 (4 x 1024, 15 on 5) 93 + 284 -> 66 +
+//    245, 480 (8 x 256, 15 on 5) backward 60 -> 62. With a group's shares to add it takes longer queries: 4 x 384, 32 on 8
+//    44 + 121 -> 31 + 111; 24 x 300, 9 on 3 52 + 139 -> 39 + 155; 8 x 256, 32 on 8 39 + 109 -> 30 + 123; without a mask
+//    16 x 256, 15 on 5 64 + 156 -> 43 + 149; 20 x 200 62 + 171 -> 44 + 180;
+//  * dK/dV per kv head, workgroups as long as the group is large, and under the mask unequal: 288 (6 x 384, 32 on 8) 67 + 175
+//    -> 48 + 167; 264 (3 x 700) 86 + 241 -> 62 + 264, 176 (4 x 700, 32 on 4) 101 + 312 -> 73 + 450. Without a mask
+//    they are equal, and one round of them is as good as several: 256 (8 x 512, 32 on 4) 158 + 538 -> 104 + 420, 132
+//    (3 x 700) 140 + 498 -> 93 + 490; 88 (4 x 700, 32 on 2) 632 -> 830;
+//  * tiles: 129 tokens (8 sequences, 32 heads) 23 + 70 -> 18 + 70, 90 (12) 23 + 62 -> 18 + 64, 80 21 + 54 -> 17 + 61; one tile
+//    alone wants to be full: 64 (24) 24 + 72 -> 21 + 70, 48 20 + 56 -> 18 + 63.
 bool split_backward_pays(const ft_context* ctx, const AttnArgs& a) {
-    const size_t cus = (size_t)ctx->num_cus, G = (size_t)a.H / a.Hkv;
-    auto full = [](int rows) { return 4 * (size_t)rows >= 3 * 64 * (size_t)ft_div_up(rows, 64); };
+    const size_t cus = (size_t)ctx->num_cus;
+    auto full = [](int rows) { return rows <= 64 ? rows >= 56 : 3 * (size_t)rows >= 2 * 64 * (size_t)ft_div_up(rows, 64); };
     if (ctx->f32_chain || !full(a.Sq) || !full(a.Sk) || ft_div_up(a.Sq, 128) * (size_t)a.B * a.H * 2 < 3 * cus) return false;
     const DkdvUnits u = split_dkdv_units(a);
-    if (!u.per_head) return u.workgroups * 3 >= 4 * cus;
-    return u.workgroups >= 3 * cus && (G == 1 || a.Sq >= (a.causal ? 384 : 256));
+    if (!u.per_head) return u.workgroups * 8 >= 9 * cus || (!a.causal && u.workgroups * 2 >= cus && u.workgroups <= cus);
+    return u.workgroups >= 3 * cus && (a.H == a.Hkv || a.Sq >= (a.causal ? 320 : 256));
 }
 // Alone the forward on bf16 parts beats the f32 kernels nearly everywhere, the 32-row ones too (1 x 96 tokens, 15 heads, 7.0
 // us against 8.0; 2 x 160, 9 heads 8.7 against 11.4; 1 x 8, 9 heads 4.6 against 6.5), but not the 16-row ones with half a tile
